@@ -270,7 +270,9 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
           X[k * MLP_TA + t] = w[k] * d * mlp_slope<T>(hact, h);
         }
       }
-      if (nl == 1) parts[t] = mlp_slope<T>(act, y);   // (every thread of an atom holds the same value)
+      // (every thread of an atom holds the same value; it goes where the input was, which nobody reads any more -- the
+      // shares are still being added by other waves)
+      if (nl == 1) X[t] = mlp_slope<T>(act, y);
     }
     if (act != 0 || nl == 1) __syncthreads();
   }
@@ -284,7 +286,7 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
     if (i < n_af && live) (i < S.Ar ? S.g2 + (atom * S.Ar + i) : S.g3 + (atom * S.Aa + (i - S.Ar)))[0] = g;
   };
   if (nl == 1) {
-    const T d = (X + rows0 * MLP_TA)[my];
+    const T d = X[my];
     for (int i = tid / MLP_TA; i < n_af; i += (int)blockDim.x / MLP_TA)
       put(i, net.fw[0][i] * d, af_at(i));
     return;

@@ -419,6 +419,38 @@ def test_device_mlp_stack_shapes(tmp_path, prec, tol, hidden, last):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("prec,tol", [("double", 1e-11), ("float", 2e-5)])
+@pytest.mark.parametrize("last", ["tanh", "relu", "linear"])
+def test_one_layer_network_beside_a_wide_one(tmp_path, prec, tol, last):
+    """A species without hidden layers in the launch of one whose 300 features give every workgroup sixteen waves: all of
+    them add up the output neuron's shares while the first of them already knows its slope.  Against the host evaluation,
+    and the same bits on every call; tolerances as above."""
+    from alphanesgpu_amd import libstaf, model_dir, synth
+    from test_oracle_pins import cluster
+    rng = np.random.Generator(np.random.Philox(33))
+    ps = synth.fingerprint_params(nt=2, ar_map=(5, 4), aa_map=(4, 3, 5), seed=3, dense_embedding=True)
+    for p, hidden in zip(ps, ([], [300, 33])):
+        dims = [p["mu"].shape[0]] + hidden + [1]
+        acts = ["tanh"] * len(hidden) + [last]
+        p["layers"] = [(rng.normal(0, 1 / np.sqrt(a), (a, b)), rng.normal(0.3, 0.1, b), act)
+                       for a, b, act in zip(dims[:-1], dims[1:], acts)]
+    pos, box, tipos, type_map = cluster([33, 17], seed=9, spread=5.0)
+    model_dir.write_model_dir(str(tmp_path), ps, rc=4.5, rc_ang=3.2, rs=1.6, radial_buffer=50, angular_buffer=1225,
+                              tipos=tipos, precision=prec)
+    p = 1 if prec == "double" else 0
+    m = libstaf.StafModel(str(tmp_path), precision=p, full_virial=True, host_mlp=True)
+    e0, f0, v0 = m.compute(pos.reshape(-1, 3), box[0], type_map)
+    m.close()
+    m = libstaf.StafModel(str(tmp_path), precision=p, full_virial=True)
+    got = [m.compute(pos.reshape(-1, 3), box[0], type_map) for _ in range(8)]
+    m.close()
+    e1, f1, v1 = got[0]
+    assert abs(e1 - e0) <= tol * max(1.0, abs(e0)) and nerr(f1, f0) <= tol and nerr(v1, v0) <= tol
+    for e, f, v in got[1:]:
+        assert e == e1 and np.array_equal(f, f1) and np.array_equal(v, v1)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("counts,nr", [([16, 17, 5], 40), ([1, 0, 9], 24), ([0, 3, 0], 60), ([40, 30, 3], 100)])
 @pytest.mark.parametrize("callers_list", [False, True])
 def test_all_species_in_one_launch(tmp_path, counts, nr, callers_list):
