@@ -405,8 +405,14 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
             m->raddescr.reserve(L * nr) && m->des3bsupp.reserve(L * nr) && m->der2b.reserve(L * 3 * nr) &&
             m->der3bsupp.reserve(L * 3 * nr) && m->unit.reserve(L * 4 * nr) && m->intmap2b.reserve(L * (nr + 1)) &&
             m->numtriplet.reserve(L) && m->type_map.reserve(nall) && m->tipos.reserve(nt) && m->actual_type.reserve(nt);
-  if (m->dev_mlp)
-    ok = ok && m->slotf.reserve(L * nr * 3) && m->selff.reserve(L * 3) && m->e_atom.reserve(L) && m->vpart.reserve(L * 9);
+  // Slot forces of both bodies and all species from one launch, or, for neighbour buffers and parameter rows that leave no
+  // room for both bodies in a workgroup's LDS (three species: 250 slots), an op per body and species.
+  bool one_force_launch = m->dev_mlp;
+  for (int k = 0; k < nt; k++)
+    if (tipos[k] > 0) one_force_launch = one_force_launch && staf::step_forces_fits<double>(nr, nt, m->Ar[k], m->Aa[k]);
+  if (m->dev_mlp) ok = ok && m->e_atom.reserve(L);
+  if (one_force_launch)
+    ok = ok && m->slotf.reserve(L * nr * 3) && m->selff.reserve(L * 3) && m->vpart.reserve(L * 9);
   else
     ok = ok && m->force_op.reserve((size_t)nall * 3) && m->virial_op.reserve(9);
   if (!ok) return -1;
@@ -450,6 +456,23 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   const int n3 = nall * 3;
   const bool want_w = virial != nullptr;
   const int skip_pbc = ext ? 1 : 0;   // the caller's neighbours are explicit periodic images
+  // The force op of one body of species k, whose owned atoms start at o, added to the forces; its virial in virial_op.
+  auto force_op = [&](int body, int k, size_t o, const double* g2, const double* g3, bool with_virial) -> int {
+    double* const w = with_virial ? m->virial_op.p : nullptr;
+    const double* const px = with_virial ? d_pos : nullptr;
+    const double* const bx = with_virial ? d_box : nullptr;
+    const int r = body == 2
+        ? staf::force_doublets<double>(g2, m->raddescr.p + o * nr, m->der2b.p + o * 3 * nr, m->intmap2b.p + o * (nr + 1), nr,
+                                       nall, 1, m->Ar[k], m->alpha2b[k].p, m->emb2b[k].p, nt, m->tipos.p,
+                                       m->actual_type.p + k, m->force_op.p, m->type_map.p, tipos[k], w, px, bx, nlocal,
+                                       skip_pbc, st)
+        : staf::force_tripl<double>(g3, m->des3bsupp.p + o * nr, nullptr, m->der3bsupp.p + o * 3 * nr, nullptr,
+                                    m->unit.p + o * 4 * nr, m->intmap2b.p + o * (nr + 1), nullptr, nr, na, nall, 1, m->Aa[k],
+                                    m->emb3b[k].p, nt, m->tipos.p, m->actual_type.p + k, m->force_op.p, m->numtriplet.p + o,
+                                    m->alpha3b[k].p, m->type_map.p, tipos[k], w, px, bx, nlocal, skip_pbc, st);
+    if (r == STAF_OK) hipLaunchKernelGGL(add_into_kernel, dim3((n3 + 255) / 256), dim3(256), 0, st, d_force, m->force_op.p, n3);
+    return r;
+  };
   // ---- everything stays on the device, five launches one behind the other (six with a cell list or a caller's
   // list): descriptors -> fingerprints -> networks -> slot forces -> collection, each over the centres of all species;
   // one synchronisation at the end of the call.  A chain per species on a stream of its own, with a launch per body, was
@@ -475,16 +498,28 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     }
     const staf::StepRows<double> rows = {m->raddescr.p, m->des3bsupp.p, m->der2b.p, m->der3bsupp.p, m->unit.p, m->intmap2b.p,
                                          m->numtriplet.p, nr, na, 1, nlocal};
-    double* const vpart = want_w ? m->vpart.p : nullptr;
+    double* const vpart = want_w && one_force_launch ? m->vpart.p : nullptr;
     if ((rc = staf::step_fingerprints(sp.data(), ns, rows, m->type_map.p, nt, st)) != STAF_OK) return gpu_failure(__LINE__, rc);
     if ((rc = staf::dev_mlp_eval(nets.data(), ns, st)) != STAF_OK) return gpu_failure(__LINE__, rc);
-    if ((rc = staf::step_forces(sp.data(), ns, rows, m->type_map.p, nt, m->slotf.p, m->selff.p, vpart, st)) != STAF_OK)
+    if (one_force_launch &&
+        (rc = staf::step_forces(sp.data(), ns, rows, m->type_map.p, nt, m->slotf.p, m->selff.p, vpart, st)) != STAF_OK)
       return gpu_failure(__LINE__, rc);
-    const staf::StepCollect<double> out = {m->slotf.p, m->selff.p, vpart, m->e_atom.p, d_force, d_parts, nullptr, nullptr,
-                                           nparts};
+    const staf::StepCollect<double> out = {m->slotf.p, m->selff.p, vpart, m->e_atom.p, one_force_launch ? d_force : nullptr,
+                                           d_parts, nullptr, nullptr, nparts};
     if ((rc = staf::step_collect(sp.data(), ns, rows, nall, out, st)) != STAF_OK)
       return gpu_failure(__LINE__, rc);
-    return 0;
+    if (one_force_launch) return 0;
+    // the virials go to the first share's row, which holds an energy sum and zeros
+    staf::launch_fill_zero<double>(d_force, n3, st);
+    for (int c = 0, k = 0; c < ns; c++, k++) {
+      while (tipos[k] == 0) k++;
+      const size_t o = (size_t)sp[c].first;
+      for (int body = 2; body <= 3; body++) {
+        if ((rc = force_op(body, k, o, sp[c].g2, sp[c].g3, want_w)) != STAF_OK) return gpu_failure(__LINE__, rc);
+        if (want_w) hipLaunchKernelGGL(add_into_kernel, dim3(1), dim3(256), 0, st, d_parts, m->virial_op.p, 9);
+      }
+    }
+    return hipGetLastError() == hipSuccess ? 0 : gpu_failure(__LINE__, 0);
   };
   if (m->dev_mlp) {
     if (device_sequence() != 0) return -20;
@@ -571,19 +606,7 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
       STAF_HIP_OK(hipMemcpyAsync(m->g3.p, m->tmp3.data(), m->tmp3.size() * sizeof(double), hipMemcpyHostToDevice, st));
       STAF_HIP_OK(hipStreamSynchronize(st));
       for (int body = 2; body <= 3; body++) {
-        if (body == 2)
-          rc = staf::force_doublets<double>(m->g2.p, m->raddescr.p + o * nr, m->der2b.p + o * 3 * nr,
-                                            m->intmap2b.p + o * (nr + 1), nr, nall, 1, Ar, m->alpha2b[k].p,
-                                            m->emb2b[k].p, nt, m->tipos.p, m->actual_type.p + k, m->force_op.p,
-                                            m->type_map.p, Nl, m->virial_op.p, d_pos, d_box, nlocal, skip_pbc, st);
-        else
-          rc = staf::force_tripl<double>(m->g3.p, m->des3bsupp.p + o * nr, nullptr, m->der3bsupp.p + o * 3 * nr, nullptr,
-                                         m->unit.p + o * 4 * nr, m->intmap2b.p + o * (nr + 1), nullptr, nr, na, nall, 1,
-                                         Aa, m->emb3b[k].p, nt, m->tipos.p, m->actual_type.p + k, m->force_op.p,
-                                         m->numtriplet.p + o, m->alpha3b[k].p, m->type_map.p, Nl, m->virial_op.p,
-                                         d_pos, d_box, nlocal, skip_pbc, st);
-        if (rc != STAF_OK) return gpu_failure(__LINE__, rc);
-        hipLaunchKernelGGL(add_into_kernel, dim3((n3 + 255) / 256), dim3(256), 0, st, d_force, m->force_op.p, n3);
+        if ((rc = force_op(body, k, o, m->g2.p, m->g3.p, true)) != STAF_OK) return gpu_failure(__LINE__, rc);
         STAF_HIP_OK(hipMemcpyAsync(Wk, m->virial_op.p, 9 * sizeof(double), hipMemcpyDeviceToHost, st));
         STAF_HIP_OK(hipStreamSynchronize(st));
         for (int c = 0; c < 9; c++) W[c] += Wk[c];

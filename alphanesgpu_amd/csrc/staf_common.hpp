@@ -468,6 +468,10 @@ struct StepRows {             // what the radial-only descriptor launch leaves, 
 template <typename real>
 int step_fingerprints(const StepSpecies<real>* sp, int n, const StepRows<real>& R, const int* type_map, int nt,
                       hipStream_t stream);
+// True: step_forces takes a species of these sizes.  Its workgroups hold the parameter rows of both bodies; sizes close to
+// a CU's LDS that it does not take may still fit force_doublets and force_tripl, an op per body.
+template <typename real>
+bool step_forces_fits(int nr, int nt, int Ar, int Aa);
 // forces on the centres' slots [nf, nlocal, nr, 3] and on the centres [nf, nlocal, 3]; vpart [nf, nlocal, 9]: their
 // virials, or null
 template <typename real>

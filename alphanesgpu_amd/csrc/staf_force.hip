@@ -803,11 +803,18 @@ static int gradforce_tripl(const real* Q, const real* G, const real* Dsup, const
 // atom -- owned or ghost -- collects what acts on it and further workgroups add up the centres' virials and energies.
 // ---------------------------------------------------------------------------
 template <typename real>
+bool step_forces_fits(int nr, int nt, int Ar, int Aa) {
+  using L = Force3Cfg<real, 4>;
+  return L::fits(nr, nt) && L::bytes(nr, Aa, nt, true, Ar) <= 160 * 1024;
+}
+
+template <typename real>
 int step_forces(const StepSpecies<real>* sp, int n, const StepRows<real>& R, const int* type_map, int nt, real* slots,
                 real* self, real* vpart, hipStream_t stream) {
   using L = Force3Cfg<real, 4>;
   using Wide = Force3Cfg<real, 8>;
-  if (!L::fits(R.nr, nt)) return STAF_E_LIMIT;
+  for (int c = 0; c < n; c++)
+    if (sp[c].Nl > 0 && !step_forces_fits<real>(R.nr, nt, sp[c].Ar, sp[c].Aa)) return STAF_E_LIMIT;
   Force3Species<real> M = {};
   size_t lds = 0, lds_wide = 0;
   int wg = 0;
@@ -954,6 +961,7 @@ int step_collect(const StepSpecies<real>* sp, int n, const StepRows<real>& R, in
 }
 
 #define STAF_STEP_INSTANCES(real)                                                                                      \
+  template bool step_forces_fits<real>(int, int, int, int);                                                            \
   template int step_forces<real>(const StepSpecies<real>*, int, const StepRows<real>&, const int*, int, real*, real*,  \
                                  real*, hipStream_t);                                                                  \
   template int step_collect<real>(const StepSpecies<real>*, int, const StepRows<real>&, int, const StepCollect<real>&, \

@@ -95,6 +95,8 @@ static int frames(const real* pos, const real* box, int nf, int N, int nt, const
   int rc = frames_plan<real>(c, nf, N, nt, sp, &P);
   if (rc != STAF_OK) return rc;
   if (!pos || !box || !type_map || !work || work_bytes < P.bytes || !energy || !virial) return STAF_E_BAD_ARG;
+  for (int k = 0; k < nt; k++)   // (known before anything is launched: the caller has another way)
+    if (force && sp[k].n_local > 0 && !step_forces_fits<real>(c.nr, nt, sp[k].nalpha_r, sp[k].nsmooth_a)) return STAF_E_LIMIT;
   char* const w = (char*)work;
   auto at = [&](size_t offset) { return (real*)(w + offset); };
   StepSpecies<real> S[NT_MAX];

@@ -486,6 +486,50 @@ def test_all_species_in_one_launch(tmp_path, counts, nr, callers_list):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("callers_list", [False, True])
+def test_neighbour_buffers_whose_slots_leave_no_room_for_both_bodies(tmp_path, callers_list):
+    """250 slots and three species: a force workgroup holds the 3-body rows (154 of 160 KB) but not the 2-body ones beside
+    them, and the forces come from an op per body.  Buffers beyond the neighbours an atom has change nothing, so the same
+    model with 60 slots, whose forces come from one launch, is the reference; sums in another order, 1e-11.  The batch
+    inference takes such a model through its layers."""
+    import torch
+    from alphanesgpu_amd import inference, libstaf, model_dir
+    from test_oracle_pins import cluster, small_model
+    ps = small_model(3, (5, 4, 6), (4, 3, 5, 3, 4, 3), seed=5, hidden=20, dense=True)
+    pos, box, tipos, types = cluster([16, 17, 5], seed=17, spread=5.0)
+    x = pos.reshape(-1, 3)
+    extra = {}
+    if callers_list:
+        d = np.linalg.norm(x[:, None] - x[None], axis=-1)
+        rows = [[j for j in np.argsort(r, kind="stable")[1:] if r[j] < 4.5] for r in d]
+        neigh = np.zeros((len(x), 40), np.int32)
+        for i, r in enumerate(rows):
+            neigh[i, :len(r)] = r
+        extra = dict(nlocal=len(x), howmany=np.array([len(r) for r in rows], np.int32), neigh=neigh)
+    out = []
+    for nr in (60, 250):
+        d = tmp_path / str(nr)
+        d.mkdir()
+        model_dir.write_model_dir(str(d), ps, rc=4.5, rc_ang=3.2, rs=1.6, radial_buffer=nr, angular_buffer=780, tipos=tipos,
+                                  precision="double")
+        m = libstaf.StafModel(str(d), precision=1, full_virial=True)
+        for want in (False, True):
+            e, f, v = m.compute(x, box[0], types, want_virial=want, **extra)
+        m.close()
+        out.append((e, f, v))
+        if not callers_list:
+            g = inference.staf_full_inference(str(d), dtype=torch.float64)
+            T = lambda a: torch.as_tensor(a, device="cuda")
+            out.append(tuple(t.cpu().numpy() for t in g.full_test(T(pos), T(box))))
+    e0, f0, v0 = out[0]
+    full = lambda v: np.array([v[0], v[4], v[8], (v[1] + v[3]) / 2, (v[2] + v[6]) / 2, (v[5] + v[7]) / 2])
+    for e, f, v in out[1:]:
+        if np.ndim(e):
+            e, f, v = e[0], f.reshape(-1, 3), full(v.reshape(-1))
+        assert abs(e - e0) <= 1e-11 * max(1.0, abs(e0)) and nerr(f, f0) <= 1e-11 and nerr(v, v0) <= 1e-11
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("cells", [(4, 4, 2), (8, 7, 3), (8, 8, 4), (9, 8, 4)])
 def test_device_path_on_both_sides_of_the_workgroup_sizes_lines(cells):
     """96, 504, 768 and 864 centres: wider workgroups for the fingerprints of up to 512 and the slot forces of up to 768.  Against the
