@@ -228,9 +228,12 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
 #pragma unroll
       for (int v = 0; v < 4; v++) y[v] += acc[v];
       mlp_act<T, 4>(act, y);
-      // (features beyond the last: zero weights, zero bias, value 0)
+      // (features beyond the last are 0 whatever their zero weights were multiplied with: an infinite value gives no number)
 #pragma unroll
-      for (int v = 0; v < 4; v++) Y[(tile * 16 + M::row(lane, v)) * MLP_TA + my] = y[v];
+      for (int v = 0; v < 4; v++) {
+        const int j = tile * 16 + M::row(lane, v);
+        Y[j * MLP_TA + my] = j < out_f ? y[v] : T(0);
+      }
     }
     if (l + 2 < nl) {
       if (wave < mlp_tiles(net.out_f[l + 1])) request(net.fw[l + 1], wave, mlp_pieces<T>(out_f));
@@ -306,7 +309,7 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
       const acc_t acc = product(net.bw[l], tile, np, D);
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        if (l > 0) at[M::row(lane, v) * MLP_TA] = acc[v] * mlp_slope<T>(act, other[v]);
+        if (l > 0) at[M::row(lane, v) * MLP_TA] = tile * 16 + M::row(lane, v) < in_f ? acc[v] * mlp_slope<T>(act, other[v]) : T(0);
         else put(tile * 16 + M::row(lane, v), acc[v], other[v]);
       }
     }

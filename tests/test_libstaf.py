@@ -451,6 +451,36 @@ def test_one_layer_network_beside_a_wide_one(tmp_path, prec, tol, last):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("prec,tol", [("double", 1e-11), ("float", 2e-5)])
+def test_infinite_activations_stay_out_of_the_padded_features(tmp_path, prec, tol):
+    """A feature of a linear layer that overflows saturates the tanh layer behind it (slope 0, so that gradients are
+    finite too).  Layers of 5 and 7 features leave most of their 16-feature tiles empty: infinity times the zero weights
+    of the empty ones must not reach the energy.  Against the host evaluation, which has no such features."""
+    from alphanesgpu_amd import libstaf, model_dir, synth
+    from test_oracle_pins import cluster
+    rng = np.random.Generator(np.random.Philox(35))
+    ps = synth.fingerprint_params(nt=2, ar_map=(5, 4), aa_map=(4, 3, 5), seed=3, dense_embedding=True)
+    for p in ps:
+        n = p["mu"].shape[0]
+        p["mu"][2] += 50.0     # |log(af + 1e-3) - mu| of this fingerprint is far above 2
+        W = [rng.normal(0, 1 / np.sqrt(a), (a, b)) for a, b in ((n, 5), (5, 7), (7, 6), (6, 1))]
+        W[0][:, 3] = 0
+        W[0][2, 3] = 0.9 * (np.finfo(np.float64).max if prec == "double" else float(np.finfo(np.float32).max))
+        p["layers"] = [(w, rng.normal(0.3, 0.1, w.shape[1]), a) for w, a in zip(W, ("linear", "tanh", "tanh", "linear"))]
+    pos, box, tipos, type_map = cluster([16, 17], seed=9, spread=4.4)
+    model_dir.write_model_dir(str(tmp_path), ps, rc=4.5, rc_ang=3.2, rs=1.6, radial_buffer=40, angular_buffer=780,
+                              tipos=tipos, precision=prec)
+    got = []
+    for host in (True, False):
+        m = libstaf.StafModel(str(tmp_path), precision=1 if prec == "double" else 0, full_virial=True, host_mlp=host)
+        got.append(m.compute(pos.reshape(-1, 3), box[0], type_map))
+        m.close()
+    (e0, f0, v0), (e1, f1, v1) = got
+    assert np.isfinite(e0) and np.isfinite(f0).all()
+    assert abs(e1 - e0) <= tol * max(1.0, abs(e0)) and nerr(f1, f0) <= tol and nerr(v1, v0) <= tol
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("counts,nr", [([16, 17, 5], 40), ([1, 0, 9], 24), ([0, 3, 0], 60), ([40, 30, 3], 100)])
 @pytest.mark.parametrize("callers_list", [False, True])
 def test_all_species_in_one_launch(tmp_path, counts, nr, callers_list):
