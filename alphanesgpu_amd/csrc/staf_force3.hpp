@@ -647,8 +647,9 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
       }
     }
     if constexpr (W2B) {
-      // the pair force of slot tid (zero weight beyond the radial neighbours); slots beyond the angular cutoff carry it alone
-      if (tid < nr) {
+      // the pair force of slot tid; slots beyond the angular cutoff carry it alone, and what a caller's rows hold beyond the
+      // radial neighbours is not read
+      if (tid < cnt2) {
         real w = 0;
 #pragma unroll
         for (int w_ = 0; w_ < NW; w_++) w += w2p[w_ * nr + tid];

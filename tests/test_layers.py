@@ -201,3 +201,42 @@ def test_forces_in_one_op_agree_with_the_two_force_ops(dtype, nr, na, counts, ow
                 bound = terms * torch.finfo(dt).eps * (x.abs().max() + y.abs().max())
                 assert (z - (x + y)).abs().max() <= bound, (k, virial != (), (z - (x + y)).abs().max(), bound)
         o += n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+def test_forces_in_one_op_do_not_read_the_padding_of_the_rows(dtype):
+    """Descriptor rows of another origin may hold anything beyond an atom's neighbours (the force ops take the counts from
+    the map): with NaN there, ops.compute_forces and the force layers give the same bits as with the descriptor op's
+    zeros, as the two ops do."""
+    import torch
+    from alphanesgpu_amd import layers, ops, synth
+    dev, dt = torch.device("cuda:0"), getattr(torch, dtype)
+    b = synth.water_batch("water96")
+    counts, nr, na, N = [int(c) for c in b["tipos"]], 60, 1770, len(b["type_map"])
+    T = lambda a: torch.as_tensor(np.ascontiguousarray(a)).to(dev)
+    tpos, tbox = (T(np.tile(b[q][:1], (2, 1))).to(dt) for q in ("pos", "box"))
+    tm, tp = T(b["type_map"].astype(np.int32)), T(np.array(counts, np.int32))
+    ops.construct_descriptors_light(synth.RC, nr, na, N, tbox, synth.RS, synth.RA, 2, dtype=dt)
+    rad, ang, sup, im2, im3, d2, d3, d3s, ntr = ops.compute_descriptors_light(tpos, tbox)
+    pad = torch.arange(nr, device=dev) >= im2[..., :1]
+    assert bool(pad.any())
+    nan = lambda t: t.masked_fill(pad.unsqueeze(2) if t.dim() == 4 else pad, float("nan"))
+    P = {q: T(v) for q, v in synth.fingerprint_params(2, dtype=getattr(np, dtype))[0].items()}
+    g = torch.Generator(device=dev)
+    g.manual_seed(5)
+    n = counts[0]
+    G2 = torch.randn((2, n, P["emb2b"].shape[1]), dtype=dt, device=dev, generator=g)
+    G3 = torch.randn((2, n, P["emb3b"].shape[1]), dtype=dt, device=dev, generator=g)
+    layer = layers.force_virial_layer(nr, na)
+    out = []
+    for f in (lambda t: t, nan):
+        c = lambda t: t[:, :n]
+        R, S, D2, D3s = (c(f(t)) for t in (rad, sup, d2.reshape(2, N, 3, nr), d3s.reshape(2, N, 3, nr)))
+        D2, D3s = D2.reshape(c(d2).shape), D3s.reshape(c(d3s).shape)
+        out.append(ops.compute_forces(G3, G2, S, c(ang), D3s, c(d3), R, D2, c(im2), c(im3), P["alpha3b"], P["emb3b"],
+                                      P["alpha2b"], P["emb2b"], tm, tp, 0, c(ntr), tpos, tbox) +
+                   layer(G2, R, D2, c(im2), P["alpha2b"], G3, c(ang), S, c(d3), D3s, c(im3), c(ntr), P["alpha3b"],
+                         P["emb2b"].sqrt(), P["emb3b"].sqrt(), tm, tp, 0, tpos, tbox))
+    for x, y in zip(*out):
+        assert bool(torch.isfinite(x).all()) and torch.equal(x, y)
