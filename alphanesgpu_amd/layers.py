@@ -63,14 +63,18 @@ class _Forces(torch.autograd.Function):
                 intder3bsupp, intmap3b, numtriplet, alpha3b, emb3b_sq, type_map, tipos, type_now, pos, box):
         ctx.save_for_backward(netderiv2b, netderiv3b, x2b, intder2b, intmap2b, alpha2b, emb2b_sq, x3b, x3bsupp, intder3b,
                               intder3bsupp, intmap3b, numtriplet, alpha3b, emb3b_sq, type_map, tipos, type_now, pos, box)
-        try:
-            out = ops.compute_forces(netderiv3b, netderiv2b, x3bsupp, x3b, intder3bsupp, intder3b, x2b, intder2b,
-                                     intmap2b, intmap3b, alpha3b, emb3b_sq, alpha2b, emb2b_sq, type_map, tipos, type_now,
-                                     numtriplet, pos, box)
-        except _lib.StafError as e:
-            if e.code != -12:
-                raise
-            # parameter rows of both kinds do not fit one workgroup's LDS: the two ops, nothing has been launched yet
+        out = None
+        if x2b.dtype == x3b.dtype:
+            try:
+                out = ops.compute_forces(netderiv3b, netderiv2b, x3bsupp, x3b, intder3bsupp, intder3b, x2b, intder2b,
+                                         intmap2b, intmap3b, alpha3b, emb3b_sq, alpha2b, emb2b_sq, type_map, tipos, type_now,
+                                         numtriplet, pos, box)
+            except _lib.StafError as e:
+                if e.code != -12:
+                    raise
+        if out is None:
+            # the two bodies in two precisions, or parameter rows of both kinds that do not fit one workgroup's LDS (nothing
+            # has been launched yet): the two ops
             out = ops.compute_force_radial(netderiv2b, intder2b, intmap2b, x2b, alpha2b, emb2b_sq, type_map, tipos,
                                            type_now, pos, box)
             out3 = ops.compute_force_tripl(netderiv3b, x3bsupp, x3b, intder3bsupp, intder3b, intmap2b, intmap3b, alpha3b,
@@ -96,16 +100,16 @@ class _Forces(torch.autograd.Function):
         if need[0] or need[5] or need[6]:
             args = (netderiv2b, intder2b, intmap2b, x2b, alpha2b, emb2b_sq, type_map, tipos, type_now)
             if pos is None:
-                gn2, ga2, ge2 = ops.compute_force_radial_grad(gf, *args)
+                gn2, ga2, ge2 = ops.compute_force_radial_grad(gf.to(x2b.dtype), *args)
             else:
-                gn2, ga2, ge2 = ops.compute_force_radial_virial_grad(gf, gv, *args, pos, box)
+                gn2, ga2, ge2 = ops.compute_force_radial_virial_grad(gf.to(x2b.dtype), gv.to(x2b.dtype), *args, pos, box)
         if need[1] or need[13] or need[14]:
             args = (netderiv3b, x3bsupp, x3b, intder3bsupp, intder3b, intmap2b, intmap3b, alpha3b, emb3b_sq, type_map, tipos,
                     type_now, numtriplet)
             if pos is None:
-                gn3, ga3, ge3 = ops.compute_force_tripl_grad(gf, *args)
+                gn3, ga3, ge3 = ops.compute_force_tripl_grad(gf.to(x3b.dtype), *args)
             else:
-                gn3, ga3, ge3 = ops.compute_force_tripl_virial_grad(gf, gv, *args, pos, box)
+                gn3, ga3, ge3 = ops.compute_force_tripl_virial_grad(gf.to(x3b.dtype), gv.to(x3b.dtype), *args, pos, box)
         return (gn2, gn3, None, None, None, ga2, ge2, None, None, None, None, None, None, ga3, ge3, None, None, None, None,
                 None)
 

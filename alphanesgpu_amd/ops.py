@@ -458,6 +458,8 @@ def compute_forces(netderiv3b, netderiv2b, radial_descriptor, angular_descriptor
     (force, virial [nf,9]), the sums of what the two virial ops return.  Arguments as compute_forces_slots."""
     dtype = angular_descriptor.dtype
     s, _ = sfx(dtype)
+    if radial_descriptor_2b.dtype != dtype:
+        raise TypeError("compute_forces takes both bodies in one precision")
     dev = angular_descriptor.device
     nf, Nl, na = angular_descriptor.shape
     nr = radial_descriptor.shape[2]

@@ -157,6 +157,37 @@ def test_layer_classes_have_the_reference_signatures():
     assert sig(layers.force_virial_layer.forward) == call + ["pos", "box"]
 
 
+@pytest.mark.parametrize("two,three,want", [
+    ("float64", "float64", ["staf_op_forces_f64"]), ("float32", "float32", ["staf_op_forces_f32"]),
+    ("float32", "float64", ["staf_op_force_doublets_f32", "staf_op_force_tripl_f64"]),
+    ("float64", "float32", ["staf_op_force_doublets_f64", "staf_op_force_tripl_f32"])])
+def test_force_layer_takes_the_bodies_in_precisions_of_their_own(monkeypatch, two, three, want):
+    """2-body and 3-body tensors of different precisions go to the two force ops, each in its own (one op for both would
+    read one body's memory as the other's); the forces are their sum in the wider one, and its gradient goes back to each
+    body in the body's precision.  Which library calls are made, on host tensors with the calls themselves replaced."""
+    import torch
+    from alphanesgpu_amd import layers, ops
+    d2, d3 = getattr(torch, two), getattr(torch, three)
+    nf, N, nr, na, Ar, Aa = 1, 3, 4, 6, 2, 3
+    z = lambda dt, *sh: torch.ones(sh, dtype=dt)
+    zi = lambda *sh: torch.zeros(sh, dtype=torch.int32)
+    layer = layers.force_layer(nr, na)
+    made = []
+    monkeypatch.setattr(ops, "call", lambda name, *args: made.append(name))
+    monkeypatch.setattr(ops, "_stream", lambda: None)
+    g2, g3 = z(d2, nf, N, Ar).requires_grad_(True), z(d3, nf, N, Aa).requires_grad_(True)
+    f = layer(g2, z(d2, nf, N, nr), z(d2, nf, N, 3 * nr), zi(nf, N, nr + 1), z(d2, 1, Ar), g3, z(d3, nf, N, na),
+              z(d3, nf, N, nr), z(d3, nf, N, 3 * na * 2), z(d3, nf, N, 3 * nr), zi(nf, N, na * 2), zi(nf, N), z(d3, 1, 3 * Aa),
+              z(d2, 1, Ar), z(d3, 1, Aa), zi(N), zi(1), 0)
+    assert made == want
+    came = {}
+    monkeypatch.setattr(ops, "compute_force_radial_grad", lambda q, g, *a: came.update(two=q.dtype) or (g, a[3], a[4]))
+    monkeypatch.setattr(ops, "compute_force_tripl_grad", lambda q, g, *a: came.update(three=q.dtype) or (g, a[6], a[7]))
+    torch.autograd.grad(f.sum(), [g2, g3])
+    assert came == dict(two=d2, three=d3)
+    assert f.dtype == torch.promote_types(d2, d3) and f.shape == (nf, 3 * N)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["float32", "float64"])
 @pytest.mark.parametrize("nr,na,counts,own_map", [(60, 1770, (32, 64), True), (60, 1770, (32, 64), False),
