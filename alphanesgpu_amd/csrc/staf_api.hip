@@ -134,6 +134,10 @@ struct StafModel {
   DevBuf<double> raddescr, des3bsupp, der2b, der3bsupp, unit;   // nr-wide rows per owned atom; unit = (u, 1/r)
   DevBuf<double> slotf, selff;   // slot forces [nlocal, nr, 3] and centres' own forces [nlocal, 3]
   DevBuf<int> intmap2b, numtriplet, type_map, tipos, actual_type;
+  // a caller's list transposed (atom -> the centres and slots that list it): counters, which read zero between builds (tr_clear:
+  // they do), counts and keys
+  DevBuf<int> tr_build, tr_cnt, tr_keys;
+  bool tr_clear = false;
   // host staging
   std::vector<double> af_h, gr_h, tmp2, tmp3;
   std::vector<float> af_f, gr_f;
@@ -232,7 +236,8 @@ void staf_free(StafModel* m) {
                             &m->e_atom, &m->vpart, &m->raddescr, &m->des3bsupp, &m->der2b, &m->der3bsupp, &m->unit,
                             &m->slotf, &m->selff})
     b->release();
-  for (DevBuf<int>* b : {&m->intmap2b, &m->numtriplet, &m->type_map, &m->tipos, &m->actual_type})
+  for (DevBuf<int>* b : {&m->intmap2b, &m->numtriplet, &m->type_map, &m->tipos, &m->actual_type, &m->tr_build, &m->tr_cnt,
+                         &m->tr_keys})
     b->release();
   delete m;
 }
@@ -415,6 +420,12 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     ok = ok && m->slotf.reserve(L * nr * 3) && m->selff.reserve(L * 3) && m->vpart.reserve(L * 9);
   else
     ok = ok && m->force_op.reserve((size_t)nall * 3) && m->virial_op.reserve(9);
+  const int tr_cap = 4 * nr;   // centres that may list an atom
+  if (ext) {   // (the number of ghosts varies from call to call: room for a quarter more)
+    auto room = [](DevBuf<int>& b, size_t want) { return want <= b.n || b.reserve(want + want / 4); };
+    if ((size_t)nall > m->tr_build.n) m->tr_clear = false;
+    ok = ok && room(m->tr_build, nall) && room(m->tr_cnt, nall) && room(m->tr_keys, (size_t)nall * tr_cap);
+  }
   if (!ok) return -1;
   if (m->type_map.p != type_map_before) m->type_map_up.clear();   // a new block holds nothing yet
   hipStream_t st = m->stream;
@@ -445,10 +456,20 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   staf::DeferStatus defer;   // conditions the kernels detect are read once, after the last kernel
 
   // ---- descriptors (own minimum-image list, or the caller's list with explicit images)
+  staf::TransposeRef tr;
+  if (ext) {
+    tr.build_cnt = m->tr_build.p; tr.cnt = m->tr_cnt.p; tr.keys = m->tr_keys.p; tr.cap = tr_cap;
+  } else {
+    tr.symmetric = 1; tr.full = m->intmap2b.p;
+  }
   auto descriptors = [&]() -> int {
-    return staf::desc_launch<double>(m->cfg, d_pos, d_box, 1, nlocal, nall, ext ? &list : nullptr, ext ? 1 : 0,
-                                     m->raddescr.p, nullptr, m->des3bsupp.p, m->intmap2b.p, nullptr, m->der2b.p, nullptr,
-                                     m->der3bsupp.p, m->numtriplet.p, m->unit.p, st) == STAF_OK ? 0 : -20;
+    if (ext && !m->tr_clear) staf::launch_fill_zero<int>(m->tr_build.p, (int)m->tr_build.n, st);
+    if (ext) m->tr_clear = false;
+    const int r = staf::desc_launch<double>(m->cfg, d_pos, d_box, 1, nlocal, nall, ext ? &list : nullptr, &tr, ext ? 1 : 0,
+                                            m->raddescr.p, nullptr, m->des3bsupp.p, m->intmap2b.p, nullptr, m->der2b.p,
+                                            nullptr, m->der3bsupp.p, m->numtriplet.p, m->unit.p, st);
+    if (ext) m->tr_clear = r == STAF_OK;
+    return r == STAF_OK ? 0 : -20;
   };
   int rc = 0;
   double energy = 0.0;
@@ -461,15 +482,18 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     double* const w = with_virial ? m->virial_op.p : nullptr;
     const double* const px = with_virial ? d_pos : nullptr;
     const double* const bx = with_virial ? d_box : nullptr;
+    staf::TransposeRef known = tr;
+    known.key_shift = (int)o;
     const int r = body == 2
         ? staf::force_doublets<double>(g2, m->raddescr.p + o * nr, m->der2b.p + o * 3 * nr, m->intmap2b.p + o * (nr + 1), nr,
                                        nall, 1, m->Ar[k], m->alpha2b[k].p, m->emb2b[k].p, nt, m->tipos.p,
                                        m->actual_type.p + k, m->force_op.p, m->type_map.p, tipos[k], w, px, bx, nlocal,
-                                       skip_pbc, st)
+                                       skip_pbc, st, &known)
         : staf::force_tripl<double>(g3, m->des3bsupp.p + o * nr, nullptr, m->der3bsupp.p + o * 3 * nr, nullptr,
                                     m->unit.p + o * 4 * nr, m->intmap2b.p + o * (nr + 1), nullptr, nr, na, nall, 1, m->Aa[k],
                                     m->emb3b[k].p, nt, m->tipos.p, m->actual_type.p + k, m->force_op.p, m->numtriplet.p + o,
-                                    m->alpha3b[k].p, m->type_map.p, tipos[k], w, px, bx, nlocal, skip_pbc, st);
+                                    m->alpha3b[k].p, m->type_map.p, tipos[k], w, px, bx, nlocal, skip_pbc, st, nullptr,
+                                    nullptr, nullptr, &known);
     if (r == STAF_OK) hipLaunchKernelGGL(add_into_kernel, dim3((n3 + 255) / 256), dim3(256), 0, st, d_force, m->force_op.p, n3);
     return r;
   };
@@ -497,7 +521,7 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
                       sp[c].Nl});
     }
     const staf::StepRows<double> rows = {m->raddescr.p, m->des3bsupp.p, m->der2b.p, m->der3bsupp.p, m->unit.p, m->intmap2b.p,
-                                         m->numtriplet.p, nr, na, 1, nlocal};
+                                         m->numtriplet.p, nr, na, 1, nlocal, tr};
     double* const vpart = want_w && one_force_launch ? m->vpart.p : nullptr;
     if ((rc = staf::step_fingerprints(sp.data(), ns, rows, m->type_map.p, nt, st)) != STAF_OK) return gpu_failure(__LINE__, rc);
     if ((rc = staf::dev_mlp_eval(nets.data(), ns, st)) != STAF_OK) return gpu_failure(__LINE__, rc);

@@ -292,16 +292,15 @@ struct TransposeRef {
   int key_shift = 0;         // centre number (row in `full`) of row 0 of the map the force op was handed
 };
 
-// Transpose the descriptor op keeps beside an intmap2b tensor it has written.
-struct Transpose {
-  const int* im2 = nullptr;  // the intmap2b tensor [nf, N, nr+1] it was built from
-  int nf = 0, N = 0, Nrecv = 0, nr = 0;
+// An intmap2b tensor the descriptor op has written: symmetric, with the checksums of its rows beside it.
+struct KnownMap {
+  const int* im2 = nullptr;      // the tensor [nf, N, nr+1]
+  int nf = 0, N = 0, nr = 0;
   TransposeRef ref;
-  Workspace buf;
-  size_t cap_recv = 0, cap_keys = 0;   // capacities of buf, in ints, of a counter part and of the key part
-  unsigned long long stamp = 0;        // last use, for replacement
+  Workspace sums;                // [nf * N] words
+  unsigned long long stamp = 0;  // last use, for replacement
 };
-constexpr int TRANSPOSE_SLOTS = 8;     // descriptor output tensors whose transposes are kept at a time
+constexpr int KNOWN_MAPS = 8;    // descriptor output tensors remembered at a time
 constexpr int STATUS_WORDS = 64;       // error words of a device, one per stream
 
 struct DeviceState {
@@ -313,9 +312,9 @@ struct DeviceState {
   int* status_h = nullptr;   // pinned host mirror, [STATUS_WORDS]
   std::unordered_map<hipStream_t, int> status_slot;
   std::unordered_map<hipStream_t, StreamWork> work;
-  Transpose transposes[TRANSPOSE_SLOTS];
+  KnownMap maps[KNOWN_MAPS];
   std::vector<void*> retired;   // outgrown blocks, freed by staf_ops_release
-  unsigned long long transpose_clock = 0;
+  unsigned long long map_clock = 0;
 };
 
 // For the current device, created on the first call (which allocates and synchronises: refused with null while
@@ -340,14 +339,12 @@ void* scratch_reserve(DeviceState* st, hipStream_t stream, size_t bytes);
 bool cells_reserve(DeviceState* st, hipStream_t stream, size_t counters, size_t rest_bytes, CellBlock* out);
 // Transpose a force op builds for itself (n_recv receiving atoms, cap keys each), in the stream's own work area.
 bool bucket_reserve(DeviceState* st, size_t n_recv, int cap, hipStream_t stream, TransposeRef* out);
-// What the library keeps beside the intmap2b tensor `im2` the descriptor op is about to write (nf frames, N centres,
-// Nrecv receiving atoms): for its own neighbour search (symmetric) only the fact, for a caller's list a transposed
-// map of cap keys per receiver.  No block to be had -> false.
-bool transpose_for_descriptor(DeviceState* st, const int* im2, int nf, int N, int Nrecv, int nr, int cap,
-                              bool symmetric, hipStream_t stream, TransposeRef* out);
-// The transpose that covers the map view a force op was handed (pointer into a descriptor output, frame stride ld),
-// if the library holds one.
-bool transpose_find(DeviceState* st, const int* im2_view, int nf, int Nrecv, int Nl, int ld, int nr, TransposeRef* out);
+// Remembers the intmap2b tensor `im2` [nf, N, nr+1] that the descriptor op is about to write with its own neighbour search.
+// No block for the checksums to be had -> false.
+bool remember_map(DeviceState* st, const int* im2, int nf, int N, int nr, hipStream_t stream, TransposeRef* out);
+// What is known of the map view a force op was handed (pointer into a descriptor output of N atoms, frame stride ld), if
+// it is remembered.
+bool find_map(DeviceState* st, const int* im2_view, int nf, int N, int Nl, int ld, int nr, TransposeRef* out);
 int finish_op(DeviceState* st, hipStream_t stream);            // launch check (+ optional sync & status fetch)
 // STAF_E_CAPTURE when the stream is being captured, else STAF_E_HIP: the code for a work area that could not be had
 int reserve_failure(hipStream_t stream);
@@ -399,6 +396,11 @@ template <typename real>
 DescConfig<real> desc_current();
 // A caller's neighbour list of one frame in the caller's order: centre i (a slot, 0 <= i < N) has howmany[row_of[i]]
 // neighbours, the atoms slot_of[with[row_of[i] * pitch + k]].  The entries have been checked on the host.
+// Where the forces on an atom are found is the caller's too (`tr` of desc_launch): for the own search the tensor the map
+// goes to, for a list the build
+// counters [Npos] (all zero), counts [Npos] and keys [Npos * cap] that the launch fills.  A
+// call of several stages holds these itself: what the library remembers by a tensor's address is little, and other
+// threads' calls take its place.
 struct NeighList {
   const int* howmany;   // null: the library's own search
   const int* with;
@@ -408,19 +410,20 @@ struct NeighList {
 };
 template <typename real>
 int desc_launch(const DescConfig<real>& c, const real* pos, const real* box, int nf, int N, int Npos,
-                const NeighList* inj, int skip_pbc, real* raddescr, real* angdescr,
+                const NeighList* inj, const TransposeRef* tr, int skip_pbc, real* raddescr, real* angdescr,
                 real* des3bsupp, int* intmap2b, int* intmap3b, real* der2b, real* der3b, real* der3bsupp,
                 int* numtriplet, real* unit, hipStream_t stream);
 
 
 // Force ops with the wrap switch of the virial forms given per call (skip_pbc = 1: neighbour positions already are
 // periodic images; the extern "C" entry points pass the process-wide setting of staf_op_force_set_skip_pbc, the MD
-// entry its own per call).  Argument lists as in include/staf_ops.h.
+// entry its own per call).  Argument lists as in include/staf_ops.h.  known != null: what the caller holds of the map
+// (key_shift: the first row of the view); null: looked up, or the view is transposed first.
 template <typename real>
 int force_doublets(const real* G, const real* D, const real* dD, const int* im2, int nr, int N, int nf, int Ar,
                    const real* alpha2b, const real* emb2b, int nt, const int* tipos, const int* actual_type,
                    real* force, const int* type_map, int Nl, real* virial, const real* pos, const real* box, int ld,
-                   int skip_pbc, void* stream);
+                   int skip_pbc, void* stream, const TransposeRef* known = nullptr);
 // unit != null: the fused forms of the MD entry (T and its Jacobian rebuilt from the radial-only descriptor call's
 // unit vectors; Tang, d3b, im3 are not read and may be null).
 template <typename real>
@@ -445,7 +448,7 @@ int force_tripl(const real* G, const real* Dsup, const real* Tang, const real* d
                 const int* tipos, const int* actual_type, real* force, const int* numtriplet, const real* alpha3b,
                 const int* type_map, int Nl, real* virial, const real* pos, const real* box, int ld, int skip_pbc,
                 void* stream, real* slots_out = nullptr, real* self_out = nullptr,
-                const Force2In<real>* two_body = nullptr);
+                const Force2In<real>* two_body = nullptr, const TransposeRef* known = nullptr);
 template <typename real>
 int force_total(const int* im2_full, int nr, int N, int nf, int nt, const int* n_local, const real* const* slot_forces,
                 const real* const* self_forces, const real* const* force_2b, real* total, void* stream);
@@ -463,6 +466,7 @@ struct StepRows {             // what the radial-only descriptor launch leaves, 
   const real *raddescr, *des3bsupp, *der2b, *der3bsupp, *unit;
   const int *intmap2b, *numtriplet;
   int nr, na, nf, nlocal;     // nlocal rows per frame
+  TransposeRef tr;            // what desc_launch was given
 };
 // 2-body and 3-body fingerprints
 template <typename real>

@@ -803,14 +803,14 @@ struct FingerprintStep {
 
 template <typename real>
 static int desc_launch_impl(const DescConfig<real>& c, const real* pos, const real* box, int nf, int N, int Npos,
-                            const NeighList* inj, int skip_pbc, real* raddescr,
+                            const NeighList* inj, const TransposeRef* tr, int skip_pbc, real* raddescr,
                             real* angdescr, real* des3bsupp, int* intmap2b, int* intmap3b, real* der2b, real* der3b,
                             real* der3bsupp, int* numtriplet, real* unit, hipStream_t stream,
                             const FingerprintStep<real>* fp) {
   if (!c.ready) return STAF_E_NOT_CONSTRUCTED;
   const bool angular = unit == nullptr;   // with `unit` the call is radial-only
   if (!pos || !box || !raddescr || !des3bsupp || !intmap2b || !der2b || !der3bsupp || !numtriplet || nf <= 0 ||
-      N <= 0 || Npos < N || (inj && nf != 1) || (angular && (!angdescr || !intmap3b || !der3b)))
+      N <= 0 || Npos < N || (inj && (nf != 1 || !tr)) || (!tr && Npos != N) || (angular && (!angdescr || !intmap3b || !der3b)))
     return STAF_E_BAD_ARG;
   DeviceState* st = device_state(stream);
   if (!st) return reserve_failure(stream);
@@ -828,8 +828,8 @@ static int desc_launch_impl(const DescConfig<real>& c, const real* pos, const re
   // the negated difference vector: same bits), so the map it writes needs no transposing; a caller's list may name
   // ghost atoms, which list nobody, and from more centres than nr.
   const bool symmetric = inj == nullptr;
-  if (!transpose_for_descriptor(st, intmap2b, nf, N, Npos, c.nr, 4 * c.nr, symmetric, stream, &A.tr))
-    return reserve_failure(stream);
+  if (tr) A.tr = *tr;
+  else if (!remember_map(st, intmap2b, nf, N, c.nr, stream, &A.tr)) return reserve_failure(stream);
   A.cell_dims = A.cell_counts = A.cell_of = nullptr;
   A.cell_recs = nullptr;
   const int cell_from = g_cell_threshold;
@@ -907,18 +907,18 @@ static int desc_launch_impl(const DescConfig<real>& c, const real* pos, const re
 
 template <typename real>
 int desc_launch(const DescConfig<real>& c, const real* pos, const real* box, int nf, int N, int Npos,
-                const NeighList* inj, int skip_pbc, real* raddescr, real* angdescr,
+                const NeighList* inj, const TransposeRef* tr, int skip_pbc, real* raddescr, real* angdescr,
                 real* des3bsupp, int* intmap2b, int* intmap3b, real* der2b, real* der3b, real* der3bsupp,
                 int* numtriplet, real* unit, hipStream_t stream) {
-  return desc_launch_impl<real>(c, pos, box, nf, N, Npos, inj, skip_pbc, raddescr, angdescr,
+  return desc_launch_impl<real>(c, pos, box, nf, N, Npos, inj, tr, skip_pbc, raddescr, angdescr,
                                 des3bsupp, intmap2b, intmap3b, der2b, der3b, der3bsupp, numtriplet, unit, stream,
                                 (const FingerprintStep<real>*)nullptr);
 }
 template int desc_launch<float>(const DescConfig<float>&, const float*, const float*, int, int, int, const NeighList*,
-                                int, float*, float*, float*, int*, int*, float*, float*, float*, int*,
+                                const TransposeRef*, int, float*, float*, float*, int*, int*, float*, float*, float*, int*,
                                 float*, hipStream_t);
 template int desc_launch<double>(const DescConfig<double>&, const double*, const double*, int, int, int, const NeighList*,
-                                 int, double*, double*, double*, int*, int*, double*, double*, double*,
+                                 const TransposeRef*, int, double*, double*, double*, int*, int*, double*, double*, double*,
                                  int*, double*, hipStream_t);
 
 template <typename real>
@@ -946,7 +946,7 @@ static int compute(const real* pos, const real* box, int nf, int N, real* raddes
                    int* intmap2b, int* intmap3b, real* der2b, real* der3b, real* der3bsupp, int* numtriplet,
                    void* stream_) {
   const DescConfig<real> c = desc_current<real>();
-  return desc_launch<real>(c, pos, box, nf, N, N, nullptr, 0, raddescr, angdescr, des3bsupp, intmap2b,
+  return desc_launch<real>(c, pos, box, nf, N, N, nullptr, nullptr, 0, raddescr, angdescr, des3bsupp, intmap2b,
                            intmap3b, der2b, der3b, der3bsupp, numtriplet, (real*)nullptr, (hipStream_t)stream_);
 }
 
@@ -975,7 +975,7 @@ static int compute_with_fingerprints(const real* pos, const real* box, int nf, i
   if (sum != N) return STAF_E_BAD_ARG;
   const DescConfig<real> c = desc_current<real>();
   FingerprintStep<real> fp = {nt, first_species, n_species, n_local, type_map, Aa, alpha3b, emb3b, af3, Ar, alpha2b, emb2b, af2};
-  return desc_launch_impl<real>(c, pos, box, nf, N, N, nullptr, 0, raddescr, angdescr, des3bsupp, intmap2b,
+  return desc_launch_impl<real>(c, pos, box, nf, N, N, nullptr, nullptr, 0, raddescr, angdescr, des3bsupp, intmap2b,
                                 intmap3b, der2b, der3b, der3bsupp, numtriplet, (real*)nullptr,
                                 (hipStream_t)stream_, &fp);
 }

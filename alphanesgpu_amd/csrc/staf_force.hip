@@ -535,11 +535,12 @@ static inline int grad_blocks_f(int atoms) {
   return nb < GRAD_MAX_BLOCKS_F ? nb : GRAD_MAX_BLOCKS_F;
 }
 
-// The transposed neighbour map for a force op: the one the descriptor op left beside the tensor `im2` points into,
-// or, for any other copy of the map, one built here in the stream's work area (push + sort launches).
+// The transposed neighbour map for a force op: what the caller holds (known), what is remembered of the tensor `im2` points
+// into, or, for any other copy of a map, a transpose built here in the stream's work area (push + sort launches).
 static int force_transpose(DeviceState* st, const int* im2, int nf, int N, int Nl, int ld, int nr, hipStream_t stream,
-                           TransposeRef* tr, bool* cached) {
-  *cached = transpose_find(st, im2, nf, N, Nl, ld, nr, tr);
+                           const TransposeRef* known, TransposeRef* tr, bool* cached) {
+  if (known) *tr = *known;
+  *cached = known || find_map(st, im2, nf, N, Nl, ld, nr, tr);
   if (*cached) return STAF_OK;
   const int cap = 4 * nr;
   if ((size_t)TR_WAVES * cap * sizeof(int) > 64 * 1024) return STAF_E_LIMIT;
@@ -571,7 +572,7 @@ template <typename real>
 int force_doublets(const real* G, const real* D, const real* dD, const int* im2, int nr, int N, int nf, int Ar,
                    const real* alpha2b, const real* emb2b, int nt, const int* tipos, const int* actual_type,
                    real* force, const int* type_map, int Nl, real* virial, const real* pos, const real* box, int ld,
-                   int skip_pbc, void* stream_) {
+                   int skip_pbc, void* stream_, const TransposeRef* known) {
   if ((virial || pos || box) && !(virial && pos && box)) return STAF_E_BAD_ARG;
   if (Nl == 0 && nf > 0 && N > 0 && force) return empty_species_force<real>(force, virial, nf, N, stream_);
   if (!G || !D || !dD || !im2 || !alpha2b || !emb2b || !tipos || !actual_type || !force || !type_map || nr <= 0 ||
@@ -584,7 +585,7 @@ int force_doublets(const real* G, const real* D, const real* dD, const int* im2,
   hipStream_t stream = (hipStream_t)stream_;
   Force2Args<real> A;
   bool cached = false;
-  int rc = force_transpose(st, im2, nf, N, Nl, ld, nr, stream, &A.tr, &cached);
+  int rc = force_transpose(st, im2, nf, N, Nl, ld, nr, stream, known, &A.tr, &cached);
   if (rc) return rc;
   A.G = G; A.D = D; A.dD = dD; A.im2 = im2; A.alpha2b = alpha2b; A.emb2b = emb2b; A.type_map = type_map;
   A.tipos = tipos; A.actual_type = actual_type; A.force = force; A.vpart = nullptr; A.pos = pos; A.box = box;
@@ -619,7 +620,8 @@ int force_tripl(const real* G, const real* Dsup, const real* Tang, const real* d
                 const real* emb3b, int nt,
                 const int* tipos, const int* actual_type, real* force, const int* numtriplet, const real* alpha3b,
                 const int* type_map, int Nl, real* virial, const real* pos, const real* box, int ld, int skip_pbc,
-                void* stream_, real* slots_out, real* self_out, const Force2In<real>* two_body) {
+                void* stream_, real* slots_out, real* self_out, const Force2In<real>* two_body,
+                const TransposeRef* known) {
   (void)im3;
   if ((virial || pos || box) && !(virial && pos && box)) return STAF_E_BAD_ARG;
   // slots_out / self_out: the slot forces [nf, Nl, nr, 3] and the centres' own forces [nf, Nl, 3] go to the caller
@@ -649,7 +651,7 @@ int force_tripl(const real* G, const real* Dsup, const real* Tang, const real* d
   if (!Force3Cfg<real, 4>::fits(nr, nt) || N >= (1 << (31 - KEY_SLOT_BITS))) return STAF_E_LIMIT;
   TransposeRef tr;
   bool cached = false;
-  int rc = deferred ? STAF_OK : force_transpose(st, im2, nf, N, Nl, ld, nr, stream, &tr, &cached);
+  int rc = deferred ? STAF_OK : force_transpose(st, im2, nf, N, Nl, ld, nr, stream, known, &tr, &cached);
   if (rc) return rc;
   const size_t ng = (size_t)nf * Nl * nr * 3, ns = (size_t)nf * Nl * 3, nv = virial ? (size_t)nf * Nl * 9 : 0;
   real* gslot = deferred ? slots_out : (real*)scratch_reserve(st, stream, (ng + ns + nv) * sizeof(real));
@@ -708,13 +710,13 @@ int force_tripl(const real* G, const real* Dsup, const real* Tang, const real* d
 
 template int force_doublets<double>(const double*, const double*, const double*, const int*, int, int, int, int,
                                     const double*, const double*, int, const int*, const int*, double*, const int*,
-                                    int, double*, const double*, const double*, int, int, void*);
+                                    int, double*, const double*, const double*, int, int, void*, const TransposeRef*);
 template int force_tripl<double>(const double*, const double*, const double*, const double*, const double*,
                                  const double*, const int*, const int*, int, int, int, int, int, const double*, int,
                                  const int*,
                                  const int*, double*, const int*, const double*, const int*, int, double*,
                                  const double*, const double*, int, int, void*, double*, double*,
-                                 const Force2In<double>*);
+                                 const Force2In<double>*, const TransposeRef*);
 
 template <typename real>
 static int gradforce_2b(const real* Q, const real* D, int nr, const real* alpha2b, int Ar, const real* dD,
@@ -945,7 +947,7 @@ int step_collect(const StepSpecies<real>* sp, int n, const StepRows<real>& R, in
   StepCollectArgs<real> A = {};
   A.io = out;
   if (out.force) {
-    if (!transpose_find(st, R.intmap2b, R.nf, nall, R.nlocal, R.nlocal, R.nr, &A.tr)) return STAF_E_BAD_ARG;
+    A.tr = R.tr;
     A.atom_blocks = (R.nf * nall + F_WAVES - 1) / F_WAVES;
   }
   A.status = status_word(st, stream);
@@ -1007,7 +1009,7 @@ int force_total(const int* im2_full, int nr, int N, int nf, int nt, const int* n
   // the slots that list an atom are found through the atom's own row: only a map the library's own neighbour search
   // wrote, and remembers, is known to be symmetric
   TransposeRef tr;
-  if (!transpose_find(st, im2_full, nf, N, N, N, nr, &tr) || !tr.symmetric || tr.key_shift != 0) return STAF_E_BAD_ARG;
+  if (!find_map(st, im2_full, nf, N, N, N, nr, &tr) || tr.key_shift != 0) return STAF_E_BAD_ARG;
   A.full = im2_full; A.total = total; A.status = status_word(st, stream); A.rowsum = tr.rowsum;
   A.nf = nf; A.N = N; A.nr = nr; A.nt = nt;
   {

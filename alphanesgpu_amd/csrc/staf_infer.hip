@@ -35,6 +35,14 @@ static DevMlpSource net_source(const StafFramesSpecies& s) {
   return n;
 }
 
+// the map that the library's own search writes to `im2`
+static TransposeRef own_map(const void* im2) {
+  TransposeRef t;
+  t.symmetric = 1;
+  t.full = (const int*)im2;
+  return t;
+}
+
 // Where everything lies in the caller's block; STAF_E_LIMIT: a model or a geometry the launches do not take.
 template <typename real>
 static int frames_plan(const DescConfig<real>& c, int nf, int N, int nt, const StafFramesSpecies* sp, FramesPlan<real>* P) {
@@ -125,11 +133,11 @@ static int frames(const real* pos, const real* box, int nf, int N, int nt, const
   DeviceState* st = device_state(stream);
   if (!st) return reserve_failure(stream);
   const StepRows<real> R = {at(P.raddescr), at(P.des3bsupp), at(P.der2b), at(P.der3bsupp), at(P.unit),
-                            (int*)(w + P.intmap2b), (int*)(w + P.numtriplet), c.nr, c.na, nf, N};
+                            (int*)(w + P.intmap2b), (int*)(w + P.numtriplet), c.nr, c.na, nf, N, own_map(w + P.intmap2b)};
   {
     DeferStatus defer;   // conditions the kernels detect are read once, behind the last launch
     if ((rc = dev_mlp_pack<real>(parts.data(), (int)parts.size(), stream)) != STAF_OK) return rc;
-    rc = desc_launch<real>(c, pos, box, nf, N, N, nullptr, 0, at(P.raddescr), nullptr, at(P.des3bsupp),
+    rc = desc_launch<real>(c, pos, box, nf, N, N, nullptr, &R.tr, 0, at(P.raddescr), nullptr, at(P.des3bsupp),
                            (int*)(w + P.intmap2b), nullptr, at(P.der2b), nullptr, at(P.der3bsupp),
                            (int*)(w + P.numtriplet), at(P.unit), stream);
     if (rc != STAF_OK) return rc;

@@ -158,62 +158,42 @@ bool bucket_reserve(DeviceState* st, size_t n_recv, int cap, hipStream_t stream,
   return true;
 }
 
-bool transpose_for_descriptor(DeviceState* st, const int* im2, int nf, int N, int Nrecv, int nr, int cap,
-                              bool symmetric, hipStream_t stream, TransposeRef* out) {
+bool remember_map(DeviceState* st, const int* im2, int nf, int N, int nr, hipStream_t stream, TransposeRef* out) {
   std::lock_guard<std::mutex> lock(g_mu);
-  // a symmetric map needs no transpose, only one word per row for the rows' checksums (the counter part of a block)
-  const size_t want_recv = (size_t)nf * Nrecv, want_keys = symmetric ? 0 : want_recv * cap;
-  Transpose* t = nullptr;
-  for (auto& e : st->transposes)
+  const size_t want = (size_t)nf * N * sizeof(unsigned);
+  KnownMap* t = nullptr;
+  for (auto& e : st->maps)
     if (e.im2 == im2) { t = &e; break; }
-  if (!t) {
-    // A tensor not seen before takes the place that has not been used for the longest time.  Under capture nothing
-    // can be allocated, so only places whose block is already large enough qualify (a graph recorded earlier with
-    // such a place rebuilds the transpose in it on every replay, before it reads it).
-    const bool capturing = stream_is_capturing(stream);
-    for (auto& e : st->transposes) {
-      if (capturing && !symmetric && (e.cap_recv < want_recv || e.cap_keys < want_keys)) continue;
+  if (!t)   // a tensor not seen before takes the place that has not been used for the longest time
+    for (auto& e : st->maps)
       if (!t || e.stamp < t->stamp) t = &e;
-    }
-    if (!t) return false;
+  // (a map whose place has no block for the checksums and cannot get one now -- a tensor first seen while its stream is
+  // captured -- goes without them)
+  bool have_block = t->sums.bytes >= want;
+  if (!have_block && !stream_is_capturing(stream)) {
+    if (!grow(st, &t->sums, want, stream)) return false;
+    have_block = true;
   }
-  // (a symmetric map whose place has no block for the checksums and cannot get one now -- a tensor first seen while
-  // its stream is captured -- goes without them)
-  bool have_block = true;
-  if (symmetric && stream_is_capturing(stream) && (t->cap_recv < want_recv))
-    have_block = false;
-  else if (!transpose_block(st, &t->buf, &t->cap_recv, &t->cap_keys, want_recv, want_keys, stream))
-    return false;
-  t->im2 = im2; t->nf = nf; t->N = N; t->Nrecv = Nrecv; t->nr = nr;
+  t->im2 = im2; t->nf = nf; t->N = N; t->nr = nr;
   t->ref = TransposeRef();
-  t->ref.symmetric = symmetric ? 1 : 0;
+  t->ref.symmetric = 1;
   t->ref.full = im2;
-  // The checksums lie where a transposed map keeps its counts, which every build rewrites -- never in the build
-  // counters, which a later build of the same place expects to read zero (a checksum taken for a counter sends the
-  // build's stores up to 8 GB away from the block).
-  if (symmetric && have_block) t->ref.rowsum = (const unsigned*)t->buf.buf + t->cap_recv;
-  if (!symmetric) {
-    t->ref.build_cnt = (int*)t->buf.buf;
-    t->ref.cnt = t->ref.build_cnt + t->cap_recv;
-    t->ref.keys = t->ref.cnt + t->cap_recv;
-    t->ref.cap = cap;
-  }
-  t->stamp = ++st->transpose_clock;
+  if (have_block) t->ref.rowsum = (const unsigned*)t->sums.buf;
+  t->stamp = ++st->map_clock;
   *out = t->ref;
   return true;
 }
 
-bool transpose_find(DeviceState* st, const int* im2_view, int nf, int Nrecv, int Nl, int ld, int nr,
-                    TransposeRef* out) {
+bool find_map(DeviceState* st, const int* im2_view, int nf, int N, int Nl, int ld, int nr, TransposeRef* out) {
   std::lock_guard<std::mutex> lock(g_mu);
-  for (auto& e : st->transposes) {
-    if (!e.im2 || e.nr != nr || e.nf != nf || e.Nrecv != Nrecv || e.N != ld) continue;
+  for (auto& e : st->maps) {
+    if (!e.im2 || e.nr != nr || e.nf != nf || e.N != N || e.N != ld) continue;
     if (im2_view < e.im2) continue;
     const size_t off = (size_t)(im2_view - e.im2);
     if (off % (size_t)(nr + 1)) continue;
     const size_t first = off / (size_t)(nr + 1);
     if (first + (size_t)Nl > (size_t)e.N) continue;
-    e.stamp = ++st->transpose_clock;
+    e.stamp = ++st->map_clock;
     *out = e.ref;
     out->key_shift = (int)first;
     return true;
@@ -274,7 +254,7 @@ static int fetch_status(DeviceState* st, hipStream_t stream, bool all) {
       // A remembered neighbour map no longer holds what the descriptor op wrote: nothing remembered is trusted any
       // more.  Force ops then transpose the map they are handed themselves until the descriptor op writes again.
       std::lock_guard<std::mutex> lock2(g_mu);
-      for (auto& e : st->transposes) e.im2 = nullptr;
+      for (auto& e : st->maps) e.im2 = nullptr;
     }
   }
   return decode_status(bits);
@@ -336,8 +316,8 @@ void staf_ops_release(void) {
     if (kv.second.buckets.buf) (void)hipFree(kv.second.buckets.buf);
     if (kv.second.cells.buf) (void)hipFree(kv.second.cells.buf);
   }
-  for (auto& t : st->transposes)
-    if (t.buf.buf) (void)hipFree(t.buf.buf);
+  for (auto& t : st->maps)
+    if (t.sums.buf) (void)hipFree(t.sums.buf);
   for (void* p : st->retired) (void)hipFree(p);
   if (st->status_d) (void)hipFree(st->status_d);
   if (st->status_h) (void)hipHostFree(st->status_h);

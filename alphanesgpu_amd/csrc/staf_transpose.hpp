@@ -2,18 +2,18 @@
 //
 // The reference scatters pair forces with floating-point atomicAdd (STAF/src/force/rad/reforce.cu.cc:112-131,
 // STAF/src/force/ang/reforce.cu.cc:206-231).  Here the force on an atom is gathered by the atom itself from the
-// slots that point at it, which needs intmap2b transposed: receiver -> sorted list of keys (centre, slot).  The
-// transpose depends on intmap2b alone, so it is built once by the descriptor op that writes intmap2b (pushes from
-// desc_kernel, one sort launch) and kept by the library beside that tensor; every force op that is handed a view of
-// that tensor finds it by address.  A force op that is handed some other copy of the map builds a transpose of its
-// own first (push + sort launches).
+// slots that point at it, which needs intmap2b transposed: receiver -> sorted list of keys (centre, slot).  A caller's
+// list of the MD entry is transposed by the descriptor launch that reads it (pushes from its workgroups, one sort
+// launch) into a block of the model.  A force op that is handed a map that is not remembered builds a transpose of its own
+// first (push + sort launches).
 //
 // Building uses integer atomics only (the arrival order they leave is removed by the sort); every list ends up in
 // ascending (centre, slot) order, so sums taken over it have a fixed order.
 //
 // None of this is needed for the maps the library's own neighbour search writes: those are symmetric, the centres
 // that list an atom are the atom's own neighbours, and the slot is found by looking the atom up in the centre's row
-// (slots_of below).  Sums then run in the order of the atom's own (distance-sorted) row.
+// (slots_of below).  Sums then run in the order of the atom's own (distance-sorted) row.  The descriptor op remembers by its
+// address that a tensor holds such a map, and every force op that is handed a view of that tensor finds it.
 #pragma once
 #include "staf_common.hpp"
 

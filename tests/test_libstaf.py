@@ -679,6 +679,46 @@ def test_three_handles_on_three_host_threads():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("host_mlp", [False, True])
+def test_more_handles_on_threads_than_maps_are_remembered(host_mlp):
+    """Twelve handles on twelve host threads, every other one with a caller's list: more than the neighbour maps the ops
+    remember by address, so a call may rely only on what its own handle holds between its launches.  Every call returns the
+    bits a single handle returned for the same frame."""
+    import threading
+    from alphanesgpu_amd import libstaf
+    pos, box, types = load_water_smoke(np.float64)
+    pos = pos.reshape(-1, 3)
+    x, allx, alltypes, _, howmany, neigh = _ghost_configuration(pos, box[0], types, RC)
+    d = os.path.join(GOLDEN, "model_double")
+    frames = [((pos, box[0], types), {}), ((allx, box[0], alltypes), dict(nlocal=len(x), howmany=howmany, neigh=neigh))]
+    make = lambda: libstaf.StafModel(d, precision=1, full_virial=True, host_mlp=host_mlp)
+    m = make()
+    want = [m.compute(*a, **kw) for a, kw in frames]
+    m.close()
+    bad = []
+
+    def worker(t):
+        try:
+            m = make()
+            for rep in range(4 if host_mlp else 25):
+                which = (t + rep // 3) % 2
+                a, kw = frames[which]
+                got = m.compute(*a, **kw)
+                if not all(np.array_equal(g, w) for g, w in zip(got, want[which])):
+                    bad.append((t, rep))
+            m.close()
+        except Exception as ex:   # a thread's exception would otherwise be lost
+            bad.append((t, repr(ex)))
+
+    threads = [threading.Thread(target=worker, args=(t,)) for t in range(12)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not bad, bad[:10]
+
+
+@pytest.mark.gpu
 def test_compute_return_codes():
     """Validation order and codes of libstaf/src/staf_api.cpp:196-337."""
     from alphanesgpu_amd import libstaf
