@@ -228,11 +228,14 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
 #pragma unroll
       for (int v = 0; v < 4; v++) y[v] += acc[v];
       mlp_act<T, 4>(act, y);
-      // (features beyond the last are 0 whatever their zero weights were multiplied with: an infinite value gives no number)
+      // (features beyond the last are 0 whatever their zero weights were multiplied with: an infinite value gives no number.  Asked
+      // of the last tile alone: as a select of every value this costs the single-precision kernel eight registers and, with
+      // the eighth wave per SIMD, 50.9 -> 56.5 us for 24576 atoms)
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int j = tile * 16 + M::row(lane, v);
-        Y[j * MLP_TA + my] = j < out_f ? y[v] : T(0);
+        if (tile * 16 + 16 > out_f && j >= out_f) y[v] = 0;
+        Y[j * MLP_TA + my] = y[v];
       }
     }
     if (l + 2 < nl) {
@@ -309,8 +312,11 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
       const acc_t acc = product(net.bw[l], tile, np, D);
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        if (l > 0) at[M::row(lane, v) * MLP_TA] = tile * 16 + M::row(lane, v) < in_f ? acc[v] * mlp_slope<T>(act, other[v]) : T(0);
-        else put(tile * 16 + M::row(lane, v), acc[v], other[v]);
+        if (l > 0) {
+          T d = acc[v] * mlp_slope<T>(act, other[v]);
+          if (tile * 16 + 16 > in_f && tile * 16 + M::row(lane, v) >= in_f) d = 0;
+          at[M::row(lane, v) * MLP_TA] = d;
+        } else put(tile * 16 + M::row(lane, v), acc[v], other[v]);
       }
     }
     if (l > 0) {
