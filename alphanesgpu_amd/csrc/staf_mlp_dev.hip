@@ -7,9 +7,10 @@
 // The Dense layers are small matrix products ([out, in] x [in, atoms]) and run on the matrix cores: a workgroup takes
 // 16 atoms, which are the columns of its 16x16x4 tiles, and a wave takes tiles of 16 output features over the whole
 // inner dimension, so that no partial sums meet in LDS and a layer costs one barrier per direction.  Activations lie in
-// LDS as [feature][16 atoms]: a tile step's read and the result's write are runs of consecutive words.  A layer's
-// delta takes the place of its activations (the derivative needs nothing else), and the input the place of the second
-// hidden layer: 39 KB for the reference's stack in double precision, four workgroups per CU.  The weights are kept in
+// LDS as [feature][16 atoms] (8 atoms for stacks with more features than fit that way): a tile step's read and the
+// result's write are runs of consecutive words.  A layer's delta takes the place of its activations (the derivative needs
+// nothing else), and the input the place of the second hidden layer: 39 KB for the reference's stack in double
+// precision, four workgroups per CU.  The weights are kept in
 // the order in which a wave reads them -- 16 bytes per lane, zero-padded to whole tiles -- forwards and transposed; a
 // wave requests the first pieces of its next product ahead of the barrier it waits at and stays six pieces ahead.
 // Bound: matrix cores and vector units in turn (16384 atoms in double precision: 25 us of matrix instructions, 16 us of
@@ -23,7 +24,6 @@
 
 namespace staf {
 
-constexpr int MLP_TA = 16;       // atoms per workgroup
 constexpr int MLP_AHEAD = 6;     // 16-byte weight pieces a lane has in flight
 constexpr int MLP_WAVES_MAX = 16;
 
@@ -145,14 +145,16 @@ __device__ inline T mlp_slope(int act, T y) {
   return act == 1 ? T(1) - y * y : relu;
 }
 
-template <typename T, typename real>
+// TA: atoms per workgroup, 16, or 8 for stacks whose rows of 16 do not fit the LDS -- an atom then holds two columns of the
+// tiles, whose lanes compute and store the same values.
+template <typename T, typename real, int TA>
 __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs<T, real> A) {
   using M = MlpTile<T>;
   using piece_t = typename M::piece_t;
   using acc_t = typename M::acc_t;
   constexpr int STEPS = mlp_steps<T>();
   extern __shared__ __align__(16) unsigned char smem[];
-  // [rows of the hidden layers][16 atoms], then the parts of the energy sums; the input lies where the second hidden
+  // [rows of the hidden layers][TA atoms], then the parts of the energy sums; the input lies where the second hidden
   // layer will
   T* const H = (T*)smem;
   const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = uniform(tid / WAVE), nw = blockDim.x / WAVE;
@@ -160,9 +162,9 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
   while (s + 1 < A.ns && (int)blockIdx.x >= A.sp[s + 1].first) s++;
   const MlpSpecies<real>& S = A.sp[s];
   const MlpNet<T>& net = A.net[s];
-  const int a0 = ((int)blockIdx.x - S.first) * MLP_TA;
+  const int a0 = ((int)blockIdx.x - S.first) * TA;
   const int nl = net.nl, n_af = net.n_af;
-  const int my = lane & 15;                                    // the lane's atom in a tile
+  const int my = lane & (TA - 1);                              // the lane's atom in a tile
   const bool live = a0 + my < S.Nl;
   const size_t atom = (size_t)(live ? a0 + my : S.Nl - 1);     // (lanes without an atom follow the last one, storing nothing)
 
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
     const piece_t* f = (const piece_t*)frag + (size_t)tile * np * WAVE + lane;
     acc_t acc = {0, 0, 0, 0};
     const int whole = np / MLP_AHEAD, rest = np - whole * MLP_AHEAD;
-    X += lane;
+    X += (lane / 16) * TA + my;
     for (int g = 0; g < whole; g++) {
       f += MLP_AHEAD * WAVE;
 #pragma unroll
@@ -187,15 +189,15 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
         const piece_t w = ring[u];
         ring[u] = f[u * WAVE];
 #pragma unroll
-        for (int j = 0; j < STEPS; j++) acc = M::run(w[j], X[(u * STEPS + j) * WAVE], acc);
+        for (int j = 0; j < STEPS; j++) acc = M::run(w[j], X[(u * STEPS + j) * 4 * TA], acc);
       }
-      X += MLP_AHEAD * STEPS * WAVE;
+      X += MLP_AHEAD * STEPS * 4 * TA;
     }
 #pragma unroll
     for (int u = 0; u + 1 < MLP_AHEAD; u++) {
       if (u >= rest) break;
 #pragma unroll
-      for (int j = 0; j < STEPS; j++) acc = M::run(ring[u][j], X[(u * STEPS + j) * WAVE], acc);
+      for (int j = 0; j < STEPS; j++) acc = M::run(ring[u][j], X[(u * STEPS + j) * 4 * TA], acc);
     }
     return acc;
   };
@@ -203,14 +205,14 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
   const int np0 = mlp_pieces<T>(n_af);
   if (nl > 1 && wave < mlp_tiles(net.out_f[0])) request(net.fw[0], wave, np0);
   const int rows0 = mlp_rows(n_af);
-  T* const input = H + (nl > 1 ? mlp_rows(net.out_f[0]) * MLP_TA : 0);
-  for (int i = tid / MLP_TA; i < rows0; i += (int)blockDim.x / MLP_TA) {
+  T* const input = H + (nl > 1 ? mlp_rows(net.out_f[0]) * TA : 0);
+  for (int i = tid / TA; i < rows0; i += (int)blockDim.x / TA) {
     T v = 0;
     if (i < n_af && live) {
       const T afv = (T)(i < S.Ar ? S.af2[atom * S.Ar + i] : S.af3[atom * S.Aa + (i - S.Ar)]);
       v = m_log(afv + T(1e-3)) - net.mu[i];
     }
-    input[i * MLP_TA + my] = v;
+    input[i * TA + my] = v;
   }
   __syncthreads();
   // ---- forward through the hidden layers
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
   for (int l = 0; l + 1 < nl; l++) {
     const int in_f = net.in_f[l], out_f = net.out_f[l], act = net.act[l];
     const int np = mlp_pieces<T>(in_f), tiles = mlp_tiles(out_f);
-    T* Y = l == 0 ? H : X + mlp_rows(in_f) * MLP_TA;
+    T* Y = l == 0 ? H : X + mlp_rows(in_f) * TA;
     for (int tile = wave; tile < tiles; tile += nw) {
       if (tile != wave) request(net.fw[l], tile, np);
       T y[4];
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
       for (int v = 0; v < 4; v++) {
         const int j = tile * 16 + M::row(lane, v);
         if (tile * 16 + 16 > out_f && j >= out_f) y[v] = 0;
-        Y[j * MLP_TA + my] = y[v];
+        Y[j * TA + my] = y[v];
       }
     }
     if (l + 2 < nl) {
@@ -252,28 +254,28 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
     const int in_f = net.in_f[nl - 1], act = net.act[nl - 1], hact = nl > 1 ? net.act[nl - 2] : 0;
     const int rows = mlp_rows(in_f);
     const T* w = net.fw[nl - 1];
-    T* parts = X + (nl == 2 ? rows + rows0 : rows) * MLP_TA;
-    const int np = (int)blockDim.x / MLP_TA, t = tid % MLP_TA, part = tid / MLP_TA;
+    T* parts = X + (nl == 2 ? rows + rows0 : rows) * TA;
+    const int np = (int)blockDim.x / TA, t = tid % TA, part = tid / TA;
     T sum = 0;
     for (int k = part; k < in_f; k += np) {
-      const T h = X[k * MLP_TA + t];
+      const T h = X[k * TA + t];
       sum += h * w[k];
-      if (act == 0 && nl > 1) X[k * MLP_TA + t] = w[k] * mlp_slope<T>(hact, h);
+      if (act == 0 && nl > 1) X[k * TA + t] = w[k] * mlp_slope<T>(hact, h);
     }
-    parts[part * MLP_TA + t] = sum;
+    parts[part * TA + t] = sum;
     __syncthreads();
-    if (tid < MLP_TA || act != 0) {
+    if (tid < TA || act != 0) {
       T y = net.b[nl - 1][0];
-      for (int p = 0; p < np; p++) y += parts[p * MLP_TA + t];
+      for (int p = 0; p < np; p++) y += parts[p * TA + t];
       T ys[1] = {y};
       mlp_act<T, 1>(act, ys);
       y = ys[0];
-      if (tid < MLP_TA && a0 + t < S.Nl) S.e_atom[a0 + t] = (real)y;
+      if (tid < TA && a0 + t < S.Nl) S.e_atom[a0 + t] = (real)y;
       if (act != 0 && nl > 1) {
         const T d = mlp_slope<T>(act, y);
         for (int k = part; k < in_f; k += np) {
-          const T h = X[k * MLP_TA + t];
-          X[k * MLP_TA + t] = w[k] * d * mlp_slope<T>(hact, h);
+          const T h = X[k * TA + t];
+          X[k * TA + t] = w[k] * d * mlp_slope<T>(hact, h);
         }
       }
       // (every thread of an atom holds the same value; it goes where the input was, which nobody reads any more -- the
@@ -293,7 +295,7 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
   };
   if (nl == 1) {
     const T d = X[my];
-    for (int i = tid / MLP_TA; i < n_af; i += (int)blockDim.x / MLP_TA)
+    for (int i = tid / TA; i < n_af; i += (int)blockDim.x / TA)
       put(i, net.fw[0][i] * d, af_at(i));
     return;
   }
@@ -301,21 +303,21 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
     const int in_f = net.in_f[l], out_f = net.out_f[l];
     const int np = mlp_pieces<T>(out_f), rows = mlp_rows(in_f), tiles = mlp_tiles(in_f);
     T* const D = X;                           // the layer's deltas
-    if (l > 0) X = X - rows * MLP_TA;         // the layer's inputs
+    if (l > 0) X = X - rows * TA;         // the layer's inputs
     const int act = l > 0 ? net.act[l - 1] : 0;
     for (int tile = wave; tile < tiles; tile += nw) {
       if (tile != wave) request(net.bw[l], tile, np);
       T other[4];   // what the product is multiplied with: the inputs' values, or the fingerprints behind them
-      T* const at = X + (tile * 16) * MLP_TA + my;
+      T* const at = X + (tile * 16) * TA + my;
 #pragma unroll
-      for (int v = 0; v < 4; v++) other[v] = l > 0 ? at[M::row(lane, v) * MLP_TA] : af_at(tile * 16 + M::row(lane, v));
+      for (int v = 0; v < 4; v++) other[v] = l > 0 ? at[M::row(lane, v) * TA] : af_at(tile * 16 + M::row(lane, v));
       const acc_t acc = product(net.bw[l], tile, np, D);
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         if (l > 0) {
           T d = acc[v] * mlp_slope<T>(act, other[v]);
           if (tile * 16 + 16 > in_f && tile * 16 + M::row(lane, v) >= in_f) d = 0;
-          at[M::row(lane, v) * MLP_TA] = d;
+          at[M::row(lane, v) * TA] = d;
         } else put(tile * 16 + M::row(lane, v), acc[v], other[v]);
       }
     }
@@ -328,8 +330,17 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
 
 // LDS of a workgroup: the rows of all layers' activations, and a part of the energy sums per thread
 template <typename T>
-static size_t mlp_lds(int rows, int waves) {
-  return ((size_t)rows * MLP_TA + (size_t)waves * WAVE) * sizeof(T);
+static size_t mlp_lds(int rows, int waves, int ta) {
+  return ((size_t)rows * ta + (size_t)waves * WAVE) * sizeof(T);
+}
+// Atoms per workgroup for stacks of `rows`: 16 up to about 1200 features in all layers in double precision and 2480 in
+// single, 8 up to twice as many (six layers of 430 in single precision, 768 atoms: 160 us, where the host takes 258 ms);
+// 0: too many.
+template <typename T>
+static int mlp_atoms(int rows) {
+  for (int ta : {16, 8})
+    if (mlp_lds<T>(rows, MLP_WAVES_MAX, ta) <= 160 * 1024) return ta;
+  return 0;
 }
 
 template <typename T>
@@ -387,10 +398,7 @@ static bool upload_net(const StafMlp* mlp, int type, DevMlpNet* net, hipStream_t
   if (nl <= 2) rows += mlp_rows(net->n_af);
   net->tiles = tiles;
   net->rows = rows;
-  if (!lds_request(mlp_kernel<T, double>, mlp_lds<T>(rows, MLP_WAVES_MAX))) {   // a stack too wide for the kernel's LDS is left to the host evaluation
-    (void)hipGetLastError();
-    return false;
-  }
+  if (mlp_atoms<T>(rows) == 0) return false;   // a stack too wide for the kernel's LDS is left to the host evaluation
   (void)place((size_t)MLP_AHEAD * WAVE * mlp_steps<T>());   // the pieces a wave requests beyond the last matrix
   T* block = nullptr;
   if (hipMalloc((void**)&block, host.size() * sizeof(T)) != hipSuccess) return false;
@@ -437,7 +445,7 @@ static bool mlp_shape(const DevMlpSource& src, DevMlpNet* net) {
     net->tiles = std::max(net->tiles, std::max(mlp_tiles(in_f), mlp_tiles(out_f)));
     net->rows += l == 1 ? std::max(mlp_rows(out_f), mlp_rows(src.n_af)) : mlp_rows(out_f);
   }
-  return mlp_lds<T>(net->rows, MLP_WAVES_MAX) <= 160 * 1024;
+  return mlp_atoms<T>(net->rows) != 0;
 }
 
 // elements of matrix [K, J] in tile order
@@ -549,10 +557,10 @@ int dev_mlp_pack(const PackPart* parts, int n, hipStream_t stream) {
 template int dev_mlp_pack<float>(const PackPart*, int, hipStream_t);
 template int dev_mlp_pack<double>(const PackPart*, int, hipStream_t);
 
-template <typename T, typename real>
-static int eval_nets(const DevMlpCall<real>* calls, int n, hipStream_t stream) {
+template <typename T, typename real, int TA>
+static int eval_nets_by(const DevMlpCall<real>* calls, int n, int rows, int tiles, hipStream_t stream) {
   MlpArgs<T, real> A = {};
-  int blocks = 0, tiles = 1, rows = 0;
+  int blocks = 0;
   for (int c = 0; c < n; c++) {
     const DevMlpCall<real>& C = calls[c];
     if (C.Nl <= 0) continue;
@@ -560,26 +568,37 @@ static int eval_nets(const DevMlpCall<real>* calls, int n, hipStream_t stream) {
     MlpSpecies<real>& S = A.sp[A.ns];
     S.af2 = C.af2; S.af3 = C.af3; S.e_atom = C.e_atom; S.g2 = C.g2; S.g3 = C.g3;
     S.Ar = C.Ar; S.Aa = C.Aa; S.Nl = C.Nl; S.first = blocks;
-    blocks += (C.Nl + MLP_TA - 1) / MLP_TA;
+    blocks += (C.Nl + TA - 1) / TA;
     MlpNet<T>& N = A.net[A.ns++];
     N.nl = net.nl; N.n_af = net.n_af; N.mu = (const T*)net.mu;
     for (int l = 0; l < net.nl; l++) {
       N.act[l] = net.act[l]; N.in_f[l] = net.in_f[l]; N.out_f[l] = net.out_f[l];
       N.fw[l] = (const T*)net.fw[l]; N.bw[l] = (const T*)net.bw[l]; N.b[l] = (const T*)net.b[l];
     }
-    tiles = std::max(tiles, net.tiles);
-    rows = std::max(rows, net.rows);
   }
   if (blocks == 0) return STAF_OK;
   // A wave per tile of the widest product while a CU has one workgroup at most (double precision, 60-140-140-1: 22.0
   // us with nine waves, 24.2 with five); two tiles per wave where it has several, whose products and activations then
   // overlap (1024 workgroups: 76.7 us with nine waves, 60.3 with five, 72 with three).
   const int waves = std::min(MLP_WAVES_MAX, std::max(2, blocks <= 256 ? tiles : (tiles + 1) / 2));
-  const size_t lds = mlp_lds<T>(rows, waves);
-  if (!lds_request(mlp_kernel<T, real>, lds)) return STAF_E_LIMIT;
+  const size_t lds = mlp_lds<T>(rows, waves, TA);
+  if (!lds_request(mlp_kernel<T, real, TA>, lds)) return STAF_E_LIMIT;
   KernelTimer kt_("mlp_kernel", stream);
-  hipLaunchKernelGGL((mlp_kernel<T, real>), dim3(blocks), dim3(waves * WAVE), lds, stream, A);
+  hipLaunchKernelGGL((mlp_kernel<T, real, TA>), dim3(blocks), dim3(waves * WAVE), lds, stream, A);
   return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
+}
+
+template <typename T, typename real>
+static int eval_nets(const DevMlpCall<real>* calls, int n, hipStream_t stream) {
+  int rows = 0, tiles = 1;
+  for (int c = 0; c < n; c++) {
+    if (calls[c].Nl <= 0) continue;
+    rows = std::max(rows, calls[c].net->rows);
+    tiles = std::max(tiles, calls[c].net->tiles);
+  }
+  const int ta = mlp_atoms<T>(rows);
+  return ta == 16 ? eval_nets_by<T, real, 16>(calls, n, rows, tiles, stream)
+       : ta == 8 ? eval_nets_by<T, real, 8>(calls, n, rows, tiles, stream) : STAF_E_LIMIT;
 }
 
 template <typename real>

@@ -419,6 +419,43 @@ def test_device_mlp_stack_shapes(tmp_path, prec, tol, hidden, last):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("prec,tol,hidden,on_gpu", [("float", 2e-5, [400] * 6, True), ("float", 2e-5, [430] * 6, True),
+                                                    ("double", 1e-11, [200] * 6, True), ("double", 1e-11, [420] * 6, False)])
+def test_deep_stacks_around_the_limits_of_a_workgroup(tmp_path, capfd, prec, tol, hidden, on_gpu):
+    """Stacks whose activations of 16 atoms just fit a workgroup's LDS, fit it for 8 atoms only, and do not fit: the first
+    two are evaluated on the GPU, the last one on the host (a line on stderr says so) and, in the batch inference, by the
+    layers.  17 atoms of a species: two, three and one workgroups, the last one with a single atom.  Against the host
+    evaluation; float64: rounding of sums of at most 420 terms, float32: as above."""
+    import torch
+    from alphanesgpu_amd import inference, libstaf, model_dir, synth
+    from test_oracle_pins import cluster
+    rng = np.random.Generator(np.random.Philox(37))
+    ps = synth.fingerprint_params(nt=2, ar_map=(5, 4), aa_map=(4, 3, 5), seed=3, dense_embedding=True)
+    for p, h in zip(ps, (hidden, [9])):
+        dims = [p["mu"].shape[0]] + h + [1]
+        acts = ["tanh"] * len(h) + ["linear"]
+        p["layers"] = [(rng.normal(0, 1 / np.sqrt(a), (a, b)), rng.normal(0, 0.1, b), act)
+                       for a, b, act in zip(dims[:-1], dims[1:], acts)]
+    pos, box, tipos, type_map = cluster([17, 16], seed=9, spread=4.4)
+    model_dir.write_model_dir(str(tmp_path), ps, rc=4.5, rc_ang=3.2, rs=1.6, radial_buffer=40, angular_buffer=780,
+                              tipos=tipos, precision=prec)
+    p = 1 if prec == "double" else 0
+    m = libstaf.StafModel(str(tmp_path), precision=p, full_virial=True, host_mlp=True)
+    e0, f0, v0 = m.compute(pos.reshape(-1, 3), box[0], type_map)
+    m.close()
+    capfd.readouterr()
+    m = libstaf.StafModel(str(tmp_path), precision=p, full_virial=True)
+    assert ("on the host" not in capfd.readouterr().err) == on_gpu
+    e1, f1, v1 = m.compute(pos.reshape(-1, 3), box[0], type_map)
+    m.close()
+    assert abs(e1 - e0) <= tol * max(1.0, abs(e0)) and nerr(f1, f0) <= tol and nerr(v1, v0) <= tol
+    inf = inference.staf_full_inference(str(tmp_path), dtype=torch.float64 if p else torch.float32)
+    e2, f2, _ = inf.full_test(pos, box)
+    tol2 = tol if p else 5e-5       # (everything in float32)
+    assert abs(float(e2[0]) - e0) <= tol2 * max(1.0, abs(e0)) and nerr(f2.cpu().numpy().reshape(-1, 3), f0) <= tol2
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("prec,tol", [("double", 1e-11), ("float", 2e-5)])
 @pytest.mark.parametrize("last", ["tanh", "relu", "linear"])
 def test_one_layer_network_beside_a_wide_one(tmp_path, prec, tol, last):
