@@ -318,23 +318,21 @@ def run_md(args, workload):
         torch.cuda.synchronize()     # every call ends with its own synchronisation; this one finds nothing to wait for
         block_s.append(time.perf_counter() - t0)
     el = float(np.median(block_s))
-    # per-kernel times from the library's events: a handle that launches every call eagerly (replayed graphs hold no events)
-    me = libstaf.StafModel(tmp, precision=1, eager=True)
-    for _ in range(3):
-        e2, f2, _ = me.compute(x, box, type_map)
-    if not (e2 == e and np.array_equal(f2, f)):
-        print("bench.py: replayed and eager calls of staf_compute differ", file=sys.stderr)
+    # a call depends on its arguments alone: one of a handle just loaded against the last of the timed handle
+    me = libstaf.StafModel(tmp, precision=1)
+    e, f, vir = m.compute(x, box, type_map)
+    e2, f2, vir2 = me.compute(x, box, type_map)
+    if not (e2 == e and np.array_equal(f2, f) and np.array_equal(vir2, vir)):
+        print("bench.py: the first call of a handle and a later one of another handle differ", file=sys.stderr)
         sys.exit(1)
+    # per-kernel times from the library's events, in calls of their own
     nprof = max(3, min(args.steps, 20))
-    t1 = time.perf_counter()
     ops.kernel_timing(True)
     for _ in range(nprof):
         me.compute(x, box, type_map)
     ops.kernel_timing(False)
-    el_eager = (time.perf_counter() - t1) / nprof
     kern = {}
-    for name in ("cell_build_kernel", "desc_kernel", "af2_kernel", "af3_kernel", "force2_kernel", "force3_kernel",
-                 "gather_kernel", "force_total_kernel"):
+    for name in ("cell_build_kernel", "desc_kernel", "af3_kernel", "mlp_kernel", "force3_kernel", "step_collect_kernel"):
         ms, n = ops.kernel_time(name)
         if n:
             kern[name] = dict(ms_per_step=ms / nprof, launches_per_step=n // nprof, avg_launch_ms=ms / n)
@@ -350,10 +348,10 @@ def run_md(args, workload):
     torch.cuda.empty_cache()
     # Bytes the call's kernels move once through HBM by their signatures (no tensor of the angular buffer's width
     # exists on this path).  In rows of N x nr doubles: the radial-only descriptor kernel writes 12 (raddescr,
-    # des3bsupp, der2b x3, der3bsupp x3, unit x4) and the neighbour map; the 2-body fingerprints read 1 and the map,
-    # the fused 3-body fingerprints 5 (des3bsupp, unit), the force launch 12 (raddescr, der2b, des3bsupp, der3bsupp,
-    # unit) -- counted as 4 + 8 below; the slot forces are written and read once (3 rows); fingerprints and their
-    # gradients are written and read once each; positions in, forces out (and the virial pass over the slot forces).
+    # des3bsupp, der2b x3, der3bsupp x3, unit x4) and the neighbour map; of the fingerprint launch the 2-body part reads 1
+    # and the map, the 3-body part 5 (des3bsupp, unit) and the map; the force launch 12 (raddescr, der2b, des3bsupp,
+    # der3bsupp, unit) -- counted as 4 + 8 below; the slot forces are written and read once (3 rows); fingerprints and their
+    # gradients are written and read once each; positions in, forces out, the centres' own forces and virials once each way.
     s = 8
     row = N * nr * s
     imap = N * (nr + 1) * 4
@@ -389,12 +387,11 @@ def run_md(args, workload):
                    "launch": "five launches (six with a cell list) over all species, issued on one stream",
                    "timing": f"median of {REPEATS} blocks of {args.steps} calls"},
         "block_ms_per_step": [b / args.steps * 1e3 for b in block_s],
-        "eager_ms_per_step": el_eager * 1e3,
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": md_bytes / (el / args.steps) / 1e9,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": md_bytes / (el / args.steps) / 1e9 / HBM_PEAK_GBS,
                      "frac_is": "bytes of the whole call (nr-wide tensors only: this path holds no tensor of the angular "
                                 "buffer's width) over the call's time over peak: low by construction, the call is bound "
-                                "by vector-ALU issue and by the latency of its ~25 dependent launches",
+                                "by vector-ALU issue and by the latency of its five dependent launches",
                      "traffic": None, "algorithmic_bytes_per_call": md_bytes,
                      "valu": {"bound": "valu", "unit": "wave instructions/s", "kernel": dom,
                               "algorithmic_inst_per_item": alg.get(dom), "items_per_call": items,
@@ -408,6 +405,9 @@ def run_md(args, workload):
         "kernel_valu_frac_algorithmic": valu_frac,
         "kernel_ms_per_step": {k: v["ms_per_step"] for k, v in kern.items()},
         "kernels_sum_ms": sum(v["ms_per_step"] for v in kern.values()),
+        "kernels_note": "af3_kernel: 2-body and 3-body fingerprints of all species; mlp_kernel: their networks; force3_kernel: "
+                        "2-body and 3-body slot forces with the centres' virials; step_collect_kernel: total forces and the "
+                        "sums of energies and virials",
         "active_slots": {"pairs_per_atom": pairs / N, "triplet_channel_items": items},
         "ms_per_frame": el / args.steps * 1e3,
     }
@@ -422,7 +422,9 @@ def profile_valu_share_md(kernel, workload):
     path = os.path.join(PROFILES, f"md_step_{workload}_sq_counters.txt")
     if not os.path.exists(path):
         raise ProfileMissing(f"{path} not found")
-    want = PROFILED_NAME[({"af3_kernel": "af3_fused", "force3_kernel": "force3_fused"}.get(kernel, kernel), "f64")]
+    want = PROFILED_NAME.get(({"af3_kernel": "af3_fused", "force3_kernel": "force3_fused"}.get(kernel, kernel), "f64"))
+    if want is None:
+        raise ProfileMissing(f"no profiled name of {kernel}")
     want = want.replace("staf::", "")
     num = den = 0.0
     for line in open(path):
