@@ -198,12 +198,11 @@ def test_forces_in_one_op_agree_with_the_two_force_ops(dtype, nr, na, counts, ow
     counts around a wave, an empty and a one-atom species, the descriptor op's map and a copy of it (a caller's map)."""
     import torch
     from alphanesgpu_amd import ops, synth
-    from perf.cases import _water
     dev, dt = torch.device("cuda:0"), getattr(torch, dtype)
-    pos, edge, _ = _water(dict(nx=4, ny=4, nz=2, frames=2), 3)
-    N = pos.shape[1]
+    frames = [synth.water_frame((4, 4, 2), 9.86, 0.05, seed) for seed in (3, 4)]
+    N = 96
     T = lambda a: torch.as_tensor(np.ascontiguousarray(a)).to(dev)
-    tpos, tbox = T(pos.reshape(2, -1)).to(dt), T(np.tile([edge[0], 0, 0, edge[1], 0, edge[2]], (2, 1))).to(dt)
+    tpos, tbox = (T(np.stack(a)).to(dt) for a in zip(*frames))
     tm, tp = T(np.repeat(np.arange(2, dtype=np.int32), counts)), T(np.array(counts, np.int32))
     ops.construct_descriptors_light(synth.RC, nr, na, N, tbox, synth.RS, synth.RA, 2, dtype=dt)
     rad, ang, sup, im2, im3, d2, d3, d3s, ntr = ops.compute_descriptors_light(tpos, tbox)

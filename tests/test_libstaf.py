@@ -275,15 +275,15 @@ def test_compute_with_injected_list_and_ghosts_matches_own_list():
 
 @pytest.mark.gpu
 def test_callers_list_after_own_list_after_callers_list():
-    """A handle that goes from the caller's list to its own and back keeps its neighbour map at one address, so the place
-    the library remembers that map in serves a transposed map, then a row of checksums, then a transposed map again:
-    the third call must find cleared build counters there.  Same bits as the first call; the own-list calls too."""
+    """A handle that goes from the caller's list to its own and back writes both neighbour maps to one place, and transposes
+    the caller's in a block whose counters every build must find cleared.  Same bits as the first call; the own-list calls
+    too."""
     from alphanesgpu_amd import libstaf
     pos, box, types = load_water_smoke(np.float64)
     pos = pos.reshape(-1, 3)
     n = len(pos)
     wrapped, allx, alltypes, _, howmany, neigh = _ghost_configuration(pos, box[0], types, RC)
-    m = libstaf.StafModel(os.path.join(GOLDEN, "model_double"), precision=1, full_virial=True, eager=True)
+    m = libstaf.StafModel(os.path.join(GOLDEN, "model_double"), precision=1, full_virial=True)
     theirs = lambda: m.compute(allx, box[0], alltypes, nlocal=n, howmany=howmany, neigh=neigh)
     ours = lambda: m.compute(wrapped, box[0], types)
     e0, f0, v0 = theirs()
@@ -342,30 +342,21 @@ def test_device_mlp_matches_host_mlp(prec, tol):
     host = libstaf.StafModel(os.path.join(GOLDEN, f"model_{prec}"), precision=p, full_virial=True, host_mlp=True)
     e0, f0, v0 = host.compute(pos, box[0], types)
     host.close()
-    # the kernel the library picks by itself, then each of its two device kernels (a handle of its own each: a
-    # handle replays what its first calls recorded)
-    for force in (None, "STAF_MLP_MATRIX", "STAF_MLP_VECTOR"):
-        if force:
-            os.environ[force] = "1"
-        try:
-            dev = libstaf.StafModel(os.path.join(GOLDEN, f"model_{prec}"), precision=p, full_virial=True)
-            e1, f1, v1 = dev.compute(pos, box[0], types)
-            dev.close()
-        finally:
-            if force:
-                os.environ.pop(force, None)
-        assert abs(e1 - e0) <= max(tol, 1e-6 if p == 0 else 0) * abs(e0), force
-        assert nerr(f1, f0) <= tol, force
-        assert nerr(v1, v0) <= tol, force
+    dev = libstaf.StafModel(os.path.join(GOLDEN, f"model_{prec}"), precision=p, full_virial=True)
+    e1, f1, v1 = dev.compute(pos, box[0], types)
+    dev.close()
+    assert abs(e1 - e0) <= max(tol, 1e-6 if p == 0 else 0) * abs(e0)
+    assert nerr(f1, f0) <= tol
+    assert nerr(v1, v0) <= tol
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec,tol", [("double", 1e-11), ("float", 2e-5)])
-def test_device_mlp_kernels_on_small_widths_and_ragged_atom_counts(tmp_path, prec, tol):
-    """Both device kernels of the network (the matrix-core one, 16 atoms per workgroup, and the vector one) against
-    the host evaluation on a written three-species model whose widths (fingerprints 9/7/11, hidden 20) are no
-    multiples of the tile sizes and whose atom counts (7, 9, 3) leave every workgroup partly empty: a wrong row
-    layout of the matrix tiles or a padding row entering a sum shows here, not on the 256/512-atom frames."""
+def test_device_mlp_on_small_widths_and_ragged_atom_counts(tmp_path, prec, tol):
+    """The network kernel (matrix cores, 16 atoms per workgroup) against the host evaluation on a written three-species
+    model whose widths (fingerprints 9/7/11, hidden 20) are no multiples of the tile sizes and whose atom counts
+    (7, 9, 3) leave every workgroup partly empty: a wrong row layout of the matrix tiles or a padding row entering a sum
+    shows here, not on the 256/512-atom frames."""
     from alphanesgpu_amd import libstaf, model_dir
     from test_oracle_pins import cluster, small_model
     ps = small_model(3, (5, 4, 6), (4, 3, 5, 3, 4, 3), seed=5, hidden=20, dense=True)
@@ -376,16 +367,11 @@ def test_device_mlp_kernels_on_small_widths_and_ragged_atom_counts(tmp_path, pre
     host = libstaf.StafModel(str(tmp_path), precision=p, full_virial=True, host_mlp=True)
     e0, f0, v0 = host.compute(pos.reshape(-1, 3), box[0], type_map)
     host.close()
-    for force in ("STAF_MLP_MATRIX", "STAF_MLP_VECTOR"):      # the library picks by size and precision otherwise
-        os.environ[force] = "1"
-        try:
-            dev = libstaf.StafModel(str(tmp_path), precision=p, full_virial=True)
-            e1, f1, v1 = dev.compute(pos.reshape(-1, 3), box[0], type_map)
-            dev.close()
-        finally:
-            os.environ.pop(force, None)
-        assert abs(e1 - e0) <= max(tol, 1e-6 if p == 0 else 0) * abs(e0), force
-        assert nerr(f1, f0) <= tol and nerr(v1, v0) <= tol, force
+    dev = libstaf.StafModel(str(tmp_path), precision=p, full_virial=True)
+    e1, f1, v1 = dev.compute(pos.reshape(-1, 3), box[0], type_map)
+    dev.close()
+    assert abs(e1 - e0) <= max(tol, 1e-6 if p == 0 else 0) * abs(e0)
+    assert nerr(f1, f0) <= tol and nerr(v1, v0) <= tol
 
 
 @pytest.mark.gpu
@@ -599,17 +585,16 @@ def test_neighbour_buffers_whose_slots_leave_no_room_for_both_bodies(tmp_path, c
 @pytest.mark.gpu
 @pytest.mark.parametrize("cells", [(4, 4, 2), (8, 7, 3), (8, 8, 4), (9, 8, 4)])
 def test_device_path_on_both_sides_of_the_workgroup_sizes_lines(cells):
-    """96, 504, 768 and 864 centres: wider workgroups for the fingerprints of up to 512 and the slot forces of up to 768.  Against the
-    op-by-op path the host network takes; float64, sums in another order, 1e-11."""
-    from alphanesgpu_amd import libstaf
-    from perf.cases import _water
-    x, edge, counts = _water(dict(nx=cells[0], ny=cells[1], nz=cells[2], frames=1), 11)
-    types = np.repeat(np.arange(2, dtype=np.int32), counts)
-    box = np.array([edge[0], 0.0, 0.0, edge[1], 0.0, edge[2]])
+    """96, 504, 768 and 864 centres: wider workgroups for the fingerprints of up to 512 and the slot forces of up to 768.
+    Against the op-by-op path the host network takes; float64, sums in another order, 1e-11."""
+    from alphanesgpu_amd import libstaf, synth
+    molecules = int(np.prod(cells))
+    x, box = synth.water_frame(cells, (29.9 * molecules) ** (1 / 3), 0.05, 11)
+    types = np.repeat(np.arange(2, dtype=np.int32), (molecules, 2 * molecules))
     out = []
     for host in (True, False):
         m = libstaf.StafModel(os.path.join(GOLDEN, "model_double"), precision=1, full_virial=True, host_mlp=host)
-        out.append(m.compute(x[0], box, types))
+        out.append(m.compute(x.reshape(-1, 3), box, types))
         m.close()
     (e0, f0, v0), (e1, f1, v1) = out
     assert abs(e1 - e0) <= 1e-11 * max(1.0, abs(e0)) and nerr(f1, f0) <= 1e-11 and nerr(v1, v0) <= 1e-11
@@ -629,48 +614,53 @@ def test_compute_without_virial_gives_the_same_energy_and_forces():
 
 
 @pytest.mark.gpu
-def test_replayed_calls_give_the_bits_of_eager_calls_and_follow_shape_changes():
-    """From the second call of a shape the library replays a recorded HIP graph.  A handle that replays and one that
-    launches eagerly walk through the same sequence of configurations -- the 768-atom frame moving from call to
-    call, then the water_smoke frame (other atom count and order), then the first one again, with and without
-    virial -- and must agree bit for bit on every call (all sums have a fixed order)."""
+def test_a_handle_that_follows_shape_changes_gives_the_bits_of_a_fresh_one():
+    """A handle walks through a sequence of configurations -- the 768-atom frame moving from call to call, then the
+    water_smoke frame (other atom count and order) with the library's list and with a caller's, then the first one again,
+    with and without virial -- and every call must agree bit for bit with the first call of a handle that has just been
+    loaded: what a handle holds between calls (blocks of an earlier size, the species it has sent, a list's transpose)
+    does not enter a result."""
     from alphanesgpu_amd import libstaf
     d = os.path.join(GOLDEN, "model_double")
     a = libstaf.StafModel(d, precision=1, full_virial=True)
-    b = libstaf.StafModel(d, precision=1, full_virial=True, eager=True)
     posA, boxA, _, tmA = load_frame_mbpol(np.float64)
     posB, boxB, typB = load_water_smoke(np.float64)
     rng = np.random.default_rng(17)
-    # (a shape is recorded after 2 calls in a row at first, after 4 and 8 once graphs have been dropped young: the
-    # runs below are long enough to be recorded and replayed each time)
-    plan = [("A", True)] * 4 + [("B", True)] * 3 + [("A", True)] * 7 + [("A", False)] * 10 + [("B", False)] * 2
-    first = {}
+    plan = ([("A", True)] * 2 + [("B", True)] * 2 + [("list", True)] * 2 + [("A", True)] + [("A", False)] * 2 +
+            [("list", False)] + [("B", False)] * 2 + [("list", True)] + [("A", True)])
     for step, (which, want_w) in enumerate(plan):
         pos, box, types = (posA, boxA[0], tmA) if which == "A" else (posB, boxB[0], typB)
         x = pos.reshape(-1, 3) + 0.02 * rng.standard_normal((pos.shape[1] // 3, 3))   # the atoms move every step
-        ea, fa, wa = a.compute(x, box, types, want_virial=want_w)
-        eb, fb, wb = b.compute(x, box, types, want_virial=want_w)
+        extra = {}
+        if which == "list":
+            n = len(x)
+            _, x, types, _, howmany, neigh = _ghost_configuration(x, box, types, RC)
+            extra = dict(nlocal=n, howmany=howmany, neigh=neigh)
+        elif step % 2:
+            flip = rng.permutation(len(x))       # (another order of the same species counts)
+            x, types = x[flip], np.asarray(types)[flip]
+        ea, fa, wa = a.compute(x, box, types, want_virial=want_w, **extra)
+        b = libstaf.StafModel(d, precision=1, full_virial=True)
+        eb, fb, wb = b.compute(x, box, types, want_virial=want_w, **extra)
+        b.close()
         assert ea == eb and np.array_equal(fa, fb), (step, which)
         assert (wa is None and wb is None) or np.array_equal(wa, wb), (step, which)
         assert np.isfinite(ea) and np.abs(fa).max() > 0
-        first.setdefault(which, ea)
         if step and plan[step - 1][0] == which:
-            assert ea != prev_e          # the inputs did change: a replay that re-used old inputs would show here
+            assert ea != prev_e          # the inputs did change: a call that re-used old inputs would show here
         prev_e = ea
     a.close()
-    b.close()
 
 
 @pytest.mark.gpu
-def test_release_of_the_ops_state_between_replayed_calls():
-    """staf_ops_release (the op interface's call that frees the library's work areas) while a handle of the MD entry
-    holds a recorded graph: the graph points into freed memory, so the handle drops it, evaluates eagerly and
-    records again -- same bits on every call."""
+def test_release_of_the_ops_state_between_calls():
+    """staf_ops_release (the op interface's call that frees the library's work areas) between calls of a handle of the MD
+    entry: the next call sizes the areas again -- same bits on every call."""
     from alphanesgpu_amd import libstaf, ops
     pos, box, _, type_map = load_frame_mbpol(np.float64)
     m = libstaf.StafModel(os.path.join(GOLDEN, "model_double"), precision=1, full_virial=True)
     x = pos.reshape(-1, 3)
-    ref = [m.compute(x, box[0], type_map) for _ in range(4)][-1]      # recorded and replayed by now
+    ref = [m.compute(x, box[0], type_map) for _ in range(4)][-1]
     for _ in range(2):
         ops.release()
         for _ in range(4):
@@ -681,8 +671,8 @@ def test_release_of_the_ops_state_between_replayed_calls():
 
 @pytest.mark.gpu
 def test_three_handles_on_three_host_threads():
-    """Three handles, each used by a host thread of its own at the same time (every handle records and replays its
-    own graph on its own streams): every call returns the bits a single handle returned for the same positions."""
+    """Three handles, each used by a host thread of its own at the same time (every handle has a stream of its own): every
+    call returns the bits a single handle returned for the same positions."""
     import threading
     from alphanesgpu_amd import libstaf
     pos, box, _, type_map = load_frame_mbpol(np.float64)
