@@ -146,10 +146,12 @@ __device__ inline T mlp_slope(int act, T y) {
   return act == 1 ? T(1) - y * y : relu;
 }
 
+// (Single precision is held to the eight waves per SIMD that 64 registers admit: with 70 and seven waves a launch of 24576
+// atoms takes 54.8 instead of 49.7 us.)
 // TA: atoms per workgroup, 16, or 8 for stacks whose rows of 16 do not fit the LDS -- an atom then holds two columns of the
 // tiles, whose lanes compute and store the same values.
 template <typename T, typename real, int TA>
-__global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs<T, real> A) {
+__global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void mlp_kernel(const MlpArgs<T, real> A) {
   using M = MlpTile<T>;
   using piece_t = typename M::piece_t;
   using acc_t = typename M::acc_t;
@@ -231,15 +233,15 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
 #pragma unroll
       for (int v = 0; v < 4; v++) y[v] += acc[v];
       mlp_act<T, 4>(act, y);
-      // (features beyond the last are 0 whatever their zero weights were multiplied with: an infinite value gives no number.  Asked
-      // of the last tile alone: as a select of every value this costs the single-precision kernel eight registers and, with
-      // the eighth wave per SIMD, 50.9 -> 56.5 us for 24576 atoms)
+      // (features beyond the last are 0 whatever their zero weights were multiplied with: an infinite value gives no number.
+      // Only a layer's last tile has such, and writes them again behind the others' values: as a select of every value
+      // this takes 2 % of the launch in double precision)
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int j = tile * 16 + M::row(lane, v);
-        if (tile * 16 + 16 > out_f && j >= out_f) y[v] = 0;
-        Y[j * TA + my] = y[v];
-      }
+      for (int v = 0; v < 4; v++) Y[(tile * 16 + M::row(lane, v)) * TA + my] = y[v];
+      if (tile * 16 + 16 > out_f)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          if (tile * 16 + M::row(lane, v) >= out_f) Y[(tile * 16 + M::row(lane, v)) * TA + my] = 0;
     }
     if (l + 2 < nl) {
       if (wave < mlp_tiles(net.out_f[l + 1])) request(net.fw[l + 1], wave, mlp_pieces<T>(out_f));
@@ -315,12 +317,13 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE) void mlp_kernel(const MlpArgs
       const acc_t acc = product(net.bw[l], tile, np, D);
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        if (l > 0) {
-          T d = acc[v] * mlp_slope<T>(act, other[v]);
-          if (tile * 16 + 16 > in_f && tile * 16 + M::row(lane, v) >= in_f) d = 0;
-          at[M::row(lane, v) * TA] = d;
-        } else put(tile * 16 + M::row(lane, v), acc[v], other[v]);
+        if (l > 0) at[M::row(lane, v) * TA] = acc[v] * mlp_slope<T>(act, other[v]);
+        else put(tile * 16 + M::row(lane, v), acc[v], other[v]);
       }
+      if (l > 0 && tile * 16 + 16 > in_f)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          if (tile * 16 + M::row(lane, v) >= in_f) at[M::row(lane, v) * TA] = 0;
     }
     if (l > 0) {
       if (wave < mlp_tiles(net.in_f[l - 1])) request(net.bw[l - 1], wave, mlp_pieces<T>(in_f));
