@@ -98,11 +98,22 @@ template <int CTRL, int ROW_MASK>
 __device__ inline unsigned dpp_get(unsigned v) {
   return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xf, false);
 }
-template <int CTRL, int ROW_MASK>
-__device__ inline double dpp_get(double v) {
+// Doubles move in two halves.  The hardware writes the 0 itself for a lane without a source (bound_ctrl) as long as every
+// row takes part; a result that starts as a register holding 0 costs two more moves per value.
+template <int CTRL>
+__device__ inline double dpp_row(double v) {
   const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, ROW_MASK, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROW_MASK, 0xf, false);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+// The same with rows that take no part: they keep `keep`, which holds 0 there.  The result serves as `keep` of the next
+// value, so that a sequence of moves needs one pair of zeroes.
+template <int CTRL, int ROW_MASK>
+__device__ inline double dpp_rows(double keep, double v) {
+  const long long b = __double_as_longlong(v), k = __double_as_longlong(keep);
+  const int lo = __builtin_amdgcn_update_dpp((int)(k & 0xffffffffll), (int)(b & 0xffffffffll), CTRL, ROW_MASK, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(k >> 32), (int)(b >> 32), CTRL, ROW_MASK, 0xf, false);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 // The two steps that carry a prefix across the rows of 16 lanes: s += (lane 15 of the row before) in rows 1 and 3,
@@ -141,25 +152,74 @@ __device__ inline void dpp_rows_carry(unsigned& a) {
       : "+v"(a));
 }
 __device__ inline void dpp_rows_carry(double& s) {
-  s += dpp_get<0x142, 0xa>(s);   // lane 15 of a row -> every lane of the next row (rows 1 and 3 take it)
-  s += dpp_get<0x143, 0xc>(s);   // lane 31 -> rows 2 and 3
+  s += dpp_rows<0x142, 0xa>(0.0, s);   // lane 15 of a row -> every lane of the next row (rows 1 and 3 take it)
+  s += dpp_rows<0x143, 0xc>(0.0, s);   // lane 31 -> rows 2 and 3
 }
-__device__ inline void dpp_rows_carry(double& a, double& b, double& c, double& d) {
-  a += dpp_get<0x142, 0xa>(a); b += dpp_get<0x142, 0xa>(b); c += dpp_get<0x142, 0xa>(c); d += dpp_get<0x142, 0xa>(d);
-  a += dpp_get<0x143, 0xc>(a); b += dpp_get<0x143, 0xc>(b); c += dpp_get<0x143, 0xc>(c); d += dpp_get<0x143, 0xc>(d);
+// several values, step by step: the moves of one fill the wait states of the others
+template <int N>
+__device__ inline void dpp_rows_carry(double (&s)[N]) {
+  double t = 0;
+#pragma unroll
+  for (int c = 0; c < N; c++) { t = dpp_rows<0x142, 0xa>(t, s[c]); s[c] += t; }
+  t = 0;
+#pragma unroll
+  for (int c = 0; c < N; c++) { t = dpp_rows<0x143, 0xc>(t, s[c]); s[c] += t; }
 }
 
-// Sum over the 64 lanes with register-to-register lane moves only; the total is valid in lane 63 alone.
-// Fixed tree: prefix steps 1,2,3,4,8 inside each row of 16, then row 0->1, 2->3, and rows 0-1 -> 2-3.
+// Inclusive prefix sums over the 64 lanes with register-to-register lane moves only, of N values at once: inside each
+// row of 16, then row 0->1, 2->3, and rows 0-1 -> 2-3.  Single precision: prefix steps 1, 2, 3 of the value itself, then 4
+// and 8 of the sum (an add takes its move along, and this is the shorter chain); double precision: 1, 2, 4 and 8 of the sum
+// (a step is two moves and an add).
+template <int N>
+__device__ inline void wave_scan(float (&v)[N]) {
+  float s[N];
+#pragma unroll
+  for (int c = 0; c < N; c++) s[c] = v[c] + dpp_get<0x111, 0xf>(v[c]);
+#pragma unroll
+  for (int c = 0; c < N; c++) s[c] += dpp_get<0x112, 0xf>(v[c]);
+#pragma unroll
+  for (int c = 0; c < N; c++) s[c] += dpp_get<0x113, 0xf>(v[c]);
+#pragma unroll
+  for (int c = 0; c < N; c++) s[c] += dpp_get<0x114, 0xf>(s[c]);
+#pragma unroll
+  for (int c = 0; c < N; c++) s[c] += dpp_get<0x118, 0xf>(s[c]);
+  if constexpr (N == 4) {
+    dpp_rows_carry(s[0], s[1], s[2], s[3]);
+  } else {
+#pragma unroll
+    for (int c = 0; c < N; c++) dpp_rows_carry(s[c]);
+  }
+#pragma unroll
+  for (int c = 0; c < N; c++) v[c] = s[c];
+}
+template <int N>
+__device__ inline void wave_scan(double (&s)[N]) {
+#pragma unroll
+  for (int c = 0; c < N; c++) s[c] += dpp_row<0x111>(s[c]);
+#pragma unroll
+  for (int c = 0; c < N; c++) s[c] += dpp_row<0x112>(s[c]);
+#pragma unroll
+  for (int c = 0; c < N; c++) s[c] += dpp_row<0x114>(s[c]);
+#pragma unroll
+  for (int c = 0; c < N; c++) s[c] += dpp_row<0x118>(s[c]);
+  dpp_rows_carry(s);
+}
+// Sum over the 64 lanes by the same steps; the total is valid in lane 63 alone.
 template <typename T>
 __device__ inline T wave_sum_to_last(T v) {
-  T s = v + dpp_get<0x111, 0xf>(v);
-  s += dpp_get<0x112, 0xf>(v);
-  s += dpp_get<0x113, 0xf>(v);
-  s += dpp_get<0x114, 0xf>(s);
-  s += dpp_get<0x118, 0xf>(s);
-  dpp_rows_carry(s);
-  return s;
+  if constexpr (sizeof(T) == 8) {
+    double s[1] = {v};
+    wave_scan(s);
+    return s[0];
+  } else {
+    T s = v + dpp_get<0x111, 0xf>(v);
+    s += dpp_get<0x112, 0xf>(v);
+    s += dpp_get<0x113, 0xf>(v);
+    s += dpp_get<0x114, 0xf>(s);
+    s += dpp_get<0x118, 0xf>(s);
+    dpp_rows_carry(s);
+    return s;
+  }
 }
 // Wave-uniform value loaded through a vector path (e.g. from LDS) moved to a scalar register, so that loop
 // bounds and addresses derived from it stay scalar.

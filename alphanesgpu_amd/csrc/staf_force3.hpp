@@ -36,27 +36,6 @@
 
 namespace staf {
 
-// register-to-register inclusive prefix sums over the 64 lanes of four values at once (same tree as
-// wave_sum_to_last; the four chains are interleaved step by step, so that the wait states a lane move needs after
-// the instruction that wrote its source are filled by the other chains)
-template <typename T>
-__device__ inline void wave_scan4(T (&v)[4]) {
-  T s[4];
-#pragma unroll
-  for (int c = 0; c < 4; c++) s[c] = v[c] + dpp_get<0x111, 0xf>(v[c]);
-#pragma unroll
-  for (int c = 0; c < 4; c++) s[c] += dpp_get<0x112, 0xf>(v[c]);
-#pragma unroll
-  for (int c = 0; c < 4; c++) s[c] += dpp_get<0x113, 0xf>(v[c]);
-#pragma unroll
-  for (int c = 0; c < 4; c++) s[c] += dpp_get<0x114, 0xf>(s[c]);
-#pragma unroll
-  for (int c = 0; c < 4; c++) s[c] += dpp_get<0x118, 0xf>(s[c]);
-  dpp_rows_carry(s[0], s[1], s[2], s[3]);
-#pragma unroll
-  for (int c = 0; c < 4; c++) v[c] = s[c];
-}
-
 // NW_: waves per workgroup, 4 or 8 (step_forces takes 8 for few centres; for the others see force_tripl).  A sweep takes 16 passes of 64 triplets
 // either way; with eight waves a wave holds two of them, so that a centre's critical path and a wave's registers
 // are about half of what they are with four.
@@ -595,7 +574,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
       }
       // slot j: the lanes of a row are contiguous.  Row sum = prefix at the row's last lane minus prefix
       // before its first lane of this pass (taken with a lane read: no memory is involved).
-      wave_scan4(vj);
+      wave_scan(vj);
       const int first = lane - (k - j - 1);   // lane of the row's first triplet (not positive: starts earlier)
       const int before = first > 0 ? first - 1 : 0;   // lanes past the last triplet hold j = k = 0: their own lane
       real pre[4];
@@ -658,11 +637,11 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
         for (int c = 0; c < 3; c++) f3[c] += w * B2.dD[rowAtom * 3 * nr + c * nr + tid];
       }
     }
+    real tot[3] = {f3[0], f3[1], f3[2]};
+    wave_scan(tot);
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-      const real t = wave_sum_to_last(f3[c]);
-      if (lane == WAVE - 1) xch[wave * 4 + c] = t;
-    }
+    for (int c = 0; c < 3; c++)
+      if (lane == WAVE - 1) xch[wave * 4 + c] = tot[c];
     if constexpr (VIR) {
       // virial of the slot forces, - sum_s f_s (x) (r_centre - r_s): the separations are the unit vectors times r
       // (nine sums in a wave that has its operands, 2-3 us of launches per 6144 atoms less than a pass over the
@@ -672,11 +651,11 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
 #pragma unroll
         for (int e = 0; e < 3; e++) {
           const real re = tid < cnt2 ? -(r * sU[e * nr + tid]) : real(0);
+          real w[3] = {f3[0] * re, f3[1] * re, f3[2] * re};
+          wave_scan(w);
 #pragma unroll
-          for (int c = 0; c < 3; c++) {
-            const real t = wave_sum_to_last(f3[c] * re);
-            if (lane == WAVE - 1) xv[wave * 9 + c * 3 + e] = t;
-          }
+          for (int c = 0; c < 3; c++)
+            if (lane == WAVE - 1) xv[wave * 9 + c * 3 + e] = w[c];
         }
       }
     }
