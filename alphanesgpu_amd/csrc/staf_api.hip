@@ -48,27 +48,54 @@ struct DevBuf {
 };
 
 // Pinned host staging (allocated pinned, never registered): one block for everything a call sends, one for what it
-// brings back, so that a call makes one copy each way.
+// brings back.  Kernels copy them (call_in_kernel, call_out_kernel).
 template <typename T>
 struct PinBuf {
   T* p = nullptr;
+  T* dev = nullptr;   // the block as the device sees it
   size_t n = 0;
   bool reserve(size_t want) {
     if (want <= n) return true;
-    if (p) (void)hipHostFree(p);
-    p = nullptr;
-    n = 0;
+    release();
     want += want / 4;
-    if (hipHostMalloc((void**)&p, want * sizeof(T), hipHostMallocDefault) != hipSuccess) return false;
+    if (hipHostMalloc((void**)&p, want * sizeof(T), hipHostMallocDefault) != hipSuccess) {
+      p = nullptr;
+      return false;
+    }
+    if (hipHostGetDevicePointer((void**)&dev, p, 0) != hipSuccess) {
+      release();
+      return false;
+    }
     n = want;
     return true;
   }
   void release() {
     if (p) (void)hipHostFree(p);
-    p = nullptr;
+    p = dev = nullptr;
     n = 0;
   }
 };
+
+// A call's input block from the pinned host memory, and its results back.  Bound by latency: three copies by the runtime
+// (input; results; error words) and the wait for the stream took 40 us of a 768-atom call and 44 of a 6144-atom one around
+// an otherwise empty chain of kernels, the two kernels and flags that the host watches 19 and 24 (24576 atoms: 60 and 43).
+// MD calls of 96, 768, 6144 and 24576 atoms: 90 -> 82, 136 -> 107, 417 -> 387 and 1340 -> 1313 us; with a caller's list,
+// 1500 and 6144 atoms: 223 -> 213 and 553 -> 529.
+constexpr int IO_THREADS = 256, IN_BLOCKS = 256, OUT_BLOCKS = 64;
+__global__ __launch_bounds__(IO_THREADS) void call_in_kernel(const double2* __restrict__ host, double2* __restrict__ dev, int n) {
+  for (int i = blockIdx.x * IO_THREADS + threadIdx.x; i < n; i += gridDim.x * IO_THREADS) dev[i] = host[i];
+}
+// The error words go along.  A workgroup's flag says that everything it copied has arrived: its threads' stores are released
+// to the host before the flag is written.
+__global__ __launch_bounds__(IO_THREADS) void call_out_kernel(const double2* __restrict__ dev, double2* __restrict__ host, int n,
+                                                              int* status, int* status_h, unsigned* flags, unsigned call) {
+  for (int i = blockIdx.x * IO_THREADS + threadIdx.x; i < n; i += gridDim.x * IO_THREADS) host[i] = dev[i];
+  if (blockIdx.x == 0 && threadIdx.x < staf::STATUS_WORDS)
+    status_h[threadIdx.x] = __hip_atomic_load(&status[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(&flags[blockIdx.x], call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 __global__ void add_into_kernel(double* dst, const double* src, int n) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
@@ -126,6 +153,8 @@ struct StafModel {
   // out_d = [force nall*3 | rows of (virial 9, energy), sums over shares of the centres]  (mirror of out_h, one copy)
   DevBuf<double> in_d, out_d, force_op, virial_op, af2, af3, g2, g3, e_atom, vpart;
   PinBuf<double> in_h, out_h;
+  PinBuf<unsigned> done_h;   // [OUT_BLOCKS flags of call_out_kernel | error words]
+  unsigned calls = 0;
   std::vector<int> type_map_up, tipos_up;   // what the device copies of type_map and tipos hold
   bool actual_type_up = false;
   // device-resident MLP (default); false: the host evaluation of staf_mlp.cpp between the kernels
@@ -232,6 +261,7 @@ void staf_free(StafModel* m) {
     for (auto& b : *v) b.release();
   m->in_h.release();
   m->out_h.release();
+  m->done_h.release();
   for (DevBuf<double>* b : {&m->in_d, &m->out_d, &m->force_op, &m->virial_op, &m->af2, &m->af3, &m->g2, &m->g3,
                             &m->e_atom, &m->vpart, &m->raddescr, &m->des3bsupp, &m->der2b, &m->der3bsupp, &m->unit,
                             &m->slotf, &m->selff})
@@ -360,10 +390,14 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   if (ext)
     for (int i = 0; i < nlocal; i++) pitch = std::max(pitch, std::min(howmany[i], row_max));
   const size_t n_in_i = ext ? 2 * L + nall + L * pitch : 0;                   // ints behind them
-  const size_t n_in = n_in_d + (n_in_i + 1) / 2;
+  const size_t n_in = (n_in_d + (n_in_i + 1) / 2 + 1) & ~(size_t)1;           // (copied by twos)
   const int nparts = std::min(64, (nlocal + 255) / 256);   // shares of the centres' virial and energy sums
-  const size_t n_out = (size_t)nall * 3 + (size_t)nparts * 10;
+  const size_t n_out = ((size_t)nall * 3 + (size_t)nparts * 10 + 1) & ~(size_t)1;
   if (!m->in_h.reserve(n_in) || !m->out_h.reserve(n_out)) return -1;
+  if (!m->done_h.p) {
+    if (!m->done_h.reserve(OUT_BLOCKS + staf::STATUS_WORDS)) return -1;
+    memset(m->done_h.p, 0, (OUT_BLOCKS + staf::STATUS_WORDS) * sizeof(unsigned));
+  }
   double* pos_h = m->in_h.p;
   int* how_h = (int*)(m->in_h.p + n_in_d);
   int* slot_of_h = how_h + L;
@@ -435,7 +469,12 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   const staf::NeighList list = {d_how, d_how + L + nall + L, d_how + L + nall, d_how + L, pitch};
   double* const d_force = m->out_d.p;
   double* const d_parts = d_force + (size_t)nall * 3;
-  STAF_HIP_OK(hipMemcpyAsync(m->in_d.p, m->in_h.p, n_in * sizeof(double), hipMemcpyHostToDevice, st));
+  {
+    const int n = (int)(n_in / 2);
+    hipLaunchKernelGGL(call_in_kernel, dim3(std::min(IN_BLOCKS, (n + IO_THREADS - 1) / IO_THREADS)), dim3(IO_THREADS), 0, st,
+                       (const double2*)m->in_h.dev, (double2*)m->in_d.p, n);
+    STAF_HIP_OK(hipGetLastError());
+  }
   // species of the slots and atoms per species: sent when they differ from what the device holds (in MD they change
   // when atoms migrate, not every step); the blocking copies read host vectors that the next lines may replace
   if (m->type_map_up != m->type_map_h) {
@@ -637,12 +676,40 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
       }
     }
   }
-  // forces, and on the device path the virial and energy sums behind them, in one copy
-  const size_t n_back = m->dev_mlp ? n_out : (size_t)n3;
-  STAF_HIP_OK(hipMemcpyAsync(m->out_h.p, m->out_d.p, n_back * sizeof(double), hipMemcpyDeviceToHost, st));
+  // forces, on the device path the virial and energy sums behind them, and the error words
+  staf::DeviceState* const state = staf::device_state(st);
+  if (!state) return gpu_failure(__LINE__, 0);
+  const unsigned call = ++m->calls ? m->calls : ++m->calls;   // (never what the flags start with)
+  unsigned* const flags = m->done_h.p;
+  int* const status_h = (int*)(m->done_h.p + OUT_BLOCKS);
+  int out_blocks = 0;
+  {
+    const int n = (int)(((m->dev_mlp ? n_out : (size_t)n3) + 1) / 2);
+    out_blocks = std::min(OUT_BLOCKS, (n + IO_THREADS - 1) / IO_THREADS);
+    hipLaunchKernelGGL(call_out_kernel, dim3(out_blocks), dim3(IO_THREADS), 0, st, (const double2*)m->out_d.p,
+                       (double2*)m->out_h.dev, n, state->status_d, (int*)(m->done_h.dev + OUT_BLOCKS), m->done_h.dev, call);
+    STAF_HIP_OK(hipGetLastError());
+  }
   const double* force_h = m->out_h.p;
-  // the call's synchronisation: results are on the host, and so is what the kernels reported
-  rc = staf_ops_poll_status(st);
+  // the call's synchronisation: results are on the host, and so is what the kernels reported.  The stream is asked now and
+  // then, and ends the wait where a kernel failed.
+  for (unsigned round = 1; ; round++) {
+    int b = 0;
+    while (b < out_blocks && __atomic_load_n(&flags[b], __ATOMIC_ACQUIRE) == call) b++;
+    if (b == out_blocks) break;
+    if (round % 8192 == 0) {
+      const hipError_t e = hipStreamQuery(st);
+      if (e == hipErrorNotReady) continue;
+      if (e != hipSuccess) return gpu_failure(__LINE__, (int)e);
+      for (b = 0; b < out_blocks; b++)
+        if (__atomic_load_n(&flags[b], __ATOMIC_ACQUIRE) != call) return gpu_failure(__LINE__, b);
+      break;
+    }
+    __builtin_ia32_pause();
+  }
+  bool reported = false;
+  for (int w = 0; w < staf::STATUS_WORDS; w++) reported = reported || status_h[w] != 0;
+  rc = reported ? staf_ops_poll_status(st) : STAF_OK;   // (reads the words again, and clears what it has read)
   if (rc == STAF_E_RADIAL_OVERFLOW) return -10;
   if (rc == STAF_E_SCATTER_OVERFLOW) return -11;
   if (rc != STAF_OK) return gpu_failure(__LINE__, rc);

@@ -821,3 +821,38 @@ def test_c_caller_reproduces_recorded_energy():
     assert abs(e[1] - e[0]) < 1e-5 * abs(e[0]) and abs(rms[1] - rms[0]) < 2e-5
     vir = [float(x) for x in lines[0][9:15]]
     assert vir[3] == vir[4] == vir[5] == 0.0 and all(v != 0.0 for v in vir[:3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 3, 170, 171, 10922, 10925])
+def test_every_atom_of_a_call_arrives_and_returns(n):
+    """Input and results are copied by kernels in pieces of two doubles, 256 to a workgroup and 64 workgroups to a round of
+    results: pairs of atoms in a row, each the same to the last bit (offsets are whole numbers, box edges a power of two), have
+    the first pair's forces to the last bit wherever they lie in the blocks, and the energies add up (n 2^-53 of the sum of n
+    equal terms)."""
+    from alphanesgpu_amd import libstaf
+    model = libstaf.StafModel(os.path.join(GOLDEN, "model_double"), precision=1)
+    x = np.zeros((n, 3))
+    x[:, 0] = 16.0 * (np.arange(n) // 2) + 2.5 * (np.arange(n) % 2)
+    howmany = np.array([min(1, n - 1 - i) if i % 2 == 0 else 1 for i in range(n)], np.int32)
+    neigh = (np.arange(n) ^ 1).reshape(-1, 1).astype(np.int32)
+    neigh[howmany == 0] = 0
+    types = (np.arange(n) % 2).astype(np.int32)
+    box = 2.0 ** 20 * np.array([1.0, 0.0, 0.0, 1.0, 0.0, 1.0])   # (a power of two: fractions of it are exact)
+    for _ in range(2):
+        e, f, _ = model.compute(x, box, types, nlocal=n, howmany=howmany, neigh=neigh)
+        pairs = n // 2
+        if pairs:
+            e2, f2, _ = model.compute(x[:2], box, types[:2], nlocal=2, howmany=howmany[:2], neigh=neigh[:2])
+            assert np.abs(f2).max() > 0
+            assert np.array_equal(f[:2 * pairs], np.tile(f[:2], (pairs, 1)))
+            assert np.abs(f[:2] - f2).max() <= 1e-13 * np.abs(f2).max()   # (other workgroup sizes: sums of 140 terms in another order)
+        else:
+            e2 = 0.0
+        e1 = 0.0
+        if n % 2:
+            e1, f1, _ = model.compute(x[:1], box, types[:1], nlocal=1, howmany=np.zeros(1, np.int32), neigh=np.zeros((1, 1), np.int32))
+            assert np.array_equal(f[-1:], f1) and np.abs(f1).max() == 0
+        want = pairs * e2 + e1
+        assert abs(e - want) <= (n + 2) * 2.0 ** -53 * (pairs * abs(e2) + abs(e1)) * 4
+    model.close()
