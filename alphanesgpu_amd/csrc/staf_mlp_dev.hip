@@ -5,9 +5,9 @@
 // libstaf/src/mlp/staf_mlp_ort.cc:186-233).
 //
 // The Dense layers are small matrix products ([out, in] x [in, atoms]) and run on the matrix cores: a workgroup takes
-// 16 atoms, which are the columns of its 16x16x4 tiles, and a wave takes tiles of 16 output features over the whole
+// 16 atoms, which are the columns of its 16x16x4 tiles (8 or 4 in launches of few atoms: columns of 4x4 tiles), and a wave takes tiles of 16 output features over the whole
 // inner dimension, so that no partial sums meet in LDS and a layer costs one barrier per direction.  Activations lie in
-// LDS as [feature][16 atoms] (8 atoms for stacks with more features than fit that way): a tile step's read and the
+// LDS as [feature][16 atoms] (8 atoms also for stacks with more features than fit that way): a tile step's read and the
 // result's write are runs of consecutive words.  A layer's delta takes the place of its activations (the derivative needs
 // nothing else), and the input the place of the second hidden layer: 39 KB for the reference's stack in double
 // precision, four workgroups per CU.  The weights are kept in
@@ -15,7 +15,8 @@
 // wave requests the first pieces of its next product ahead of the barrier it waits at and stays six pieces ahead.
 // Bound: matrix cores and vector units in turn (16384 atoms in double precision: 25 us of matrix instructions, 16 us of
 // activations and the rest, 60 us measured; 150 us before, when the inner dimension was sliced over sixteen waves and
-// weights were read row by row), and for a single workgroup the chain of four products (22 us; 25 before).  Asking for
+// weights were read row by row), and for a single workgroup the chain of four products (22 us, with four atoms 14; 25 before
+// either).  Asking for
 // the weights' lines ahead of everything, and more than six pieces in flight, are slower.
 #include "staf_mlp_dev.hpp"
 
@@ -29,18 +30,80 @@ constexpr int MLP_WAVES_MAX = 16;
 
 template <typename T> struct MlpTile;
 // operand layout of the 16x16x4 tiles: A[row = lane % 16][k = lane / 16], B[k = lane / 16][col = lane % 16];
-// accumulator element v of a lane: col = lane % 16, row = row(lane, v) (the two precisions differ)
+// accumulator element v of a lane: (row(lane, v), col(lane, v)) (the two precisions differ); NV elements
 template <> struct MlpTile<double> {
   typedef double acc_t __attribute__((ext_vector_type(4)));
   typedef double piece_t __attribute__((ext_vector_type(2)));
-  __device__ static acc_t run(double a, double b, acc_t c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+  static constexpr int NV = 4;
+  __device__ static acc_t run(double a, const double* X, acc_t c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, *X, c, 0, 0, 0); }
   __device__ static int row(int lane, int v) { return lane / 16 + 4 * v; }
+  __device__ static void values(const acc_t& c, int, double (&y)[NV]) {
+#pragma unroll
+    for (int v = 0; v < NV; v++) y[v] = c[v];
+  }
+  __device__ static int col(int lane, int) { return lane & 15; }
 };
 template <> struct MlpTile<float> {
   typedef float acc_t __attribute__((ext_vector_type(4)));
   typedef float piece_t __attribute__((ext_vector_type(4)));
-  __device__ static acc_t run(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+  static constexpr int NV = 4;
+  __device__ static acc_t run(float a, const float* X, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, *X, c, 0, 0, 0); }
+  __device__ static void values(const acc_t& c, int, float (&y)[NV]) {
+#pragma unroll
+    for (int v = 0; v < NV; v++) y[v] = c[v];
+  }
   __device__ static int row(int lane, int v) { return 4 * (lane / 16) + v; }
+  __device__ static int col(int lane, int) { return lane & 15; }
+};
+
+// Workgroups of few atoms: four atoms to a tile, TA / 4 tiles beside each other, with the large tiles' operands: A[feature
+// 4 b + i][k] and B[k][atom j] in lane 16 k + 4 b + (i or j).  Double precision: 4x4x4 tiles in four blocks b, element
+// (feature 4 b + i, atom j) in lane 16 i + 4 b + j.  Single precision: 4x4x1 tiles in sixteen blocks, a block for every (k,
+// b): the four k of an element are added at the end, and the lane of k keeps element i = k, as in double precision.  The
+// matrix cores do four atoms at the rate of sixteen (measured 17 cycles an instruction, 66 for the large tile's four times
+// the work; single precision 10 to 12 and 32).
+template <typename T, int TILES> struct MlpTiles4;
+template <int TILES>
+struct MlpTiles4<double, TILES> {
+  struct acc_t { double v[TILES]; };
+  typedef double piece_t __attribute__((ext_vector_type(2)));
+  static constexpr int NV = TILES;
+  __device__ static acc_t run(double a, const double* X, acc_t c) {
+#pragma unroll
+    for (int t = 0; t < TILES; t++) c.v[t] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, X[4 * t], c.v[t], 0, 0, 0);
+    return c;
+  }
+  __device__ static void values(const acc_t& c, int, double (&y)[NV]) {
+#pragma unroll
+    for (int t = 0; t < TILES; t++) y[t] = c.v[t];
+  }
+  __device__ static int row(int lane, int) { return (lane & 12) + lane / 16; }
+  __device__ static int col(int lane, int v) { return 4 * v + (lane & 3); }
+};
+template <int TILES>
+struct MlpTiles4<float, TILES> {
+  typedef float four __attribute__((ext_vector_type(4)));
+  struct acc_t { four v[TILES]; };
+  typedef four piece_t;
+  static constexpr int NV = TILES;
+  __device__ static acc_t run(float a, const float* X, acc_t c) {
+#pragma unroll
+    for (int t = 0; t < TILES; t++) c.v[t] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, X[4 * t], c.v[t], 0, 0, 0);
+    return c;
+  }
+  __device__ static void values(const acc_t& c, int lane, float (&y)[NV]) {
+    const bool hi2 = lane & 32, hi1 = lane & 16;
+#pragma unroll
+    for (int t = 0; t < TILES; t++) {
+      // each half of the lanes keeps two elements and hands the other two on, then each quarter one
+      const four& e = c.v[t];
+      const float p = (hi2 ? e[2] : e[0]) + __shfl_xor(hi2 ? e[0] : e[2], 32, WAVE);
+      const float q = (hi2 ? e[3] : e[1]) + __shfl_xor(hi2 ? e[1] : e[3], 32, WAVE);
+      y[t] = (hi1 ? q : p) + __shfl_xor(hi1 ? p : q, 16, WAVE);
+    }
+  }
+  __device__ static int row(int lane, int) { return (lane & 12) + lane / 16; }
+  __device__ static int col(int lane, int v) { return 4 * v + (lane & 3); }
 };
 
 template <typename T> __host__ __device__ constexpr int mlp_steps() { return 16 / (int)sizeof(T); }   // tile steps per piece
@@ -146,16 +209,16 @@ __device__ inline T mlp_slope(int act, T y) {
   return act == 1 ? T(1) - y * y : relu;
 }
 
-// (Single precision is held to the eight waves per SIMD that 64 registers admit: with 70 and seven waves a launch of 24576
-// atoms takes 54.8 instead of 49.7 us.)
-// TA: atoms per workgroup, 16, or 8 for stacks whose rows of 16 do not fit the LDS -- an atom then holds two columns of the
-// tiles, whose lanes compute and store the same values.
+// (Single precision with 16 atoms is held to the eight waves per SIMD that 64 registers admit: with 70 and seven waves a launch
+// of 24576 atoms takes 54.8 instead of 49.7 us.  With 8 atoms it would spill there.)
+// TA: atoms per workgroup, 16, 8 or 4 (mlp_atoms).
 template <typename T, typename real, int TA>
-__global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void mlp_kernel(const MlpArgs<T, real> A) {
-  using M = MlpTile<T>;
+__global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? (TA == 16 ? 8 : 5) : 4) void mlp_kernel(const MlpArgs<T, real> A) {
+  static_assert(TA == 4 || TA == 8 || TA == 16, "columns of the tiles");
+  using M = std::conditional_t<(TA < 16), MlpTiles4<T, TA / 4>, MlpTile<T>>;
   using piece_t = typename M::piece_t;
   using acc_t = typename M::acc_t;
-  constexpr int STEPS = mlp_steps<T>();
+  constexpr int STEPS = mlp_steps<T>(), NV = M::NV;
   extern __shared__ __align__(16) unsigned char smem[];
   // [rows of the hidden layers][TA atoms], then the parts of the energy sums; the input lies where the second hidden
   // layer will
@@ -167,9 +230,10 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void 
   const MlpNet<T>& net = A.net[s];
   const int a0 = ((int)blockIdx.x - S.first) * TA;
   const int nl = net.nl, n_af = net.n_af;
-  const int my = lane & (TA - 1);                              // the lane's atom in a tile
+  const int my = lane & (TA - 1);                              // the lane's atom outside the products
   const bool live = a0 + my < S.Nl;
   const size_t atom = (size_t)(live ? a0 + my : S.Nl - 1);     // (lanes without an atom follow the last one, storing nothing)
+  auto col = [&](int v) -> int { return M::col(lane, v); };   // atom of a product's value v
 
   // The pieces requested ahead may lie beyond the tile's last one: in the next tile or, behind the last matrix, in the
   // spare pieces at the end of the block; they are not used.
@@ -180,11 +244,11 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void 
 #pragma unroll
     for (int u = 0; u < MLP_AHEAD; u++) ring[u] = f[u * WAVE];
   };
-  auto product = [&](const T* frag, int tile, int np, const T* X) -> acc_t {
+  auto product = [&](const T* frag, int tile, int np, const T* X, T (&out)[NV]) {
     const piece_t* f = (const piece_t*)frag + (size_t)tile * np * WAVE + lane;
-    acc_t acc = {0, 0, 0, 0};
+    acc_t acc = {};
     const int whole = np / MLP_AHEAD, rest = np - whole * MLP_AHEAD;
-    X += (lane / 16) * TA + my;
+    X += (lane / 16) * TA + col(0);
     for (int g = 0; g < whole; g++) {
       f += MLP_AHEAD * WAVE;
 #pragma unroll
@@ -192,7 +256,7 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void 
         const piece_t w = ring[u];
         ring[u] = f[u * WAVE];
 #pragma unroll
-        for (int j = 0; j < STEPS; j++) acc = M::run(w[j], X[(u * STEPS + j) * 4 * TA], acc);
+        for (int j = 0; j < STEPS; j++) acc = M::run(w[j], X + (u * STEPS + j) * 4 * TA, acc);
       }
       X += MLP_AHEAD * STEPS * 4 * TA;
     }
@@ -200,9 +264,9 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void 
     for (int u = 0; u + 1 < MLP_AHEAD; u++) {
       if (u >= rest) break;
 #pragma unroll
-      for (int j = 0; j < STEPS; j++) acc = M::run(ring[u][j], X[(u * STEPS + j) * 4 * TA], acc);
+      for (int j = 0; j < STEPS; j++) acc = M::run(ring[u][j], X + (u * STEPS + j) * 4 * TA, acc);
     }
-    return acc;
+    M::values(acc, lane, out);
   };
 
   const int np0 = mlp_pieces<T>(n_af);
@@ -226,22 +290,23 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void 
     T* Y = l == 0 ? H : X + mlp_rows(in_f) * TA;
     for (int tile = wave; tile < tiles; tile += nw) {
       if (tile != wave) request(net.fw[l], tile, np);
-      T y[4];
+      T y[NV];
 #pragma unroll
-      for (int v = 0; v < 4; v++) y[v] = net.b[l][tile * 16 + M::row(lane, v)];
-      const acc_t acc = product(net.fw[l], tile, np, X);
+      for (int v = 0; v < NV; v++) y[v] = net.b[l][tile * 16 + M::row(lane, v)];
+      T acc[NV];
+      product(net.fw[l], tile, np, X, acc);
 #pragma unroll
-      for (int v = 0; v < 4; v++) y[v] += acc[v];
-      mlp_act<T, 4>(act, y);
+      for (int v = 0; v < NV; v++) y[v] += acc[v];
+      mlp_act<T, NV>(act, y);
       // (features beyond the last are 0 whatever their zero weights were multiplied with: an infinite value gives no number.
       // Only a layer's last tile has such, and writes them again behind the others' values: as a select of every value
       // this takes 2 % of the launch in double precision)
 #pragma unroll
-      for (int v = 0; v < 4; v++) Y[(tile * 16 + M::row(lane, v)) * TA + my] = y[v];
+      for (int v = 0; v < NV; v++) Y[(tile * 16 + M::row(lane, v)) * TA + col(v)] = y[v];
       if (tile * 16 + 16 > out_f)
 #pragma unroll
-        for (int v = 0; v < 4; v++)
-          if (tile * 16 + M::row(lane, v) >= out_f) Y[(tile * 16 + M::row(lane, v)) * TA + my] = 0;
+        for (int v = 0; v < NV; v++)
+          if (tile * 16 + M::row(lane, v) >= out_f) Y[(tile * 16 + M::row(lane, v)) * TA + col(v)] = 0;
     }
     if (l + 2 < nl) {
       if (wave < mlp_tiles(net.out_f[l + 1])) request(net.fw[l + 1], wave, mlp_pieces<T>(out_f));
@@ -251,8 +316,8 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void 
     __syncthreads();
     X = Y;
   }
-  // ---- the output neuron: every thread takes one atom's share of the features, the shares are added in ascending
-  // order; the delta of the last hidden layer takes the place of its values
+  // ---- the output neuron: every thread takes one atom's share of the features, the shares are added in a fixed order; the
+  // delta of the last hidden layer takes the place of its values
   {
     const int in_f = net.in_f[nl - 1], act = net.act[nl - 1], hact = nl > 1 ? net.act[nl - 2] : 0;
     const int rows = mlp_rows(in_f);
@@ -265,11 +330,14 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void 
       sum += h * w[k];
       if (act == 0 && nl > 1) X[k * TA + t] = w[k] * mlp_slope<T>(hact, h);
     }
-    parts[part * TA + t] = sum;
+    // the wave's shares of an atom (lanes TA apart) first, then the waves in ascending order
+#pragma unroll
+    for (int o = TA; o < WAVE; o *= 2) sum += __shfl_xor(sum, o, WAVE);
+    if (lane < TA) parts[wave * TA + t] = sum;
     __syncthreads();
     if (tid < TA || act != 0) {
       T y = net.b[nl - 1][0];
-      for (int p = 0; p < np; p++) y += parts[p * TA + t];
+      for (int p = 0; p < nw; p++) y += parts[p * TA + t];
       T ys[1] = {y};
       mlp_act<T, 1>(act, ys);
       y = ys[0];
@@ -288,18 +356,20 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void 
     if (act != 0 || nl == 1) __syncthreads();
   }
   // ---- backward: d sum(e) / d af = delta / (af + 1e-3)
-  auto af_at = [&](int i) -> T {   // (beyond the last fingerprint: the last one)
+  auto af_at = [&](int c, int i) -> T {   // (beyond the last atom or fingerprint: the last one)
+    const size_t at = (size_t)(a0 + c < S.Nl ? a0 + c : S.Nl - 1);
     i = i < n_af ? i : n_af - 1;
-    return (T)(i < S.Ar ? S.af2[atom * S.Ar + i] : S.af3[atom * S.Aa + (i - S.Ar)]);
+    return (T)(i < S.Ar ? S.af2[at * S.Ar + i] : S.af3[at * S.Aa + (i - S.Ar)]);
   };
-  auto put = [&](int i, T delta, T afv) {
+  auto put = [&](int c, int i, T delta, T afv) {
     const real g = (real)(delta / (afv + T(1e-3)));
-    if (i < n_af && live) (i < S.Ar ? S.g2 + (atom * S.Ar + i) : S.g3 + (atom * S.Aa + (i - S.Ar)))[0] = g;
+    const size_t at = (size_t)(a0 + c);
+    if (i < n_af && a0 + c < S.Nl) (i < S.Ar ? S.g2 + (at * S.Ar + i) : S.g3 + (at * S.Aa + (i - S.Ar)))[0] = g;
   };
   if (nl == 1) {
     const T d = X[my];
     for (int i = tid / TA; i < n_af; i += (int)blockDim.x / TA)
-      put(i, net.fw[0][i] * d, af_at(i));
+      put(my, i, net.fw[0][i] * d, af_at(my, i));
     return;
   }
   for (int l = nl - 2; l >= 0; l--) {
@@ -310,20 +380,21 @@ __global__ __launch_bounds__(MLP_WAVES_MAX * WAVE, sizeof(T) == 4 ? 8 : 4) void 
     const int act = l > 0 ? net.act[l - 1] : 0;
     for (int tile = wave; tile < tiles; tile += nw) {
       if (tile != wave) request(net.bw[l], tile, np);
-      T other[4];   // what the product is multiplied with: the inputs' values, or the fingerprints behind them
-      T* const at = X + (tile * 16) * TA + my;
+      T other[NV];   // what the product is multiplied with: the inputs' values, or the fingerprints behind them
+      T* const at = X + (tile * 16) * TA;
 #pragma unroll
-      for (int v = 0; v < 4; v++) other[v] = l > 0 ? at[M::row(lane, v) * TA] : af_at(tile * 16 + M::row(lane, v));
-      const acc_t acc = product(net.bw[l], tile, np, D);
+      for (int v = 0; v < NV; v++) other[v] = l > 0 ? at[M::row(lane, v) * TA + col(v)] : af_at(col(v), tile * 16 + M::row(lane, v));
+      T acc[NV];
+      product(net.bw[l], tile, np, D, acc);
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        if (l > 0) at[M::row(lane, v) * TA] = acc[v] * mlp_slope<T>(act, other[v]);
-        else put(tile * 16 + M::row(lane, v), acc[v], other[v]);
+      for (int v = 0; v < NV; v++) {
+        if (l > 0) at[M::row(lane, v) * TA + col(v)] = acc[v] * mlp_slope<T>(act, other[v]);
+        else put(col(v), tile * 16 + M::row(lane, v), acc[v], other[v]);
       }
       if (l > 0 && tile * 16 + 16 > in_f)
 #pragma unroll
-        for (int v = 0; v < 4; v++)
-          if (tile * 16 + M::row(lane, v) >= in_f) at[M::row(lane, v) * TA] = 0;
+        for (int v = 0; v < NV; v++)
+          if (tile * 16 + M::row(lane, v) >= in_f) at[M::row(lane, v) * TA + col(v)] = 0;
     }
     if (l > 0) {
       if (wave < mlp_tiles(net.in_f[l - 1])) request(net.bw[l - 1], wave, mlp_pieces<T>(in_f));
@@ -337,7 +408,7 @@ template <typename T>
 static size_t mlp_lds(int rows, int waves, int ta) {
   return ((size_t)rows * ta + (size_t)waves * WAVE) * sizeof(T);
 }
-// Atoms per workgroup for stacks of `rows`: 16 up to about 1200 features in all layers in double precision and 2480 in
+// Most atoms per workgroup for stacks of `rows`: 16 up to about 1200 features in all layers in double precision and 2480 in
 // single, 8 up to twice as many (six layers of 430 in single precision, 768 atoms: 160 us, where the host takes 258 ms);
 // 0: too many.
 template <typename T>
@@ -581,10 +652,10 @@ static int eval_nets_by(const DevMlpCall<real>* calls, int n, int rows, int tile
     }
   }
   if (blocks == 0) return STAF_OK;
-  // A wave per tile of the widest product while a CU has one workgroup at most (double precision, 60-140-140-1: 22.0
-  // us with nine waves, 24.2 with five); two tiles per wave where it has several, whose products and activations then
-  // overlap (1024 workgroups: 76.7 us with nine waves, 60.3 with five, 72 with three).
-  const int waves = std::min(MLP_WAVES_MAX, std::max(2, blocks <= 256 ? tiles : (tiles + 1) / 2));
+  // A wave per tile of the widest product while a CU has one workgroup at most, or two small ones (double precision,
+  // 60-140-140-1: 22.0 us with nine waves, 24.2 with five); two tiles per wave where it has several, whose products and
+  // activations then overlap (1024 workgroups: 76.7 us with nine waves, 60.3 with five, 72 with three).
+  const int waves = std::min(MLP_WAVES_MAX, std::max(2, blocks <= (TA == 16 ? 256 : 512) ? tiles : (tiles + 1) / 2));
   const size_t lds = mlp_lds<T>(rows, waves, TA);
   if (!lds_request(mlp_kernel<T, real, TA>, lds)) return STAF_E_LIMIT;
   KernelTimer kt_("mlp_kernel", stream);
@@ -594,15 +665,24 @@ static int eval_nets_by(const DevMlpCall<real>* calls, int n, int rows, int tile
 
 template <typename T, typename real>
 static int eval_nets(const DevMlpCall<real>* calls, int n, hipStream_t stream) {
-  int rows = 0, tiles = 1;
+  int rows = 0, tiles = 1, by4 = 0, by8 = 0;   // workgroups of four and of eight atoms
   for (int c = 0; c < n; c++) {
     if (calls[c].Nl <= 0) continue;
     rows = std::max(rows, calls[c].net->rows);
     tiles = std::max(tiles, calls[c].net->tiles);
+    by4 += (calls[c].Nl + 3) / 4;
+    by8 += (calls[c].Nl + 7) / 8;
   }
-  const int ta = mlp_atoms<T>(rows);
-  return ta == 16 ? eval_nets_by<T, real, 16>(calls, n, rows, tiles, stream)
-       : ta == 8 ? eval_nets_by<T, real, 8>(calls, n, rows, tiles, stream) : STAF_E_LIMIT;
+  // A launch of few atoms lasts as long as a workgroup's chain of products, which is shorter for fewer atoms as long as the
+  // workgroups find a CU each: double precision by fours up to 256 workgroups (96 to 768 atoms 22.5 -> 14.1 us) and by
+  // eights up to as many (1500 atoms by 16 / 8 / 4: 23.3 / 17.8 / 23.6; 3072: 24 / 29 / 34).  In single precision, whose
+  // weights are half the bytes, two small workgroups share a CU (96 to 768 atoms 17.3 -> 12.3, 1500 atoms 17.8 / 15.7 / 15.2,
+  // 3072 18.4 / 19.8 / 18.8).  (Times between the library's events.)
+  const int most = mlp_atoms<T>(rows);
+  if (most == 0) return STAF_E_LIMIT;
+  if (by4 <= (sizeof(T) == 8 ? 256 : 512)) return eval_nets_by<T, real, 4>(calls, n, rows, tiles, stream);
+  if (most == 8 || (sizeof(T) == 8 && by8 <= 256)) return eval_nets_by<T, real, 8>(calls, n, rows, tiles, stream);
+  return eval_nets_by<T, real, 16>(calls, n, rows, tiles, stream);
 }
 
 template <typename real>

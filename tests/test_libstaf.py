@@ -856,3 +856,27 @@ def test_every_atom_of_a_call_arrives_and_returns(n):
         want = pairs * e2 + e1
         assert abs(e - want) <= (n + 2) * 2.0 ** -53 * (pairs * abs(e2) + abs(e1)) * 4
     model.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,tol", [("double", 1e-11), ("float", 2e-5)])
+@pytest.mark.parametrize("n", [1021, 1027, 2043, 2053])
+def test_network_on_both_sides_of_the_atoms_per_workgroup_lines(prec, tol, n):
+    """256 workgroups of four atoms, 256 of eight, 512 of four (n atoms of two species, ragged last tiles): device network
+    against the host's, tolerances of test_device_mlp_matches_host_mlp."""
+    from alphanesgpu_amd import libstaf
+    rng = np.random.Generator(np.random.Philox(n))
+    edge = 4 * round(n ** (1 / 3) + 1)
+    cells = rng.permutation((edge // 4) ** 3)[:n]
+    x = 4.0 * np.stack(np.unravel_index(cells, (edge // 4,) * 3), 1) + rng.uniform(0, 1.5, (n, 3))
+    types = rng.integers(0, 2, n).astype(np.int32)
+    box = edge * np.array([1.0, 0.0, 0.0, 1.0, 0.0, 1.0])
+    d = os.path.join(GOLDEN, f"model_{prec}")
+    out = []
+    for host in (False, True):
+        m = libstaf.StafModel(d, precision=1 if prec == "double" else 0, full_virial=True, host_mlp=host)
+        out.append(m.compute(x, box, types))
+        m.close()
+    (e, f, w), (eh, fh, wh) = out
+    assert abs(e - eh) <= tol * abs(eh)
+    assert nerr(f, fh) <= tol and nerr(w, wh) <= tol
