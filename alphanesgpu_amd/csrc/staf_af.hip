@@ -32,13 +32,14 @@ __global__ __launch_bounds__(AF_BLOCK) void af2_kernel(const real* __restrict__ 
                                                        const real* __restrict__ alpha2b,
                                                        const real* __restrict__ emb2b,
                                                        const int* __restrict__ type_map, real* __restrict__ out,
-                                                       int nf, int Nl, int ld, int nr, int Ar, int nt) {
+                                                       int nf, int Nl, int ld, int nr, int Ar, int nt, int raw_emb,
+                                                       int out_ld) {
   extern __shared__ __align__(16) unsigned char smem[];
   real* p_al = (real*)smem;          // [nt*Ar] alpha in the units of the hot exponential
   real* p_c2 = p_al + nt * Ar;       // [nt*Ar]
   real* w_D = p_c2 + nt * Ar;        // [AF_WAVES][nr]
   int* w_t = (int*)(w_D + AF_WAVES * nr);  // [AF_WAVES][nr]
-  af2_tables(alpha2b, emb2b, nt * Ar, p_al, p_c2);
+  af2_tables(alpha2b, emb2b, nt * Ar, p_al, p_c2, raw_emb);
   const int wave = threadIdx.x / WAVE, lane = lane_id();
   real* myD = w_D + wave * nr;
   int* myT = w_t + wave * nr;
@@ -51,7 +52,7 @@ __global__ __launch_bounds__(AF_BLOCK) void af2_kernel(const real* __restrict__ 
   }
   __syncthreads();
   if (atom >= nf * Nl) return;
-  af2_wave_sum(p_al, p_c2, myD, myT, cnt, Ar, out + (size_t)atom * Ar, lane);
+  af2_wave_sum(p_al, p_c2, myD, myT, cnt, Ar, out + (size_t)atom * out_ld, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -66,7 +67,8 @@ __global__ __launch_bounds__(AF_BLOCK) void grad2_kernel(const real* __restrict_
                                                          const real* __restrict__ emb2b,
                                                          const int* __restrict__ type_map,
                                                          const real* __restrict__ P, real* __restrict__ partial,
-                                                         int nf, int Nl, int ld, int nr, int Ar, int nt) {
+                                                         int nf, int Nl, int ld, int nr, int Ar, int nt, int raw_emb,
+                                                         int P_ld) {
   using HE = HotExp<real>;
   extern __shared__ __align__(16) unsigned char smem[];
   real* p_al = (real*)smem;                 // [nt*Ar] alpha in the units of the hot exponential
@@ -76,7 +78,11 @@ __global__ __launch_bounds__(AF_BLOCK) void grad2_kernel(const real* __restrict_
   int* w_t = (int*)(w_D + AF_WAVES * nr);   // [AF_WAVES][nr] species of the slot
   int* w_l = w_t + AF_WAVES * nr;           // [AF_WAVES][nr] slots grouped by species
   int* w_o = w_l + AF_WAVES * nr;           // [AF_WAVES][NT_MAX+1] first grouped position of a species
-  for (int q = threadIdx.x; q < nt * Ar; q += blockDim.x) { p_al[q] = HE::scale(alpha2b[q]); p_c2[q] = emb2b[q]; }
+  for (int q = threadIdx.x; q < nt * Ar; q += blockDim.x) {
+    const real c = emb2b[q];
+    p_al[q] = HE::scale(alpha2b[q]);
+    p_c2[q] = raw_emb ? c * c : c;
+  }
   const int wave = threadIdx.x / WAVE, lane = lane_id();
   real* myD = w_D + wave * nr;
   int* myT = w_t + wave * nr;
@@ -106,7 +112,7 @@ __global__ __launch_bounds__(AF_BLOCK) void grad2_kernel(const real* __restrict_
     for (int a0 = 0; a0 < Ar; a0 += cs.chunk) {
       const int a = a0 + cs.a;
       const bool on = cs.sub < cs.nsub && a < Ar;
-      const real pg = on ? P[(size_t)atom * Ar + a] : real(0);
+      const real pg = on ? P[(size_t)atom * P_ld + a] : real(0);
       for (int t = 0; t < nt; t++) {
         const int q0 = uniform(myO[t]), q1 = uniform(myO[t + 1]);
         if (q0 == q1) continue;
@@ -149,7 +155,8 @@ static inline int grad_blocks(int atoms) {
 
 template <typename real>
 static int radial_afs(const real* D, int nr, const real* alpha2b, int Ar, real* out, int nf, int Nl, const int* im2,
-                      const real* emb2b, const int* type_map, int nt, int ld, void* stream_) {
+                      const real* emb2b, const int* type_map, int nt, int ld, void* stream_, int raw_emb = 0,
+                      int out_ld = 0) {
   if (Nl == 0 && nf > 0 && Ar > 0) return STAF_OK;   // a species without atoms in these frames: nothing to write
   if (!D || !alpha2b || !out || !im2 || !emb2b || !type_map || nr <= 0 || Ar <= 0 || nf <= 0 || Nl <= 0 || nt <= 0)
     return STAF_E_BAD_ARG;
@@ -161,7 +168,8 @@ static int radial_afs(const real* D, int nr, const real* alpha2b, int Ar, real* 
   {
     KernelTimer kt_("af2_kernel", (hipStream_t)stream_);
     hipLaunchKernelGGL(af2_kernel<real>, dim3((atoms + AF_WAVES - 1) / AF_WAVES), dim3(AF_BLOCK), lds,
-                       (hipStream_t)stream_, D, im2, alpha2b, emb2b, type_map, out, nf, Nl, ld, nr, Ar, nt);
+                       (hipStream_t)stream_, D, im2, alpha2b, emb2b, type_map, out, nf, Nl, ld, nr, Ar, nt, raw_emb,
+                       out_ld ? out_ld : Ar);
   }
   return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
 }
@@ -192,7 +200,8 @@ static int alpha_dist_grad_check(const real* D, int nr, const real* alpha2b, int
 template <typename real>
 static int alpha_dist_grad_launch(const real* D, int nr, const real* alpha2b, int Ar, real* g_alpha, int nf, int Nl,
                                   const int* im2, const real* P, const real* emb2b, const int* type_map, real* g_emb,
-                                  int nt, int ld, real* work, bool timed, hipStream_t stream) {
+                                  int nt, int ld, real* work, bool timed, hipStream_t stream, int raw_emb = 0,
+                                  int P_ld = 0) {
   const int nout = 2 * nt * Ar;
   const int nb = grad_blocks(nf * Nl);
   real* partial = work;
@@ -202,19 +211,20 @@ static int alpha_dist_grad_launch(const real* D, int nr, const real* alpha2b, in
   if (timed) {
     KernelTimer kt_("grad2_kernel", stream);
     hipLaunchKernelGGL(grad2_kernel<real>, dim3(nb), dim3(AF_BLOCK), lds, stream, D, im2, alpha2b, emb2b, type_map, P,
-                       partial, nf, Nl, ld, nr, Ar, nt);
+                       partial, nf, Nl, ld, nr, Ar, nt, raw_emb, P_ld ? P_ld : Ar);
   } else {
     hipLaunchKernelGGL(grad2_kernel<real>, dim3(nb), dim3(AF_BLOCK), lds, stream, D, im2, alpha2b, emb2b, type_map, P,
-                       partial, nf, Nl, ld, nr, Ar, nt);
+                       partial, nf, Nl, ld, nr, Ar, nt, raw_emb, P_ld ? P_ld : Ar);
   }
-  launch_reduce_partials<real>(partial, nb, nout, g_alpha, nt * Ar, nt * Ar, g_emb, nt * Ar, nt * Ar, red_tmp, stream);
+  launch_reduce_partials<real>(partial, nb, nout, g_alpha, nt * Ar, nt * Ar, g_emb, nt * Ar, nt * Ar, red_tmp, stream,
+                               (real*)nullptr, 0, 0, raw_emb ? emb2b : (const real*)nullptr);
   return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
 }
 
 template <typename real>
 static int alpha_dist_grad(const real* D, int nr, const real* alpha2b, int Ar, real* g_alpha, int nf, int Nl,
                            const int* im2, const real* P, const real* emb2b, const int* type_map, real* g_emb, int nt,
-                           int ld, void* stream_) {
+                           int ld, void* stream_, int raw_emb = 0, int P_ld = 0) {
   hipStream_t stream = (hipStream_t)stream_;
   if (Nl == 0 && nf > 0 && Ar > 0 && nt > 0 && g_alpha && g_emb) {
     // a species without atoms in these frames: its sums are empty
@@ -230,7 +240,7 @@ static int alpha_dist_grad(const real* D, int nr, const real* alpha2b, int Ar, r
   real* work = (real*)scratch_reserve(st, stream, grad2_work_reals(nf, Nl, nt, Ar) * sizeof(real));
   if (!work) return reserve_failure(stream);
   return alpha_dist_grad_launch<real>(D, nr, alpha2b, Ar, g_alpha, nf, Nl, im2, P, emb2b, type_map, g_emb, nt, ld,
-                                      work, true, stream);
+                                      work, true, stream, raw_emb, P_ld);
 }
 
 // ---- the same op for callers that cannot allocate -------------------------------------------------------------
@@ -290,7 +300,7 @@ static int alpha_dist_grad_noalloc(const double* D, int nr, const double* alpha2
 template <typename real>
 int angular_afs(const real* Dsup, const real* Tang, const real* unit, int nr, int na, real* out, int nf, int Nl,
                 const int* im3, const int* im2, const real* alpha3b, int Aa, const real* emb3b, const int* type_map,
-                const int* numtriplet, int nt, int ld, void* stream_) {
+                const int* numtriplet, int nt, int ld, void* stream_, int raw_emb, int out_ld) {
   (void)im3;
   if (Nl == 0 && nf > 0 && Aa > 0) return STAF_OK;   // a species without atoms in these frames: nothing to write
   if (!Dsup || (!Tang && !unit) || !out || !im2 || !alpha3b || !emb3b || !type_map || !numtriplet || nr <= 0 ||
@@ -303,7 +313,7 @@ int angular_afs(const real* Dsup, const real* Tang, const real* unit, int nr, in
     return STAF_E_LIMIT;
   TriArgs<real> A = {};
   A.Dsup = Dsup; A.Tang = Tang; A.unit = unit; A.im2 = im2; A.alpha3b = alpha3b; A.emb3b = emb3b;
-  A.type_map = type_map; A.numtriplet = numtriplet; A.out = out;
+  A.type_map = type_map; A.numtriplet = numtriplet; A.out = out; A.raw_emb = raw_emb; A.out_ld = out_ld;
   A.nf = nf; A.Nl = Nl; A.ld = ld; A.nr = nr; A.na = na; A.Aa = Aa; A.nt = nt;
   {
     KernelTimer kt_("af3_kernel", (hipStream_t)stream_);
@@ -321,7 +331,7 @@ int angular_afs(const real* Dsup, const real* Tang, const real* unit, int nr, in
 }
 template int angular_afs<double>(const double*, const double*, const double*, int, int, double*, int, int, const int*,
                                  const int*, const double*, int, const double*, const int*, const int*, int, int,
-                                 void*);
+                                 void*, int, int);
 
 // ---------------------------------------------------------------------------
 // Fingerprints of a whole evaluation: 2-body and 3-body of all species in one launch.  Workgroups first2[e] .. take four
@@ -442,7 +452,7 @@ template <typename real>
 static int alphagrad_ang(const real* Dsup, const real* Tang, int nr, int na, const real* P, int nf, int Nl,
                          const int* im3, const int* im2, const real* alpha3b, int Aa, real* g_alpha,
                          const real* emb3b, const int* type_map, real* g_emb, const int* numtriplet, int ntc, int nt,
-                         int ld, void* stream_) {
+                         int ld, void* stream_, int raw_emb = 0, int P_ld = 0) {
   (void)im3;
   if (Nl == 0 && nf > 0 && Aa > 0 && nt > 0 && ntc >= 2 * nt - 1 && g_alpha && g_emb) {
     // a species without atoms in these frames: its sums are empty
@@ -471,7 +481,7 @@ static int alphagrad_ang(const real* Dsup, const real* Tang, int nr, int na, con
   const int nall = ntc * Aa * 3;
   TriArgs<real> A = {};
   A.Dsup = Dsup; A.Tang = Tang; A.im2 = im2; A.alpha3b = alpha3b; A.emb3b = emb3b; A.type_map = type_map;
-  A.numtriplet = numtriplet; A.P = P; A.partial = partial;
+  A.numtriplet = numtriplet; A.P = P; A.partial = partial; A.raw_emb = raw_emb; A.P_ld = P_ld;
   A.nf = nf; A.Nl = Nl; A.ld = ld; A.nr = nr; A.na = na; A.Aa = Aa; A.nt = nt;
   {
     KernelTimer kt_("grad3_kernel", stream);
@@ -482,9 +492,59 @@ static int alphagrad_ang(const real* Dsup, const real* Tang, int nr, int na, con
   return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
 }
 
+// The physics layer of a species: fingerprints [nf, Nl, Ar + Aa] of both bodies from the embeddings as they are trained (not
+// squared), and the gradients of all its parameters from dL/dfingerprints.
+template <typename real>
+static int layer_fingerprints(const real* D, const real* Dsup, const real* Tang, int nr, int na, int nf, int Nl,
+                              const int* im2, const real* alpha2b, int Ar, const real* emb2b, const real* alpha3b, int Aa,
+                              const real* emb3b, const int* type_map, const int* numtriplet, int nt, real* out, int ld,
+                              void* stream) {
+  if (Ar <= 0 || Aa <= 0 || (!out && Nl != 0)) return STAF_E_BAD_ARG;
+  if (Nl == 0 && nf > 0) return STAF_OK;   // a species without atoms in these frames: nothing to write
+  int rc = radial_afs<real>(D, nr, alpha2b, Ar, out, nf, Nl, im2, emb2b, type_map, nt, ld, stream, 1, Ar + Aa);
+  if (rc == STAF_OK)
+    rc = angular_afs<real>(Dsup, Tang, nullptr, nr, na, out + Ar, nf, Nl, nullptr, im2, alpha3b, Aa, emb3b, type_map,
+                           numtriplet, nt, ld, stream, 1, Ar + Aa);
+  return rc;
+}
+template <typename real>
+static int layer_fingerprints_grad(const real* P, const real* D, const real* Dsup, const real* Tang, int nr, int na, int nf,
+                                   int Nl, const int* im2, const real* alpha2b, int Ar, const real* emb2b,
+                                   const real* alpha3b, int Aa, const real* emb3b, const int* type_map,
+                                   const int* numtriplet, int nt, real* g_alpha2b, real* g_emb2b, real* g_alpha3b,
+                                   real* g_emb3b, int ld, void* stream) {
+  if (Ar <= 0 || Aa <= 0 || nt <= 0 || (!P && Nl != 0)) return STAF_E_BAD_ARG;
+  int rc = alpha_dist_grad<real>(D, nr, alpha2b, Ar, g_alpha2b, nf, Nl, im2, P, emb2b, type_map, g_emb2b, nt, ld, stream, 1,
+                                 Ar + Aa);
+  if (rc == STAF_OK)
+    rc = alphagrad_ang<real>(Dsup, Tang, nr, na, Nl ? P + Ar : P, nf, Nl, nullptr, im2, alpha3b, Aa, g_alpha3b, emb3b, type_map,
+                             g_emb3b, numtriplet, nt * (nt + 1) / 2, nt, ld, stream, 1, Ar + Aa);
+  return rc;
+}
+
 }  // namespace staf
 
 extern "C" {
+
+#define STAF_LAYER_FINGERPRINTS(SFX, real)                                                                             \
+  int staf_op_layer_fingerprints_##SFX(const real* D, const real* Dsup, const real* Tang, int nr, int na, int nf, int Nl, \
+                                       const int* im2, const real* alpha2b, int Ar, const real* emb2b,                 \
+                                       const real* alpha3b, int Aa, const real* emb3b, const int* type_map,            \
+                                       const int* numtriplet, int nt, real* out, int ld, void* stream) {               \
+    return staf::layer_fingerprints<real>(D, Dsup, Tang, nr, na, nf, Nl, im2, alpha2b, Ar, emb2b, alpha3b, Aa, emb3b,  \
+                                          type_map, numtriplet, nt, out, ld, stream);                                  \
+  }                                                                                                                    \
+  int staf_op_layer_fingerprints_grad_##SFX(const real* P, const real* D, const real* Dsup, const real* Tang, int nr,  \
+                                            int na, int nf, int Nl, const int* im2, const real* alpha2b, int Ar,       \
+                                            const real* emb2b, const real* alpha3b, int Aa, const real* emb3b,         \
+                                            const int* type_map, const int* numtriplet, int nt, real* g_alpha2b,       \
+                                            real* g_emb2b, real* g_alpha3b, real* g_emb3b, int ld, void* stream) {     \
+    return staf::layer_fingerprints_grad<real>(P, D, Dsup, Tang, nr, na, nf, Nl, im2, alpha2b, Ar, emb2b, alpha3b, Aa, \
+                                               emb3b, type_map, numtriplet, nt, g_alpha2b, g_emb2b, g_alpha3b,         \
+                                               g_emb3b, ld, stream);                                                   \
+  }
+STAF_LAYER_FINGERPRINTS(f32, float)
+STAF_LAYER_FINGERPRINTS(f64, double)
 
 int staf_op_radial_afs_f32(const float* D, int nr, const float* alpha2b, int Ar, float* out, int nf, int Nl,
                            const int* im2, const float* emb2b, const int* type_map, int nt, int ld, void* stream) {

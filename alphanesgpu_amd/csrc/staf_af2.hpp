@@ -10,13 +10,14 @@
 namespace staf {
 
 // Parameter tables of a workgroup in LDS: p_al[nt*Ar] = alpha in the units of the hot exponential, p_c2[nt*Ar].
-// All threads of the workgroup call; a barrier must follow before the tables are read.
+// raw_emb: emb2b is to be squared.  All threads of the workgroup call; a barrier must follow before the tables are read.
 template <typename real>
 __device__ inline void af2_tables(const real* __restrict__ alpha2b, const real* __restrict__ emb2b, int n,
-                                  real* p_al, real* p_c2) {
+                                  real* p_al, real* p_c2, int raw_emb = 0) {
   for (int q = threadIdx.x; q < n; q += blockDim.x) {
     p_al[q] = HotExp<real>::scale(alpha2b[q]);
-    p_c2[q] = emb2b[q];
+    const real c = emb2b[q];
+    p_c2[q] = raw_emb ? c * c : c;
   }
 }
 

@@ -489,7 +489,7 @@ int force_doublets(const real* G, const real* D, const real* dD, const int* im2,
 template <typename real>
 int angular_afs(const real* Dsup, const real* Tang, const real* unit, int nr, int na, real* out, int nf, int Nl,
                 const int* im3, const int* im2, const real* alpha3b, int Aa, const real* emb3b, const int* type_map,
-                const int* numtriplet, int nt, int ld, void* stream);
+                const int* numtriplet, int nt, int ld, void* stream, int raw_emb = 0, int out_ld = 0);
 // The 2-body inputs of the force launch that adds the pair forces to the 3-body slot forces (staf_force3.hpp).
 template <typename real>
 struct Force2In {
@@ -508,7 +508,7 @@ int force_tripl(const real* G, const real* Dsup, const real* Tang, const real* d
                 const int* tipos, const int* actual_type, real* force, const int* numtriplet, const real* alpha3b,
                 const int* type_map, int Nl, real* virial, const real* pos, const real* box, int ld, int skip_pbc,
                 void* stream, real* slots_out = nullptr, real* self_out = nullptr,
-                const Force2In<real>* two_body = nullptr, const TransposeRef* known = nullptr);
+                const Force2In<real>* two_body = nullptr, const TransposeRef* known = nullptr, int raw_emb = 0);
 template <typename real>
 int force_total(const int* im2_full, int nr, int N, int nf, int nt, const int* n_local, const real* const* slot_forces,
                 const real* const* self_forces, const real* const* force_2b, real* total, void* stream);

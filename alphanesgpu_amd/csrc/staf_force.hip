@@ -425,7 +425,7 @@ __global__ __launch_bounds__(F_BLOCK) void gradforce2_kernel(
     const int* __restrict__ type_map, const int* __restrict__ tipos, const int* __restrict__ actual_type,
     real* __restrict__ gnet, real* __restrict__ partial, const real* __restrict__ Qvir,
     const real* __restrict__ pos, const real* __restrict__ box, int skip_pbc, int nf, int N, int Nl, int ld, int nr,
-    int Ar, int nt) {
+    int Ar, int nt, int raw_emb) {
   using HE = HotExp<real>;
   extern __shared__ __align__(16) unsigned char smem[];
   real* p_al = (real*)smem;                     // [nt*Ar]
@@ -436,7 +436,11 @@ __global__ __launch_bounds__(F_BLOCK) void gradforce2_kernel(
   int* w_t = (int*)(w_w + F_WAVES * nr);        // [F_WAVES][nr]  species of the slot
   int* w_l = w_t + F_WAVES * nr;                // [F_WAVES][nr]  slots grouped by species
   int* w_o = w_l + F_WAVES * nr;                // [F_WAVES][NT_MAX+1]
-  for (int q = threadIdx.x; q < nt * Ar; q += blockDim.x) { p_al[q] = alpha2b[q]; p_c2[q] = emb2b[q]; }
+  for (int q = threadIdx.x; q < nt * Ar; q += blockDim.x) {
+    const real c = emb2b[q];
+    p_al[q] = alpha2b[q];
+    p_c2[q] = raw_emb ? c * c : c;
+  }
   const int wave = threadIdx.x / WAVE, lane = lane_id();
   real* myD = w_D + wave * nr;
   real* myW = w_w + wave * nr;
@@ -621,7 +625,7 @@ int force_tripl(const real* G, const real* Dsup, const real* Tang, const real* d
                 const int* tipos, const int* actual_type, real* force, const int* numtriplet, const real* alpha3b,
                 const int* type_map, int Nl, real* virial, const real* pos, const real* box, int ld, int skip_pbc,
                 void* stream_, real* slots_out, real* self_out, const Force2In<real>* two_body,
-                const TransposeRef* known) {
+                const TransposeRef* known, int raw_emb) {
   (void)im3;
   if ((virial || pos || box) && !(virial && pos && box)) return STAF_E_BAD_ARG;
   // slots_out / self_out: the slot forces [nf, Nl, nr, 3] and the centres' own forces [nf, Nl, 3] go to the caller
@@ -680,6 +684,7 @@ int force_tripl(const real* G, const real* Dsup, const real* Tang, const real* d
     A.G = G; A.Dsup = Dsup; A.Tang = Tang; A.dDsup = dDsup; A.d3b = d3b; A.unit = unit; A.im2 = im2; A.alpha3b = alpha3b;
     A.emb3b = emb3b; A.type_map = type_map; A.numtriplet = numtriplet; A.gslot = gslot; A.self = self;
     A.Nl = Nl; A.ld = ld; A.ldo = Nl; A.nr = nr; A.na = na; A.Aa = Aa; A.nt = nt;
+    A.raw_emb = raw_emb;
     if (two_body) A.B2 = *two_body;
     KernelTimer kt_("force3_kernel", stream);
     hipLaunchKernelGGL((force3_kernel<real, FUSED, NWV, W2B>), dim3(nf * Nl), dim3(L::THREADS), lds, stream, A);
@@ -716,14 +721,14 @@ template int force_tripl<double>(const double*, const double*, const double*, co
                                  const int*,
                                  const int*, double*, const int*, const double*, const int*, int, double*,
                                  const double*, const double*, int, int, void*, double*, double*,
-                                 const Force2In<double>*, const TransposeRef*);
+                                 const Force2In<double>*, const TransposeRef*, int);
 
 template <typename real>
 static int gradforce_2b(const real* Q, const real* D, int nr, const real* alpha2b, int Ar, const real* dD,
                         const int* im2, int nf, int N, int Nl, const real* G, const real* emb2b, int nt,
                         const int* type_map, const int* tipos, const int* actual_type, real* gnet, real* g_alpha,
                         real* g_emb, const real* Qvir, const real* pos, const real* box, int ld, int skip_pbc,
-                        void* stream_) {
+                        void* stream_, int raw_emb = 0) {
   if ((Qvir || pos || box) && !(Qvir && pos && box)) return STAF_E_BAD_ARG;
   if (Nl == 0 && nf > 0 && Ar > 0 && nt > 0 && g_alpha && g_emb)
     return empty_species_grad<real>(g_alpha, nt * Ar, g_emb, nt * Ar, stream_);
@@ -747,9 +752,10 @@ static int gradforce_2b(const real* Q, const real* D, int nr, const real* alpha2
     KernelTimer kt_("gradforce2_kernel", stream);
     hipLaunchKernelGGL(gradforce2_kernel<real>, dim3(nb), dim3(F_BLOCK), lds, stream, Q, G, D, dD, im2, alpha2b, emb2b,
                        type_map, tipos, actual_type, gnet, partial, Qvir, pos, box, skip_pbc, nf, N, Nl, ld, nr,
-                       Ar, nt);
+                       Ar, nt, raw_emb);
   }
-  launch_reduce_partials<real>(partial, nb, nout, g_alpha, nt * Ar, nt * Ar, g_emb, nt * Ar, nt * Ar, red_tmp, stream);
+  launch_reduce_partials<real>(partial, nb, nout, g_alpha, nt * Ar, nt * Ar, g_emb, nt * Ar, nt * Ar, red_tmp, stream,
+                               (real*)nullptr, 0, 0, raw_emb ? emb2b : (const real*)nullptr);
   return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
 }
 
@@ -758,7 +764,8 @@ static int gradforce_tripl(const real* Q, const real* G, const real* Dsup, const
                            const real* d3b, const int* im2, const int* im3, int nr, int na, int N, int nf, int Aa,
                            const real* emb3b, int nt, const int* tipos, const int* actual_type, const int* numtriplet,
                            const real* alpha3b, const int* type_map, int Nl, real* gnet, real* g_alpha, real* g_emb,
-                           const real* Qvir, const real* pos, const real* box, int ld, int skip_pbc, void* stream_) {
+                           const real* Qvir, const real* pos, const real* box, int ld, int skip_pbc, void* stream_,
+                           int raw_emb = 0) {
   (void)im3;
   if ((Qvir || pos || box) && !(Qvir && pos && box)) return STAF_E_BAD_ARG;
   if (Nl == 0 && nf > 0 && Aa > 0 && nt > 0 && g_alpha && g_emb) {
@@ -789,7 +796,7 @@ static int gradforce_tripl(const real* Q, const real* G, const real* Dsup, const
   A.Dsup = Dsup; A.Tang = Tang; A.im2 = im2; A.alpha3b = alpha3b; A.emb3b = emb3b; A.type_map = type_map;
   A.numtriplet = numtriplet; A.P = G; A.Q = Q; A.dDsup = dDsup; A.d3b = d3b; A.tipos = tipos;
   A.actual_type = actual_type; A.out = gnet; A.partial = partial; A.Qvir = Qvir; A.pos = pos; A.box = box;
-  A.skip_pbc = skip_pbc;
+  A.skip_pbc = skip_pbc; A.raw_emb = raw_emb;
   A.nf = nf; A.N = N; A.Nl = Nl; A.ld = ld; A.nr = nr; A.na = na; A.Aa = Aa; A.nt = nt;
   {
     KernelTimer kt_("gradforce3_kernel", stream);
@@ -1190,6 +1197,42 @@ void staf_op_force_set_skip_pbc(int skip) { staf::g_force_skip_pbc = skip ? 1 : 
 
 STAF_FORCE_ENTRY(float, f32)
 STAF_FORCE_ENTRY(double, f64)
+
+// The force layer of a species: staf_op_forces and the gradients of both bodies from the embeddings as they are trained.
+#define STAF_LAYER_FORCE_ENTRY(real, SFX)                                                                              \
+  int staf_op_layer_forces_##SFX(const real* G2, const real* G3, const real* D, const real* dD, const real* Dsup,      \
+                                 const real* Tang, const real* dDsup, const real* d3b, const int* im2, int nr, int na, \
+                                 int N, int nf, int Nl, const real* alpha2b, int Ar, const real* emb2b,                \
+                                 const real* alpha3b, int Aa, const real* emb3b, int nt, const int* tipos,             \
+                                 const int* actual_type, const int* numtriplet, const int* type_map, real* force,      \
+                                 real* virial, const real* pos, const real* box, int ld, void* stream) {               \
+    staf::Force2In<real> two;                                                                                          \
+    two.G2 = G2; two.D = D; two.dD = dD; two.alpha2b = alpha2b; two.emb2b = emb2b; two.Ar = Ar;                        \
+    return staf::force_tripl<real>(G3, Dsup, Tang, dDsup, d3b, (const real*)nullptr, im2, (const int*)nullptr, nr, na, \
+                                   N, nf, Aa, emb3b, nt, tipos, actual_type, force, numtriplet, alpha3b, type_map, Nl, \
+                                   virial, pos, box, ld, staf::g_force_skip_pbc, stream, (real*)nullptr,               \
+                                   (real*)nullptr, &two, (const staf::TransposeRef*)nullptr, 1);                       \
+  }                                                                                                                    \
+  int staf_op_layer_forces_grad_##SFX(                                                                                 \
+      const real* Q, const real* G2, const real* G3, const real* D, const real* dD, const real* Dsup,                  \
+      const real* Tang, const real* dDsup, const real* d3b, const int* im2, int nr, int na, int N, int nf, int Nl,     \
+      const real* alpha2b, int Ar, const real* emb2b, const real* alpha3b, int Aa, const real* emb3b, int nt,          \
+      const int* tipos, const int* actual_type, const int* numtriplet, const int* type_map, real* gnet2,               \
+      real* g_alpha2b, real* g_emb2b, real* gnet3, real* g_alpha3b, real* g_emb3b, const real* Qvir, const real* pos,  \
+      const real* box, int ld, void* stream) {                                                                         \
+    int rc = STAF_OK;                                                                                                  \
+    if (g_alpha2b)                                                                                                     \
+      rc = staf::gradforce_2b<real>(Q, D, nr, alpha2b, Ar, dD, im2, nf, N, Nl, G2, emb2b, nt, type_map, tipos,         \
+                                    actual_type, gnet2, g_alpha2b, g_emb2b, Qvir, pos, box, ld,                        \
+                                    staf::g_force_skip_pbc, stream, 1);                                                \
+    if (rc == STAF_OK && g_alpha3b)                                                                                    \
+      rc = staf::gradforce_tripl<real>(Q, G3, Dsup, Tang, dDsup, d3b, im2, (const int*)nullptr, nr, na, N, nf, Aa,     \
+                                       emb3b, nt, tipos, actual_type, numtriplet, alpha3b, type_map, Nl, gnet3,        \
+                                       g_alpha3b, g_emb3b, Qvir, pos, box, ld, staf::g_force_skip_pbc, stream, 1);     \
+    return rc;                                                                                                         \
+  }
+STAF_LAYER_FORCE_ENTRY(float, f32)
+STAF_LAYER_FORCE_ENTRY(double, f64)
 
 #define STAF_FUSED_GRAD_ENTRY(real, SFX)                                                                               \
   int staf_op_grads_tripl_fused_##SFX(                                                                                 \

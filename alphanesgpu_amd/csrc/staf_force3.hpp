@@ -114,6 +114,7 @@ struct Force3Args {   // one centre species
   real* vpart;            // FUSED with W2B: [nf, ldo, 9] virial of the centre's slot forces, or null
   int Nl, ld, nr, na, Aa, nt;
   int ldo;                // rows per frame of gslot, self and vpart (Nl where these hold one species)
+  int raw_emb;            // emb3b and B2.emb2b are to be squared
   Force2In<real> B2;      // W2B
 };
 
@@ -249,6 +250,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
       if (a < Aa) {
         const real* al = alpha3b + ((size_t)sgm * Aa + a) * 3;
         c = emb3b[sgm * Aa + a];
+        if (A.raw_emb) c *= c;
         al0 = al[0]; al1 = al[1]; al2 = al[2];
         gv = G[(size_t)atom * Aa + a];
       }
@@ -285,7 +287,8 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
         real al = 0, w = 0;
         if (a < Ar) {
           al = B2.alpha2b[t * Ar + a];
-          w = B2.G2[(size_t)atom * Ar + a] * B2.emb2b[t * Ar + a];
+          const real c = B2.emb2b[t * Ar + a];
+          w = B2.G2[(size_t)atom * Ar + a] * (A.raw_emb ? c * c : c);
         }
         const bool on = !(w == real(0));
         const unsigned long long mask = __ballot(on);

@@ -15,8 +15,10 @@ constexpr int RED_SLICES = 32;  // rows callers still reserve behind their parti
 // partial rows are a few MB and a segment's column a few hundred KB, which one CU reads in the time a launch costs.
 // The padded output space is a sequence of up to three pieces: piece i takes the next n[i] columns of the partial
 // rows and is z[i] >= n[i] elements long, the rest written as zero (a piece with n = 0 is a zero fill).
+// chain != null: the piece is the gradient of squares, and what is written is that of their roots chain[0 .. n).
 struct ReduceOut {
   void* out[3];
+  const void* chain[3];
   int n[3], z[3];
 };
 template <typename real>
@@ -53,6 +55,7 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_partials_kernel(const real
     real t = 0;
 #pragma unroll
     for (int w = 0; w < NWV; w++) t += sh[w][tid];
+    if (src >= 0 && O.chain[piece]) t *= real(2) * ((const real*)O.chain[piece])[at];
     if (at < O.z[piece]) ((real*)O.out[piece])[at] = t;
   }
 }
@@ -61,11 +64,13 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_partials_kernel(const real
 template <typename real>
 inline void launch_reduce_partials(const real* partial, int nblocks, int nout, real* out0, int n0, int z0, real* out1,
                                    int n1, int z1, real* tmp, hipStream_t stream, real* out2 = nullptr, int n2 = 0,
-                                   int z2 = 0) {
+                                   int z2 = 0, const real* chain1 = nullptr) {
   (void)tmp;
   constexpr int EL = 64 / (int)sizeof(real);
   const int etot = z0 + z1 + z2;
   ReduceOut O;
+  O.chain[0] = O.chain[2] = nullptr;
+  O.chain[1] = chain1;
   O.out[0] = out0; O.n[0] = n0; O.z[0] = z0;
   O.out[1] = out1; O.n[1] = n1; O.z[1] = z1;
   O.out[2] = out2; O.n[2] = n2; O.z[2] = z2;

@@ -35,9 +35,9 @@ struct ChanTable {
     // the next carve-out may hold doubles: keep 16-byte alignment
     return p + ((((size_t)nsig * Aa * (4 * sizeof(real) + sizeof(int)) + (size_t)nsig * sizeof(int)) + 15) & ~(size_t)15);
   }
-  // alpha3b [ntc, 3*Aa] as (alpha1, alpha2, beta) per channel, emb3b [ntc, Aa].
+  // alpha3b [ntc, 3*Aa] as (alpha1, alpha2, beta) per channel, emb3b [ntc, Aa], squared or (raw) to be squared here.
   // Waves of the block split the rows; a __syncthreads() must follow.
-  __device__ void build(const real* alpha3b, const real* emb3b) {
+  __device__ void build(const real* alpha3b, const real* emb3b, int raw) {
     const int lane = lane_id();
     const int wave = threadIdx.x / WAVE, nwaves = blockDim.x / WAVE;
     for (int sg = wave; sg < nsig; sg += nwaves) {
@@ -46,6 +46,7 @@ struct ChanTable {
         const int a = a0 + lane;
         real c = 0;
         if (a < Aa) c = emb3b[sg * Aa + a];
+        if (raw) c *= c;
         const bool on = (a < Aa) && (c != real(0));
         const unsigned long long mask = __ballot(on);
         if (on) {

@@ -53,6 +53,68 @@ class _SortProj3body(torch.autograd.Function):
         return None, None, None, None, ga, ge, None, None
 
 
+class _LayerFingerprints(torch.autograd.Function):
+    """Both fingerprint ops of a species on the embeddings as they are trained, and their gradient ops, as one call each way
+    (ops.layer_fingerprints): the values and gradients of _SortProj and _SortProj3body on the squares, beside each other."""
+
+    @staticmethod
+    def forward(ctx, x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb3b, type_map, numtriplet):
+        ctx.save_for_backward(x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb3b, type_map, numtriplet)
+        return ops.layer_fingerprints(x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb3b, type_map, numtriplet)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad):
+        ga2, ge2, ga3, ge3 = ops.layer_fingerprints_grad(grad, *ctx.saved_tensors)
+        return None, None, ga2, ge2, None, None, ga3, ge3, None, None
+
+
+class _LayerForces(torch.autograd.Function):
+    """_Forces on the embeddings as they are trained (ops.layer_forces, ops.layer_forces_grad)."""
+
+    @staticmethod
+    def forward(ctx, netderiv2b, netderiv3b, x2b, intder2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, intder3b, intder3bsupp,
+                numtriplet, alpha3b, emb3b, type_map, tipos, type_now, pos, box):
+        ctx.save_for_backward(netderiv2b, netderiv3b, x2b, intder2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, intder3b,
+                              intder3bsupp, numtriplet, alpha3b, emb3b, type_map, tipos, type_now, pos, box)
+        out = ops.layer_forces(netderiv2b, netderiv3b, x2b, intder2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, intder3b,
+                               intder3bsupp, numtriplet, alpha3b, emb3b, type_map, tipos, type_now, pos, box)
+        if pos is not None:
+            ctx.shapes = (out[0].shape, out[1].shape)
+        return out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad_force, grad_virial=None):
+        saved = ctx.saved_tensors
+        pos, box = saved[-2:]
+        need = ctx.needs_input_grad
+        if pos is not None:
+            # a missing branch counts as zero (register_force_2bAFs_virial_grad.py:15-18)
+            x2b = saved[2]
+            grad_force = grad_force if grad_force is not None else x2b.new_zeros(ctx.shapes[0])
+            grad_virial = grad_virial if grad_virial is not None else x2b.new_zeros(ctx.shapes[1])
+        gn2, ga2, ge2, gn3, ga3, ge3 = ops.layer_forces_grad(grad_force, *saved[:-2], grad_virial, pos, box,
+                                                             (need[0] or need[5] or need[6], need[1] or need[12] or need[13]))
+        return (gn2, gn3, None, None, None, ga2, ge2, None, None, None, None, None, ga3, ge3, None, None, None, None, None)
+
+
+def _forces(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, type_emb_2b, x3b, x3bsupp, intder3b, intder3bsupp, int3b,
+            numtriplet, alpha3b, type_emb_3b, type_map, tipos, tn, pos, box):
+    # One call a species each way.  (Squares and their gradients as torch operations, an op per body and the sums around
+    # them were 250 of the 2500 us of host time that a step of a small box takes.)
+    tensors = (net_der_r, net_der_a, alpha2b, type_emb_2b, alpha3b, type_emb_3b)
+    if x2b.is_cuda and x2b.dtype == x3b.dtype and all(t.dtype == x2b.dtype for t in tensors):
+        try:
+            return _LayerForces.apply(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, type_emb_2b, x3b, x3bsupp, intder3b,
+                                      intder3bsupp, numtriplet, alpha3b, type_emb_3b, type_map, tipos, tn, pos, box)
+        except _lib.StafError as e:
+            if e.code != -12:   # (parameter rows of both bodies that do not fit one workgroup: nothing was launched)
+                raise
+    return _Forces.apply(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, torch.square(type_emb_2b), x3b, x3bsupp, intder3b,
+                         intder3bsupp, int3b, numtriplet, alpha3b, torch.square(type_emb_3b), type_map, tipos, tn, pos, box)
+
+
 class _Forces(torch.autograd.Function):
     """ComputeForceRadial + ComputeForceTripl of one centre species, or their Virial forms when pos and box are given
     (two outputs then).  One op (ops.compute_forces) adds the pair forces to the 3-body kernel's slot forces; the
@@ -195,6 +257,15 @@ class physics_layer(torch.nn.Module):
         self.output_dim = self.nalpha_r + self.nalpha_a
 
     def forward(self, x2b, x3bsupp, intmap2b, x3b, intmap3b, numtriplet, type_map):
+        tensors = (x3b, self.alpha2b, self.type_emb_2b, self.alpha3b, self.type_emb_3b)
+        if x2b.is_cuda and all(t.dtype == x2b.dtype for t in tensors) and self.alpha3b.shape[0] == self.alpha2b.shape[0] * (
+                self.alpha2b.shape[0] + 1) // 2:
+            try:
+                return _LayerFingerprints.apply(x2b, intmap2b, self.alpha2b, self.type_emb_2b, x3b, x3bsupp, self.alpha3b,
+                                                self.type_emb_3b, type_map, numtriplet)
+            except _lib.StafError as e:
+                if e.code != -12:
+                    raise
         emb2 = torch.square(self.type_emb_2b)
         emb3 = torch.square(self.type_emb_3b)
         af2 = _SortProj.apply(x2b, intmap2b, self.alpha2b, emb2, type_map)
@@ -263,9 +334,8 @@ class force_layer(torch.nn.Module):
     def forward(self, net_der_r, x2b, intder2b, int2b, alpha2b, net_der_a, x3b, x3bsupp, intder3b, intder3bsupp, int3b,
                 numtriplet, alpha3b, type_emb_2b, type_emb_3b, type_map, tipos, type_now):
         tn = _type_now(type_now, x2b.device)
-        return _Forces.apply(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, torch.square(type_emb_2b), x3b, x3bsupp,
-                             intder3b, intder3bsupp, int3b, numtriplet, alpha3b, torch.square(type_emb_3b), type_map, tipos,
-                             tn, None, None)
+        return _forces(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, type_emb_2b, x3b, x3bsupp, intder3b, intder3bsupp,
+                       int3b, numtriplet, alpha3b, type_emb_3b, type_map, tipos, tn, None, None)
 
 
 class force_virial_layer(torch.nn.Module):
@@ -282,6 +352,5 @@ class force_virial_layer(torch.nn.Module):
     def forward(self, net_der_r, x2b, intder2b, int2b, alpha2b, net_der_a, x3b, x3bsupp, intder3b, intder3bsupp, int3b,
                 numtriplet, alpha3b, type_emb_2b, type_emb_3b, type_map, tipos, type_now, pos, box):
         tn = _type_now(type_now, x2b.device)
-        return _Forces.apply(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, torch.square(type_emb_2b), x3b, x3bsupp,
-                             intder3b, intder3bsupp, int3b, numtriplet, alpha3b, torch.square(type_emb_3b), type_map, tipos,
-                             tn, pos, box)
+        return _forces(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, type_emb_2b, x3b, x3bsupp, intder3b, intder3bsupp,
+                       int3b, numtriplet, alpha3b, type_emb_3b, type_map, tipos, tn, pos, box)

@@ -550,6 +550,127 @@ def compute_force_tripl_virial(netderiv, radial_descriptor, angular_descriptor, 
                                pos, box)
 
 
+# --------------------------------------------------------------------------- the layers of a species as single calls
+
+_entries = {}
+
+
+def _entry(name, dtype, pointers_and_ints):
+    """C entry with its argument types set ('p' pointer, 'i' int): plain integers, and None for NULL, are passed as they
+    are, which for the forty arguments of these calls takes a third of the time of ctypes objects made one by one."""
+    key = (name, dtype)
+    if key not in _entries:
+        fn = getattr(_lib.lib(), f"{name}_{sfx(dtype)[0]}")
+        fn.argtypes = [C.c_void_p if a == "p" else C.c_int for a in pointers_and_ints]
+        fn.restype = C.c_int
+        _entries[key] = fn
+    return _entries[key]
+
+
+def _checked(rc, name):
+    if rc != _lib.STAF_OK:
+        raise _lib.StafError(rc, name)
+
+
+def _addr(t):
+    if t is None:
+        return None
+    if not t.is_contiguous():
+        raise ValueError("STAF ops need contiguous tensors")
+    return t.data_ptr()
+
+
+def _stream_addr():
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+def layer_fingerprints(x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb3b, type_map, numtriplet):
+    """Fingerprints [nf,Nl,Ar+Aa] of one centre species as physics_layer_mod.py:23-45 gives them: compute_sort_proj and
+    compute_sort_proj3body with the squares of emb2b, emb3b, one beside the other."""
+    dtype = x2b.dtype
+    nf, Nl, nr = x2b.shape
+    na = x3b.shape[2]
+    nt, Ar = alpha2b.shape
+    Aa = alpha3b.shape[1] // 3
+    v = _Views()
+    pD, pT, pS, pI, pN = v(x2b), v(x3b), v(x3bsupp), v(_i32(intmap2b)), v(_i32(numtriplet))
+    out = torch.empty((nf, Nl, Ar + Aa), dtype=dtype, device=x2b.device)
+    fn = _entry("staf_op_layer_fingerprints", dtype, "ppp" "iiii" "p" "pippip" "pp" "i" "p" "ip")
+    _checked(fn(pD, pS, pT, nr, na, nf, Nl, pI, _addr(_dense(alpha2b)), Ar, _addr(_dense(emb2b)), _addr(_dense(alpha3b)), Aa,
+                _addr(_dense(emb3b)), _addr(_i32(type_map)), pN, nt, out.data_ptr(), v.ld, _stream_addr()),
+             "staf_op_layer_fingerprints")
+    return out
+
+
+def layer_fingerprints_grad(grad, x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb3b, type_map, numtriplet):
+    """dL/dalpha2b, dL/demb2b, dL/dalpha3b, dL/demb3b (zero) of layer_fingerprints from dL/dfingerprints."""
+    dtype = x2b.dtype
+    nf, Nl, nr = x2b.shape
+    na = x3b.shape[2]
+    nt, Ar = alpha2b.shape
+    Aa = alpha3b.shape[1] // 3
+    v = _Views()
+    pD, pT, pS, pI, pN = v(x2b), v(x3b), v(x3bsupp), v(_i32(intmap2b)), v(_i32(numtriplet))
+    e = lambda t: torch.empty(t.shape, dtype=dtype, device=x2b.device)
+    ga2, ge2, ga3, ge3 = e(alpha2b), e(emb2b), e(alpha3b), e(emb3b)
+    fn = _entry("staf_op_layer_fingerprints_grad", dtype, "pppp" "iiii" "p" "pippip" "pp" "i" "pppp" "ip")
+    _checked(fn(_addr(_dense(grad)), pD, pS, pT, nr, na, nf, Nl, pI, _addr(_dense(alpha2b)), Ar, _addr(_dense(emb2b)),
+                _addr(_dense(alpha3b)), Aa, _addr(_dense(emb3b)), _addr(_i32(type_map)), pN, nt, ga2.data_ptr(),
+                ge2.data_ptr(), ga3.data_ptr(), ge3.data_ptr(), v.ld, _stream_addr()), "staf_op_layer_fingerprints_grad")
+    return ga2, ge2, ga3, ge3
+
+
+def layer_forces(netderiv2b, netderiv3b, x2b, intder2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, intder3b, intder3bsupp,
+                 numtriplet, alpha3b, emb3b, type_map, tipos, type_now, pos=None, box=None):
+    """compute_forces with the squares of emb2b, emb3b: force [nf,3N], or with pos and box (force, virial [nf,9])."""
+    dtype, dev = x3b.dtype, x3b.device
+    nf, Nl, na = x3b.shape
+    nr, N, nt = x3bsupp.shape[2], type_map.shape[0], tipos.shape[0]
+    Ar, Aa = alpha2b.shape[1], alpha3b.shape[1] // 3
+    v = _Views()
+    rows = [v(t) for t in (x2b, intder2b, x3bsupp, x3b, intder3bsupp, intder3b)]
+    pI, pN = v(_i32(intmap2b)), v(_i32(numtriplet))
+    force = torch.empty((nf, 3 * N), dtype=dtype, device=dev)
+    virial = torch.empty((nf, 9), dtype=dtype, device=dev) if pos is not None else None
+    at = _scalar_dev(type_now, dev)
+    fn = _entry("staf_op_layer_forces", dtype, "pp" "pppppp" "p" "iiiii" "pippip" "i" "pppp" "pppp" "ip")
+    _checked(fn(_addr(_dense(netderiv2b)), _addr(_dense(netderiv3b)), *rows, pI, nr, na, N, nf, Nl, _addr(_dense(alpha2b)), Ar,
+                _addr(_dense(emb2b)), _addr(_dense(alpha3b)), Aa, _addr(_dense(emb3b)), nt, _addr(_i32(tipos)), _addr(at), pN,
+                _addr(_i32(type_map)), force.data_ptr(), _addr(virial), _addr(None if pos is None else _dense(pos)),
+                _addr(None if box is None else _dense(box)), v.ld, _stream_addr()), "staf_op_layer_forces")
+    return force if pos is None else (force, virial)
+
+
+def layer_forces_grad(prevgrad, netderiv2b, netderiv3b, x2b, intder2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, intder3b,
+                      intder3bsupp, numtriplet, alpha3b, emb3b, type_map, tipos, type_now, prevgrad_virial=None, pos=None,
+                      box=None, bodies=(True, True)):
+    """Gradients of layer_forces: (gradnet2b, dL/dalpha2b, dL/demb2b, gradnet3b, dL/dalpha3b, dL/demb3b), None for a body that
+    is not asked for."""
+    dtype, dev = x3b.dtype, x3b.device
+    nf, Nl, na = x3b.shape
+    nr, N, nt = x3bsupp.shape[2], type_map.shape[0], tipos.shape[0]
+    Ar, Aa = alpha2b.shape[1], alpha3b.shape[1] // 3
+    v = _Views()
+    rows = [v(t) for t in (x2b, intder2b, x3bsupp, x3b, intder3bsupp, intder3b)]
+    pI, pN = v(_i32(intmap2b)), v(_i32(numtriplet))
+    e = lambda *sh: torch.empty(sh, dtype=dtype, device=dev)
+    out = [None] * 6
+    if bodies[0]:
+        out[:3] = e(nf, Nl, Ar), e(*alpha2b.shape), e(*emb2b.shape)
+    if bodies[1]:
+        out[3:] = e(nf, Nl, Aa), e(*alpha3b.shape), e(*emb3b.shape)
+    at = _scalar_dev(type_now, dev)
+    fn = _entry("staf_op_layer_forces_grad", dtype,
+                "ppp" "pppppp" "p" "iiiii" "pippip" "i" "pppp" "pppppp" "ppp" "ip")
+    _checked(fn(_addr(_dense(prevgrad)), _addr(_dense(netderiv2b)), _addr(_dense(netderiv3b)), *rows, pI, nr, na, N, nf, Nl,
+                _addr(_dense(alpha2b)), Ar, _addr(_dense(emb2b)), _addr(_dense(alpha3b)), Aa, _addr(_dense(emb3b)), nt,
+                _addr(_i32(tipos)), _addr(at), pN, _addr(_i32(type_map)), *[_addr(t) for t in out],
+                _addr(None if prevgrad_virial is None else _dense(prevgrad_virial)),
+                _addr(None if pos is None else _dense(pos)), _addr(None if box is None else _dense(box)), v.ld,
+                _stream_addr()), "staf_op_layer_forces_grad")
+    return tuple(out)
+
+
 # --------------------------------------------------------------------------- parameter gradients (energy branch)
 
 

@@ -488,6 +488,66 @@ int staf_op_frames_f64(const double* positions, const double* boxer, int nf, int
                        const StafFramesSpecies* species, const int* type_map, void* work, size_t work_bytes,
                        double* energy, double* force, double* virial, void* stream);
 
+/* The physics and force layers of one centre species as single calls (STAF/source_routine/physics_layer_mod.py:23-45,
+ * force_layer_mod.py:22-44 and :92-103): the embeddings are given as they are trained, squared where they are read, and
+ * their gradients come back with respect to them (what tf.square's gradient makes of the ops').  Arrays as for the single
+ * ops; fingerprints and dL/dfingerprints are [nf, N_local, Ar + Aa], 2-body first.
+ * staf_op_layer_fingerprints_grad: dL/dalpha2b, dL/demb2b [nt,Ar], dL/dalpha3b [ntc,3Aa], dL/demb3b [ntc,Aa] (zero).
+ * staf_op_layer_forces: forces [nf,3N] and, when virial, pos and box are given, virial [nf,9], as staf_op_forces.
+ * staf_op_layer_forces_grad: the outputs of both gradient ops of the forces; a null grad_alpha2b or grad_alpha3b leaves that
+ * body out; prevgrad_virial, pos and box: the virial forms.
+ * Limits as for the single ops and staf_op_forces. */
+int staf_op_layer_fingerprints_f32(const float* raddescr, const float* des3bsupp, const float* angdescr, int nr, int na, int dimbat,
+                                   int N_local, const int* intmap_r, const float* alpha2b, int nalpha_r,
+                                   const float* type_emb2b, const float* alpha3b, int nsmooth_a, const float* type_emb3b,
+                                   const int* type_map, const int* num_triplets, int nt, float* fingerprints, int ld_atoms,
+                                   void* stream);
+int staf_op_layer_fingerprints_grad_f32(const float* prevgrad, const float* raddescr, const float* des3bsupp,
+                                        const float* angdescr, int nr, int na, int dimbat, int N_local, const int* intmap_r,
+                                        const float* alpha2b, int nalpha_r, const float* type_emb2b, const float* alpha3b,
+                                        int nsmooth_a, const float* type_emb3b, const int* type_map, const int* num_triplets,
+                                        int nt, float* grad_alpha2b, float* grad_emb2b, float* grad_alpha3b, float* grad_emb3b,
+                                        int ld_atoms, void* stream);
+int staf_op_layer_forces_f32(const float* netderiv2b, const float* netderiv3b, const float* raddescr, const float* der2b,
+                             const float* des3bsupp, const float* angdescr, const float* der3bsupp, const float* der3b,
+                             const int* intmap_r, int nr, int na, int N, int dimbat, int N_local, const float* alpha2b,
+                             int nalpha_r, const float* type_emb2b, const float* alpha3b, int nsmooth_a, const float* type_emb3b,
+                             int nt, const int* tipos, const int* actual_type, const int* num_triplets, const int* type_map,
+                             float* forces, float* virial, const float* pos, const float* box, int ld_atoms, void* stream);
+int staf_op_layer_forces_grad_f32(const float* prevgrad, const float* netderiv2b, const float* netderiv3b, const float* raddescr,
+                                  const float* der2b, const float* des3bsupp, const float* angdescr, const float* der3bsupp,
+                                  const float* der3b, const int* intmap_r, int nr, int na, int N, int dimbat, int N_local,
+                                  const float* alpha2b, int nalpha_r, const float* type_emb2b, const float* alpha3b, int nsmooth_a,
+                                  const float* type_emb3b, int nt, const int* tipos, const int* actual_type,
+                                  const int* num_triplets, const int* type_map, float* gradnet_2b, float* grad_alpha2b,
+                                  float* grad_emb2b, float* gradnet_3b, float* grad_alpha3b, float* grad_emb3b,
+                                  const float* prevgrad_virial, const float* pos, const float* box, int ld_atoms, void* stream);
+int staf_op_layer_fingerprints_f64(const double* raddescr, const double* des3bsupp, const double* angdescr, int nr, int na, int dimbat,
+                                   int N_local, const int* intmap_r, const double* alpha2b, int nalpha_r,
+                                   const double* type_emb2b, const double* alpha3b, int nsmooth_a, const double* type_emb3b,
+                                   const int* type_map, const int* num_triplets, int nt, double* fingerprints, int ld_atoms,
+                                   void* stream);
+int staf_op_layer_fingerprints_grad_f64(const double* prevgrad, const double* raddescr, const double* des3bsupp,
+                                        const double* angdescr, int nr, int na, int dimbat, int N_local, const int* intmap_r,
+                                        const double* alpha2b, int nalpha_r, const double* type_emb2b, const double* alpha3b,
+                                        int nsmooth_a, const double* type_emb3b, const int* type_map, const int* num_triplets,
+                                        int nt, double* grad_alpha2b, double* grad_emb2b, double* grad_alpha3b, double* grad_emb3b,
+                                        int ld_atoms, void* stream);
+int staf_op_layer_forces_f64(const double* netderiv2b, const double* netderiv3b, const double* raddescr, const double* der2b,
+                             const double* des3bsupp, const double* angdescr, const double* der3bsupp, const double* der3b,
+                             const int* intmap_r, int nr, int na, int N, int dimbat, int N_local, const double* alpha2b,
+                             int nalpha_r, const double* type_emb2b, const double* alpha3b, int nsmooth_a, const double* type_emb3b,
+                             int nt, const int* tipos, const int* actual_type, const int* num_triplets, const int* type_map,
+                             double* forces, double* virial, const double* pos, const double* box, int ld_atoms, void* stream);
+int staf_op_layer_forces_grad_f64(const double* prevgrad, const double* netderiv2b, const double* netderiv3b, const double* raddescr,
+                                  const double* der2b, const double* des3bsupp, const double* angdescr, const double* der3bsupp,
+                                  const double* der3b, const int* intmap_r, int nr, int na, int N, int dimbat, int N_local,
+                                  const double* alpha2b, int nalpha_r, const double* type_emb2b, const double* alpha3b, int nsmooth_a,
+                                  const double* type_emb3b, int nt, const int* tipos, const int* actual_type,
+                                  const int* num_triplets, const int* type_map, double* gradnet_2b, double* grad_alpha2b,
+                                  double* grad_emb2b, double* gradnet_3b, double* grad_alpha3b, double* grad_emb3b,
+                                  const double* prevgrad_virial, const double* pos, const double* box, int ld_atoms, void* stream);
+
 /* Sum of up to four arrays of n elements, dst[e] = ((a[e] + b[e]) + c[e]) + d[e] (c, d may be null), in one launch:
  * what the callers do with the per-op force arrays (force_radial + force_angular in
  * STAF/source_routine/force_layer_mod.py:43, tf.math.add_n over the species in

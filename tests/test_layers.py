@@ -270,3 +270,58 @@ def test_forces_in_one_op_do_not_read_the_padding_of_the_rows(dtype):
                          P["emb2b"].sqrt(), P["emb3b"].sqrt(), tm, tp, 0, tpos, tbox))
     for x, y in zip(*out):
         assert bool(torch.isfinite(x).all()) and torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("counts", [(32, 64), (96, 0), (1, 95)])
+@pytest.mark.parametrize("virial", [False, True])
+def test_layers_as_single_calls_give_the_bits_of_the_ops_on_squared_embeddings(dtype, counts, virial):
+    """physics_layer, force_layer and force_virial_layer square the embeddings where the kernels read them and write the
+    gradients of the unsquared ones; the values and gradients of the op-by-op route on torch's squares, to the last bit
+    (the same sums, and g (2 e) is one rounding either way), with a species without atoms and one of a single atom."""
+    import torch
+    from alphanesgpu_amd import layers, ops, synth
+    dev, dt = torch.device("cuda:0"), getattr(torch, dtype)
+    nr, na, N = 60, 1770, 96
+    frames = [synth.water_frame((4, 4, 2), 9.86, 0.05, seed) for seed in (3, 4)]
+    T = lambda a: torch.as_tensor(np.ascontiguousarray(a)).to(dev)
+    tpos, tbox = (T(np.stack(a)).to(dt) for a in zip(*frames))
+    tm, tp = T(np.repeat(np.arange(2, dtype=np.int32), counts)), T(np.array(counts, np.int32))
+    ops.construct_descriptors_light(synth.RC, nr, na, N, tbox, synth.RS, synth.RA, 2, dtype=dt)
+    rad, ang, sup, im2, im3, d2, d3, d3s, ntr = ops.compute_descriptors_light(tpos, tbox)
+    g = torch.Generator(device=dev)
+    g.manual_seed(5)
+    rand = lambda *sh: torch.randn(sh, dtype=dt, device=dev, generator=g)
+    o = 0
+    for k, (p, n) in enumerate(zip(synth.fingerprint_params(2, dtype=getattr(np, dtype)), counts)):
+        c = lambda t: t[:, o:o + n]
+        ph = layers.physics_layer(T(p["alpha2b"]), T(p["alpha3b"]), [0.5 + rand(*p["emb2b"].shape).abs(),
+                                                                      T(p["emb3b"]) * (0.5 + rand(*p["emb3b"].shape).abs())])
+        par = list(ph.parameters())
+        U, Q, Qw = rand(2, n, ph.output_dim), rand(2, 3 * N), rand(2, 9)
+        G = [rand(2, n, w).requires_grad_(True) for w in (ph.nalpha_r, ph.nalpha_a)]
+        af = ph(c(rad), c(sup), c(im2), c(ang), c(im3), c(ntr), tm)
+        af_ops = torch.cat([layers._SortProj.apply(c(rad), c(im2), ph.alpha2b, torch.square(ph.type_emb_2b), tm),
+                            layers._SortProj3body.apply(c(ang), c(sup), c(im3), c(im2), ph.alpha3b,
+                                                        torch.square(ph.type_emb_3b), tm, c(ntr))], dim=2)
+        assert torch.equal(af, af_ops)
+        for x, y in zip(torch.autograd.grad(af, par, U), torch.autograd.grad(af_ops, par, U)):
+            assert torch.equal(x, y)
+        layer = layers.force_virial_layer(nr, na) if virial else layers.force_layer(nr, na)
+        box = (tpos, tbox) if virial else (None, None)
+        F = layer(G[0], c(rad), c(d2), c(im2), ph.alpha2b, G[1], c(ang), c(sup), c(d3), c(d3s), c(im3), c(ntr), ph.alpha3b,
+                  ph.type_emb_2b, ph.type_emb_3b, tm, tp, k, *(box if virial else ()))
+        tn = T(np.array([k], np.int32))
+        F_ops = layers._Forces.apply(G[0], G[1], c(rad), c(d2), c(im2), ph.alpha2b, torch.square(ph.type_emb_2b), c(ang), c(sup),
+                                     c(d3), c(d3s), c(im3), c(ntr), ph.alpha3b, torch.square(ph.type_emb_3b), tm, tp, tn, *box)
+        F, F_ops = ([t] if not virial else list(t) for t in (F, F_ops))
+        assert all(torch.equal(x, y) for x, y in zip(F, F_ops))
+        up = [Q, Qw][:len(F)]
+        wanted = G + [ph.alpha2b, ph.alpha3b, ph.type_emb_2b, ph.type_emb_3b]
+        for x, y in zip(torch.autograd.grad(F, wanted, up, retain_graph=True), torch.autograd.grad(F_ops, wanted, up)):
+            assert torch.equal(x, y)
+        x, = torch.autograd.grad(F, G[1:], up)   # (one body alone, one output alone)
+        if n:
+            assert bool(x.abs().max() > 0)
+        o += n
