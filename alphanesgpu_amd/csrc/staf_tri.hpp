@@ -42,7 +42,6 @@ namespace staf {
 
 constexpr int TRI_BLOCK = 256;
 constexpr int TRI_CAP = 16;    // channels tabulated per pass = lanes of a subset
-constexpr int TRI_CAPP = TRI_CAP + 1;   // table row pitch: the entry after a row's channels holds (D, V) of its slot
 // BLOCK: threads per workgroup, 256 or, for the fingerprints of a small launch (step_fingerprints), 512.
 template <typename real, int MODE, bool FUSED = false, int BLOCK = TRI_BLOCK>
 struct TriCfg {
@@ -51,19 +50,25 @@ struct TriCfg {
   // pieces of 1280 bytes a CU hands out, which is exactly a fourth (192, counted on 40 KB per workgroup, was the
   // earlier choice: 336.7 -> 333.3 us per fp64 training step; 272, not a power of two, is slower again).
   // The fused double-precision fingerprint kernel (the MD entry: thousands of centres per launch, several per
-  // workgroup) stages 160: five workgroups per CU instead of four.  The plain double-precision fingerprint kernel
-  // stages 448: a CU hands out its 160 KB of LDS in pieces of 1280 bytes, so the 32496 bytes that 512 staged triplets
+  // workgroup) stages 128, and its registers are held to six waves per SIMD: 26832 bytes of LDS and six workgroups per
+  // CU (160 and five before: with the table's rows of sixteen below, 426 -> 409 us for 24576 centres, 118 -> 113 for
+  // 6144).  The plain double-precision fingerprint kernel stages 448: a CU hands out its 160 KB of LDS in pieces of 1280 bytes, so the 32496 bytes that 512 staged triplets
   // make count as 33280 and four workgroups fit, not the five that the occupancy query of the runtime reports
   // (measured with a kernel that counts its resident workgroups per CU); with 448 it is 31472 bytes and five
   // (6144-atom step 360.6 -> 356.8 us).
-  static constexpr int QB = BLOCK > TRI_BLOCK ? 512 : sizeof(real) == 8 ? (MODE == 3 ? 256 : MODE == 2 ? 448 : FUSED ? 160 : MODE == 0 ? 448 : 512) : 512;
+  static constexpr int QB = BLOCK > TRI_BLOCK ? 512 : sizeof(real) == 8 ? (MODE == 3 ? 256 : MODE == 2 ? 448 : FUSED ? 128 : MODE == 0 ? 448 : 512) : 512;
   // waves per SIMD the register allocation is held to: without a bound the allocation comes out a few registers
   // above the next occupancy step.  The
   // single-precision pass for both gradients is held to six (80 registers, 56 bytes of spill per lane outside the
   // item loop) where it would take 95 and run four: 146 against 168 us per 8-frame step; seven (with a staging block
   // of 256 so that seven workgroups fit a CU's LDS) is slower again (156 us).
-  static constexpr int MIN_WAVES = BLOCK > TRI_BLOCK ? 4 : sizeof(real) == 8 ? (MODE == 0 ? 5 : 4)   // also the fused fingerprint kernel's
+  static constexpr int MIN_WAVES = BLOCK > TRI_BLOCK ? 4 : sizeof(real) == 8 ? (MODE == 0 ? (FUSED ? 6 : 5) : 4)
                                                      : (MODE == 0 ? 8 : MODE == 1 ? 7 : MODE == 3 ? 6 : 5);
+  // Entries of a table row.  Of the gradient modes' rows the one after the channels holds (D, V) of its slot; the
+  // fingerprints' rows are the sixteen channels alone, 256 bytes in double precision, so that the sixteen lanes of every
+  // subset read the same banks in the same order whichever rows they are at (a 16-byte read per lane of four rows 272
+  // bytes apart takes 8.3 clocks of a CU's LDS, of whole rows of 256 bytes 4.7; the launch of 24576 centres 430 -> 420 us).
+  static constexpr int PITCH = MODE == 0 ? TRI_CAP : TRI_CAP + 1;
   static constexpr bool FORCE_BRANCH = MODE == 2 || MODE == 3;    // dL/dF comes in: der3b, der3bsupp are read
   static constexpr bool ENERGY_BRANCH = MODE == 1 || MODE == 3;   // dL/dAF3 comes in
 };
@@ -306,7 +311,7 @@ struct TriLds {
   static constexpr int QB = TriCfg<real, MODE, FUSED, BLOCK>::QB, WAVES = BLOCK / WAVE;
   __host__ __device__ static size_t n_reals(int nr, int Aa, int nt, bool fused = false) {
     const int nsig = 2 * nt - 1;
-    size_t r = (size_t)nr * TRI_CAPP * 2;                   // pair tables (real2 per (row, channel)), + (D, V) per row
+    size_t r = (size_t)nr * TriCfg<real, MODE>::PITCH * 2;  // pair tables (real2 per (row, channel)), + (D, V) per row
     if (fused) r += (size_t)3 * nr;                         // unit vectors of the slots
     r += nr;                                                // sD
     r += (size_t)NG * Aa;                                   // sP (and sPE)
@@ -341,6 +346,7 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
   constexpr int WAVES = BLOCK / WAVE, SUBS = BLOCK / TRI_CAP;
   constexpr int TRI_QB = TriCfg<real, MODE, FUSED, BLOCK>::QB;
   constexpr bool FB = TriCfg<real, MODE>::FORCE_BRANCH;
+  constexpr int TRI_CAPP = TriCfg<real, MODE>::PITCH;
   extern __shared__ __align__(16) unsigned char smem[];
   const int nr = A.nr, na = A.na, Aa = A.Aa, nt = A.nt;
   const int nsig = 2 * nt - 1;
@@ -532,7 +538,7 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
               v.y = HE::eval(a2s * d, etab);
               tabE[row * TRI_CAPP + ia] = v;
             }
-            if (ia == 0) {
+            if (MODE != 0 && ia == 0) {
               real2 v;
               v.x = d;
               v.y = FB ? sV[s] : real(0);
