@@ -81,15 +81,52 @@ struct PinBuf {
 // an otherwise empty chain of kernels, the two kernels and flags that the host watches 19 and 24 (24576 atoms: 60 and 43).
 // MD calls of 96, 768, 6144 and 24576 atoms: 90 -> 82, 136 -> 107, 417 -> 387 and 1340 -> 1313 us; with a caller's list,
 // 1500 and 6144 atoms: 223 -> 213 and 553 -> 529.
+// They also take the positions from the caller's order to the species-sorted slots and the forces back, and a changed order
+// and species along, which the host did in loops over the atoms and with a copy of its own: calls of 768, 6144 and 24576
+// atoms in an order that changes every time 101 -> 99, 386 -> 370 and 1299 -> 1245 us, with a caller's list, whose ghosts
+// change species, 1500 and 6144 atoms 209 -> 170 and 533 -> 490.
 constexpr int IO_THREADS = 256, IN_BLOCKS = 256, OUT_BLOCKS = 64;
-__global__ __launch_bounds__(IO_THREADS) void call_in_kernel(const double2* __restrict__ host, double2* __restrict__ dev, int n) {
-  for (int i = blockIdx.x * IO_THREADS + threadIdx.x; i < n; i += gridDim.x * IO_THREADS) dev[i] = host[i];
+// The first n3 doubles are positions in the caller's order and go to the atoms' slots; the rest is copied as it is.  new_order:
+// the slots have changed; their numbers and the atoms' species lie in host memory too, and further workgroups keep them on
+// the device for the calls that follow: order_d (and behind it the owned slots' atoms) and the slots' species.
+struct CallOrder {
+  const int* new_order;   // [slot of every atom nall | species of every atom nall] or null
+  int *order_d, *type_map;
+  int nall, nlocal, blocks;   // blocks: workgroups that copy the first part
+};
+__global__ __launch_bounds__(IO_THREADS) void call_in_kernel(const double2* __restrict__ host, double* __restrict__ dev, int n3,
+                                                             int n, const CallOrder O) {
+  if ((int)blockIdx.x < O.blocks) {
+    const int* const slot_of = O.new_order ? O.new_order : O.order_d;
+    for (int i = blockIdx.x * IO_THREADS + threadIdx.x; i < n; i += O.blocks * IO_THREADS) {
+      const double2 v = host[i];
+      const int e = 2 * i;
+      dev[e < n3 ? 3 * slot_of[e / 3] + e % 3 : e] = v.x;
+      dev[e + 1 < n3 ? 3 * slot_of[(e + 1) / 3] + (e + 1) % 3 : e + 1] = v.y;
+    }
+  } else {
+    const int step = (gridDim.x - O.blocks) * IO_THREADS;
+    for (int i = (blockIdx.x - O.blocks) * IO_THREADS + threadIdx.x; i < O.nall; i += step) {
+      const int s = O.new_order[i], t = O.new_order[O.nall + i];
+      O.order_d[i] = s;
+      O.type_map[s] = t;
+      if (i < O.nlocal) O.order_d[O.nall + s] = i;
+    }
+  }
 }
+// Forces in the caller's order, the rest as it is.
 // The error words go along.  A workgroup's flag says that everything it copied has arrived: its threads' stores are released
 // to the host before the flag is written.
-__global__ __launch_bounds__(IO_THREADS) void call_out_kernel(const double2* __restrict__ dev, double2* __restrict__ host, int n,
-                                                              int* status, int* status_h, unsigned* flags, unsigned call) {
-  for (int i = blockIdx.x * IO_THREADS + threadIdx.x; i < n; i += gridDim.x * IO_THREADS) host[i] = dev[i];
+__global__ __launch_bounds__(IO_THREADS) void call_out_kernel(const double* __restrict__ dev, double2* __restrict__ host,
+                                                              const int* __restrict__ slot_of, int n3, int n, int* status,
+                                                              int* status_h, unsigned* flags, unsigned call) {
+  for (int i = blockIdx.x * IO_THREADS + threadIdx.x; i < n; i += gridDim.x * IO_THREADS) {
+    double2 v;
+    const int e = 2 * i;
+    v.x = dev[e < n3 ? 3 * slot_of[e / 3] + e % 3 : e];
+    v.y = dev[e + 1 < n3 ? 3 * slot_of[(e + 1) / 3] + (e + 1) % 3 : e + 1];
+    host[i] = v;
+  }
   if (blockIdx.x == 0 && threadIdx.x < staf::STATUS_WORDS)
     status_h[threadIdx.x] = __hip_atomic_load(&status[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __threadfence_system();
@@ -148,14 +185,20 @@ struct StafModel {
   hipStream_t stream = nullptr;            // the call's stream
   // device buffers
   // in_d  = [pos nall*3 | box 6], with a caller's list behind them, in ints,
-  //         [howmany nlocal | slot of every atom nall | atom of every owned slot nlocal | rows nlocal*pitch]
-  //         (mirror of in_h, one copy per call)
-  // out_d = [force nall*3 | rows of (virial 9, energy), sums over shares of the centres]  (mirror of out_h, one copy)
+  //         [howmany nlocal | rows nlocal*pitch]
+  //         (in_h the same with the positions in the caller's order, and a changed order, as in `order`, behind them)
+  // out_d = [force nall*3 | rows of (virial 9, energy), sums over shares of the centres]  (out_h: forces in the caller's order)
   DevBuf<double> in_d, out_d, force_op, virial_op, af2, af3, g2, g3, e_atom, vpart;
   PinBuf<double> in_h, out_h;
   PinBuf<unsigned> done_h;   // [OUT_BLOCKS flags of call_out_kernel | error words]
   unsigned calls = 0;
-  std::vector<int> type_map_up, tipos_up;   // what the device copies of type_map and tipos hold
+  // The atoms' order: made for the types of a call and kept for the calls that follow with the same ones (in MD they change
+  // when atoms migrate, not every step).  order_ready: tipos_h, order and type_map are those of
+  // types_seen.
+  std::vector<int> types_seen, tipos_h;
+  int nlocal_seen = 0;
+  bool order_ready = false;
+  std::vector<int> tipos_up;   // what the device's tipos holds
   bool actual_type_up = false;
   // device-resident MLP (default); false: the host evaluation of staf_mlp.cpp between the kernels
   bool dev_mlp = false;
@@ -163,6 +206,7 @@ struct StafModel {
   DevBuf<double> raddescr, des3bsupp, der2b, der3bsupp, unit;   // nr-wide rows per owned atom; unit = (u, 1/r)
   DevBuf<double> slotf, selff;   // slot forces [nlocal, nr, 3] and centres' own forces [nlocal, 3]
   DevBuf<int> intmap2b, numtriplet, type_map, tipos, actual_type;
+  DevBuf<int> order;   // [slot of every atom nall | atom of every owned slot nlocal]
   // a caller's list transposed (atom -> the centres and slots that list it): counters, which read zero between builds (tr_clear:
   // they do), counts and keys
   DevBuf<int> tr_build, tr_cnt, tr_keys;
@@ -170,7 +214,6 @@ struct StafModel {
   // host staging
   std::vector<double> af_h, gr_h, tmp2, tmp3;
   std::vector<float> af_f, gr_f;
-  std::vector<int> order_to_slot, slot_to_order, type_map_h;
 };
 
 static bool load_species_params(StafModel* m) {
@@ -266,7 +309,7 @@ void staf_free(StafModel* m) {
                             &m->e_atom, &m->vpart, &m->raddescr, &m->des3bsupp, &m->der2b, &m->der3bsupp, &m->unit,
                             &m->slotf, &m->selff})
     b->release();
-  for (DevBuf<int>* b : {&m->intmap2b, &m->numtriplet, &m->type_map, &m->tipos, &m->actual_type, &m->tr_build, &m->tr_cnt,
+  for (DevBuf<int>* b : {&m->intmap2b, &m->numtriplet, &m->type_map, &m->tipos, &m->actual_type, &m->order, &m->tr_build, &m->tr_cnt,
                          &m->tr_keys})
     b->release();
   delete m;
@@ -352,33 +395,32 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   const int nt = m->nt, nr = m->nr, na = m->na;
 
   // ---- owned atoms species-sorted into slots [0, nlocal), ghosts keep their order behind them
-  std::vector<int> tipos(nt, 0), cursor(nt, 0);
-  for (int i = 0; i < nlocal; i++) {
-    const int sp = type ? type[i] : 0;
-    if (sp < 0 || sp >= nt) {
-      fprintf(stderr, "staf_compute: unsupported type %d at atom %d\n", sp, i);
+  const bool same_order = m->order_ready && m->nlocal_seen == nlocal && m->types_seen.size() == (size_t)nall &&
+                          (type ? memcmp(type, m->types_seen.data(), (size_t)nall * sizeof(int)) == 0
+                                : std::all_of(m->types_seen.begin(), m->types_seen.end(), [](int t) { return t == 0; }));
+  if (!same_order) {
+    m->order_ready = false;
+    m->tipos_h.assign(nt, 0);
+    int known = 0;
+    for (int t = 0; t < nt; t++) {
+      int n = 0;
+      for (int i = 0; i < nlocal; i++) n += (type ? type[i] : 0) == t;
+      m->tipos_h[t] = n;
+      known += n;
+    }
+    if (known != nlocal) {
+      int i = 0;
+      while (type[i] >= 0 && type[i] < nt) i++;
+      fprintf(stderr, "staf_compute: unsupported type %d at atom %d\n", type[i], i);
       return -8;
     }
-    tipos[sp]++;
+    for (int i = nlocal; i < nall; i++)
+      if (type && (type[i] < 0 || type[i] >= nt)) return -8;
+    if (type) m->types_seen.assign(type, type + nall);
+    else m->types_seen.assign(nall, 0);
+    m->nlocal_seen = nlocal;
   }
-  for (int t = 1; t < nt; t++) cursor[t] = cursor[t - 1] + tipos[t - 1];
-  m->order_to_slot.resize(nall);
-  m->slot_to_order.resize(nall);
-  m->type_map_h.resize(nall);
-  for (int i = 0; i < nlocal; i++) {
-    const int sp = type ? type[i] : 0;
-    const int slot = cursor[sp]++;
-    m->order_to_slot[i] = slot;
-    m->slot_to_order[slot] = i;
-    m->type_map_h[slot] = sp;
-  }
-  for (int i = nlocal; i < nall; i++) {
-    const int sp = type ? type[i] : 0;
-    if (sp < 0 || sp >= nt) return -8;
-    m->order_to_slot[i] = i;
-    m->slot_to_order[i] = i;
-    m->type_map_h[i] = sp;
-  }
+  const std::vector<int>& tipos = m->tipos_h;
   // ---- the call's input block, written straight into pinned memory
   const size_t L = (size_t)nlocal;
   const size_t n_in_d = (size_t)nall * 3 + 6;                                 // doubles
@@ -389,23 +431,19 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   const int row_max = std::min(nr, maxneigh);   // truncated like the reference (staf_api.cpp:321-323)
   if (ext)
     for (int i = 0; i < nlocal; i++) pitch = std::max(pitch, std::min(howmany[i], row_max));
-  const size_t n_in_i = ext ? 2 * L + nall + L * pitch : 0;                   // ints behind them
+  const size_t n_in_i = ext ? L + L * pitch : 0;                              // ints behind them
   const size_t n_in = (n_in_d + (n_in_i + 1) / 2 + 1) & ~(size_t)1;           // (copied by twos)
   const int nparts = std::min(64, (nlocal + 255) / 256);   // shares of the centres' virial and energy sums
   const size_t n_out = ((size_t)nall * 3 + (size_t)nparts * 10 + 1) & ~(size_t)1;
-  if (!m->in_h.reserve(n_in) || !m->out_h.reserve(n_out)) return -1;
+  if (!m->in_h.reserve(n_in + (same_order ? 0 : (size_t)nall)) || !m->out_h.reserve(n_out)) return -1;
   if (!m->done_h.p) {
     if (!m->done_h.reserve(OUT_BLOCKS + staf::STATUS_WORDS)) return -1;
     memset(m->done_h.p, 0, (OUT_BLOCKS + staf::STATUS_WORDS) * sizeof(unsigned));
   }
   double* pos_h = m->in_h.p;
   int* how_h = (int*)(m->in_h.p + n_in_d);
-  int* slot_of_h = how_h + L;
-  int* row_of_h = slot_of_h + nall;
-  int* with_h = row_of_h + L;
+  int* with_h = how_h + L;
   if (ext) {
-    memcpy(slot_of_h, m->order_to_slot.data(), (size_t)nall * sizeof(int));
-    memcpy(row_of_h, m->slot_to_order.data(), L * sizeof(int));
     for (int i = 0; i < nlocal; i++) {
       const int nn = std::max(0, std::min(howmany[i], row_max));
       how_h[i] = nn;
@@ -427,23 +465,39 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
       }
     }
   }
-  for (int i = 0; i < nall; i++) {
-    const int s = m->order_to_slot[i];
-    pos_h[3 * s] = x[3 * i];
-    pos_h[3 * s + 1] = x[3 * i + 1];
-    pos_h[3 * s + 2] = x[3 * i + 2];
-  }
+  memcpy(pos_h, x, (size_t)nall * 3 * sizeof(double));
   memcpy(pos_h + (size_t)nall * 3, box, 6 * sizeof(double));
+  if (!same_order) {
+    // the slots, in the caller's order within a species.  (Two species: one running number; with a table of running numbers
+    // every atom waits for the one before it to be stored, 40 us for 24576 atoms.)
+    int* const slot = (int*)(m->in_h.p + n_in);
+    const int* const t = m->types_seen.data();
+    if (nt <= 2) {
+      int zeros = 0;
+      const int n0 = tipos[0];
+      for (int i = 0; i < nlocal; i++) {
+        const int one = t[i];
+        slot[i] = one ? n0 + i - zeros : zeros;
+        zeros += 1 - one;
+      }
+    } else {
+      std::vector<int> cursor(nt, 0);
+      for (int k = 1; k < nt; k++) cursor[k] = cursor[k - 1] + tipos[k - 1];
+      for (int i = 0; i < nlocal; i++) slot[i] = cursor[t[i]]++;
+    }
+    for (int i = nlocal; i < nall; i++) slot[i] = i;
+    memcpy(slot + nall, t, (size_t)nall * sizeof(int));
+  }
 
   // ---- device buffers
   int amax2 = 0, amax3 = 0;
   for (int k = 0; k < nt; k++) { amax2 = m->Ar[k] > amax2 ? m->Ar[k] : amax2; amax3 = m->Aa[k] > amax3 ? m->Aa[k] : amax3; }
-  const int* type_map_before = m->type_map.p;
   bool ok = m->in_d.reserve(n_in) && m->out_d.reserve(n_out) && m->af2.reserve(L * amax2) &&
             m->af3.reserve(L * amax3) && m->g2.reserve(L * amax2) && m->g3.reserve(L * amax3) &&
             m->raddescr.reserve(L * nr) && m->des3bsupp.reserve(L * nr) && m->der2b.reserve(L * 3 * nr) &&
             m->der3bsupp.reserve(L * 3 * nr) && m->unit.reserve(L * 4 * nr) && m->intmap2b.reserve(L * (nr + 1)) &&
-            m->numtriplet.reserve(L) && m->type_map.reserve(nall) && m->tipos.reserve(nt) && m->actual_type.reserve(nt);
+            m->numtriplet.reserve(L) && m->type_map.reserve(nall) && m->tipos.reserve(nt) && m->actual_type.reserve(nt) &&
+            m->order.reserve((size_t)nall + L);
   // Slot forces of both bodies and all species from one launch, or, for neighbour buffers and parameter rows that leave no
   // room for both bodies in a workgroup's LDS (three species: 250 slots), an op per body and species.
   bool one_force_launch = m->dev_mlp;
@@ -461,26 +515,24 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     ok = ok && room(m->tr_build, nall) && room(m->tr_cnt, nall) && room(m->tr_keys, (size_t)nall * tr_cap);
   }
   if (!ok) return -1;
-  if (m->type_map.p != type_map_before) m->type_map_up.clear();   // a new block holds nothing yet
   hipStream_t st = m->stream;
   double* const d_pos = m->in_d.p;
   double* const d_box = d_pos + (size_t)nall * 3;
   int* const d_how = (int*)(m->in_d.p + n_in_d);
-  const staf::NeighList list = {d_how, d_how + L + nall + L, d_how + L + nall, d_how + L, pitch};
+  const staf::NeighList list = {d_how, d_how + L, m->order.p + nall, m->order.p, pitch};
   double* const d_force = m->out_d.p;
   double* const d_parts = d_force + (size_t)nall * 3;
   {
-    const int n = (int)(n_in / 2);
-    hipLaunchKernelGGL(call_in_kernel, dim3(std::min(IN_BLOCKS, (n + IO_THREADS - 1) / IO_THREADS)), dim3(IO_THREADS), 0, st,
-                       (const double2*)m->in_h.dev, (double2*)m->in_d.p, n);
+    const int n = (int)(n_in / 2), blocks = std::min(IN_BLOCKS, (n + IO_THREADS - 1) / IO_THREADS);
+    const CallOrder order = {same_order ? nullptr : (const int*)(m->in_h.dev + n_in), m->order.p, m->type_map.p, nall, nlocal,
+                             blocks};
+    const int more = same_order ? 0 : std::min(IN_BLOCKS, (nall + IO_THREADS - 1) / IO_THREADS);
+    hipLaunchKernelGGL(call_in_kernel, dim3(blocks + more), dim3(IO_THREADS), 0, st, (const double2*)m->in_h.dev, m->in_d.p,
+                       nall * 3, n, order);
     STAF_HIP_OK(hipGetLastError());
   }
-  // species of the slots and atoms per species: sent when they differ from what the device holds (in MD they change
-  // when atoms migrate, not every step); the blocking copies read host vectors that the next lines may replace
-  if (m->type_map_up != m->type_map_h) {
-    if (!upload_sync(m->type_map.p, m->type_map_h.data(), (size_t)nall * sizeof(int), st)) return gpu_failure(__LINE__, 0);
-    m->type_map_up = m->type_map_h;
-  }
+  // atoms per species: sent when they differ from what the device holds; the blocking copies read host vectors that the next
+  // lines may replace
   if (m->tipos_up != tipos) {
     if (!upload_sync(m->tipos.p, tipos.data(), nt * sizeof(int), st)) return gpu_failure(__LINE__, 0);
     m->tipos_up = tipos;
@@ -491,6 +543,7 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     if (!upload_sync(m->actual_type.p, ats.data(), nt * sizeof(int), st)) return gpu_failure(__LINE__, 0);
     m->actual_type_up = true;
   }
+  m->order_ready = true;
   // No synchronisation here: the pinned input block outlives the call's final synchronisation.
   staf::DeferStatus defer;   // conditions the kernels detect are read once, after the last kernel
 
@@ -686,8 +739,8 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   {
     const int n = (int)(((m->dev_mlp ? n_out : (size_t)n3) + 1) / 2);
     out_blocks = std::min(OUT_BLOCKS, (n + IO_THREADS - 1) / IO_THREADS);
-    hipLaunchKernelGGL(call_out_kernel, dim3(out_blocks), dim3(IO_THREADS), 0, st, (const double2*)m->out_d.p,
-                       (double2*)m->out_h.dev, n, state->status_d, (int*)(m->done_h.dev + OUT_BLOCKS), m->done_h.dev, call);
+    hipLaunchKernelGGL(call_out_kernel, dim3(out_blocks), dim3(IO_THREADS), 0, st, m->out_d.p, (double2*)m->out_h.dev,
+                       m->order.p, n3, n, state->status_d, (int*)(m->done_h.dev + OUT_BLOCKS), m->done_h.dev, call);
     STAF_HIP_OK(hipGetLastError());
   }
   const double* force_h = m->out_h.p;
@@ -725,13 +778,7 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   }
 
   if (e_rank) *e_rank = energy;
-  if (f)
-    for (int s = 0; s < nall; s++) {
-      const int i = m->slot_to_order[s];
-      f[3 * i] = force_h[3 * s];
-      f[3 * i + 1] = force_h[3 * s + 1];
-      f[3 * i + 2] = force_h[3 * s + 2];
-    }
+  if (f) memcpy(f, force_h, (size_t)n3 * sizeof(double));
   if (virial) {
     virial[0] = W[0];
     virial[1] = W[4];

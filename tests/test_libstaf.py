@@ -880,3 +880,35 @@ def test_network_on_both_sides_of_the_atoms_per_workgroup_lines(prec, tol, n):
     (e, f, w), (eh, fh, wh) = out
     assert abs(e - eh) <= tol * abs(eh)
     assert nerr(f, fh) <= tol and nerr(w, wh) <= tol
+
+
+@pytest.mark.gpu
+def test_a_handle_keeps_the_order_of_the_types_it_was_last_given():
+    """The slots of the atoms are worked out for the types of a call and kept for calls with the same ones: after other types,
+    other ghosts' types, no types at all and a refused call the results are those of a fresh handle, to the last bit."""
+    from alphanesgpu_amd import libstaf, synth
+    pos, box = synth.water_frame((4, 4, 2), 9.86, 0.05, 5)
+    pos, H = _wrap(pos.reshape(-1, 3), box)
+    water = np.repeat(np.arange(2, dtype=np.int32), (32, 64))
+    rng = np.random.Generator(np.random.Philox(8))
+    own = [(pos, t) for t in (water, water[::-1].copy(), rng.permutation(water), np.zeros(96, np.int32), None, water, None)]
+    listed = []
+    for t in (water, rng.permutation(water)):
+        x, allx, alltypes, _, howmany, neigh = _ghost_configuration(pos, box, t, RC)
+        listed += [(allx, alltypes, 96, howmany, neigh), (allx, np.concatenate([t, rng.permutation(alltypes[96:])]), 96, howmany, neigh)]
+    calls = own[:3] + listed[:2] + own[3:5] + ["refused"] + own[5:] + listed[2:] + own[:1]
+    make = lambda: libstaf.StafModel(os.path.join(GOLDEN, "model_double"), precision=1)
+    used = make()
+    for c in calls:
+        if c == "refused":
+            bad = water.copy()
+            bad[50] = 2
+            with pytest.raises(libstaf.StafComputeError):
+                used.compute(pos, box, bad)
+            continue
+        args = (c[0], box, c[1]) if len(c) == 2 else (c[0], box, c[1], *c[2:])
+        fresh = make()
+        want, got = fresh.compute(*args), used.compute(*args)
+        fresh.close()
+        assert got[0] == want[0] and np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2])
+    used.close()
