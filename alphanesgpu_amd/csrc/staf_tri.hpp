@@ -52,7 +52,7 @@ struct TriCfg {
   // The fused double-precision fingerprint kernel (the MD entry: thousands of centres per launch, several per
   // workgroup) stages 128, and its registers are held to six waves per SIMD: 26832 bytes of LDS and six workgroups per
   // CU (160 and five before: with the table's rows of sixteen below, 426 -> 409 us for 24576 centres, 118 -> 113 for
-  // 6144).  The plain double-precision fingerprint kernel stages 448: a CU hands out its 160 KB of LDS in pieces of 1280 bytes, so the 32496 bytes that 512 staged triplets
+  // 6144; 394 and 108.5 with the exponential of HotExp::Factor).  The plain double-precision fingerprint kernel stages 448: a CU hands out its 160 KB of LDS in pieces of 1280 bytes, so the 32496 bytes that 512 staged triplets
   // make count as 33280 and four workgroups fit, not the five that the occupancy query of the runtime reports
   // (measured with a kernel that counts its resident workgroups per CU); with 448 it is 31472 bytes and five
   // (6144-atom step 360.6 -> 356.8 us).
@@ -136,6 +136,11 @@ template <> struct HotExp<float> {
   __device__ static float eval(float t, const float*) { return __builtin_amdgcn_exp2f(t); }
   __device__ static float unscale() { return 0.693147180559945309f; }   // scaled argument -> natural argument
   __device__ static void fill(float*, int, int) {}
+  // e^(a y) for a factor a that is used with many y
+  struct Factor { float a; };
+  __device__ static Factor factor(float a) { return {scale(a)}; }
+  template <bool ONCE>
+  __device__ static float eval(Factor f, float y, const float*) { return __builtin_amdgcn_exp2f(f.a * y); }
 };
 // 2^(i/128), i = 0..127, correctly rounded
 static __device__ const double exp2_frac_128[128] = {
@@ -213,6 +218,35 @@ template <> struct HotExp<double> {
     p = fma(p, r, 1.0);
     return ldexp(f * p, i >> 7);
   }
+  // e^(a y) for a factor a that is used with many y, for the fingerprints and their gradient: a is held as hi + lo in units
+  // of ln2/128, so that a y comes out as t + r, t its integer part and r exact but for its own last bit: no multiplication
+  // by 128/ln2, no product rounded ahead of the reduction.  2^((128 k + i + r)/128) = 2^k (g + g q(r)), g from the table, q
+  // of degree 4 through zero and the values of 2^(r/128) - 1 at the other four zeros of the Chebyshev polynomial T5 on
+  // |r| <= 1/2 (truncation 7.6e-17); 14 vector instructions with the product, 16 in the form above.  Maximum relative error
+  // 2.8e-16 for |a y| up to 600; the form above has 3.0e-16 and what the rounding of a y adds (3.4e-16 up to 2, 9.7e-16 up to
+  // 10).  Fingerprints of 96 atoms against long double: 1.16e-16 rms instead of 1.20e-16 (parameters four times as large:
+  // 1.9e-16 instead of 2.7e-16).  The passes with dL/dF need a y itself and have no registers to spare: they keep that form.
+  // With the row offsets below, 21 instead of 25 instructions per item: fingerprint launch of 24576, 6144 and 3072 centres
+  // 420 -> 394, 116 -> 108.5 and 62.1 -> 58.6 us, of 73728 centres without the 2-body ones (two launches) 412 -> 380.
+  // ONCE: the call stands outside the loop, which would have its constants in vector registers of their own (six, spilled).
+  struct Factor { double hi, lo; };
+  __device__ static Factor factor(double a) {
+    const double hi = a * 184.6649652337873;
+    return {hi, fma(a, 2.6054750388391722e-15, fma(a, 184.6649652337873, -hi))};
+  }
+  template <bool ONCE>
+  __device__ static double eval(Factor f, double y, const double* tab) {
+    auto c = [](double v) { return ONCE ? scalar(v) : v; };
+    const double t = rint(y * f.hi);
+    double r = fma(y, f.hi, -t);
+    r = fma(y, f.lo, r);
+    const int i = (int)t;
+    const double g = tab[i & 127];
+    double q = fma(r, c(3.5830333998870575e-11), ONCE ? vector(2.6466433571133577e-08) : 2.6466433571133577e-08);
+    q = fma(q, r, c(1.466226238763974e-05));
+    q = fma(q, r, c(0.0054152123481238145));
+    return ldexp(fma(g, q * r, g), i >> 7);
+  }
   __device__ static double unscale() { return 1.0; }
   __device__ static void fill(double* tab, int tid, int nthreads) {
     for (int i = tid; i < TABLE_REALS; i += nthreads) tab[i] = exp2_frac_128[i];
@@ -260,7 +294,7 @@ struct TriArgs {
 // gradient, whose LDS budget has no room for padding): every lane of a subset reads the same record.
 //   float,  fingerprint / its gradient: {ab, T}          8 bytes
 //   float,  force gradient:             {ab, T, U, -}   16 bytes
-//   double, fingerprint / its gradient: {ab, -, T}      16 bytes
+//   double, fingerprint / its gradient: {a, b, T}       16 bytes, a and b in bytes: an addition per row and item
 //   double, force gradient:             {T, U} 16 bytes in one array, ab in a second one
 template <typename real, int MODE>
 struct TriStage {
@@ -269,7 +303,9 @@ struct TriStage {
   static constexpr int BYTES = SPLIT ? 20 : ((sizeof(real) == 4 && !WITH_U) ? 8 : 16);
   unsigned char* base;   // 16-byte aligned; SPLIT: QB records of 16 bytes, then QB words
   int qb;
-  __device__ void put(int qq, unsigned ab, real T, real U) const {
+  // a, b: the rows' first entries
+  __device__ void put(int qq, unsigned a, unsigned b, real T, real U) const {
+    const unsigned ab = a | (b << 16);
     if constexpr (SPLIT) {
       double2 v;
       v.x = T; v.y = U;
@@ -281,10 +317,13 @@ struct TriStage {
       ((uint4*)base)[qq] = make_uint4(ab, __float_as_uint((float)T), __float_as_uint((float)U), 0u);
     } else {
       const unsigned long long t = (unsigned long long)__double_as_longlong((double)T);
-      ((uint4*)base)[qq] = make_uint4(ab, 0u, (unsigned)(t & 0xffffffffull), (unsigned)(t >> 32));
+      ((uint4*)base)[qq] = make_uint4(a * 16u, b * 16u, (unsigned)(t & 0xffffffffull), (unsigned)(t >> 32));
     }
   }
-  __device__ void get(int qq, unsigned& ab, real& T, real& U) const {
+  // the rows in tabE, T, U
+  template <typename real2>
+  __device__ void get(int qq, const real2* tabE, const real2*& r1, const real2*& r2, real& T, real& U) const {
+    unsigned ab;
     if constexpr (SPLIT) {
       const double2 v = ((const double2*)base)[qq];
       T = (real)v.x; U = (real)v.y;
@@ -297,10 +336,14 @@ struct TriStage {
       ab = v.x; T = (real)__uint_as_float(v.y); U = (real)__uint_as_float(v.z);
     } else {
       const uint4 v = ((const uint4*)base)[qq];
-      ab = v.x;
+      r1 = (const real2*)((const unsigned char*)tabE + v.x);
+      r2 = (const real2*)((const unsigned char*)tabE + v.y);
       T = (real)__longlong_as_double((long long)(((unsigned long long)v.w << 32) | v.z));
       U = 0;
+      return;
     }
+    r1 = tabE + (ab & 0xffffu);
+    r2 = tabE + (ab >> 16);
   }
 };
 
@@ -523,6 +566,7 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
           real a1 = 0, a2 = 0, be = 0;
           if (chan) { a1 = tab.a1[pb + c0 + ia]; a2 = tab.a2[pb + c0 + ia]; be = tab.be[pb + c0 + ia]; }
           const real a1s = HE::scale(a1), a2s = HE::scale(a2), bes = HE::scale(be);
+          const typename HE::Factor a1f = HE::factor(a1), a2f = HE::factor(a2), bef = HE::factor(be);
           if (!first) {
             __syncthreads();   // tables and staged block of the previous pass fully consumed
             flush_pass();
@@ -534,8 +578,8 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
             const real d = sD[s];
             if (chan) {
               real2 v;
-              v.x = HE::eval(a1s * d, etab);
-              v.y = HE::eval(a2s * d, etab);
+              v.x = FB ? HE::eval(a1s * d, etab) : HE::template eval<false>(a1f, d, etab);
+              v.y = FB ? HE::eval(a2s * d, etab) : HE::template eval<false>(a2f, d, etab);
               tabE[row * TRI_CAPP + ia] = v;
             }
             if (MODE != 0 && ia == 0) {
@@ -556,7 +600,7 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
             const int nq_pad = (nq + SUBS - 1) & ~(SUBS - 1);
             if (q0 > 0) __syncthreads();   // previous block consumed
             // ---- stage a block of triplets
-            for (int qq = nq + tid; qq < nq_pad; qq += BLOCK) stage.put(qq, 0u, real(0), real(0));
+            for (int qq = nq + tid; qq < nq_pad; qq += BLOCK) stage.put(qq, 0u, 0u, real(0), real(0));
             for (int qq = tid; qq < nq; qq += BLOCK) {
               const int q = q0 + qq;
               int x, y;
@@ -566,7 +610,6 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
               const int j = s1 < s2 ? s1 : s2, k = s1 < s2 ? s2 : s1;
               const int nn = tri_rowstart(j, m) + k - j - 1;
               const bool ok = nn < na;
-              const unsigned ab = (unsigned)(x * TRI_CAPP) | ((unsigned)((rowB0 + y) * TRI_CAPP) << 16);
               real T = 0, U = 0;
               if (ok) {
                 if constexpr (FUSED) {
@@ -585,23 +628,21 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
                   }
                 }
               }
-              stage.put(qq, ab, T, U);
+              stage.put(qq, (unsigned)(x * TRI_CAPP), (unsigned)((rowB0 + y) * TRI_CAPP), T, U);
             }
             __syncthreads();
-            // ---- thread <-> (channel ia, subset sub)
+            // ---- thread <-> (channel ia, subset sub), two steps at a time
             if (chan) {
               const int rounds = nq_pad / SUBS;
-#pragma unroll 2
-              for (int it = 0; it < rounds; it++) {
+              auto item = [&](int it, auto last_c) {
+                constexpr bool LAST = decltype(last_c)::value;
                 const int qq = sub + it * SUBS;
-                unsigned ab;
+                const real2 *r1, *r2;
                 real T, U;
-                stage.get(qq, ab, T, U);
-                const real2* r1 = tabE + (ab & 0xffffu);
-                const real2* r2 = tabE + (ab >> 16);
+                stage.get(qq, tabE, r1, r2, T, U);
                 const real2 e1 = r1[ia];
                 const real2 e2 = r2[ia];
-                const real ebt = HE::eval(bes * T, etab);
+                const real ebt = FB ? HE::eval(bes * T, etab) : HE::template eval<LAST>(bef, T, etab);
                 const real sim2 = e1.x * e2.y;   // exp(a1 D1 + a2 D2)
                 const real sim1 = e1.y * e2.x;   // exp(a2 D1 + a1 D2)
                 if constexpr (MODE == 0) {
@@ -648,7 +689,13 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
                     acc[6] = r_fma(ss * hT, T, acc[6]);
                   }
                 }
+              };
+              int it = 0;
+              for (; it + 2 <= rounds; it += 2) {
+                item(it, std::false_type{});
+                item(it + 1, std::false_type{});
               }
+              if (it < rounds) item(it, std::true_type{});
             }
           }
           // ---- the wave's four subsets of every channel, then the wave's own accumulators (fixed order)
