@@ -161,6 +161,13 @@ bool bucket_reserve(DeviceState* st, size_t n_recv, int cap, hipStream_t stream,
 bool remember_map(DeviceState* st, const int* im2, int nf, int N, int nr, hipStream_t stream, TransposeRef* out) {
   std::lock_guard<std::mutex> lock(g_mu);
   const size_t want = (size_t)nf * N * sizeof(unsigned);
+  // Memory that this tensor takes up holds no earlier one any more: a map remembered from before somewhere else in it would
+  // be found first by a view whose distance from it happens to be whole rows.
+  const uintptr_t begin = (uintptr_t)im2, end = begin + (size_t)nf * N * (nr + 1) * sizeof(int);
+  for (auto& e : st->maps) {
+    const uintptr_t b = (uintptr_t)e.im2;
+    if (e.im2 && e.im2 != im2 && b < end && begin < b + (size_t)e.nf * e.N * (e.nr + 1) * sizeof(int)) e.im2 = nullptr;
+  }
   KnownMap* t = nullptr;
   for (auto& e : st->maps)
     if (e.im2 == im2) { t = &e; break; }

@@ -1325,3 +1325,31 @@ def test_changed_row_of_a_remembered_map_is_reported_by_its_checksum():
     rad, ang, sup, im2, im3, d2, d3, d3s, ntr = ops.compute_descriptors_light(T(b["pos"]), T(b["box"]))
     ops.compute_force_radial(G2, d2[:, :n0], im2[:, :n0], rad[:, :n0], T(p0["alpha2b"]), T(p0["emb2b"]), tm, tp, at)
     ops.poll_status()
+
+
+def test_a_map_in_the_memory_of_an_earlier_one_is_not_taken_for_it():
+    """Descriptor outputs of two calls, the second map sixteen rows further in the memory of the first (a recycled block): a
+    force op on a view of the second one finds that, not the rows the earlier map had at this distance."""
+    import torch
+    from alphanesgpu_amd import ops
+    b = _synth("water96")
+    dev, dt = torch.device("cuda:0"), torch.float64
+    N, n0 = b["N"], int(b["tipos"][0])
+    T = lambda a: torch.as_tensor(np.ascontiguousarray(a)).to(dev)
+    p = _params(np.dtype(np.float64))[0]
+    ops.construct_descriptors_light(4.5, NR, NA, N, None, 2.25, 4.5, 1, dtype=dt)
+    memory = torch.zeros((2 * N * (NR + 1),), dtype=torch.int32, device=dev)
+    first = list(ops.compute_descriptors_light(T(b["pos"]), T(b["box"])))
+    maps = [memory[r * (NR + 1):(r + N) * (NR + 1)].view(1, N, NR + 1) for r in (0, 16)]
+    tm, tp, at = T(b["type_map"]), T(b["tipos"]), torch.tensor([0], dtype=torch.int32, device=dev)
+    G2 = torch.ones(1, n0, p["alpha2b"].shape[1], dtype=dt, device=dev)
+    moved = torch.roll(T(b["pos"]).view(1, N, 3), 1, 1).reshape(1, 3 * N).contiguous()
+    for im2, pos in zip(maps, (T(b["pos"]), moved)):
+        out = [torch.empty_like(t) for t in first]
+        out[3] = im2
+        rad, _, _, im2, _, d2, _, _, _ = ops.compute_descriptors_light(pos, T(b["box"]), out=tuple(out))
+        args = lambda m: (G2, d2[:, :n0], m, rad[:, :n0], T(p["alpha2b"]), T(p["emb2b"]), tm, tp, at)
+        f = ops.compute_force_radial(*args(im2[:, :n0]))
+        g = ops.compute_force_radial(*args(im2.clone()[:, :n0]))
+        # the same pair forces, at most 2 x 60 of them on an atom, in another order
+        assert (f - g).abs().max() <= 120 * 2.0 ** -52 * max(1.0, float(g.abs().max()))
