@@ -73,9 +73,12 @@ def call(name, *args):
 
 
 def ptr(t):
-    """Device pointer of a contiguous torch tensor (None -> NULL)."""
+    """Device pointer of a contiguous torch tensor (None -> NULL), which lives as long as the pointer: a copy made for a call's
+    argument list is held until the call has been made."""
     if t is None:
         return C.c_void_p(0)
     if not t.is_contiguous():
         raise ValueError("STAF ops need contiguous tensors")
-    return C.c_void_p(t.data_ptr())
+    p = C.c_void_p(t.data_ptr())
+    p.tensor = t
+    return p

@@ -502,8 +502,8 @@ def force_total(interaction_map_rad_full, n_local, slot_forces, self_forces, for
     some = next(t for t in list(slot_forces) + list(forces2b or []) if t is not None)
     dtype, dev = some.dtype, some.device
     s, _ = sfx(dtype)
-    arr = lambda ts: (C.c_void_p * nt)(*[None if t is None else _dense(t).data_ptr() for t in ts])
-    keep = [None if t is None else _dense(t) for t in list(slot_forces) + list(self_forces) + list(forces2b or [])]
+    keep = _Dense()
+    arr = lambda ts: (C.c_void_p * nt)(*[keep(t) for t in ts])
     total = torch.empty((nf, 3 * N), dtype=dtype, device=dev) if out is None else out
     call(f"staf_op_force_total_{s}", ptr(im), _I(nr1 - 1), _I(N), _I(nf), _I(nt), (C.c_int * nt)(*[int(n) for n in n_local]),
          arr(slot_forces), arr(self_forces), arr(forces2b if forces2b is not None else [None] * nt), ptr(total),
@@ -580,6 +580,20 @@ def _addr(t):
     return t.data_ptr()
 
 
+class _Dense:
+    """Addresses of the dense forms of a call's tensors; copies live as long as this object.  (The memory of a copy that nobody
+    holds is given to the next one while the arguments are still being put together.)"""
+
+    def __init__(self):
+        self.kept = []
+
+    def __call__(self, t):
+        if t is None:
+            return None
+        self.kept.append(_dense(t))
+        return self.kept[-1].data_ptr()
+
+
 def _stream_addr():
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
@@ -592,12 +606,12 @@ def layer_fingerprints(x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb
     na = x3b.shape[2]
     nt, Ar = alpha2b.shape
     Aa = alpha3b.shape[1] // 3
-    v = _Views()
+    v, dense = _Views(), _Dense()
     pD, pT, pS, pI, pN = v(x2b), v(x3b), v(x3bsupp), v(_i32(intmap2b)), v(_i32(numtriplet))
     out = torch.empty((nf, Nl, Ar + Aa), dtype=dtype, device=x2b.device)
     fn = _entry("staf_op_layer_fingerprints", dtype, "ppp" "iiii" "p" "pippip" "pp" "i" "p" "ip")
-    _checked(fn(pD, pS, pT, nr, na, nf, Nl, pI, _addr(_dense(alpha2b)), Ar, _addr(_dense(emb2b)), _addr(_dense(alpha3b)), Aa,
-                _addr(_dense(emb3b)), _addr(_i32(type_map)), pN, nt, out.data_ptr(), v.ld, _stream_addr()),
+    _checked(fn(pD, pS, pT, nr, na, nf, Nl, pI, dense(alpha2b), Ar, dense(emb2b), dense(alpha3b), Aa, dense(emb3b),
+                _addr(_i32(type_map)), pN, nt, out.data_ptr(), v.ld, _stream_addr()),
              "staf_op_layer_fingerprints")
     return out
 
@@ -609,14 +623,14 @@ def layer_fingerprints_grad(grad, x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, a
     na = x3b.shape[2]
     nt, Ar = alpha2b.shape
     Aa = alpha3b.shape[1] // 3
-    v = _Views()
+    v, dense = _Views(), _Dense()
     pD, pT, pS, pI, pN = v(x2b), v(x3b), v(x3bsupp), v(_i32(intmap2b)), v(_i32(numtriplet))
     e = lambda t: torch.empty(t.shape, dtype=dtype, device=x2b.device)
     ga2, ge2, ga3, ge3 = e(alpha2b), e(emb2b), e(alpha3b), e(emb3b)
     fn = _entry("staf_op_layer_fingerprints_grad", dtype, "pppp" "iiii" "p" "pippip" "pp" "i" "pppp" "ip")
-    _checked(fn(_addr(_dense(grad)), pD, pS, pT, nr, na, nf, Nl, pI, _addr(_dense(alpha2b)), Ar, _addr(_dense(emb2b)),
-                _addr(_dense(alpha3b)), Aa, _addr(_dense(emb3b)), _addr(_i32(type_map)), pN, nt, ga2.data_ptr(),
-                ge2.data_ptr(), ga3.data_ptr(), ge3.data_ptr(), v.ld, _stream_addr()), "staf_op_layer_fingerprints_grad")
+    _checked(fn(dense(grad), pD, pS, pT, nr, na, nf, Nl, pI, dense(alpha2b), Ar, dense(emb2b), dense(alpha3b), Aa,
+                dense(emb3b), _addr(_i32(type_map)), pN, nt, ga2.data_ptr(), ge2.data_ptr(), ga3.data_ptr(),
+                ge3.data_ptr(), v.ld, _stream_addr()), "staf_op_layer_fingerprints_grad")
     return ga2, ge2, ga3, ge3
 
 
@@ -627,17 +641,16 @@ def layer_forces(netderiv2b, netderiv3b, x2b, intder2b, intmap2b, alpha2b, emb2b
     nf, Nl, na = x3b.shape
     nr, N, nt = x3bsupp.shape[2], type_map.shape[0], tipos.shape[0]
     Ar, Aa = alpha2b.shape[1], alpha3b.shape[1] // 3
-    v = _Views()
+    v, dense = _Views(), _Dense()
     rows = [v(t) for t in (x2b, intder2b, x3bsupp, x3b, intder3bsupp, intder3b)]
     pI, pN = v(_i32(intmap2b)), v(_i32(numtriplet))
     force = torch.empty((nf, 3 * N), dtype=dtype, device=dev)
     virial = torch.empty((nf, 9), dtype=dtype, device=dev) if pos is not None else None
     at = _scalar_dev(type_now, dev)
     fn = _entry("staf_op_layer_forces", dtype, "pp" "pppppp" "p" "iiiii" "pippip" "i" "pppp" "pppp" "ip")
-    _checked(fn(_addr(_dense(netderiv2b)), _addr(_dense(netderiv3b)), *rows, pI, nr, na, N, nf, Nl, _addr(_dense(alpha2b)), Ar,
-                _addr(_dense(emb2b)), _addr(_dense(alpha3b)), Aa, _addr(_dense(emb3b)), nt, _addr(_i32(tipos)), _addr(at), pN,
-                _addr(_i32(type_map)), force.data_ptr(), _addr(virial), _addr(None if pos is None else _dense(pos)),
-                _addr(None if box is None else _dense(box)), v.ld, _stream_addr()), "staf_op_layer_forces")
+    _checked(fn(dense(netderiv2b), dense(netderiv3b), *rows, pI, nr, na, N, nf, Nl, dense(alpha2b), Ar, dense(emb2b),
+                dense(alpha3b), Aa, dense(emb3b), nt, _addr(_i32(tipos)), _addr(at), pN, _addr(_i32(type_map)),
+                force.data_ptr(), _addr(virial), dense(pos), dense(box), v.ld, _stream_addr()), "staf_op_layer_forces")
     return force if pos is None else (force, virial)
 
 
@@ -650,7 +663,7 @@ def layer_forces_grad(prevgrad, netderiv2b, netderiv3b, x2b, intder2b, intmap2b,
     nf, Nl, na = x3b.shape
     nr, N, nt = x3bsupp.shape[2], type_map.shape[0], tipos.shape[0]
     Ar, Aa = alpha2b.shape[1], alpha3b.shape[1] // 3
-    v = _Views()
+    v, dense = _Views(), _Dense()
     rows = [v(t) for t in (x2b, intder2b, x3bsupp, x3b, intder3bsupp, intder3b)]
     pI, pN = v(_i32(intmap2b)), v(_i32(numtriplet))
     e = lambda *sh: torch.empty(sh, dtype=dtype, device=dev)
@@ -662,11 +675,10 @@ def layer_forces_grad(prevgrad, netderiv2b, netderiv3b, x2b, intder2b, intmap2b,
     at = _scalar_dev(type_now, dev)
     fn = _entry("staf_op_layer_forces_grad", dtype,
                 "ppp" "pppppp" "p" "iiiii" "pippip" "i" "pppp" "pppppp" "ppp" "ip")
-    _checked(fn(_addr(_dense(prevgrad)), _addr(_dense(netderiv2b)), _addr(_dense(netderiv3b)), *rows, pI, nr, na, N, nf, Nl,
-                _addr(_dense(alpha2b)), Ar, _addr(_dense(emb2b)), _addr(_dense(alpha3b)), Aa, _addr(_dense(emb3b)), nt,
+    _checked(fn(dense(prevgrad), dense(netderiv2b), dense(netderiv3b), *rows, pI, nr, na, N, nf, Nl,
+                dense(alpha2b), Ar, dense(emb2b), dense(alpha3b), Aa, dense(emb3b), nt,
                 _addr(_i32(tipos)), _addr(at), pN, _addr(_i32(type_map)), *[_addr(t) for t in out],
-                _addr(None if prevgrad_virial is None else _dense(prevgrad_virial)),
-                _addr(None if pos is None else _dense(pos)), _addr(None if box is None else _dense(box)), v.ld,
+                dense(prevgrad_virial), dense(pos), dense(box), v.ld,
                 _stream_addr()), "staf_op_layer_forces_grad")
     return tuple(out)
 

@@ -325,3 +325,44 @@ def test_layers_as_single_calls_give_the_bits_of_the_ops_on_squared_embeddings(d
         if n:
             assert bool(x.abs().max() > 0)
         o += n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("entry", ["layer_forces", "compute_forces", "force_total"])
+def test_arguments_that_are_not_dense_are_copied_to_places_of_their_own(entry):
+    """Halves of one tensor and strided parameters: every one is copied for the call, and the copies live until it is made."""
+    import torch
+    from alphanesgpu_amd import ops, synth
+    dev, dt = torch.device("cuda:0"), torch.float64
+    pos, box = synth.water_frame((4, 4, 2), 9.86, 0.05, 3)
+    N, n = 96, 32
+    T = lambda a: torch.as_tensor(np.ascontiguousarray(a)).to(dev)
+    tpos, tbox = T(pos[None]), T(box[None])
+    tm, tp, tn = T(np.repeat(np.arange(2, dtype=np.int32), (32, 64))), T(np.array([32, 64], np.int32)), T(np.zeros(1, np.int32))
+    ops.construct_descriptors_light(synth.RC, 60, 1770, N, tbox, synth.RS, synth.RA, 1, dtype=dt)
+    rad, ang, sup, im2, im3, d2, d3, d3s, ntr = ops.compute_descriptors_light(tpos, tbox)
+    c = lambda t: t[:, :n]
+    P = {q: T(v) for q, v in synth.fingerprint_params(2, dtype=np.float64)[0].items()}
+    g = torch.Generator(device=dev)
+    g.manual_seed(5)
+    Ar, Aa = P["emb2b"].shape[1], P["emb3b"].shape[1]
+    G = torch.randn((1, n, Ar + Aa), dtype=dt, device=dev, generator=g)
+    strided = lambda t: torch.stack([t, torch.full_like(t, float("nan"))], -1)[..., 0]
+    forms = []
+    for form in (lambda t: t.contiguous(), strided):
+        G2, G3 = form(G[..., :Ar]), form(G[..., Ar:])
+        Q = {k: form(P[k]) for k in ("alpha2b", "alpha3b", "emb2b", "emb3b")}
+        if entry == "layer_forces":
+            f = ops.layer_forces(G2, G3, c(rad), c(d2), c(im2), Q["alpha2b"], Q["emb2b"], c(ang), c(sup), c(d3), c(d3s), c(ntr),
+                                 Q["alpha3b"], Q["emb3b"], tm, tp, tn)
+        else:
+            args = (G3, G2, c(sup), c(ang), c(d3s), c(d3), c(rad), c(d2), c(im2), c(im3), Q["alpha3b"], Q["emb3b"],
+                    Q["alpha2b"], Q["emb2b"], tm, tp, tn, c(ntr))
+            if entry == "compute_forces":
+                f = ops.compute_forces(*args)
+            else:
+                slots, own = ops.compute_forces_slots(*args)
+                none = [torch.zeros((1, 64, *slots.shape[2:]), dtype=dt, device=dev), torch.zeros((1, 64, *own.shape[2:]), dtype=dt, device=dev)]
+                f = ops.force_total(im2, [32, 64], [form(slots), form(none[0])], [form(own), form(none[1])])
+        forms.append(f)
+    assert torch.equal(*forms)
