@@ -337,7 +337,7 @@ __device__ __forceinline__ void desc_body(const DescArgs<real> A, const int cent
           l = cell_cnt[c];
         }
       }
-      // groups before a lane's own: a prefix sum over the lanes, register to register (same tree as wave_scan4)
+      // groups before a lane's own: a prefix sum over the lanes, register to register (the tree of wave_scan)
       const unsigned g = (unsigned)(l + GROUP - 1) / GROUP;
       unsigned incl = g + dpp_get<0x111, 0xf>(g);
       incl += dpp_get<0x112, 0xf>(g);

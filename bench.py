@@ -384,14 +384,15 @@ def run_md(args, workload):
                    "neighbour_list": "the library's own, rebuilt on every call (cell list from 4096 atoms on)",
                    "boundary": "host arrays in (positions, box, species) and out (energy, forces, virial): the PCIe "
                                "copies and the call's one synchronisation are inside the timed region",
-                   "launch": "five launches (six with a cell list) over all species, issued on one stream",
+                   "launch": "seven launches (eight with a cell list) issued on one stream: the input's copy, five "
+                             "stages over all species, the results' copy",
                    "timing": f"median of {REPEATS} blocks of {args.steps} calls"},
         "block_ms_per_step": [b / args.steps * 1e3 for b in block_s],
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": md_bytes / (el / args.steps) / 1e9,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": md_bytes / (el / args.steps) / 1e9 / HBM_PEAK_GBS,
                      "frac_is": "bytes of the whole call (nr-wide tensors only: this path holds no tensor of the angular "
                                 "buffer's width) over the call's time over peak: low by construction, the call is bound "
-                                "by vector-ALU issue and by the latency of its five dependent launches",
+                                "by vector-ALU issue and by the latency of its dependent launches",
                      "traffic": None, "algorithmic_bytes_per_call": md_bytes,
                      "valu": {"bound": "valu", "unit": "wave instructions/s", "kernel": dom,
                               "algorithmic_inst_per_item": alg.get(dom), "items_per_call": items,
