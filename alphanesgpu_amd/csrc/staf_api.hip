@@ -589,9 +589,9 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     if (r == STAF_OK) hipLaunchKernelGGL(add_into_kernel, dim3((n3 + 255) / 256), dim3(256), 0, st, d_force, m->force_op.p, n3);
     return r;
   };
-  // ---- everything stays on the device, five launches one behind the other (six with a cell list or a caller's
-  // list): descriptors -> fingerprints -> networks -> slot forces -> collection, each over the centres of all species;
-  // one synchronisation at the end of the call.  A chain per species on a stream of its own, with a launch per body, was
+  // ---- everything stays on the device, between the copying kernels five launches one behind the other (six with a cell
+  // list or a caller's list): descriptors -> fingerprints -> networks -> slot forces -> collection, each over the centres
+  // of all species; one wait at the end of the call.  A chain per species on a stream of its own, with a launch per body, was
   // 17 to 31 launches, replayed as a recorded graph because the host could not issue them as fast as they ran, and a
   // small system's time was the gaps between them (96 atoms: 147 us a call, 100 now; 768: 168 and 140).  Five launches
   // are issued ahead of the GPU: a recorded graph of them is no faster (106 and 143 us), and costs its recording whenever

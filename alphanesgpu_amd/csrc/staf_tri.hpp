@@ -126,7 +126,7 @@ inline int tri_grid(const void* kernel, size_t lds, int centres) {
 // values of (e^r - 1 - r - r^2/2) / r^3 at the nine Chebyshev points of the interval (truncation 3.3e-17, where the Taylor
 // polynomial of degree 12 has 1.7e-16 with one instruction more), ldexp; 17 instructions, maximum relative error 1.4e-16
 // over [-60, 60] against a 60-digit evaluation (Taylor: 3.3e-16).
-// The 3-body kernels use the tabulated form below it (eval(x, table in LDS)).
+// The reduce kernels of this file use the tabulated forms below it (a table in LDS).
 // Overflow gives inf, underflow 0, NaN stays NaN; exp(+inf) gives NaN (arguments here are finite products).
 template <typename real> struct HotExp;
 template <> struct HotExp<float> {
