@@ -193,8 +193,8 @@ struct StafModel {
   PinBuf<unsigned> done_h;   // [OUT_BLOCKS flags of call_out_kernel | error words]
   unsigned calls = 0;
   // The atoms' order: made for the types of a call and kept for the calls that follow with the same ones (in MD they change
-  // when atoms migrate, not every step).  order_ready: tipos_h, order and type_map are those of
-  // types_seen.
+  // when atoms migrate, not every step).  order_ready: a call that has sent them is through, and tipos_h, order and type_map are
+  // those of types_seen.
   std::vector<int> types_seen, tipos_h;
   int nlocal_seen = 0;
   bool order_ready = false;
@@ -381,6 +381,17 @@ static int gpu_failure(int line, int code) {
   if (verbose) fprintf(stderr, "staf_compute: GPU runtime failure at staf_api.hip:%d (code %d)\n", line, code);
   return -20;
 }
+// A call from its first launch on.  One that returns before its results are there waits for what it has queued, which reads
+// the pinned blocks that the next call writes, and the next call sends the order of the atoms again.
+struct CallInFlight {
+  StafModel* m;
+  bool through = false;
+  ~CallInFlight() {
+    if (through) return;
+    (void)hipStreamSynchronize(m->stream);
+    m->order_ready = false;
+  }
+};
 #define STAF_HIP_OK(x) do { const hipError_t e_ = (x); if (e_ != hipSuccess) return gpu_failure(__LINE__, (int)e_); } while (0)
 
 int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const double* box, const int* type,
@@ -522,6 +533,7 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   const staf::NeighList list = {d_how, d_how + L, m->order.p + nall, m->order.p, pitch};
   double* const d_force = m->out_d.p;
   double* const d_parts = d_force + (size_t)nall * 3;
+  CallInFlight in_flight{m};
   {
     const int n = (int)(n_in / 2), blocks = std::min(IN_BLOCKS, (n + IO_THREADS - 1) / IO_THREADS);
     const CallOrder order = {same_order ? nullptr : (const int*)(m->in_h.dev + n_in), m->order.p, m->type_map.p, nall, nlocal,
@@ -543,7 +555,6 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     if (!upload_sync(m->actual_type.p, ats.data(), nt * sizeof(int), st)) return gpu_failure(__LINE__, 0);
     m->actual_type_up = true;
   }
-  m->order_ready = true;
   // No synchronisation here: the pinned input block outlives the call's final synchronisation.
   staf::DeferStatus defer;   // conditions the kernels detect are read once, after the last kernel
 
@@ -760,6 +771,7 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     }
     __builtin_ia32_pause();
   }
+  in_flight.through = m->order_ready = true;
   bool reported = false;
   for (int w = 0; w < staf::STATUS_WORDS; w++) reported = reported || status_h[w] != 0;
   rc = reported ? staf_ops_poll_status(st) : STAF_OK;   // (reads the words again, and clears what it has read)
