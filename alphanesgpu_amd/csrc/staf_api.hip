@@ -115,7 +115,7 @@ __global__ __launch_bounds__(IO_THREADS) void call_in_kernel(const double2* __re
   }
 }
 // Forces in the caller's order, the rest as it is.
-// The error words go along.  A workgroup's flag says that everything it copied has arrived: its threads' stores are released
+// The stream's error word goes along.  A workgroup's flag says that everything it copied has arrived: its threads' stores are released
 // to the host before the flag is written.
 __global__ __launch_bounds__(IO_THREADS) void call_out_kernel(const double* __restrict__ dev, double2* __restrict__ host,
                                                               const int* __restrict__ slot_of, int n3, int n, int* status,
@@ -127,8 +127,8 @@ __global__ __launch_bounds__(IO_THREADS) void call_out_kernel(const double* __re
     v.y = dev[e + 1 < n3 ? 3 * slot_of[(e + 1) / 3] + (e + 1) % 3 : e + 1];
     host[i] = v;
   }
-  if (blockIdx.x == 0 && threadIdx.x < staf::STATUS_WORDS)
-    status_h[threadIdx.x] = __hip_atomic_load(&status[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    *status_h = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __threadfence_system();
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(&flags[blockIdx.x], call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -190,7 +190,7 @@ struct StafModel {
   // out_d = [force nall*3 | rows of (virial 9, energy), sums over shares of the centres]  (out_h: forces in the caller's order)
   DevBuf<double> in_d, out_d, force_op, virial_op, af2, af3, g2, g3, e_atom, vpart;
   PinBuf<double> in_h, out_h;
-  PinBuf<unsigned> done_h;   // [OUT_BLOCKS flags of call_out_kernel | error words]
+  PinBuf<unsigned> done_h;   // [OUT_BLOCKS flags of call_out_kernel | the stream's error word]
   unsigned calls = 0;
   // The atoms' order: made for the types of a call and kept for the calls that follow with the same ones (in MD they change
   // when atoms migrate, not every step).  order_ready: a call that has sent them is through, and tipos_h, order and type_map are
@@ -448,8 +448,8 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   const size_t n_out = ((size_t)nall * 3 + (size_t)nparts * 10 + 1) & ~(size_t)1;
   if (!m->in_h.reserve(n_in + (same_order ? 0 : (size_t)nall)) || !m->out_h.reserve(n_out)) return -1;
   if (!m->done_h.p) {
-    if (!m->done_h.reserve(OUT_BLOCKS + staf::STATUS_WORDS)) return -1;
-    memset(m->done_h.p, 0, (OUT_BLOCKS + staf::STATUS_WORDS) * sizeof(unsigned));
+    if (!m->done_h.reserve(OUT_BLOCKS + 1)) return -1;
+    memset(m->done_h.p, 0, (OUT_BLOCKS + 1) * sizeof(unsigned));
   }
   double* pos_h = m->in_h.p;
   int* how_h = (int*)(m->in_h.p + n_in_d);
@@ -740,7 +740,7 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
       }
     }
   }
-  // forces, on the device path the virial and energy sums behind them, and the error words
+  // forces, on the device path the virial and energy sums behind them, and the stream's error word
   staf::DeviceState* const state = staf::device_state(st);
   if (!state) return gpu_failure(__LINE__, 0);
   const unsigned call = ++m->calls ? m->calls : ++m->calls;   // (never what the flags start with)
@@ -751,7 +751,7 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     const int n = (int)(((m->dev_mlp ? n_out : (size_t)n3) + 1) / 2);
     out_blocks = std::min(OUT_BLOCKS, (n + IO_THREADS - 1) / IO_THREADS);
     hipLaunchKernelGGL(call_out_kernel, dim3(out_blocks), dim3(IO_THREADS), 0, st, m->out_d.p, (double2*)m->out_h.dev,
-                       m->order.p, n3, n, state->status_d, (int*)(m->done_h.dev + OUT_BLOCKS), m->done_h.dev, call);
+                       m->order.p, n3, n, staf::status_word(state, st), (int*)(m->done_h.dev + OUT_BLOCKS), m->done_h.dev, call);
     STAF_HIP_OK(hipGetLastError());
   }
   const double* force_h = m->out_h.p;
@@ -772,9 +772,8 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
     __builtin_ia32_pause();
   }
   in_flight.through = m->order_ready = true;
-  bool reported = false;
-  for (int w = 0; w < staf::STATUS_WORDS; w++) reported = reported || status_h[w] != 0;
-  rc = reported ? staf_ops_poll_status(st) : STAF_OK;   // (reads the words again, and clears what it has read)
+  // What the results' kernel has read is what the call found; the conditions of other streams are left to them.
+  rc = *status_h ? staf::take_status(state, st, *status_h) : STAF_OK;
   if (rc == STAF_E_RADIAL_OVERFLOW) return -10;
   if (rc == STAF_E_SCATTER_OVERFLOW) return -11;
   if (rc != STAF_OK) return gpu_failure(__LINE__, rc);

@@ -393,6 +393,8 @@ inline bool lds_request(K kernel, size_t lds) {
 }
 // The error word of `stream` on this device (see DeviceState::status_d).
 int* status_word(DeviceState* st, hipStream_t stream);
+// What the stream's error word says, together with the bits `seen` that the caller has read from it; the word is cleared.
+int take_status(DeviceState* st, hipStream_t stream, int seen);
 // Both grow on demand and never shrink; under capture a request that does not fit what the stream already holds
 // returns null (the caller reports STAF_E_CAPTURE) instead of freeing and allocating.
 void* scratch_reserve(DeviceState* st, hipStream_t stream, size_t bytes);

@@ -241,8 +241,9 @@ __global__ void status_clear_kernel(int* word, StatusSeen seen, int nw) {
 }
 
 // Reads and clears, after waiting for `stream`, the stream's own error word (all = false) or every word of the
-// device (all = true: the poll, whose caller has waited for the other streams itself).
-static int fetch_status(DeviceState* st, hipStream_t stream, bool all) {
+// device (all = true: the poll, whose caller has waited for the other streams itself).  seen_bits: what the caller
+// has read from the word already, which counts whether or not it is still there (another thread's poll clears every word).
+static int fetch_status(DeviceState* st, hipStream_t stream, bool all, int seen_bits = 0) {
   static std::mutex mirror_mu;   // one pinned mirror per device
   std::lock_guard<std::mutex> lock(mirror_mu);
   int* word = all ? st->status_d : status_word(st, stream);
@@ -250,7 +251,7 @@ static int fetch_status(DeviceState* st, hipStream_t stream, bool all) {
   int* host = st->status_h + (word - st->status_d);
   if (hipMemcpyAsync(host, word, nw * sizeof(int), hipMemcpyDeviceToHost, stream) != hipSuccess) return STAF_E_HIP;
   if (hipStreamSynchronize(stream) != hipSuccess) return STAF_E_HIP;
-  int bits = 0;
+  int bits = seen_bits;
   StatusSeen seen;
   for (int w = 0; w < STATUS_WORDS; w++) seen.bits[w] = w < nw ? host[w] : 0;
   for (int w = 0; w < nw; w++) bits |= host[w];
@@ -266,6 +267,8 @@ static int fetch_status(DeviceState* st, hipStream_t stream, bool all) {
   }
   return decode_status(bits);
 }
+
+int take_status(DeviceState* st, hipStream_t stream, int seen) { return fetch_status(st, stream, false, seen); }
 
 int finish_op(DeviceState* st, hipStream_t stream) {
   if (hipGetLastError() != hipSuccess) return STAF_E_HIP;

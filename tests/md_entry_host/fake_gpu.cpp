@@ -1,7 +1,7 @@
 // The host side of staf_compute (csrc/staf_api.hip, csrc/staf_runtime.hip) over a runtime without a GPU: memory is the
 // host's, a stream is a queue whose entries run when the host waits for it or asks it, and the stages between the copying
 // kernels are replaced by one that writes a force per slot.  Conditions that a GPU gives only now and then -- a stage that
-// cannot be launched while the call's first kernel has not run yet -- are set here.
+// cannot be launched while the call's first kernel has not run yet, another thread's poll between two lines -- are set here.
 //
 //   fake_gpu MODEL_DIR SCENARIO   prints "ok" or what is wrong
 #include "../../alphanesgpu_amd/csrc/staf_common.hpp"
@@ -27,7 +27,8 @@ std::map<const void*, std::string>& names() {   // (filled before this file's ow
   static std::map<const void*, std::string> n;
   return n;
 }
-int fail_descriptors_ = 0;
+std::function<void()> after_results_;   // runs between the results' kernel and what the host does next
+int fail_descriptors_ = 0, raise_ = 0;
 
 void run_queue() {
   while (!queue_.empty()) {
@@ -100,6 +101,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, 
       for (int e = 0; e < 2 * n; e++) host[e] = dev[e < n3 ? 3 * slot_of[e / 3] + e % 3 : e];
       status_h[0] = status[0];
       for (int b = 0; b < blocks; b++) flags[b] = call;
+      if (after_results_) after_results_();
     });
   } else if (is("fill_zero_kernel")) {
     char* const p = arg<char*>(args, 0);
@@ -158,9 +160,13 @@ template <> int desc_configure<double>(DescConfig<double>& c, double, int nr, in
 }
 template <> int desc_launch<double>(const DescConfig<double>&, const double* pos, const double*, int, int, int,
                                     const NeighList*, const TransposeRef*, int, double*, double*, double*, int*, int*, double*,
-                                    double*, double*, int*, double*, hipStream_t) {
+                                    double*, double*, int*, double*, hipStream_t stream) {
   if (fail_descriptors_) return STAF_E_HIP;
   positions_ = pos;
+  if (const int bit = raise_) {
+    int* const word = status_word(device_state(stream), stream);
+    queue_.push_back([=] { *word |= bit; });
+  }
   return STAF_OK;
 }
 bool dev_mlp_upload(const StafMlp*, int, DevMlpNet*, hipStream_t) { return true; }
@@ -255,6 +261,29 @@ int main(int argc, char** argv) {
     expect(next.run(m) == 0, "call after the failed one");
     expect(next.right(), "forces after the failed call");
     expect(drained, "work in flight behind a failed call");
+  } else if (scenario == "other_poll") {
+    // another thread polls, and clears every word, between the results and what this call does next
+    staf::DeviceState* const st = staf::device_state(nullptr);
+    raise_ = 1;
+    after_results_ = [=] { for (int w = 0; w < staf::STATUS_WORDS; w++) st->status_d[w] = 0; };
+    Call c(300, -1, 1);
+    expect(c.run(m) == -10, "a condition of the call that another poll has cleared");
+    after_results_ = nullptr;
+    expect(c.run(m) == -10, "a condition of the call");
+    raise_ = 0;
+    expect(c.run(m) == 0 && c.right(), "the call after it");
+  } else if (scenario == "other_stream") {
+    // a condition of another stream is pending
+    staf::DeviceState* const st = staf::device_state(nullptr);
+    int* const word = staf::status_word(st, (hipStream_t)&queue_);
+    *word = 2;
+    Call c(300, -1, 1);
+    expect(c.run(m) == 0 && c.right(), "a call beside another stream's condition");
+    raise_ = 1;
+    expect(c.run(m) == -10, "a condition of the call");
+    raise_ = 0;
+    expect(*word == 2, "another stream's condition is gone");
+    expect(staf_ops_poll_status(nullptr) == STAF_E_SCATTER_OVERFLOW, "the poll for it");
   } else {
     return 2;
   }

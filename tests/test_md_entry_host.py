@@ -34,3 +34,13 @@ def test_a_call_whose_stage_cannot_be_launched_leaves_nothing_behind(fake_gpu):
     """The call's first kernel is queued and reads the pinned input; the call returns -20.  It has waited for the kernel, and
     the next call with the same types sends the order of the atoms again."""
     scenario(fake_gpu, "failed_launch")
+
+
+def test_a_condition_of_a_call_is_its_own(fake_gpu):
+    """Another thread's poll, which clears the words of every stream, between a call's results and its return: the call still
+    reports what its kernels found."""
+    scenario(fake_gpu, "other_poll")
+
+
+def test_a_condition_of_another_stream_is_left_to_it(fake_gpu):
+    scenario(fake_gpu, "other_stream")
