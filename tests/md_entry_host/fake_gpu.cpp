@@ -28,7 +28,8 @@ std::map<const void*, std::string>& names() {   // (filled before this file's ow
   return n;
 }
 std::function<void()> after_results_;   // runs between the results' kernel and what the host does next
-int fail_descriptors_ = 0, raise_ = 0;
+int fail_descriptors_ = 0, raise_ = 0, queries_ = 0, waits_ = 0;
+unsigned flags_ = hipDeviceScheduleAuto;
 
 void run_queue() {
   while (!queue_.empty()) {
@@ -122,6 +123,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, 
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipGetDeviceFlags(unsigned* f) { *f = flags_; return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 // (blocks are filled, so that nothing is right by the zeroes of fresh memory; freeing waits, as the runtime's does)
 hipError_t hipMalloc(void** p, size_t n) { *p = malloc(n); memset(*p, 0x7f, n); return hipSuccess; }
@@ -137,8 +139,8 @@ hipError_t hipMemset(void* p, int v, size_t n) { memset(p, v, n); return hipSucc
 hipError_t hipDeviceSynchronize() { run_queue(); return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)malloc(1); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { run_queue(); return hipSuccess; }
-hipError_t hipStreamQuery(hipStream_t) { run_queue(); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { waits_++; run_queue(); return hipSuccess; }
+hipError_t hipStreamQuery(hipStream_t) { queries_++; run_queue(); return hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) { *s = hipStreamCaptureStatusNone; return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t*) { return hipErrorUnknown; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
@@ -284,6 +286,14 @@ int main(int argc, char** argv) {
     raise_ = 0;
     expect(*word == 2, "another stream's condition is gone");
     expect(staf_ops_poll_status(nullptr) == STAF_E_SCATTER_OVERFLOW, "the poll for it");
+  } else if (scenario == "blocking_wait") {
+    queries_ = waits_ = 0;
+    Call c(300, -1, 0);
+    expect(c.run(m) == 0 && c.right() && queries_ > 0, "a call that watches the flags");
+    queries_ = waits_ = 0;
+    flags_ = hipDeviceScheduleBlockingSync | hipDeviceMapHost;
+    expect(c.run(m) == 0 && c.right(), "a call that blocks");
+    expect(queries_ == 0 && waits_ > 0, "the stream is not waited for");
   } else {
     return 2;
   }

@@ -44,3 +44,8 @@ def test_a_condition_of_a_call_is_its_own(fake_gpu):
 
 def test_a_condition_of_another_stream_is_left_to_it(fake_gpu):
     scenario(fake_gpu, "other_stream")
+
+
+def test_a_program_that_asks_for_blocking_waits_gets_them(fake_gpu):
+    """hipDeviceScheduleBlockingSync: the call sleeps until its stream is through, it does not watch the flags."""
+    scenario(fake_gpu, "blocking_wait")
