@@ -104,7 +104,8 @@ def _forces(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, type_emb_2b, x3
     # One call a species each way.  (Squares and their gradients as torch operations, an op per body and the sums around
     # them were 250 of the 2500 us of host time that a step of a small box takes.)
     tensors = (net_der_r, net_der_a, alpha2b, type_emb_2b, alpha3b, type_emb_3b)
-    if x2b.is_cuda and x2b.dtype == x3b.dtype and all(t.dtype == x2b.dtype for t in tensors):
+    if x2b.is_cuda and x2b.dtype == x3b.dtype and all(t.dtype == x2b.dtype for t in tensors) and \
+            ops.layer_widths(tipos.shape[0], alpha2b, type_emb_2b, alpha3b, type_emb_3b):
         try:
             return _LayerForces.apply(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, type_emb_2b, x3b, x3bsupp, intder3b,
                                       intder3bsupp, numtriplet, alpha3b, type_emb_3b, type_map, tipos, tn, pos, box)
@@ -257,9 +258,9 @@ class physics_layer(torch.nn.Module):
         self.output_dim = self.nalpha_r + self.nalpha_a
 
     def forward(self, x2b, x3bsupp, intmap2b, x3b, intmap3b, numtriplet, type_map):
-        tensors = (x3b, self.alpha2b, self.type_emb_2b, self.alpha3b, self.type_emb_3b)
-        if x2b.is_cuda and all(t.dtype == x2b.dtype for t in tensors) and self.alpha3b.shape[0] == self.alpha2b.shape[0] * (
-                self.alpha2b.shape[0] + 1) // 2:
+        params = (self.alpha2b, self.type_emb_2b, self.alpha3b, self.type_emb_3b)
+        if x2b.is_cuda and all(t.dtype == x2b.dtype for t in (x3b, *params)) and \
+                ops.layer_widths(self.alpha2b.shape[0], *params):
             try:
                 return _LayerFingerprints.apply(x2b, intmap2b, self.alpha2b, self.type_emb_2b, x3b, x3bsupp, self.alpha3b,
                                                 self.type_emb_3b, type_map, numtriplet)

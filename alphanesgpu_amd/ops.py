@@ -598,6 +598,23 @@ def _stream_addr():
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
+def layer_widths(nt, alpha2b, emb2b, alpha3b, emb3b):
+    """(Ar, Aa) of a species' parameters: alpha2b and emb2b [nt,Ar], alpha3b [nt(nt+1)/2,3Aa], emb3b [nt(nt+1)/2,Aa]; None for any
+    other shapes, of which the gradient calls know nothing: they write gradients of exactly these."""
+    if alpha2b.dim() != 2 or alpha3b.dim() != 2:
+        return None
+    Ar, Aa, ntc = alpha2b.shape[1], alpha3b.shape[1] // 3, nt * (nt + 1) // 2
+    shapes = [tuple(t.shape) for t in (alpha2b, emb2b, alpha3b, emb3b)]
+    return (Ar, Aa) if shapes == [(nt, Ar), (nt, Ar), (ntc, 3 * Aa), (ntc, Aa)] else None
+
+
+def _widths(*args):
+    found = layer_widths(*args)
+    if found is None:
+        raise ValueError("the gradients are of parameters [nt,Ar], [nt,Ar], [nt(nt+1)/2,3Aa] and [nt(nt+1)/2,Aa]")
+    return found
+
+
 def layer_fingerprints(x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb3b, type_map, numtriplet):
     """Fingerprints [nf,Nl,Ar+Aa] of one centre species as physics_layer_mod.py:23-45 gives them: compute_sort_proj and
     compute_sort_proj3body with the squares of emb2b, emb3b, one beside the other."""
@@ -621,8 +638,8 @@ def layer_fingerprints_grad(grad, x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, a
     dtype = x2b.dtype
     nf, Nl, nr = x2b.shape
     na = x3b.shape[2]
-    nt, Ar = alpha2b.shape
-    Aa = alpha3b.shape[1] // 3
+    nt = alpha2b.shape[0]
+    Ar, Aa = _widths(nt, alpha2b, emb2b, alpha3b, emb3b)
     v, dense = _Views(), _Dense()
     pD, pT, pS, pI, pN = v(x2b), v(x3b), v(x3bsupp), v(_i32(intmap2b)), v(_i32(numtriplet))
     e = lambda t: torch.empty(t.shape, dtype=dtype, device=x2b.device)
@@ -662,7 +679,7 @@ def layer_forces_grad(prevgrad, netderiv2b, netderiv3b, x2b, intder2b, intmap2b,
     dtype, dev = x3b.dtype, x3b.device
     nf, Nl, na = x3b.shape
     nr, N, nt = x3bsupp.shape[2], type_map.shape[0], tipos.shape[0]
-    Ar, Aa = alpha2b.shape[1], alpha3b.shape[1] // 3
+    Ar, Aa = _widths(nt, alpha2b, emb2b, alpha3b, emb3b)
     v, dense = _Views(), _Dense()
     rows = [v(t) for t in (x2b, intder2b, x3bsupp, x3b, intder3bsupp, intder3b)]
     pI, pN = v(_i32(intmap2b)), v(_i32(numtriplet))

@@ -1,0 +1,109 @@
+"""What ops.layer_* and the layers hand to the library, looked at without a GPU: the library's entries are replaced by ones that
+take note of their arguments."""
+import pytest
+import torch
+
+from alphanesgpu_amd import layers, ops
+
+NF, NL, N, NR, NA, AR, AA = 2, 3, 5, 8, 28, 4, 6
+
+
+class Calls(list):
+    """(entry, arguments) of every call."""
+
+    def entry(self, name, dtype, kinds):
+        def fn(*args):
+            assert len(args) == len(kinds.replace(" ", ""))
+            self.append((name, args))
+            return 0
+        return fn
+
+    def by_name(self, name, *args):
+        self.append((name, args))
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    seen = Calls()
+    monkeypatch.setattr(ops, "_entry", seen.entry)
+    monkeypatch.setattr(ops, "call", seen.by_name)
+    monkeypatch.setattr(ops, "_stream_addr", lambda: 0)
+    monkeypatch.setattr(ops, "_stream", lambda: None)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda t: True), raising=False)
+    return seen
+
+
+def made(nt, rows3=None, rows2=None):
+    """Arguments of ops.layer_forces of a species among nt."""
+    ntc = nt * (nt + 1) // 2
+    z = lambda *sh: torch.zeros(sh, dtype=torch.float64)
+    i = lambda *sh: torch.zeros(sh, dtype=torch.int32)
+    a = dict(netderiv2b=z(NF, NL, AR), netderiv3b=z(NF, NL, AA), x2b=z(NF, NL, NR), intder2b=z(NF, NL, 3, NR),
+             intmap2b=i(NF, NL, NR + 1), alpha2b=z(nt, AR), emb2b=z(nt, AR), x3b=z(NF, NL, NA), x3bsupp=z(NF, NL, NR),
+             intder3b=z(NF, NL, 3, 2 * NA), intder3bsupp=z(NF, NL, 3, NR), numtriplet=i(NF, NL), alpha3b=z(ntc, 3 * AA),
+             emb3b=z(ntc, AA), type_map=i(N), tipos=i(nt), type_now=i(1))
+    a["intmap3b"] = i(NF, NL, 2 * NA)
+    return a
+
+
+FORCES = ("netderiv2b", "netderiv3b", "x2b", "intder2b", "intmap2b", "alpha2b", "emb2b", "x3b", "x3bsupp", "intder3b",
+          "intder3bsupp", "numtriplet", "alpha3b", "emb3b", "type_map", "tipos", "type_now")
+FINGERPRINTS = ("x2b", "intmap2b", "alpha2b", "emb2b", "x3b", "x3bsupp", "alpha3b", "emb3b", "type_map", "numtriplet")
+# a parameter of a species among three with fewer rows than the gradient has (2-body: 3, 3-body: 6), or more, or other columns
+OTHER = [("emb2b", (2, AR)), ("alpha2b", (2, AR)), ("alpha3b", (5, 3 * AA)), ("emb3b", (5, AA)), ("emb3b", (7, AA)),
+         ("emb3b", (6, AA - 1)), ("emb2b", (3 * AR,))]
+
+
+@pytest.mark.parametrize("name,shape", OTHER)
+def test_gradients_of_other_shapes_than_the_library_writes_are_refused(calls, name, shape):
+    a = made(3)
+    a[name] = torch.zeros(shape, dtype=torch.float64)
+    with pytest.raises(ValueError):
+        ops.layer_forces_grad(torch.zeros(NF, 3 * N, dtype=torch.float64), *[a[k] for k in FORCES])
+    with pytest.raises(ValueError):
+        ops.layer_fingerprints_grad(torch.zeros(NF, NL, AR + AA, dtype=torch.float64), *[a[k] for k in FINGERPRINTS])
+    assert not calls
+
+
+@pytest.mark.parametrize("nt", [1, 2, 3])
+def test_gradients_have_the_shapes_that_the_library_writes(calls, nt):
+    a = made(nt)
+    ntc = nt * (nt + 1) // 2
+    got = ops.layer_forces_grad(torch.zeros(NF, 3 * N, dtype=torch.float64), *[a[k] for k in FORCES])
+    assert [tuple(t.shape) for t in got] == [(NF, NL, AR), (nt, AR), (nt, AR), (NF, NL, AA), (ntc, 3 * AA), (ntc, AA)]
+    got = ops.layer_fingerprints_grad(torch.zeros(NF, NL, AR + AA, dtype=torch.float64), *[a[k] for k in FINGERPRINTS])
+    assert [tuple(t.shape) for t in got] == [(nt, AR), (nt, AR), (ntc, 3 * AA), (ntc, AA)]
+    assert [c[0] for c in calls] == ["staf_op_layer_forces_grad", "staf_op_layer_fingerprints_grad"]
+
+
+def forward(a):
+    """A physics_layer's and a force_layer's call."""
+    ph = layers.physics_layer(torch.zeros(1, AR, dtype=torch.float64), torch.zeros(1, 3 * AA, dtype=torch.float64),
+                              [torch.zeros(1, AR, dtype=torch.float64), torch.zeros(1, AA, dtype=torch.float64)])
+    for own, k in (("alpha2b", "alpha2b"), ("type_emb_2b", "emb2b"), ("alpha3b", "alpha3b"), ("type_emb_3b", "emb3b")):
+        setattr(ph, own, torch.nn.Parameter(a[k]))
+    yield lambda: ph(a["x2b"], a["x3bsupp"], a["intmap2b"], a["x3b"], a["intmap3b"], a["numtriplet"], a["type_map"])
+    fl = layers.force_layer.__new__(layers.force_layer)
+    torch.nn.Module.__init__(fl)
+    yield lambda: fl(a["netderiv2b"], a["x2b"], a["intder2b"], a["intmap2b"], a["alpha2b"], a["netderiv3b"], a["x3b"], a["x3bsupp"],
+                     a["intder3b"], a["intder3bsupp"], a["intmap3b"], a["numtriplet"], a["alpha3b"], a["emb2b"], a["emb3b"],
+                     a["type_map"], a["tipos"], a["type_now"])
+
+
+def test_layers_take_the_single_calls(calls):
+    for layer in forward(made(3)):
+        layer()
+    assert [c[0] for c in calls] == ["staf_op_layer_fingerprints", "staf_op_layer_forces"]
+
+
+@pytest.mark.parametrize("name,shape", [("alpha3b", (5, 3 * AA)), ("emb3b", (5, AA)), ("emb3b", (7, AA))])
+def test_layers_of_parameters_with_other_rows_take_the_ops(calls, name, shape):
+    """The forward ops read 2 nt - 1 rows and take such parameters; autograd refuses their gradients by the shapes."""
+    a = made(3)
+    a[name] = torch.zeros(shape, dtype=torch.float64)
+    for layer in forward(a):
+        try:
+            layer()
+        except ValueError as e:   # (rows of alpha3b that are those of no number of species)
+            assert name == "alpha3b" and "is not nt(nt+1)/2" in str(e)
+    assert calls and not any("layer" in c[0] for c in calls)
