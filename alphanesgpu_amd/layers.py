@@ -106,6 +106,7 @@ def _forces(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, type_emb_2b, x3
     tensors = (net_der_r, net_der_a, alpha2b, type_emb_2b, alpha3b, type_emb_3b)
     if x2b.is_cuda and x2b.dtype == x3b.dtype and all(t.dtype == x2b.dtype for t in tensors) and \
             ops.layer_widths(tipos.shape[0], alpha2b, type_emb_2b, alpha3b, type_emb_3b):
+        ops.check_rows(x3b, int3b)
         try:
             return _LayerForces.apply(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, type_emb_2b, x3b, x3bsupp, intder3b,
                                       intder3bsupp, numtriplet, alpha3b, type_emb_3b, type_map, tipos, tn, pos, box)
@@ -261,6 +262,7 @@ class physics_layer(torch.nn.Module):
         params = (self.alpha2b, self.type_emb_2b, self.alpha3b, self.type_emb_3b)
         if x2b.is_cuda and all(t.dtype == x2b.dtype for t in (x3b, *params)) and \
                 ops.layer_widths(self.alpha2b.shape[0], *params):
+            ops.check_rows(x3b, intmap3b)
             try:
                 return _LayerFingerprints.apply(x2b, intmap2b, self.alpha2b, self.type_emb_2b, x3b, x3bsupp, self.alpha3b,
                                                 self.type_emb_3b, type_map, numtriplet)

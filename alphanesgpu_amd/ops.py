@@ -608,6 +608,12 @@ def layer_widths(nt, alpha2b, emb2b, alpha3b, emb3b):
     return (Ar, Aa) if shapes == [(nt, Ar), (nt, Ar), (ntc, 3 * Aa), (ntc, Aa)] else None
 
 
+def check_rows(x3b, intmap3b):
+    """The map of the triplets' neighbours as the ops take it: int32, and rows that lie like x3b's.  No kernel reads it."""
+    v = _Views()
+    v(x3b), v(_i32(intmap3b))
+
+
 def _widths(*args):
     found = layer_widths(*args)
     if found is None:

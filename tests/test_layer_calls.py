@@ -107,3 +107,15 @@ def test_layers_of_parameters_with_other_rows_take_the_ops(calls, name, shape):
         except ValueError as e:   # (rows of alpha3b that are those of no number of species)
             assert name == "alpha3b" and "is not nt(nt+1)/2" in str(e)
     assert calls and not any("layer" in c[0] for c in calls)
+
+
+@pytest.mark.parametrize("what,error", [(lambda m: m.long(), TypeError), (lambda m: m.transpose(0, 1).contiguous().transpose(0, 1), ValueError),
+                                        (lambda m: torch.stack([m, m], -1)[..., 0], ValueError), (lambda m: None, AttributeError)])
+def test_layers_refuse_a_map_of_the_triplets_that_the_ops_refuse(calls, what, error):
+    """Another type, rows that lie otherwise and no map at all: no kernel reads it, and the ops refuse it all the same."""
+    a = made(2)
+    a["intmap3b"] = what(a["intmap3b"])
+    for layer in forward(a):
+        with pytest.raises(error):
+            layer()
+    assert not calls
