@@ -514,9 +514,11 @@ static int layer_fingerprints_grad(const real* P, const real* D, const real* Dsu
                                    const int* numtriplet, int nt, real* g_alpha2b, real* g_emb2b, real* g_alpha3b,
                                    real* g_emb3b, int ld, void* stream) {
   if (Ar <= 0 || Aa <= 0 || nt <= 0 || (!P && Nl != 0)) return STAF_E_BAD_ARG;
-  int rc = alpha_dist_grad<real>(D, nr, alpha2b, Ar, g_alpha2b, nf, Nl, im2, P, emb2b, type_map, g_emb2b, nt, ld, stream, 1,
-                                 Ar + Aa);
-  if (rc == STAF_OK)
+  int rc = STAF_OK;   // (a body without gradients is left out)
+  if (g_alpha2b)
+    rc = alpha_dist_grad<real>(D, nr, alpha2b, Ar, g_alpha2b, nf, Nl, im2, P, emb2b, type_map, g_emb2b, nt, ld, stream, 1,
+                               Ar + Aa);
+  if (rc == STAF_OK && g_alpha3b)
     rc = alphagrad_ang<real>(Dsup, Tang, nr, na, Nl ? P + Ar : P, nf, Nl, nullptr, im2, alpha3b, Aa, g_alpha3b, emb3b, type_map,
                              g_emb3b, numtriplet, nt * (nt + 1) / 2, nt, ld, stream, 1, Ar + Aa);
   return rc;

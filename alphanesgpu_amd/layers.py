@@ -65,7 +65,8 @@ class _LayerFingerprints(torch.autograd.Function):
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, grad):
-        ga2, ge2, ga3, ge3 = ops.layer_fingerprints_grad(grad, *ctx.saved_tensors)
+        need = ctx.needs_input_grad
+        ga2, ge2, ga3, ge3 = ops.layer_fingerprints_grad(grad, *ctx.saved_tensors, (need[2] or need[3], need[6] or need[7]))
         return None, None, ga2, ge2, None, None, ga3, ge3, None, None
 
 

@@ -639,8 +639,10 @@ def layer_fingerprints(x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb
     return out
 
 
-def layer_fingerprints_grad(grad, x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb3b, type_map, numtriplet):
-    """dL/dalpha2b, dL/demb2b, dL/dalpha3b, dL/demb3b (zero) of layer_fingerprints from dL/dfingerprints."""
+def layer_fingerprints_grad(grad, x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, alpha3b, emb3b, type_map, numtriplet,
+                            bodies=(True, True)):
+    """dL/dalpha2b, dL/demb2b, dL/dalpha3b, dL/demb3b (zero) of layer_fingerprints from dL/dfingerprints, None for a body that
+    is not asked for."""
     dtype = x2b.dtype
     nf, Nl, nr = x2b.shape
     na = x3b.shape[2]
@@ -649,12 +651,16 @@ def layer_fingerprints_grad(grad, x2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, a
     v, dense = _Views(), _Dense()
     pD, pT, pS, pI, pN = v(x2b), v(x3b), v(x3bsupp), v(_i32(intmap2b)), v(_i32(numtriplet))
     e = lambda t: torch.empty(t.shape, dtype=dtype, device=x2b.device)
-    ga2, ge2, ga3, ge3 = e(alpha2b), e(emb2b), e(alpha3b), e(emb3b)
+    out = [None] * 4
+    if bodies[0]:
+        out[:2] = e(alpha2b), e(emb2b)
+    if bodies[1]:
+        out[2:] = e(alpha3b), e(emb3b)
     fn = _entry("staf_op_layer_fingerprints_grad", dtype, "pppp" "iiii" "p" "pippip" "pp" "i" "pppp" "ip")
     _checked(fn(dense(grad), pD, pS, pT, nr, na, nf, Nl, pI, dense(alpha2b), Ar, dense(emb2b), dense(alpha3b), Aa,
-                dense(emb3b), _addr(_i32(type_map)), pN, nt, ga2.data_ptr(), ge2.data_ptr(), ga3.data_ptr(),
-                ge3.data_ptr(), v.ld, _stream_addr()), "staf_op_layer_fingerprints_grad")
-    return ga2, ge2, ga3, ge3
+                dense(emb3b), _addr(_i32(type_map)), pN, nt, *[_addr(t) for t in out], v.ld, _stream_addr()),
+             "staf_op_layer_fingerprints_grad")
+    return tuple(out)
 
 
 def layer_forces(netderiv2b, netderiv3b, x2b, intder2b, intmap2b, alpha2b, emb2b, x3b, x3bsupp, intder3b, intder3bsupp,

@@ -492,7 +492,8 @@ int staf_op_frames_f64(const double* positions, const double* boxer, int nf, int
  * force_layer_mod.py:22-44 and :92-103): the embeddings are given as they are trained, squared where they are read, and
  * their gradients come back with respect to them (what tf.square's gradient makes of the ops').  Arrays as for the single
  * ops; fingerprints and dL/dfingerprints are [nf, N_local, Ar + Aa], 2-body first.
- * staf_op_layer_fingerprints_grad: dL/dalpha2b, dL/demb2b [nt,Ar], dL/dalpha3b [ntc,3Aa], dL/demb3b [ntc,Aa] (zero).
+ * staf_op_layer_fingerprints_grad: dL/dalpha2b, dL/demb2b [nt,Ar], dL/dalpha3b [ntc,3Aa], dL/demb3b [ntc,Aa] (zero); a null
+ * grad_alpha2b or grad_alpha3b leaves that body out.
  * staf_op_layer_forces: forces [nf,3N] and, when virial, pos and box are given, virial [nf,9], as staf_op_forces.
  * staf_op_layer_forces_grad: the outputs of both gradient ops of the forces; a null grad_alpha2b or grad_alpha3b leaves that
  * body out; prevgrad_virial, pos and box: the virial forms.

@@ -119,3 +119,18 @@ def test_layers_refuse_a_map_of_the_triplets_that_the_ops_refuse(calls, what, er
         with pytest.raises(error):
             layer()
     assert not calls
+
+
+@pytest.mark.parametrize("frozen", ["2", "3"])
+def test_a_body_whose_parameters_are_frozen_gets_no_gradient_kernels(calls, frozen):
+    """The library is handed null for the gradients of a body that needs none, and makes no launches for it."""
+    a = made(2)
+    ph = layers.physics_layer(a["alpha2b"], a["alpha3b"], [a["emb2b"], a["emb3b"]])
+    for name, p in ph.named_parameters():
+        p.requires_grad_(frozen not in name)
+    out = ph(a["x2b"], a["x3bsupp"], a["intmap2b"], a["x3b"], a["intmap3b"], a["numtriplet"], a["type_map"])
+    out.backward(torch.zeros_like(out))
+    name, args = calls[-1]
+    assert name == "staf_op_layer_fingerprints_grad"
+    assert [v is None for v in args[-6:-2]] == [frozen == "2"] * 2 + [frozen == "3"] * 2
+    assert [p.grad is None for _, p in ph.named_parameters()] == [frozen in n for n, _ in ph.named_parameters()]

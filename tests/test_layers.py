@@ -366,3 +366,32 @@ def test_arguments_that_are_not_dense_are_copied_to_places_of_their_own(entry):
                 f = ops.force_total(im2, [32, 64], [form(slots), form(none[0])], [form(own), form(none[1])])
         forms.append(f)
     assert torch.equal(*forms)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("frozen", ["2", "3"])
+def test_gradients_beside_a_frozen_body_have_the_bits_of_both(frozen):
+    """physics_layer with the parameters of one body frozen: the other body's gradients, to the last bit."""
+    import torch
+    from alphanesgpu_amd import layers, ops, synth
+    dev, dt = torch.device("cuda:0"), torch.float64
+    pos, box = synth.water_frame((4, 4, 2), 9.86, 0.05, 3)
+    T = lambda a: torch.as_tensor(np.ascontiguousarray(a)).to(dev)
+    ops.construct_descriptors_light(synth.RC, 60, 1770, 96, T(box[None]), synth.RS, synth.RA, 1, dtype=dt)
+    rad, ang, sup, im2, im3, _, _, _, ntr = ops.compute_descriptors_light(T(pos[None]), T(box[None]))
+    tm = T(np.repeat(np.arange(2, dtype=np.int32), (32, 64)))
+    p = synth.fingerprint_params(2, dtype=np.float64)[0]
+    ph = layers.physics_layer(T(p["alpha2b"]), T(p["alpha3b"]), [T(p["emb2b"]), T(p["emb3b"])])
+    c = lambda t: t[:, :32]
+    g = torch.Generator(device=dev)
+    g.manual_seed(5)
+    U = torch.randn((1, 32, ph.output_dim), dtype=dt, device=dev, generator=g)
+    got = []
+    for freeze in (False, True):
+        ph.zero_grad()
+        for name, q in ph.named_parameters():
+            q.requires_grad_(not freeze or frozen not in name)
+        ph(c(rad), c(sup), c(im2), c(ang), c(im3), c(ntr), tm).backward(U)
+        got.append({name: q.grad for name, q in ph.named_parameters()})
+    for name, x in got[1].items():
+        assert x is None if frozen in name else torch.equal(x, got[0][name])
