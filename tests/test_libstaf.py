@@ -353,10 +353,10 @@ def test_device_mlp_matches_host_mlp(prec, tol):
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec,tol", [("double", 1e-11), ("float", 2e-5)])
 def test_device_mlp_on_small_widths_and_ragged_atom_counts(tmp_path, prec, tol):
-    """The network kernel (matrix cores, 16 atoms per workgroup) against the host evaluation on a written three-species
-    model whose widths (fingerprints 9/7/11, hidden 20) are no multiples of the tile sizes and whose atom counts
-    (7, 9, 3) leave every workgroup partly empty: a wrong row layout of the matrix tiles or a padding row entering a sum
-    shows here, not on the 256/512-atom frames."""
+    """The network kernel (matrix cores, four atoms per workgroup in launches this small) against the host evaluation on a
+    written three-species model whose widths (fingerprints 9/7/11, hidden 20) are no multiples of the tile sizes and whose
+    atom counts (7, 9, 3) leave a workgroup of every species partly empty: a wrong row layout of the matrix tiles or a
+    padding row entering a sum shows here, not on the 256/512-atom frames."""
     from alphanesgpu_amd import libstaf, model_dir
     from test_oracle_pins import cluster, small_model
     ps = small_model(3, (5, 4, 6), (4, 3, 5, 3, 4, 3), seed=5, hidden=20, dense=True)
@@ -380,8 +380,8 @@ def test_device_mlp_on_small_widths_and_ragged_atom_counts(tmp_path, prec, tol):
                                          ([300, 33], "linear"), ([16, 48, 16, 5], "linear")])
 def test_device_mlp_stack_shapes(tmp_path, prec, tol, hidden, last):
     """The matrix-core network at the edges of its tiles: no hidden layer, one feature, exactly a tile, one more and one
-    less, more tiles than waves, an output neuron with an activation; 16 and 17 atoms of a species (a workgroup exactly
-    full, one atom in the next).  Against the host evaluation; float64: rounding of sums of at most 300 terms,
+    less, more tiles than waves, an output neuron with an activation; 16 and 17 atoms of a species (workgroups of four
+    atoms exactly full, one atom in the next).  Against the host evaluation; float64: rounding of sums of at most 300 terms,
     float32: as the test above."""
     from alphanesgpu_amd import libstaf, model_dir, synth
     from test_oracle_pins import cluster
@@ -410,8 +410,8 @@ def test_device_mlp_stack_shapes(tmp_path, prec, tol, hidden, last):
 def test_deep_stacks_around_the_limits_of_a_workgroup(tmp_path, capfd, prec, tol, hidden, on_gpu):
     """Stacks whose activations of 16 atoms just fit a workgroup's LDS, fit it for 8 atoms only, and do not fit: the first
     two are evaluated on the GPU, the last one on the host (a line on stderr says so) and, in the batch inference, by the
-    layers.  17 atoms of a species: two, three and one workgroups, the last one with a single atom.  Against the host
-    evaluation; float64: rounding of sums of at most 420 terms, float32: as above."""
+    layers.  17 atoms of a species: five workgroups of four, the last one with a single atom.  Against the host evaluation;
+    float64: rounding of sums of at most 420 terms, float32: as above."""
     import torch
     from alphanesgpu_amd import inference, libstaf, model_dir, synth
     from test_oracle_pins import cluster
@@ -912,3 +912,80 @@ def test_a_handle_keeps_the_order_of_the_types_it_was_last_given():
         fresh.close()
         assert got[0] == want[0] and np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2])
     used.close()
+
+
+def _gas(counts, seed):
+    """So many atoms of each species, one anywhere in the middle of a 4 A cell: at least 2.5 A apart, few neighbours."""
+    rng = np.random.Generator(np.random.Philox(seed))
+    n = sum(counts)
+    edge = int(np.ceil(n ** (1 / 3))) + 1
+    x = 4.0 * np.stack(np.unravel_index(rng.permutation(edge ** 3)[:n], (edge,) * 3), 1) + rng.uniform(0, 1.5, (n, 3))
+    return x, 4.0 * edge * np.array([1.0, 0.0, 0.0, 1.0, 0.0, 1.0]), np.repeat(np.arange(len(counts), dtype=np.int32), counts)
+
+
+def _device_and_host_network(folder, prec, tol, hidden, last, counts, seed, change=None):
+    """A model of two species with these hidden layers, evaluated on the GPU and by the host.  Forces and virials to tol;
+    energies to tol and, in single precision, what the host's running sum of n atoms may lose (n 2^-24), of the energy or of a
+    sixteenth per atom where they cancel."""
+    from alphanesgpu_amd import libstaf, model_dir, synth
+    rng = np.random.Generator(np.random.Philox(seed))
+    ps = synth.fingerprint_params(nt=2, ar_map=(5, 4), aa_map=(4, 3, 5), seed=3, dense_embedding=True)
+    for p, h in zip(ps, hidden):
+        dims = [p["mu"].shape[0]] + h + [1]
+        acts = ["tanh" if i % 2 == 0 or len(h) > 4 else "relu" for i in range(len(h))] + [last]
+        p["layers"] = [(rng.normal(0, 1 / np.sqrt(a), (a, b)), rng.normal(0.3, 0.1, b), act)
+                       for a, b, act in zip(dims[:-1], dims[1:], acts)]
+        if change is not None:
+            change(p, rng)
+    x, box, types = _gas(counts, seed)
+    model_dir.write_model_dir(str(folder), ps, rc=4.5, rc_ang=3.2, rs=1.6, radial_buffer=40, angular_buffer=780, tipos=counts,
+                              precision=prec)
+    got = []
+    for host in (True, False):
+        m = libstaf.StafModel(str(folder), precision=1 if prec == "double" else 0, full_virial=True, host_mlp=host)
+        got.append(m.compute(x, box, types))
+        m.close()
+    (e0, f0, v0), (e1, f1, v1) = got
+    assert np.isfinite(e0) and np.isfinite(f0).all() and (change is not None or np.abs(f0).max() > 0)
+    assert abs(e1 - e0) <= (tol + (len(x) * 2.0 ** -24 if prec == "float" else 0.0)) * max(abs(e0), len(x) / 16)
+    assert nerr(f1, f0) <= tol and nerr(v1, v0) <= tol
+
+
+# Launches of more than 1024 atoms in double precision and of more than 2048 in single take more than four to a workgroup:
+# eight (double, up to 2048; stacks that fit no more) or sixteen.  The species' last workgroups are ragged.
+LARGER = [("double", 1e-11, (1004, 521)), ("double", 1e-11, (1506, 601)), ("float", 2e-5, (1506, 601))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,tol,counts", LARGER)
+@pytest.mark.parametrize("hidden,last", [([], "linear"), ([], "tanh"), ([1], "linear"), ([16], "relu"), ([17, 15], "tanh"),
+                                         ([300, 33], "linear"), ([16, 48, 16, 5], "linear")])
+def test_network_stack_shapes_with_more_atoms_per_workgroup(tmp_path, prec, tol, counts, hidden, last):
+    """The stacks of test_device_mlp_stack_shapes, beside one without and one with another number of hidden layers in the same launch, by
+    eight and by sixteen atoms."""
+    _device_and_host_network(tmp_path, prec, tol, (hidden, [] if hidden else [300, 33]), last, counts, seed=41)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,tol,hidden,counts", [("float", 2e-5, [400] * 6, (705, 1401)), ("float", 2e-5, [430] * 6, (705, 1401)),
+                                                    ("double", 1e-11, [192] * 6, (705, 1401)), ("double", 1e-11, [200] * 6, (705, 1401)),
+                                                    ("double", 1e-11, [400] * 6, (405, 701))])
+def test_deep_stacks_with_more_atoms_per_workgroup(tmp_path, prec, tol, hidden, counts):
+    """Sixteen atoms where their activations fit (2400 of 2496 features in single, 1152 of 1216 in double precision), eight
+    where they do not (2592; 1248, 2400 of 2432: 160 KB of LDS).  float64: sums of at most 400 terms through seven layers."""
+    _device_and_host_network(tmp_path, prec, tol, (hidden, [9]), "linear", counts, seed=43)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,tol,counts", LARGER)
+def test_infinite_activations_with_more_atoms_per_workgroup(tmp_path, prec, tol, counts):
+    """As test_infinite_activations_stay_out_of_the_padded_features, by eight and by sixteen atoms.  (The infinite feature
+    saturates the whole tanh layer behind it: forces are zero.)"""
+    def overflow(p, rng):
+        n = p["mu"].shape[0]
+        p["mu"][2] += 50.0
+        W = [rng.normal(0, 1 / np.sqrt(a), (a, b)) for a, b in ((n, 5), (5, 7), (7, 6), (6, 1))]
+        W[0][:, 3] = 0
+        W[0][2, 3] = 0.9 * (np.finfo(np.float64).max if prec == "double" else float(np.finfo(np.float32).max))
+        p["layers"] = [(w, rng.normal(0.3, 0.1, w.shape[1]), a) for w, a in zip(W, ("linear", "tanh", "tanh", "linear"))]
+    _device_and_host_network(tmp_path, prec, tol, ([5], [5]), "linear", counts, seed=45, change=overflow)
