@@ -285,8 +285,10 @@ struct TriArgs {
   real* out;              // MODE 0: AF3, MODE 2, 3: gradnet  [nf, Nl, Aa] contiguous
   real* partial;          // MODE 1, 2: [gridDim.x, nsig*Aa*3]; MODE 3: [gridDim.x, 2, nsig*Aa*3] force branch, energy branch
   int nf, N, Nl, ld, nr, na, Aa, nt;
-  int raw_emb;            // emb3b is to be squared
-  int out_ld, P_ld;       // row lengths of out and P, 0: Aa
+  int raw_emb;            // emb3b is to be squared (not MODE 3)
+  // row lengths of out in MODE 0 and of P in MODE 1, 0: Aa.  The other modes have no scalar registers left for them (MODE 3 in
+  // single precision: 218 more instructions that spill and fetch scalars, 156 -> 160 us per step of 8 frames of 768 atoms).
+  int out_ld, P_ld;
 };
 
 // A staged triplet: the offsets of its two table rows (16 bits each, in one word), T and -- force gradient -- the
@@ -442,7 +444,7 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
       }
     }
   }
-  tab.build(A.alpha3b, A.emb3b, A.raw_emb);
+  tab.build(A.alpha3b, A.emb3b, MODE != 3 && A.raw_emb);
   HE::fill(etab, tid, BLOCK);
   if (MODE != 0)
     for (int q = tid; q < NG * nacc; q += BLOCK) accw[q] = 0;
@@ -523,7 +525,7 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
       }
     }
     for (int a = tid; a < Aa; a += BLOCK) {
-      if (MODE != 0) sP[a] = A.P[(size_t)atom * (A.P_ld ? A.P_ld : Aa) + a];
+      if (MODE != 0) sP[a] = A.P[(size_t)atom * (MODE == 1 && A.P_ld ? A.P_ld : Aa) + a];
       if (MODE == 3) sPE[a] = A.PE[(size_t)atom * Aa + a];
     }
     for (int q = tid; q < WAVES * Aa; q += BLOCK) outw[q] = 0;
@@ -738,7 +740,7 @@ __device__ __forceinline__ void tri_reduce_body(const TriArgs<real> A, const int
         real s = 0;
 #pragma unroll
         for (int w = 0; w < WAVES; w++) s += outw[w * Aa + a];
-        A.out[(size_t)atom * (A.out_ld ? A.out_ld : Aa) + a] = s;
+        A.out[(size_t)atom * (MODE == 0 && A.out_ld ? A.out_ld : Aa) + a] = s;
       }
     __syncthreads();
     if (stride > total - 1 - atom) break;   // (no overflow of atom + stride)
