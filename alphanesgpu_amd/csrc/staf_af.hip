@@ -426,9 +426,9 @@ static int step_fingerprints_launch(const StepSpecies<real>* sp, int n, const St
   return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
 }
 // Few centres: a launch lasts as long as one centre takes, which workgroups of 512 threads shorten (32 triplets at a time
-// instead of 16, half the rounds of tables, a class staged at once): MD call of 96 atoms 100.9 -> 94.4 us, 192 103 -> 96.5,
-// 432 110.5 -> 105.  A CU holds two such workgroups; beyond that 256 threads are as fast (576 atoms: 118.8 and 117.9 us) or
-// faster (1152: 168 and 173).
+// instead of 16, half the rounds of tables, a class staged at once): MD call of 225 atoms 87.7 -> 79.3 us, 432 93.9 -> 86.0, 504
+// 94.0 -> 88.7.  A CU holds two such workgroups; beyond that 256 threads are as fast (588 atoms: 98.5 and 98.6 us) or faster
+// (768: 99.7 and 101.0, 1080: 119.3 and 123.1, 1215: 125.2 and 130.5).
 constexpr int WIDE_FINGERPRINT_CENTRES = 512;   // two per CU
 template <typename real>
 int step_fingerprints(const StepSpecies<real>* sp, int n, const StepRows<real>& R, const int* type_map, int nt,

@@ -479,8 +479,10 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
   memcpy(pos_h, x, (size_t)nall * 3 * sizeof(double));
   memcpy(pos_h + (size_t)nall * 3, box, 6 * sizeof(double));
   if (!same_order) {
-    // the slots, in the caller's order within a species.  (Two species: one running number; with a table of running numbers
-    // every atom waits for the one before it to be stored, 40 us for 24576 atoms.)
+    // the slots, in the caller's order within a species.  With a table of running numbers an atom waits until the last one of
+    // its species has stored its own: 24576 atoms in random order, 62 / 29 / 21 / 21 us for one / two / three / four species.
+    // One running number, which one and two species need, stays in a register: 18.6.  (A pass over the atoms per species
+    // mispredicts: 67 to 220 us for two, 143 to 249 for three.)
     int* const slot = (int*)(m->in_h.p + n_in);
     const int* const t = m->types_seen.data();
     if (nt <= 2) {

@@ -848,9 +848,9 @@ int step_forces(const StepSpecies<real>* sp, int n, const StepRows<real>& R, con
   if (wg == 0) return STAF_OK;
   M.first[M.entries] = wg;
   // A launch of few centres lasts as long as one centre takes, and with eight waves a centre's passes are shared by twice
-  // as many: MD call of 96 atoms 104 -> 100 us, 288 112.6 -> 108.4, 576 119.5 -> 116.7, 768 142.7 -> 140.4.  From three
-  // centres per CU on (1152: 168.1 and 167.1) the four-wave workgroups, of which a CU holds as many waves, are no slower,
-  // and the registers and LDS of the wide ones cost residency in longer launches.
+  // as many: MD call of 225 atoms 84.8 -> 79.3 us, 432 89.7 -> 86.0, 504 91.6 -> 88.7, 588 101.2 -> 98.5, 768 103.5 -> 99.7.  A
+  // little beyond it they still are no slower (864: 105.1 and 104.1, 960: 112.1 and 109.6, 1152: 126.1 and 123.1, 1215: 125.2 and
+  // 123.8); in longer launches the registers and LDS of the wide ones cost residency.
   constexpr int FORCE3_WIDE_CENTRES = 768;   // three per CU
   if (wg <= FORCE3_WIDE_CENTRES && lds_wide <= 64 * 1024) {
     KernelTimer kt_("force3_kernel", stream);

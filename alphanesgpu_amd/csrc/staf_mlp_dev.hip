@@ -677,7 +677,12 @@ static int eval_nets(const DevMlpCall<real>* calls, int n, hipStream_t stream) {
   // workgroups find a CU each: double precision by fours up to 256 workgroups (96 to 768 atoms 22.5 -> 14.1 us) and by
   // eights up to as many (1500 atoms by 16 / 8 / 4: 23.3 / 17.8 / 23.6; 3072: 24 / 29 / 34).  In single precision, whose
   // weights are half the bytes, two small workgroups share a CU (96 to 768 atoms 17.3 -> 12.3, 1500 atoms 17.8 / 15.7 / 15.2,
-  // 3072 18.4 / 19.8 / 18.8).  (Times between the library's events.)
+  // 3072 18.4 / 19.8 / 18.8).  (Times between the library's events.)  The lines are those of 60-140-140-1 stacks.  Others, by 16 /
+  // 8 / 4, double: 60-300-300-1, 768 atoms 44.4 / 30.2 / 27.9, 1500 44.2 / 31.2 / 48.2, 2046 44.6 / 53.4 / 50.7; 60-32-32-1,
+  // 768 14.1 / 11.4 / 10.1, 1500 13.7 / 11.4 / 10.6, 2046 13.8 / 11.7 / 10.8, 4096 18.6 / 15.5 / 13.6; single: 60-300-300-1, 768
+  // 30.1 / 24.9 / 19.9, 1500 30.3 / 26.4 / 29.7, 2046 30.5 / 42.9 / 30.9; 60-32-32-1, 2046 12.9 / 11.6 / 10.3, 4096 16.4 / 14.8 / 12.4.
+  // Narrow stacks' weights cost less than their chains, and few atoms pay for more workgroups than this; so do eight for 4096
+  // atoms of 60-140-140-1 in double (34.0 / 30.6 / 42.8).
   const int most = mlp_atoms<T>(rows);
   if (most == 0) return STAF_E_LIMIT;
   if (by4 <= (sizeof(T) == 8 ? 256 : 512)) return eval_nets_by<T, real, 4>(calls, n, rows, tiles, stream);

@@ -52,10 +52,12 @@ struct TriCfg {
   // The fused double-precision fingerprint kernel (the MD entry: thousands of centres per launch, several per
   // workgroup) stages 128, and its registers are held to six waves per SIMD: 26832 bytes of LDS and six workgroups per
   // CU (160 and five before: with the table's rows of sixteen below, 426 -> 409 us for 24576 centres, 118 -> 113 for
-  // 6144; 394 and 108.5 with the exponential of HotExp::Factor).  The plain double-precision fingerprint kernel stages 448: a CU hands out its 160 KB of LDS in pieces of 1280 bytes, so the 32496 bytes that 512 staged triplets
-  // make count as 33280 and four workgroups fit, not the five that the occupancy query of the runtime reports
-  // (measured with a kernel that counts its resident workgroups per CU); with 448 it is 31472 bytes and five
-  // (6144-atom step 360.6 -> 356.8 us).
+  // 6144; 394 and 108.5 with the exponential of HotExp::Factor).  The plain double-precision fingerprint kernel stages 448:
+  // 30512 bytes of LDS (60 slots, 40 channels, two species), five workgroups per CU, which is what its registers are held to.
+  // 512 are 31536 bytes, also five: no slower (2048 / 4096 / 16384 centres 38.2 / 64.9 / 222.5 us by 448 and 37.8 / 64.6 /
+  // 221.2 by 512), for a kilobyte of what a workgroup may use.  (With table rows of seventeen entries 512 were 32496 bytes,
+  // 33280 in the pieces of 1280 that a CU hands out its 160 KB in, and four workgroups, not the five that the occupancy query
+  // of the runtime reports: 6144-atom step 360.6 -> 356.8 us with 448.)
   static constexpr int QB = BLOCK > TRI_BLOCK ? 512 : sizeof(real) == 8 ? (MODE == 3 ? 256 : MODE == 2 ? 448 : FUSED ? 128 : MODE == 0 ? 448 : 512) : 512;
   // waves per SIMD the register allocation is held to: without a bound the allocation comes out a few registers
   // above the next occupancy step.  The
@@ -68,6 +70,8 @@ struct TriCfg {
   // fingerprints' rows are the sixteen channels alone, 256 bytes in double precision, so that the sixteen lanes of every
   // subset read the same banks in the same order whichever rows they are at (a 16-byte read per lane of four rows 272
   // bytes apart takes 8.3 clocks of a CU's LDS, of whole rows of 256 bytes 4.7; the launch of 24576 centres 430 -> 420 us).
+  // Single precision reads 8 bytes per lane and takes the same time with rows of sixteen (128 bytes) and of seventeen: 64 /
+  // 2048 / 16384 centres 14.6 / 21.8 / 116.3 and 14.9 / 21.8 / 116.3 us.
   static constexpr int PITCH = MODE == 0 ? TRI_CAP : TRI_CAP + 1;
   static constexpr bool FORCE_BRANCH = MODE == 2 || MODE == 3;    // dL/dF comes in: der3b, der3bsupp are read
   static constexpr bool ENERGY_BRANCH = MODE == 1 || MODE == 3;   // dL/dAF3 comes in

@@ -102,8 +102,8 @@ class _LayerForces(torch.autograd.Function):
 
 def _forces(net_der_r, net_der_a, x2b, intder2b, int2b, alpha2b, type_emb_2b, x3b, x3bsupp, intder3b, intder3bsupp, int3b,
             numtriplet, alpha3b, type_emb_3b, type_map, tipos, tn, pos, box):
-    # One call a species each way.  (Squares and their gradients as torch operations, an op per body and the sums around
-    # them were 250 of the 2500 us of host time that a step of a small box takes.)
+    # One call a species each way.  (Host time of a species' forces and their gradients without a GPU: 215 us, as squares, ops
+    # and sums of their own 265; of its fingerprints and their gradients 165 and 265.)
     tensors = (net_der_r, net_der_a, alpha2b, type_emb_2b, alpha3b, type_emb_3b)
     if x2b.is_cuda and x2b.dtype == x3b.dtype and all(t.dtype == x2b.dtype for t in tensors) and \
             ops.layer_widths(tipos.shape[0], alpha2b, type_emb_2b, alpha3b, type_emb_3b):
