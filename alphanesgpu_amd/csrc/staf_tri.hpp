@@ -61,7 +61,7 @@ struct TriCfg {
   static constexpr int QB = BLOCK > TRI_BLOCK ? 512 : sizeof(real) == 8 ? (MODE == 3 ? 256 : MODE == 2 ? 448 : FUSED ? 128 : MODE == 0 ? 448 : 512) : 512;
   // waves per SIMD the register allocation is held to: without a bound the allocation comes out a few registers
   // above the next occupancy step.  The
-  // single-precision pass for both gradients is held to six (80 registers, 56 bytes of spill per lane outside the
+  // single-precision pass for both gradients is held to six (80 registers, 52 bytes of spill per lane outside the
   // item loop) where it would take 95 and run four: 146 against 168 us per 8-frame step; seven (with a staging block
   // of 256 so that seven workgroups fit a CU's LDS) is slower again (156 us).
   static constexpr int MIN_WAVES = BLOCK > TRI_BLOCK ? 4 : sizeof(real) == 8 ? (MODE == 0 ? (FUSED ? 6 : 5) : 4)
