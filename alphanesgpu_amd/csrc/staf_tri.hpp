@@ -54,7 +54,7 @@ struct TriCfg {
   // CU (160 and five before: with the table's rows of sixteen below, 426 -> 409 us for 24576 centres, 118 -> 113 for
   // 6144; 394 and 108.5 with the exponential of HotExp::Factor).  The plain double-precision fingerprint kernel stages 448:
   // 30512 bytes of LDS (60 slots, 40 channels, two species), five workgroups per CU, which is what its registers are held to.
-  // 512 are 31536 bytes, also five: no slower (2048 / 4096 / 16384 centres 38.2 / 64.9 / 222.5 us by 448 and 37.8 / 64.6 /
+  // 512 are 31536 bytes, also five: no slower (2048 / 4096 / 16384 centres 38.2 / 64.8 / 222.4 us by 448 and 37.8 / 64.5 /
   // 221.2 by 512), for a kilobyte of what a workgroup may use.  (With table rows of seventeen entries 512 were 32496 bytes,
   // 33280 in the pieces of 1280 that a CU hands out its 160 KB in, and four workgroups, not the five that the occupancy query
   // of the runtime reports: 6144-atom step 360.6 -> 356.8 us with 448.)
