@@ -121,6 +121,28 @@ def test_layers_refuse_a_map_of_the_triplets_that_the_ops_refuse(calls, what, er
     assert not calls
 
 
+@pytest.mark.parametrize("rows", [slice(0, NL), slice(2, N), slice(1, 1), slice(1, 2)])
+@pytest.mark.parametrize("frames", [1, 2])
+def test_a_map_of_the_triplets_is_taken_where_the_whole_test_takes_it(rows, frames):
+    """check_rows knows a map by its strides beside x3b's: the same verdict as of the test of every dimension, for slices of a
+    descriptor output, copies of them and maps of other widths."""
+    def verdict(f, *args):
+        try:
+            f(*args)
+        except (TypeError, ValueError) as e:
+            return type(e), str(e)
+
+    def whole(x3b, intmap3b):
+        v = ops._Views()
+        v(x3b), v(ops._i32(intmap3b))
+    out = {w: torch.zeros(frames, N, w, dtype=torch.int32 if w > NA else torch.float64)[:, rows] for w in (NA, 2 * NA, 2 * NA + 1)}
+    maps = [out[2 * NA], out[2 * NA].clone(), out[2 * NA + 1], out[2 * NA + 1][..., :2 * NA], out[2 * NA].flip(1), out[2 * NA].long()]
+    for x3b in (out[NA], out[NA].clone()):
+        for m in maps:
+            assert verdict(ops.check_rows, x3b, m) == verdict(whole, x3b, m)
+        assert verdict(ops.check_rows, x3b, maps[x3b.is_contiguous() and frames > 1]) is None
+
+
 @pytest.mark.parametrize("frozen", ["2", "3"])
 def test_a_body_whose_parameters_are_frozen_gets_no_gradient_kernels(calls, frozen):
     """The library is handed null for the gradients of a body that needs none, and makes no launches for it."""
