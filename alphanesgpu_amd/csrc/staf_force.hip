@@ -824,6 +824,8 @@ int step_forces(const StepSpecies<real>* sp, int n, const StepRows<real>& R, con
   using Wide = Force3Cfg<real, 8>;
   for (int c = 0; c < n; c++)
     if (sp[c].Nl > 0 && !step_forces_fits<real>(R.nr, nt, sp[c].Ar, sp[c].Aa)) return STAF_E_LIMIT;
+  bool pull = R.nr <= WAVE;
+  for (int c = 0; c < n; c++) pull = pull && Wide::bytes(R.nr, sp[c].Aa, nt, true, sp[c].Ar, true) <= 64 * 1024;
   Force3Species<real> M = {};
   size_t lds = 0, lds_wide = 0;
   int wg = 0;
@@ -839,9 +841,9 @@ int step_forces(const StepSpecies<real>* sp, int n, const StepRows<real>& R, con
     A.Nl = S.Nl; A.ld = A.ldo = R.nlocal; A.nr = R.nr; A.na = R.na; A.Aa = S.Aa; A.nt = nt;
     A.B2.G2 = S.g2; A.B2.D = R.raddescr + o * R.nr; A.B2.dD = R.der2b + o * 3 * R.nr; A.B2.alpha2b = S.alpha2b;
     A.B2.emb2b = S.emb2b; A.B2.Ar = S.Ar;
-    const size_t need = L::bytes(R.nr, S.Aa, nt, true, S.Ar);
+    const size_t need = L::bytes(R.nr, S.Aa, nt, true, S.Ar, pull);
     lds = need > lds ? need : lds;
-    lds_wide = std::max(lds_wide, Wide::bytes(R.nr, S.Aa, nt, true, S.Ar));
+    lds_wide = std::max(lds_wide, Wide::bytes(R.nr, S.Aa, nt, true, S.Ar, pull));
     M.first[M.entries++] = wg;
     wg += R.nf * S.Nl;
   }
@@ -852,15 +854,18 @@ int step_forces(const StepSpecies<real>* sp, int n, const StepRows<real>& R, con
   // little beyond it they still are no slower (864: 105.1 and 104.1, 960: 112.1 and 109.6, 1152: 126.1 and 123.1, 1215: 125.2 and
   // 123.8); in longer launches the registers and LDS of the wide ones cost residency.
   constexpr int FORCE3_WIDE_CENTRES = 768;   // three per CU
-  if (wg <= FORCE3_WIDE_CENTRES && lds_wide <= 64 * 1024) {
-    KernelTimer kt_("force3_kernel", stream);
-    hipLaunchKernelGGL((force3_species_kernel<real, true, 8, true>), dim3(wg), dim3(Wide::THREADS), lds_wide, stream, M);
-    return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
-  }
-  if (!lds_request(force3_species_kernel<real, true, 4, true>, lds)) return STAF_E_LIMIT;
   KernelTimer kt_("force3_kernel", stream);
-  hipLaunchKernelGGL((force3_species_kernel<real, true, 4, true>), dim3(wg), dim3(L::THREADS), lds, stream, M);
-  return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
+  auto launch = [&](auto pull_c) -> int {
+    constexpr bool PULL = decltype(pull_c)::value;
+    if (wg <= FORCE3_WIDE_CENTRES && lds_wide <= 64 * 1024) {
+      hipLaunchKernelGGL((force3_species_kernel<real, true, 8, true, PULL>), dim3(wg), dim3(Wide::THREADS), lds_wide, stream, M);
+    } else {
+      if (!lds_request((force3_species_kernel<real, true, 4, true, PULL>), lds)) return STAF_E_LIMIT;
+      hipLaunchKernelGGL((force3_species_kernel<real, true, 4, true, PULL>), dim3(wg), dim3(L::THREADS), lds, stream, M);
+    }
+    return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
+  };
+  return pull ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 template <typename real>

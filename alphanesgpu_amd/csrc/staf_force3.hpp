@@ -26,6 +26,12 @@
 //     accumulators row by row (inside a row the k are distinct).  One accumulator per wave and slot takes both;
 //     the waves' accumulators are added in a fixed order: results are bit-reproducible.
 //     F_s = sum_p Sd(s,p) dT/dd_s(s,p) + (sum_p SB_s(s,p)) grad fc_s
+// PULL (the fused form with up to 64 slots): the sums are taken in the lane of the slot.  With A = Sd fc_j fc_k a triplet's share
+// of the force on slot s is A (u_p - (u_s . u_p) u_s) / (2 r_s) + R_s grad fc_s, p the other slot: V_s = sum_p A u_p and sum_p R
+// are all that has to be summed, and (u_s . V_s) u_s comes off once.  The lanes of the triplets leave A, R_j and R_k in LDS, where
+// the exponential table was, in storage order, and lane s takes them for every p (dealt to the waves): reads of consecutive
+// words for p < s.  Seven operations per (slot, partner) in place of four prefix sums per pass and a loop over the rows of a pass:
+// 236 -> 215 M vector instructions for 24576 atoms (m = 37), 23 -> 15 % of the LDS cycles; launch 535 -> 486 us.
 // The slot forces go to scratch or to the caller's arrays (gslot, and the centre's own force to self); the atoms
 // that receive them collect them in gather_kernel (per op) or force_total_kernel (all species at once) through the
 // neighbour map.
@@ -72,19 +78,26 @@ struct Force3Cfg {
   // (a multiple of 128 bytes for the usual channel counts) those entries would share their banks; one entry more
   // puts consecutive rows one entry apart.
   __host__ __device__ static int rowp(int Aa) { return pitch(Aa) + 1; }
+  static constexpr int SWEEP = NW * NP * WAVE;              // triplets of a sweep
+  static constexpr int TRI = SWEEP + 2;                     // entries of a column of the sweep's triplets, one of them 0
+  __host__ __device__ static size_t table_reals(int nr, int nt, bool pull) {
+    const size_t e = ((size_t)ROWP * nt * nr + 1) & ~(size_t)1;
+    const size_t t = (size_t)3 * TRI, sums = (size_t)NW * 4 * WAVE;
+    return !pull ? e : (e > t ? (e > sums ? e : sums) : (t > sums ? t : sums));
+  }
   // Ar2 > 0: the 2-body pair forces are added (Ar2 radial channels)
-  __host__ __device__ static size_t n_reals(int nr, int Aa, int nt, bool fused = false, int Ar2 = 0) {
+  __host__ __device__ static size_t n_reals(int nr, int Aa, int nt, bool fused = false, int Ar2 = 0, bool pull = false) {
     const int nsig = 2 * nt - 1;
     return (size_t)nsig * rowp(Aa) * 4 /*prm*/ + (size_t)nsig * pitch(Aa) * 2 /*prE*/ +
-           (((size_t)ROWP * nt * nr + 1) & ~(size_t)1) /*E*/ +
-           (size_t)NW * 4 * nr /*slot sums per wave*/ + nr /*D*/ + 3 * nr /*grad fc*/ +
+           table_reals(nr, nt, pull) /*E, then the triplets*/ +
+           (pull ? 0 : (size_t)NW * 4 * nr) /*slot sums per wave*/ + nr /*D*/ + 3 * nr /*grad fc*/ +
            (size_t)NW * 4 /*the waves' shares of the centre's own force*/ + (fused ? 4 * nr : 0) /*unit vectors, 1/r*/ +
            (Ar2 > 0 ? (size_t)NW * nr + nr + (size_t)2 * nt * Ar2 : 0) /*2-body: the waves' shares of the pair
            weights, D, parameter rows*/ +
            (fused && Ar2 > 0 ? NW * 9 : 0) /*the waves' shares of the centre's virial*/;
   }
-  __host__ __device__ static size_t bytes(int nr, int Aa, int nt, bool fused = false, int Ar2 = 0) {
-    return n_reals(nr, Aa, nt, fused, Ar2) * sizeof(real) + (size_t)(16 + (Ar2 > 0 ? NT_MAX : 0) + nr) * sizeof(int);
+  __host__ __device__ static size_t bytes(int nr, int Aa, int nt, bool fused = false, int Ar2 = 0, bool pull = false) {
+    return n_reals(nr, Aa, nt, fused, Ar2, pull) * sizeof(real) + (size_t)(16 + (Ar2 > 0 ? NT_MAX : 0) + nr) * sizeof(int);
   }
 };
 
@@ -118,7 +131,7 @@ struct Force3Args {   // one centre species
   Force2In<real> B2;      // W2B
 };
 
-template <typename real, bool FUSED, int NWAVES, bool W2B>
+template <typename real, bool FUSED, int NWAVES, bool W2B, bool PULL>
 __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int atom) {
   const real* __restrict__ G = A.G;
   const real* __restrict__ Dsup = A.Dsup;
@@ -135,6 +148,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
   real* __restrict__ self = A.self;
   const int Nl = A.Nl, ld = A.ld, nr = A.nr, na = A.na, Aa = A.Aa, nt = A.nt;
   const Force2In<real>& B2 = A.B2;
+  static_assert(!PULL || FUSED, "a triplet's Jacobian as sums over slots only where the kernel forms it");
   constexpr bool VIR = FUSED && W2B;   // the form that can leave the centres' virials
   using real2 = typename Vec2<real>::type;
   using real4 = typename Vec4<real>::type;
@@ -148,8 +162,9 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
   real* prm = (real*)smem;                                 // [nsig][Apr][4] = a1+a2, a1-a2, scaled beta, 1/4 G c3 (active channels)
   real* prE = prm + (size_t)nsig * Apr * 4;                // [nsig*Ap][2] = a1, a2 in the units of the hot exponential
   real* E = prE + (size_t)nsig * Ap * 2;                   // [RT][ROWP], see Force3Cfg::ROWP
-  real* acc = E + (((size_t)RT * ROWP + 1) & ~(size_t)1);  // [NW][4 nr]: per wave, slot sums (as j and as k), see accW
-  real* sD = acc + (size_t)NW * 4 * nr;                    // [nr]
+  real* triA = E;                                          // PULL: [3][TRI] of the sweep's triplets, where the table was
+  real* acc = E + L::table_reals(nr, nt, PULL);            // [NW][4 nr]: per wave, slot sums (as j and as k), see accW
+  real* sD = acc + (PULL ? (size_t)0 : (size_t)NW * 4 * nr);   // [nr]
   real* sg = sD + nr;                                      // [3*nr] grad fc (der3bsupp)
   real* xch = sg + 3 * nr;                                 // [NW][4] the waves' shares of the centre's own force
   real* sU = xch + NW * 4;                                 // FUSED: [4][nr] unit vector, 1/r
@@ -237,7 +252,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
   int t_s = 0;
   if (slot_t) t_s = type_map[nj];
   if (tid >= nsig && tid < 16) nact[tid] = 0;
-  {
+  if constexpr (!PULL) {
     real4 z;
     z.x = z.y = z.z = z.w = 0;
     for (int q = tid; q < NW * nr; q += THREADS) ((real4*)acc)[q] = z;
@@ -358,6 +373,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
     }
   }
 
+  real pull[4] = {0, 0, 0, 0};   // PULL: this wave's share of the sums of slot `lane`: A u of the partners (x, y, z), radial
   for (int w0 = 0; w0 < ntri; w0 += NW * NP * WAVE) {
     // ---- this wave's triplets of the sweep: T, table rows of slot j and slot k, parameter row of sigma, packed j|k
     real T[NP], Sd[NP], U[NP], V[NP];
@@ -487,6 +503,41 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
       }
     }
 
+    if constexpr (PULL) {
+      // ---- slot sums
+      __syncthreads();   // readers of the table are done
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        if (p >= npass) break;
+        const int q = (p * NW + wave) * WAVE + lane;
+        const int j = jk[p] & 0xff, k = jk[p] >> 8;
+        const real cs = sU[j] * sU[k] + sU[nr + j] * sU[nr + k] + sU[2 * nr + j] * sU[2 * nr + k];
+        const real fj = sD[j], fk = sD[k], hT = real(0.5) * T[p];
+        const real sh = Sd[p] * (real(0.5) * (cs + real(1)));
+        if (w0 + q < ntri) {
+          triA[q] = Sd[p] * (fj * fk);
+          triA[L::TRI + q] = r_fma(sh, fk, (U[p] + V[p]) * hT);
+          triA[2 * L::TRI + q] = r_fma(sh, fj, (U[p] - V[p]) * hT);
+        }
+      }
+      if (tid < 3) triA[tid * L::TRI + L::SWEEP] = 0;
+      __syncthreads();
+      if (lane < m) {
+        const int left = ntri - w0, n = left < L::SWEEP ? left : L::SWEEP;
+        const int mine = tri_rowstart(lane, m) - lane - 1 - w0;
+        for (int p = wave; p < m; p += NW) {
+          const int theirs = tri_rowstart(p, m) - p - 1 - w0;
+          const bool low = lane < p;              // the pair's j is this slot
+          int q = low ? mine + p : theirs + lane;
+          q = (unsigned)q < (unsigned)n && lane != p ? q : L::SWEEP;
+          const real a = triA[q], rad = triA[(low ? L::TRI : 2 * L::TRI) + q];
+#pragma unroll
+          for (int c = 0; c < 3; c++) pull[c] = r_fma(a, sU[c * nr + p], pull[c]);
+          pull[3] += rad;
+        }
+      }
+      continue;
+    }
     // ---- contraction with der3b, slot sums of this wave.  Lanes past the last triplet hold T = 0 and finite sums
     // computed on row 0: their products are forced to 0.
     if constexpr (FUSED) {
@@ -610,6 +661,11 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
     }
   }
   __syncthreads();
+  if constexpr (PULL) {   // (the triplets of the last sweep are read)
+#pragma unroll
+    for (int c = 0; c < 4; c++) triA[(wave * 4 + c) * WAVE + lane] = pull[c];
+    __syncthreads();
+  }
 
   // ---- slot forces (waves added in a fixed order; one slot per thread: m <= nr < THREADS), centre's own force.
   // Only the waves that hold slots (the first one for up to 64 slots) form sums; the others' share is zero.
@@ -617,10 +673,22 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
   if (wave * WAVE < nr) {
     if (slot) {
       real t4[4] = {0, 0, 0, 0};
+      if constexpr (PULL) {
+#pragma unroll
+        for (int w = 0; w < NW; w++)
+#pragma unroll
+          for (int c = 0; c < 4; c++) t4[c] += triA[(w * 4 + c) * WAVE + lane];
+        // sum of A (u_p - (u_s . u_p) u_s)
+        const real u[3] = {sU[tid], sU[nr + tid], sU[2 * nr + tid]};
+        const real along = u[0] * t4[0] + u[1] * t4[1] + u[2] * t4[2];
+#pragma unroll
+        for (int c = 0; c < 3; c++) t4[c] = r_fma(-along, u[c], t4[c]);
+      } else {
 #pragma unroll
       for (int w = 0; w < NW; w++) {
         const real4 a = acc_get(acc + (size_t)w * 4 * nr, tid);
         t4[0] += a.x; t4[1] += a.y; t4[2] += a.z; t4[3] += a.w;
+      }
       }
 #pragma unroll
       for (int c = 0; c < 3; c++) {
@@ -688,10 +756,10 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
   }
 }
 
-template <typename real, bool FUSED = false, int NWAVES = 4, bool W2B = false>
+template <typename real, bool FUSED = false, int NWAVES = 4, bool W2B = false, bool PULL = false>
 __global__ __launch_bounds__((Force3Cfg<real, NWAVES>::THREADS), (Force3Cfg<real, NWAVES>::MIN_WAVES)) void force3_kernel(
     const Force3Args<real> A) {
-  force3_body<real, FUSED, NWAVES, W2B>(A, (int)blockIdx.x);
+  force3_body<real, FUSED, NWAVES, W2B, PULL>(A, (int)blockIdx.x);
 }
 
 // The centres of several species in one launch: entry e takes workgroups first[e] .. first[e + 1].
@@ -701,12 +769,12 @@ struct Force3Species {
   int first[NT_MAX + 1];
   Force3Args<real> e[NT_MAX];
 };
-template <typename real, bool FUSED, int NWAVES, bool W2B>
+template <typename real, bool FUSED, int NWAVES, bool W2B, bool PULL>
 __global__ __launch_bounds__((Force3Cfg<real, NWAVES>::THREADS), (Force3Cfg<real, NWAVES>::MIN_WAVES)) void force3_species_kernel(
     const Force3Species<real> M) {
   int e = 0;
   while (e + 1 < M.entries && (int)blockIdx.x >= M.first[e + 1]) e++;
-  force3_body<real, FUSED, NWAVES, W2B>(M.e[e], (int)blockIdx.x - M.first[e]);
+  force3_body<real, FUSED, NWAVES, W2B, PULL>(M.e[e], (int)blockIdx.x - M.first[e]);
 }
 
 }  // namespace staf
