@@ -68,9 +68,10 @@ struct Force3Cfg {
   // start to have the lines in the L2)
   static constexpr bool PREFETCH = false;
   // waves per SIMD the register allocation is held to: with four waves per workgroup what the LDS footprint of the
-  // reference's sizes admits (six workgroups per CU in single precision, four in double); with eight waves two
-  // workgroups per CU, launches of few centres hold no more
-  static constexpr int MIN_WAVES = NW == 8 ? 4 : (sizeof(real) == 8 ? 4 : 6);
+  // reference's sizes admits (six workgroups per CU in single precision, four in double); with eight waves three
+  // workgroups per CU, so that the launches that take them (FORCE3_WIDE_CENTRES) have all their centres resident: 768 atoms
+  // in double precision 33.8 us at 87 registers and two workgroups, 28.0 at 80
+  static constexpr int MIN_WAVES = NW == 8 ? 6 : (sizeof(real) == 8 ? 4 : 6);
   __host__ __device__ static bool fits(int nr, int nt) { return nr <= 255 && nt <= NT_MAX; }   // slots packed in 8 bits
   __host__ __device__ static int pitch(int Aa) { return (Aa + 3) & ~3; }   // parameter row pitch (channels)
   // Distance, in channels, between the weight rows of consecutive sigma.  The lanes of a wave read the 16- or 32-byte
