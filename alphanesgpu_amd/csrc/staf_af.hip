@@ -11,6 +11,7 @@
 #include "staf_tile.hpp"
 #include "staf_reduce.hpp"
 #include "staf_tri.hpp"
+#include "staf_step.hpp"
 #include "staf_af2.hpp"
 
 #include <stdio.h>
@@ -343,6 +344,7 @@ struct StepFingerprintArgs {
   int entries, nr, nt;
   int first2[NT_MAX + 1], first3[NT_MAX + 1];   // first2 ends where first3 starts
   TriArgs<real> tri[NT_MAX];
+  const real* table[NT_MAX];
   struct {
     const real *D, *alpha2b, *emb2b;
     real* out;
@@ -350,8 +352,8 @@ struct StepFingerprintArgs {
   } rad[NT_MAX];
 };
 
-template <typename real, int BLOCK>
-__global__ __launch_bounds__(BLOCK, (TriCfg<real, 0, true, BLOCK>::MIN_WAVES)) void step_fingerprints_kernel(
+template <typename real, int BLOCK, bool ROWS>
+__global__ __launch_bounds__(BLOCK, (ROWS ? RowsCfg<real, BLOCK / WAVE>::MIN_WAVES : TriCfg<real, 0, true, BLOCK>::MIN_WAVES)) void step_fingerprints_kernel(
     const StepFingerprintArgs<real> M) {
   constexpr int WAVES = BLOCK / WAVE;
   const int wg = (int)blockIdx.x;
@@ -380,10 +382,11 @@ __global__ __launch_bounds__(BLOCK, (TriCfg<real, 0, true, BLOCK>::MIN_WAVES)) v
     return;
   }
   while (e + 1 < M.entries && wg >= M.first3[e + 1]) e++;
-  tri_reduce_body<real, 0, true, BLOCK>(M.tri[e], wg - M.first3[e], M.first3[e + 1] - M.first3[e], 0);
+  if constexpr (ROWS) rows_body<real, BLOCK / WAVE>(M.tri[e], M.table[e], wg - M.first3[e], M.first3[e + 1] - M.first3[e]);
+  else tri_reduce_body<real, 0, true, BLOCK>(M.tri[e], wg - M.first3[e], M.first3[e + 1] - M.first3[e], 0);
 }
 
-template <typename real, int BLOCK>
+template <typename real, int BLOCK, bool ROWS>
 static int step_fingerprints_launch(const StepSpecies<real>* sp, int n, const StepRows<real>& R, const int* type_map, int nt,
                                     hipStream_t stream) {
   constexpr int WAVES = BLOCK / WAVE;
@@ -401,7 +404,8 @@ static int step_fingerprints_launch(const StepSpecies<real>* sp, int n, const St
     T.nf = R.nf; T.Nl = S.Nl; T.ld = R.nlocal; T.nr = R.nr; T.na = R.na; T.Aa = S.Aa; T.nt = nt;
     auto& Q = M.rad[M.entries];
     Q.D = R.raddescr + o * R.nr; Q.alpha2b = S.alpha2b; Q.emb2b = S.emb2b; Q.out = S.af2; Q.Ar = S.Ar;
-    const size_t need3 = TriLds<real, 0, true, BLOCK>::bytes(R.nr, S.Aa, nt, true);
+    M.table[M.entries] = S.table;
+    const size_t need3 = ROWS ? RowsCfg<real, WAVES>::bytes(R.nr, S.Aa, nt) : TriLds<real, 0, true, BLOCK>::bytes(R.nr, S.Aa, nt, true);
     const size_t need2 = (size_t)2 * nt * S.Ar * sizeof(real) + (size_t)WAVES * R.nr * (sizeof(real) + sizeof(int));
     lds = std::max(lds, std::max(need2, need3));
     M.first2[M.entries++] = wg;
@@ -411,9 +415,10 @@ static int step_fingerprints_launch(const StepSpecies<real>* sp, int n, const St
   if (total == 0) return STAF_OK;
   M.first2[M.entries] = wg;
   M.nr = R.nr; M.nt = nt;
-  if (!lds_request((step_fingerprints_kernel<real, BLOCK>), lds)) return STAF_E_LIMIT;
+  constexpr auto kernel = step_fingerprints_kernel<real, BLOCK, ROWS>;
+  if (!lds_request(kernel, lds)) return STAF_E_LIMIT;
   // the 3-body workgroups a launch of all centres would have, dealt to the species by their centres
-  const int grid = BLOCK == TRI_BLOCK ? tri_grid((const void*)step_fingerprints_kernel<real, BLOCK>, lds, total) : total;
+  const int grid = BLOCK == TRI_BLOCK ? tri_grid((const void*)kernel, lds, total) : total;
   for (int e = 0; e < M.entries; e++) {
     const int centres = R.nf * M.tri[e].Nl;
     const int share = (int)(((long long)grid * centres + total / 2) / total);
@@ -422,7 +427,7 @@ static int step_fingerprints_launch(const StepSpecies<real>* sp, int n, const St
   }
   M.first3[M.entries] = wg;
   KernelTimer kt_("af3_kernel", stream);
-  hipLaunchKernelGGL((step_fingerprints_kernel<real, BLOCK>), dim3(wg), dim3(BLOCK), lds, stream, M);
+  hipLaunchKernelGGL(kernel, dim3(wg), dim3(BLOCK), lds, stream, M);
   return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
 }
 // Few centres: a launch lasts as long as one centre takes, which workgroups of 512 threads shorten (32 triplets at a time
@@ -430,19 +435,28 @@ static int step_fingerprints_launch(const StepSpecies<real>* sp, int n, const St
 // 94.0 -> 88.7.  A CU holds two such workgroups; beyond that 256 threads are as fast (588 atoms: 98.5 and 98.6 us) or faster
 // (768: 99.7 and 101.0, 1080: 119.3 and 123.1, 1215: 125.2 and 130.5).
 constexpr int WIDE_FINGERPRINT_CENTRES = 512;   // two per CU
+// The same of rows_body, whose launches of 4 and of 8 waves per centre take 13.5 and 10.7 us for 96 centres, 13.9 and 10.8 for
+// 225, 15.6 and 13.4 for 378, 16.1 and 16.8 for 504, 17.1 and 19.0 for 576, 18.5 and 21.6 for 768.
+constexpr int WIDE_ROWS_CENTRES = 448;
 template <typename real>
 int step_fingerprints(const StepSpecies<real>* sp, int n, const StepRows<real>& R, const int* type_map, int nt,
                       hipStream_t stream) {
   int total = 0;
-  size_t lds = 0;
+  size_t lds = 0, rows_lds = 0;
+  bool rows = step_slots(R.nr, R.na, nt);
   for (int c = 0; c < n; c++) {
     total += R.nf * sp[c].Nl;
+    rows = rows && (sp[c].table || sp[c].Nl == 0);
+    rows_lds = std::max(rows_lds, RowsCfg<real, 8>::bytes(R.nr, sp[c].Aa, nt) +
+                                      (size_t)2 * nt * sp[c].Ar * sizeof(real) + (size_t)8 * R.nr * (sizeof(real) + sizeof(int)));
     lds = std::max(lds, TriLds<real, 0, true, 512>::bytes(R.nr, sp[c].Aa, nt, true) +
                             (size_t)2 * nt * sp[c].Ar * sizeof(real) + (size_t)8 * R.nr * (sizeof(real) + sizeof(int)));
   }
-  if (total <= WIDE_FINGERPRINT_CENTRES && lds <= 64 * 1024)
-    return step_fingerprints_launch<real, 512>(sp, n, R, type_map, nt, stream);
-  return step_fingerprints_launch<real, TRI_BLOCK>(sp, n, R, type_map, nt, stream);
+  if (rows && rows_lds <= 64 * 1024)
+    return total <= WIDE_ROWS_CENTRES ? step_fingerprints_launch<real, 512, true>(sp, n, R, type_map, nt, stream)
+                                      : step_fingerprints_launch<real, TRI_BLOCK, true>(sp, n, R, type_map, nt, stream);
+  if (total <= WIDE_FINGERPRINT_CENTRES && lds <= 64 * 1024) return step_fingerprints_launch<real, 512, false>(sp, n, R, type_map, nt, stream);
+  return step_fingerprints_launch<real, TRI_BLOCK, false>(sp, n, R, type_map, nt, stream);
 }
 template int step_fingerprints<float>(const StepSpecies<float>*, int, const StepRows<float>&, const int*, int, hipStream_t);
 template int step_fingerprints<double>(const StepSpecies<double>*, int, const StepRows<double>&, const int*, int,

@@ -13,6 +13,7 @@
 #include "staf_common.hpp"
 #include "staf_reduce.hpp"
 #include "staf_mlp_dev.hpp"
+#include "staf_step.hpp"
 #include "../../include/staf.h"
 #include "../../include/staf_mlp.h"
 
@@ -180,7 +181,7 @@ struct StafModel {
   int nt = 0, ntc = 0, nr = 60, na = 1770;
   double Rc = 4.5, Ra = 4.5, Rs = 2.25;
   std::vector<int> Ar, Aa;
-  std::vector<DevBuf<double>> alpha2b, alpha3b, emb2b, emb3b;
+  std::vector<DevBuf<double>> alpha2b, alpha3b, emb2b, emb3b, table;
   staf::DescConfig<double> cfg;
   hipStream_t stream = nullptr;            // the call's stream
   // device buffers
@@ -224,6 +225,7 @@ static bool load_species_params(StafModel* m) {
   m->alpha3b.resize(nt);
   m->emb2b.resize(nt);
   m->emb3b.resize(nt);
+  m->table.resize(nt);
   for (int k = 0; k < nt; k++) {
     const std::string pre = m->dir + "/type" + std::to_string(k) + "_";
     std::vector<double> a2, a3, e2, e3;
@@ -247,6 +249,12 @@ static bool load_species_params(StafModel* m) {
     for (auto& u : up) {
       if (!u.d->reserve(u.h->size())) return false;
       if (!upload_sync(u.d->p, u.h->data(), u.h->size() * sizeof(double), m->stream)) return false;
+    }
+    if (const size_t n = staf::step_table_reals<double>(nt, m->Aa[k])) {
+      if (!m->table[k].reserve(n)) return false;
+      std::vector<double> t(n, 0.0);
+      staf::step_table_host(t.data(), a3.data(), e3.data(), nt, m->Aa[k]);
+      if (!upload_sync(m->table[k].p, t.data(), n * sizeof(double), m->stream)) return false;
     }
   }
   return true;
@@ -300,7 +308,7 @@ void staf_free(StafModel* m) {
   if (m->stream) (void)hipStreamDestroy(m->stream);
   if (m->mlp) staf_mlp_destroy(m->mlp);
   for (auto& n : m->dnets) staf::dev_mlp_free(&n);
-  for (auto* v : {&m->alpha2b, &m->alpha3b, &m->emb2b, &m->emb3b})
+  for (auto* v : {&m->alpha2b, &m->alpha3b, &m->emb2b, &m->emb3b, &m->table})
     for (auto& b : *v) b.release();
   m->in_h.release();
   m->out_h.release();
@@ -616,7 +624,7 @@ int staf_compute(StafModel* m, int nlocal, int nghost, const double* x, const do
       if (tipos[k] == 0) continue;
       const size_t o = (size_t)at;
       sp.push_back({at, tipos[k], m->Ar[k], m->Aa[k], m->alpha2b[k].p, m->alpha3b[k].p, m->emb2b[k].p, m->emb3b[k].p,
-                    m->af2.p + o * amax2, m->af3.p + o * amax3, m->g2.p + o * amax2, m->g3.p + o * amax3});
+                    m->af2.p + o * amax2, m->af3.p + o * amax3, m->g2.p + o * amax2, m->g3.p + o * amax3, m->table[k].p});
     }
     const int ns = (int)sp.size();
     std::vector<staf::DevMlpCall<double>> nets;

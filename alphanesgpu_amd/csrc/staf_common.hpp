@@ -522,6 +522,7 @@ struct StepSpecies {
   int first, Nl, Ar, Aa;      // first owned atom and owned atoms in a frame, fingerprints
   const real *alpha2b, *alpha3b, *emb2b, *emb3b;
   real *af2, *af3, *g2, *g3;  // [nf, Nl, Ar], [nf, Nl, Aa]: fingerprints and dE/d fingerprint
+  const real* table;          // its parameters laid out (StepTablePart), or null
 };
 template <typename real>
 struct StepRows {             // what the radial-only descriptor launch leaves, nr-wide rows of all owned atoms
@@ -529,6 +530,15 @@ struct StepRows {             // what the radial-only descriptor launch leaves, 
   const int *intmap2b, *numtriplet;
   int nr, na, nf, nlocal;     // nlocal rows per frame
   TransposeRef tr;            // what desc_launch was given
+};
+// The parameters of a species laid out for the kernels below (staf_step.hpp; step_table_reals has the size), written by the
+// launch that lays out the networks (dev_mlp_pack).
+constexpr int STEP_CHANNELS = 1024;
+template <typename real>
+struct StepTablePart {
+  const real *alpha3b, *emb3b;
+  real* table;
+  int Aa, raw_emb;   // emb3b is to be squared
 };
 // 2-body and 3-body fingerprints
 template <typename real>

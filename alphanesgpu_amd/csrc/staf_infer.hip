@@ -9,6 +9,7 @@
 // the caller's allocator's to reuse in the order of the stream.
 #include "staf_common.hpp"
 #include "staf_mlp_dev.hpp"
+#include "staf_step.hpp"
 
 #include <vector>
 
@@ -18,7 +19,7 @@ template <typename real>
 struct FramesPlan {
   size_t bytes = 0;
   size_t raddescr, des3bsupp, der2b, der3bsupp, unit, slots, self, vpart, e_atom, intmap2b, numtriplet;
-  size_t af2[NT_MAX], af3[NT_MAX], g2[NT_MAX], g3[NT_MAX], net[NT_MAX], emb2b[NT_MAX], emb3b[NT_MAX];
+  size_t af2[NT_MAX], af3[NT_MAX], g2[NT_MAX], g3[NT_MAX], net[NT_MAX], emb2b[NT_MAX], emb3b[NT_MAX], table[NT_MAX];
 };
 
 static DevMlpSource net_source(const StafFramesSpecies& s) {
@@ -82,6 +83,7 @@ static int frames_plan(const DescConfig<real>& c, int nf, int N, int nt, const S
     P->emb2b[k] = place((size_t)nt * s.nalpha_r * sizeof(real));
     P->emb3b[k] = place((size_t)nt * (nt + 1) / 2 * s.nsmooth_a * sizeof(real));
     P->net[k] = place(block * sizeof(real));
+    P->table[k] = place(step_table_reals<real>(nt, s.nsmooth_a) * sizeof(real));
   }
   return sum == N ? STAF_OK : STAF_E_BAD_ARG;
 }
@@ -111,7 +113,8 @@ static int frames(const real* pos, const real* box, int nf, int N, int nt, const
   DevMlpNet nets[NT_MAX];
   DevMlpCall<real> calls[NT_MAX];
   std::vector<PackPart> parts;
-  int n = 0, first = 0;
+  StepTablePart<real> tables[NT_MAX];
+  int n = 0, first = 0, n_tables = 0;
   for (int k = 0; k < nt; first += sp[k].n_local, k++) {
     const StafFramesSpecies& s = sp[k];
     if (s.n_local == 0) continue;
@@ -125,7 +128,11 @@ static int frames(const real* pos, const real* box, int nf, int N, int nt, const
     const int m = dev_mlp_plan<real>(net_source(s), at(P.net[k]), &nets[n], mine + 2);
     parts.insert(parts.end(), mine, mine + 2 + m);
     S[n] = {first, s.n_local, s.nalpha_r, s.nsmooth_a, (const real*)s.alpha2b, (const real*)s.alpha3b, at(P.emb2b[k]),
-            at(P.emb3b[k]), at(P.af2[k]), at(P.af3[k]), at(P.g2[k]), at(P.g3[k])};
+            at(P.emb3b[k]), at(P.af2[k]), at(P.af3[k]), at(P.g2[k]), at(P.g3[k]), nullptr};
+    if (step_table_reals<real>(nt, s.nsmooth_a)) {
+      S[n].table = at(P.table[k]);
+      tables[n_tables++] = {S[n].alpha3b, (const real*)s.type_emb3b, at(P.table[k]), s.nsmooth_a, 1};
+    }
     calls[n] = {&nets[n], S[n].af2, S[n].af3, at(P.e_atom) + (size_t)nf * first, S[n].g2, S[n].g3, S[n].Ar, S[n].Aa,
                 nf * s.n_local};
     n++;
@@ -136,7 +143,7 @@ static int frames(const real* pos, const real* box, int nf, int N, int nt, const
                             (int*)(w + P.intmap2b), (int*)(w + P.numtriplet), c.nr, c.na, nf, N, own_map(w + P.intmap2b)};
   {
     DeferStatus defer;   // conditions the kernels detect are read once, behind the last launch
-    if ((rc = dev_mlp_pack<real>(parts.data(), (int)parts.size(), stream)) != STAF_OK) return rc;
+    if ((rc = dev_mlp_pack<real>(parts.data(), (int)parts.size(), tables, n_tables, nt, stream)) != STAF_OK) return rc;
     rc = desc_launch<real>(c, pos, box, nf, N, N, nullptr, &R.tr, 0, at(P.raddescr), nullptr, at(P.des3bsupp),
                            (int*)(w + P.intmap2b), nullptr, at(P.der2b), nullptr, at(P.der3bsupp),
                            (int*)(w + P.numtriplet), at(P.unit), stream);

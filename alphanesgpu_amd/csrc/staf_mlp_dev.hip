@@ -19,6 +19,7 @@
 // either).  Asking for
 // the weights' lines ahead of everything, and more than six pieces in flight, are slower.
 #include "staf_mlp_dev.hpp"
+#include "staf_step.hpp"
 
 #include <algorithm>
 #include <vector>
@@ -578,9 +579,13 @@ template int dev_mlp_plan<float>(const DevMlpSource&, float*, DevMlpNet*, PackPa
 template int dev_mlp_plan<double>(const DevMlpSource&, double*, DevMlpNet*, PackPart*);
 
 constexpr int PACK_BLOCK = 256;
+static_assert(PACK_BLOCK == STEP_TABLE_BLOCK, "one launch");
+template <typename T>
 struct PackArgs {
-  int n, first[PACK_PARTS + 1];   // workgroups of a part
+  int n, first[PACK_PARTS + 1];   // workgroups of a part; behind the last one's those of the tables
   PackPart part[PACK_PARTS];
+  int nt;
+  StepTablePart<T> table[NT_MAX];
 };
 template <typename T>
 __host__ __device__ inline size_t pack_elements(const PackPart& p) {
@@ -589,7 +594,12 @@ __host__ __device__ inline size_t pack_elements(const PackPart& p) {
 // A thread per element of the destination: the order of upload_net's tiles.  Bound by its launch: the two networks of a
 // 60-140-140-1 stack in double precision are 0.9 MB.
 template <typename T>
-__global__ __launch_bounds__(PACK_BLOCK) void mlp_pack_kernel(const PackArgs A) {
+__global__ __launch_bounds__(PACK_BLOCK) void mlp_pack_kernel(const PackArgs<T> A) {
+  if ((int)blockIdx.x >= A.first[A.n]) {
+    const int w = (int)blockIdx.x - A.first[A.n], q = w / STEP_TABLE_PARTS, nsig = 2 * A.nt - 1;
+    step_table_body<T>(A.table[q / nsig], A.nt, q % nsig, w % STEP_TABLE_PARTS, STEP_TABLE_PARTS);
+    return;
+  }
   int e = 0;
   while (e + 1 < A.n && (int)blockIdx.x >= A.first[e + 1]) e++;
   const PackPart& p = A.part[e];
@@ -613,9 +623,9 @@ __global__ __launch_bounds__(PACK_BLOCK) void mlp_pack_kernel(const PackArgs A) 
 }
 
 template <typename T>
-int dev_mlp_pack(const PackPart* parts, int n, hipStream_t stream) {
+int dev_mlp_pack(const PackPart* parts, int n, const StepTablePart<T>* tables, int n_tables, int nt, hipStream_t stream) {
   for (int at = 0; at < n; at += PACK_PARTS) {
-    PackArgs A = {};
+    PackArgs<T> A = {};
     size_t blocks = 0;
     for (A.n = 0; A.n < PACK_PARTS && at + A.n < n; A.n++) {
       A.part[A.n] = parts[at + A.n];
@@ -623,14 +633,19 @@ int dev_mlp_pack(const PackPart* parts, int n, hipStream_t stream) {
       blocks += (pack_elements<T>(A.part[A.n]) + PACK_BLOCK - 1) / PACK_BLOCK;
     }
     A.first[A.n] = (int)blocks;
+    A.nt = nt;
+    if (at == 0) {
+      for (int k = 0; k < n_tables; k++) A.table[k] = tables[k];
+      blocks += (size_t)n_tables * (2 * nt - 1) * STEP_TABLE_PARTS;
+    }
     if (blocks > 0x7fffffff) return STAF_E_LIMIT;
     KernelTimer kt_("mlp_pack_kernel", stream);
     if (blocks) hipLaunchKernelGGL(mlp_pack_kernel<T>, dim3((unsigned)blocks), dim3(PACK_BLOCK), 0, stream, A);
   }
   return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
 }
-template int dev_mlp_pack<float>(const PackPart*, int, hipStream_t);
-template int dev_mlp_pack<double>(const PackPart*, int, hipStream_t);
+template int dev_mlp_pack<float>(const PackPart*, int, const StepTablePart<float>*, int, int, hipStream_t);
+template int dev_mlp_pack<double>(const PackPart*, int, const StepTablePart<double>*, int, int, hipStream_t);
 
 template <typename T, typename real, int TA>
 static int eval_nets_by(const DevMlpCall<real>* calls, int n, int rows, int tiles, hipStream_t stream) {

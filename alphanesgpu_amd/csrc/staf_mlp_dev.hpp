@@ -57,7 +57,8 @@ constexpr int PACK_PARTS = 64;
 // Describes the network laid out in `block` and appends the parts that fill it (at most 3 per layer and one).
 template <typename T>
 int dev_mlp_plan(const DevMlpSource& src, T* block, DevMlpNet* net, PackPart* parts);
+// The same launch writes the tables of n_tables species (staf_step.hpp).
 template <typename T>
-int dev_mlp_pack(const PackPart* parts, int n, hipStream_t stream);
+int dev_mlp_pack(const PackPart* parts, int n, const StepTablePart<T>* tables, int n_tables, int nt, hipStream_t stream);
 
 }  // namespace staf

@@ -1,0 +1,507 @@
+// 3-body fingerprints of the paths that hold no tensor of the angular buffer's width (the MD entry, the batch inference), from
+// the nr-wide rows of the radial-only descriptor launch, for up to 64 neighbours and angular buffers that hold all their
+// pairs (step_slots); other buffers go through tri_reduce_body.
+//
+// tri_reduce_body, which also rebuilds T where no angular tensor exists, stages the triplets of a class in LDS and reads a
+// record and two table rows per (triplet, channel): its inner loop is as long as its LDS reads take, whatever it computes (the
+// exponential from the table below took 8 of its 21 instructions away and no time), and without the loop the launch still
+// takes 240 of 370 us: staging, seven to twelve barriers per centre, tables.  rows_body walks over the rows of the triplet
+// triangle instead, four rows x of a class at a time against sixteen columns y:
+//   * lane (r, l) forms T(x_r, y_l) once, and the sixteen lanes of row r, now a channel each, take it from its lane by a
+//     broadcast within the row (DPP): triplets never go through LDS;
+//   * e^(a1 D_x), e^(a2 D_x) of the lane's row are in registers, sum_y T e^(bT) e^(a2 D_y) and sum_y T e^(bT) e^(a1 D_y) are what
+//     is summed (two multiply-adds per item instead of four operations), and the row's factors are applied once per row;
+//   * one table entry per item is read from LDS, the same address for the four rows;
+//   * all classes' tables are built at once, the rows of all classes are dealt to the waves: three barriers per centre.
+// Launches of 24576, 4 x 768 (inference), 768 and 96 centres: 366 -> 329, 56.6 -> 51.6, 24.9 -> 18.5 and 12.5 -> 10.7 us in double
+// precision (157 -> 135 M vector instructions, 28 -> 12 M LDS instructions for 24576), 4 x 768 in single 31.8 -> 25.3; a vector
+// instruction in 0.71 of the issue slots, the rest is latency at four waves per SIMD (125 registers; five would need 96, and
+// less than the 36 KB of LDS that 60 slots take).
+#pragma once
+#include "staf_tri.hpp"
+
+namespace staf {
+
+// What the kernel needs of a species' parameters, laid out once for a loaded model, once a call where the
+// parameters are a caller's tensors: the channels of every sigma whose embedding is not 0, in ascending order, then
+// zeros up to the pitch.
+//   [STEP_HEAD]  N, the largest number of such channels, N', - ; [8 + sigma] the number of such channels
+//   [nsig][pitch][4]  alpha1, alpha2, embedding, channel
+//   [nsig][pitch]     beta
+//   double: [nsig][N + 1][pitch]  e^(beta i/N), and [nsig][N' + 1][pitch] of (e^(alpha1 i/N'), e^(alpha2 i/N')), N' in [2]
+// The last part: e^(beta T) = g + g p(beta (T - i/N)) with g from the row nearest to T.  What the reduction of HotExp does per
+// triplet and channel -- the integer part, the remainder, the power of two -- is done once per triplet, with exact results: i
+// and T - i/N.  N is the smallest power of two with |beta| / (2 N) <= 2^-7 for every channel (trained values are between -10 and
+// 4; beyond EXP_ROWS / 64 = 16, and where a beta is not a number, N is 0 and HotExp is used); there p, of degree 5 through 0 with
+// slope 1 and the values of e^x at four Chebyshev points, is off by at most 4e-17.
+constexpr int EXP_ROWS = 1024, STEP_HEAD = 32;
+__host__ __device__ inline int step_pitch(int Aa) { return (Aa + 15) & ~15; }
+template <typename real>
+__host__ __device__ inline size_t step_exp_at(int nsig, int Aa) { return STEP_HEAD + (size_t)nsig * step_pitch(Aa) * 5; }
+template <typename real>
+__host__ __device__ inline size_t step_pair_at(int nsig, int Aa) {
+  return step_exp_at<real>(nsig, Aa) + (size_t)nsig * (EXP_ROWS + 1) * step_pitch(Aa);
+}
+template <typename real>
+inline size_t step_table_reals(int nt, int Aa) {   // 0: more channels than a table is made for
+  if (Aa > STEP_CHANNELS || nt > NT_MAX) return 0;
+  const int nsig = 2 * nt - 1;
+  return sizeof(real) == 8 ? step_pair_at<real>(nsig, Aa) + (size_t)nsig * (EXP_ROWS + 1) * step_pitch(Aa) * 2
+                           : step_exp_at<real>(nsig, Aa);
+}
+// rows of a table for exponents up to `largest`
+__host__ __device__ inline int exp_rows(double largest) {
+  int N = largest <= EXP_ROWS / 64 ? 1 : 0;
+  while (N && N < 64 * largest) N *= 2;
+  return N;
+}
+// e^(a t): the product's rounding is made good
+__host__ __device__ inline double exp_of(double a, double t) {
+  const double hi = a * t, e = exp(hi);
+  return fma(e, fma(a, t, -hi), e);
+}
+// The table of a loaded model, on the host: t zeroed, emb3b squared.  step_table_body is the same on the device.
+inline void step_table_host(double* t, const double* alpha3b, const double* emb3b, int nt, int Aa) {
+  const int nsig = 2 * nt - 1, pitch = step_pitch(Aa);
+  double* const par = t + STEP_HEAD;
+  double* const beta = par + (size_t)nsig * pitch * 4;
+  double most[2] = {0, 0};   // of beta, of the alphas
+  int n[2 * NT_MAX] = {0};
+  for (int s = 0; s < nsig; s++) {
+    for (int a = 0; a < Aa; a++) {
+      if (emb3b[s * Aa + a] == 0) continue;
+      const double* al = alpha3b + 3 * ((size_t)s * Aa + a);
+      for (int c = 0; c < 3; c++) most[c < 2] = !(fabs(al[c]) <= 1e30) ? 1e30 : fmax(most[c < 2], fabs(al[c]));
+      const size_t at = (size_t)s * pitch + n[s]++;
+      par[4 * at] = al[0]; par[4 * at + 1] = al[1]; par[4 * at + 2] = emb3b[s * Aa + a]; par[4 * at + 3] = a;
+      beta[at] = al[2];
+    }
+    t[8 + s] = n[s];
+    t[1] = fmax(t[1], t[8 + s]);
+  }
+  const int N = exp_rows(most[0]), Np = exp_rows(most[1]);
+  t[0] = N;
+  t[2] = Np;
+  double* const rows = t + step_exp_at<double>(nsig, Aa);
+  double* const pairs = t + step_pair_at<double>(nsig, Aa);
+  for (int s = 0; s < nsig; s++)
+    for (int c = 0; c < n[s]; c++) {
+      const size_t at = (size_t)s * pitch + c;
+      for (int i = 0; N && i <= N; i++) rows[((size_t)s * (N + 1) + i) * pitch + c] = exp_of(beta[at], (double)i / N);
+      for (int i = 0; Np && i <= Np; i++)
+        for (int k = 0; k < 2; k++)
+          pairs[(((size_t)s * (Np + 1) + i) * pitch + c) * 2 + k] = exp_of(par[4 * at + k], (double)i / Np);
+    }
+}
+// where T lies: its row, and its distance from it
+__device__ inline int exp_place(double T, double n, double inv_n, int N, double& rest) {
+  const double r = rint(T * n);
+  rest = fma(-r, inv_n, T);
+  const int i = (int)r;
+  return i < 0 ? 0 : (i > N ? N : i);
+}
+// g e^x for |x| <= 2^-7
+__device__ inline double exp_near(double x, double g) {
+  double q = fma(x, 0.008333345443492365, 0.041666751437797855);
+  q = fma(q, x, 0.1666666666665743);
+  q = fma(q, x, 0.49999999999935324);
+  q = fma(q, x, 1.0);
+  return fma(g, q * x, g);
+}
+
+// A slot's entry of the pair tables, (e^(alpha1 D), e^(alpha2 D)) of one channel, by the table's rows (n > 0) or HotExp.  D is a
+// cutoff function's value, between 0 and 1.
+template <typename real>
+struct PairTable {
+  const real* rows;
+  int n, pitch;
+  __device__ PairTable(const real* table, int n_, int nsig, int Aa)
+      : rows(table + step_pair_at<real>(nsig, Aa)), n(n_), pitch(step_pitch(Aa)) {}
+  // what a slot's entries have in common: its row and its distance from it
+  __device__ int place(real D, real& rest) const {
+    if constexpr (sizeof(real) == 8) {
+      return exp_place(D, (real)n, real(1) / (real)n, n, rest);
+    } else {
+      rest = 0;
+      return 0;
+    }
+  }
+  __device__ typename Vec2<real>::type operator()(real a1, real a2, int sg, int channel, real D, int row, real rest) const {
+    using HE = HotExp<real>;
+    typename Vec2<real>::type v;
+    if constexpr (sizeof(real) == 8) {
+      if (n) {
+        const auto g = ((const typename Vec2<real>::type*)rows)[(unsigned)(sg * (n + 1) + row) * (unsigned)pitch + channel];
+        v.x = exp_near(a1 * rest, g.x);
+        v.y = exp_near(a2 * rest, g.y);
+      } else {
+        auto eval = [&](real a) { const real x = a * D, e = HE::eval(x); return r_fma(e, r_fma(a, D, -x), e); };
+        v.x = eval(a1);
+        v.y = eval(a2);
+      }
+    } else {
+      v.x = HE::eval(HE::scale(a1) * D);
+      v.y = HE::eval(HE::scale(a2) * D);
+    }
+    return v;
+  }
+};
+
+// broadcast of lane L of every row of sixteen lanes
+template <int L>
+__device__ inline double row_lane(double v) {
+  return __longlong_as_double(__builtin_amdgcn_update_dpp(0ll, __double_as_longlong(v), 0x150 + L, 0xf, 0xf, true));
+}
+template <int L>
+__device__ inline float row_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + L, 0xf, 0xf, true));
+}
+template <int L>
+__device__ inline unsigned row_lane(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + L, 0xf, 0xf, true);
+}
+// read-only memory through the scalar cache: addresses are uniform
+template <typename T>
+__device__ inline const __attribute__((address_space(4))) T* scalar_ptr(const T* p) {
+  return (const __attribute__((address_space(4))) T*)p;
+}
+
+__host__ __device__ inline bool step_slots(int nr, int na, int nt) {
+  return nr <= WAVE && na >= nr * (nr - 1) / 2 && nt <= NT_MAX;
+}
+
+// Slots grouped by species, by one full wave: lane s holds slot s (its species t_s, anything for lanes that take no part: on
+// false).  off [nt + 1]; returns the place of the lane's slot.
+__device__ inline int group_lane(int nt, int t_s, bool on, int* off) {
+  const int lane = lane_id();
+  int pos = 0, base = 0;
+  for (int t = 0; t < nt; t++) {
+    const unsigned long long mask = __ballot(on && t_s == t);
+    if (lane == 0) off[t] = base;
+    if (on && t_s == t) pos = base + __popcll(mask & ((1ull << lane) - 1ull));
+    base += __popcll(mask);
+  }
+  if (lane == 0) off[nt] = base;
+  return pos;
+}
+
+// ---------------------------------------------------------------------------
+// The table, by workgroup `part` of `parts` of sigma sg.  Every workgroup finds the largest exponents of all active channels and
+// the active channels of its sigma for itself; the first one of a sigma writes the parameters, all of them the rows.
+// ---------------------------------------------------------------------------
+constexpr int STEP_TABLE_BLOCK = 256, STEP_TABLE_PARTS = 32;
+template <typename real>
+__device__ inline void step_table_body(const StepTablePart<real>& P, int nt, int sg, int part, int parts) {
+  using real2 = typename Vec2<real>::type;
+  using real4 = typename Vec4<real>::type;
+  constexpr bool DBL = sizeof(real) == 8;
+  constexpr int WAVES = STEP_TABLE_BLOCK / WAVE;
+  __shared__ unsigned short ch[STEP_CHANNELS];
+  __shared__ real top[WAVES][2];
+  __shared__ int act[WAVES], active;
+  const int nsig = 2 * nt - 1, Aa = P.Aa, pitch = step_pitch(Aa);
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
+  real4* const par = (real4*)(P.table + STEP_HEAD) + (size_t)sg * pitch;
+  real* const beta = P.table + STEP_HEAD + (size_t)nsig * pitch * 4 + (size_t)sg * pitch;
+  const real* const alpha = P.alpha3b + (size_t)sg * Aa * 3;
+  auto weight = [&](int s, int a) {
+    const real c = a < Aa ? P.emb3b[s * Aa + a] : real(0);
+    return P.raw_emb ? c * c : c;
+  };
+  auto larger = [](real a, real v) { return !(fabs(v) <= real(1e30)) ? real(1e30) : fmax(a, fabs(v)); };
+  real most = 0, most_a = 0;
+  int channels = 0;
+  for (int s = wave; s < nsig; s += WAVES) {
+    int base = 0;
+    for (int a0 = 0; a0 < Aa; a0 += WAVE) {
+      const int a = a0 + lane;
+      const bool on = weight(s, a) != real(0);
+      base += __popcll(__ballot(on));
+      if (on) {
+        const real* al = P.alpha3b + 3 * ((size_t)s * Aa + a);
+        most_a = larger(larger(most_a, al[0]), al[1]);
+        most = larger(most, al[2]);
+      }
+    }
+    channels = base > channels ? base : channels;
+  }
+#pragma unroll
+  for (int d = WAVE / 2; d > 0; d >>= 1) {
+    most = fmax(most, __shfl_xor(most, d, WAVE));
+    most_a = fmax(most_a, __shfl_xor(most_a, d, WAVE));
+  }
+  if (lane == 0) { top[wave][0] = most; top[wave][1] = most_a; act[wave] = channels; }
+  if (wave == 0) {
+    int base = 0;
+    for (int a0 = 0; a0 < Aa; a0 += WAVE) {
+      const int a = a0 + lane;
+      const real c = weight(sg, a);
+      const bool on = c != real(0);
+      const unsigned long long mask = __ballot(on);
+      if (on) {
+        const int at = base + __popcll(mask & ((1ull << lane) - 1ull));
+        ch[at] = (unsigned short)a;
+        if (part == 0) {
+          real4 x;
+          x.x = alpha[3 * a]; x.y = alpha[3 * a + 1]; x.z = c; x.w = real(a);
+          par[at] = x;
+          beta[at] = alpha[3 * a + 2];
+        }
+      }
+      base += __popcll(mask);
+    }
+    if (part == 0) {
+      real4 z;
+      z.x = z.y = z.z = z.w = 0;
+      for (int a = base + lane; a < pitch; a += WAVE) { par[a] = z; beta[a] = 0; }
+      if (lane == 0) P.table[8 + sg] = real(base);
+    }
+    if (lane == 0) active = base;
+  }
+  __syncthreads();
+  for (int w = 0; w < WAVES; w++) {
+    most = fmax(most, top[w][0]);
+    most_a = fmax(most_a, top[w][1]);
+    channels = act[w] > channels ? act[w] : channels;
+  }
+  const int N = DBL ? exp_rows(most) : 0, Np = DBL ? exp_rows(most_a) : 0;
+  if (part == 0 && sg == 0 && tid == 0) {
+    P.table[0] = real(N);
+    P.table[1] = real(channels);
+    P.table[2] = real(Np);
+  }
+  if constexpr (DBL) {
+    real* const rows = P.table + step_exp_at<real>(nsig, Aa) + (size_t)sg * (N + 1) * pitch;
+    for (int q = part * STEP_TABLE_BLOCK + tid; N && q < (N + 1) * pitch; q += parts * STEP_TABLE_BLOCK) {
+      const int i = q / pitch, c = q - i * pitch;
+      rows[q] = c < active ? exp_of(alpha[3 * ch[c] + 2], real(i) / N) : real(0);
+    }
+    real2* const pairs = (real2*)(P.table + step_pair_at<real>(nsig, Aa)) + (size_t)sg * (Np + 1) * pitch;
+    for (int q = part * STEP_TABLE_BLOCK + tid; Np && q < (Np + 1) * pitch; q += parts * STEP_TABLE_BLOCK) {
+      const int i = q / pitch, c = q - i * pitch;
+      real2 v;
+      v.x = c < active ? exp_of(alpha[3 * ch[c]], real(i) / Np) : real(0);
+      v.y = c < active ? exp_of(alpha[3 * ch[c] + 1], real(i) / Np) : real(0);
+      pairs[q] = v;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Fingerprints
+// ---------------------------------------------------------------------------
+template <typename real, int WAVES>
+struct RowsCfg {
+  static constexpr int THREADS = WAVES * WAVE;
+  static constexpr int PAD = 3;            // rows a step of four may read beyond the last one
+  static constexpr int MIN_WAVES = sizeof(real) == 8 ? 4 : 8;
+  __host__ __device__ static size_t bytes(int nr, int Aa, int nt) {
+    size_t b = ((size_t)nt * (nr + PAD) * TRI_CAP * 2 + (size_t)5 * nr + (size_t)WAVES * Aa) * sizeof(real);
+    b += (size_t)(nr + NT_MAX + 1) * sizeof(int);
+    return (b + 15) & ~(size_t)15;
+  }
+};
+
+template <typename real, int WAVES>
+__device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __restrict__ table, const int first_centre,
+                                          const int stride) {
+  using real2 = typename Vec2<real>::type;
+  using real4 = typename Vec4<real>::type;
+  using HE = HotExp<real>;
+  using L = RowsCfg<real, WAVES>;
+  constexpr bool DBL = sizeof(real) == 8;
+  constexpr int THREADS = L::THREADS;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int nr = A.nr, Aa = A.Aa, nt = A.nt, nsig = 2 * nt - 1, pitch = step_pitch(Aa);
+  const int EP = nr + L::PAD;                      // rows of a partner species' block of the table
+  real2* E = (real2*)smem;                         // [partner species][grouped slot][channel]
+  real2* slots = E + (size_t)nt * EP * TRI_CAP;    // [grouped slot] unit vector, cutoff value
+  real* rst = (real*)(slots + 2 * nr);             // [grouped slot] distance from its row of the pair tables
+  real* outw = rst + nr;
+  int* stp = (int*)(outw + (size_t)WAVES * Aa);    // [grouped slot] species | row of the pair tables << 8
+  int* off = stp + nr;                             // [nt + 1] first grouped slot of a species
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = uniform(tid / WAVE);
+  const int ia = lane & (TRI_CAP - 1), r = lane / TRI_CAP;
+  real* const my_out = outw + wave * Aa;
+  const auto head = scalar_ptr(table);
+  const int exp_n = DBL ? (int)head[0] : 0, maxact = (int)head[1];
+  const real4* const parA = (const real4*)(table + STEP_HEAD);
+  const real* const beta = (const real*)(parA + (size_t)nsig * pitch);
+  const PairTable<real> pairs(table, (int)head[2], nsig, Aa);
+  const real exp_nr = real(exp_n), exp_inv = real(1) / exp_nr;
+  const int exp_row = pitch * (int)sizeof(real);
+
+  const int total = A.nf * A.Nl;
+  // what a centre's set-up reads from its own rows: issued while the centre before it is summed
+  int m_n = 0, nj_n = 0;
+  real d_n = 0, u_n[3] = {0, 0, 0};
+  auto request = [&](int atom) {   // (by the first wave)
+    if (wave > 0) return;
+    const int b = atom / A.Nl, p = atom - b * A.Nl;
+    const size_t row = (size_t)b * A.ld + p;
+    m_n = A.numtriplet[row];
+    if (lane < nr) {
+      nj_n = A.im2[row * (nr + 1) + 1 + lane];
+      d_n = A.Dsup[row * nr + lane];
+#pragma unroll
+      for (int c = 0; c < 3; c++) u_n[c] = A.unit[(row * 4 + c) * nr + lane];
+    }
+  };
+  request(first_centre);
+
+  for (int atom = first_centre;;) {
+    // ---- slots grouped by species
+    if (wave == 0) {
+      const int m = m_n > nr ? nr : m_n;
+      int t_s = 0;
+      if (lane < m) t_s = A.type_map[nj_n];
+      const int pos = group_lane(nt, t_s, lane < m, off);
+      if (lane < m) {
+        real2 v, w;
+        v.x = u_n[0]; v.y = u_n[1]; w.x = u_n[2]; w.y = d_n;
+        slots[2 * pos] = v;
+        slots[2 * pos + 1] = w;
+        stp[pos] = t_s | (pairs.place(d_n, rst[pos]) << 8);
+      }
+    }
+    __syncthreads();
+    const int m = uniform(off[nt]);
+    const int next = stride > total - 1 - atom ? -1 : atom + stride;
+
+    for (int c0 = 0; c0 < maxact; c0 += TRI_CAP) {
+      if (c0 > 0) __syncthreads();   // the table of the channels before is consumed
+      // ---- table: E[tb][g][ia] = (exp(a1 D), exp(a2 D)) with the parameters of sigma = species + tb
+      {
+        int g = wave * 4 + r, tb = 0;
+        const int rows = m + L::PAD;
+        for (;; g += 4 * WAVES) {
+          while (g >= rows && tb < nt) { g -= rows; tb++; }
+          if (tb >= nt) break;
+          real2 v;
+          v.x = v.y = 0;
+          if (g < m) {
+            const int at = stp[g], sg = (at & 255) + tb;
+            const real2 par = *(const real2*)(parA + sg * pitch + c0 + ia);
+            v = pairs(par.x, par.y, sg, c0 + ia, slots[2 * g + 1].y, at >> 8, rst[g]);
+          }
+          E[(tb * EP + g) * TRI_CAP + ia] = v;
+        }
+      }
+      __syncthreads();
+      if (c0 == 0)
+        for (int a = lane; a < Aa; a += WAVE) my_out[a] = 0;
+      if (c0 + TRI_CAP >= maxact && next >= 0) request(next);
+      // ---- rows, four at a time, of every class, dealt to the waves
+      int turn = 0;
+      for (int ta = 0; ta < nt; ta++) {
+        const int oa = uniform(off[ta]), na_ = uniform(off[ta + 1]) - oa;
+        for (int tb = ta; tb < nt; tb++) {
+          const int ob = uniform(off[tb]), nb_ = uniform(off[tb + 1]) - ob;
+          const bool same = ta == tb;
+          if (same ? na_ < 2 : na_ * nb_ == 0) continue;
+          const int sg = ta + tb;
+          if (c0 >= (int)head[8 + sg]) continue;
+          // rows x of one species, columns y of the other one (the same: y < x)
+          const bool flip = !same && ((na_ + 3) >> 2) * nb_ > ((nb_ + 3) >> 2) * na_;
+          const int nx = flip ? nb_ : na_, ny = flip ? na_ : nb_;
+          const int ox = flip ? ob : oa, oy = flip ? oa : ob;
+          const int tx = flip ? tb : ta, ty = flip ? ta : tb;
+          const int blocks = ((same ? nx - 1 : nx) + 3) >> 2;
+          int blk = (wave - turn) & (WAVES - 1);
+          turn = (turn + blocks) & (WAVES - 1);
+          if (blk >= blocks) continue;
+          const int at = sg * pitch + c0 + ia;
+          const real be = beta[at], bes = HE::scale(be);
+          const real4 par = parA[at];
+          const unsigned char* const exp_base =
+              (const unsigned char*)(table + step_exp_at<real>(nsig, Aa) + c0) + (size_t)sg * (exp_n + 1) * exp_row;
+          const unsigned exp_lane = (unsigned)ia * sizeof(real);
+          real acc = 0;
+          for (; blk < blocks; blk += WAVES) {
+            const int x = same ? nx - 1 - 4 * blk - r : 4 * blk + r;
+            const int len = same ? nx - 1 - 4 * blk : ny;          // of the block's longest row
+            const bool row_ok = x >= 0 && x < nx;
+            const int mine = row_ok ? (same ? x : ny) : 0;
+            const int gx = ox + (row_ok ? x : 0);
+            const real2 x01 = slots[2 * gx], x23 = slots[2 * gx + 1];
+            const real2 e1 = E[(ty * EP + gx) * TRI_CAP + ia];
+            const real2* Ey = E + (tx * EP + oy) * TRI_CAP + ia;
+            real F1 = 0, F2 = 0;
+            for (int y0 = 0; y0 < len; y0 += 16, Ey += 16 * TRI_CAP) {
+              // T of row r and column y0 + (lane & 15)
+              const int y = y0 + ia, gy = oy + (y < ny ? y : ny - 1);
+              const real2 y01 = slots[2 * gy], y23 = slots[2 * gy + 1];
+              const real cs = x01.x * y01.x + x01.y * y01.y + x23.x * y23.x;
+              real T = (real(0.5) * (cs + real(1))) * (x23.y * y23.y);
+              T = y < mine ? T : real(0);
+              real rest = 0;
+              unsigned row = 0;
+              if constexpr (DBL) row = (unsigned)mul24(exp_place(T, exp_nr, exp_inv, exp_n, rest), exp_row);
+              const int left = len - y0;
+              auto four = [&](auto q_c, auto near_c) {
+                constexpr int Q = decltype(q_c)::value;
+                constexpr bool NEAR = decltype(near_c)::value;
+                real2 e2[4];
+                real g[4], Tb[4], rb[4];
+                auto load = [&](auto u_c) {
+                  constexpr int u = decltype(u_c)::value;
+                  Tb[u] = row_lane<Q + u>(T);
+                  if constexpr (NEAR) {
+                    g[u] = *(const real*)(exp_base + (row_lane<Q + u>(row) + exp_lane));
+                    rb[u] = row_lane<Q + u>(rest);
+                  }
+                  e2[u] = Ey[(Q + u) * TRI_CAP];
+                };
+                load(std::integral_constant<int, 0>{});
+                load(std::integral_constant<int, 1>{});
+                load(std::integral_constant<int, 2>{});
+                load(std::integral_constant<int, 3>{});
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                  real e;
+                  if constexpr (NEAR) e = exp_near(be * rb[u], g[u]);
+                  else e = HE::eval(bes * Tb[u]);
+                  const real w = Tb[u] * e;
+                  F2 = r_fma(w, e2[u].y, F2);
+                  F1 = r_fma(w, e2[u].x, F1);
+                }
+              };
+              auto sixteen = [&](auto near_c) {
+                four(std::integral_constant<int, 0>{}, near_c);
+                if (left > 4) four(std::integral_constant<int, 4>{}, near_c);
+                if (left > 8) four(std::integral_constant<int, 8>{}, near_c);
+                if (left > 12) four(std::integral_constant<int, 12>{}, near_c);
+              };
+              if constexpr (DBL) {
+                if (exp_n) sixteen(std::true_type{});
+                else sixteen(std::false_type{});
+              } else {
+                sixteen(std::false_type{});
+              }
+            }
+            acc = r_fma(e1.x, F2, acc);
+            acc = r_fma(e1.y, F1, acc);
+          }
+          acc += __shfl_xor(acc, 16, WAVE);
+          acc += __shfl_xor(acc, 32, WAVE);
+          if (lane < TRI_CAP && par.z != real(0)) my_out[(int)par.w] += acc * (par.z * real(0.5));
+        }
+      }
+    }
+    if (maxact == 0) {   // (no channel has a weight)
+      for (int a = lane; a < Aa; a += WAVE) my_out[a] = 0;
+      if (next >= 0) request(next);
+    }
+    __syncthreads();
+    for (int a = (tid + THREADS - WAVE) % THREADS; a < Aa; a += THREADS) {   // (not by the first wave)
+      real s = 0;
+#pragma unroll
+      for (int w = 0; w < WAVES; w++) s += outw[w * Aa + a];
+      A.out[(size_t)atom * Aa + a] = s;
+    }
+    if (next < 0) break;
+    atom = next;
+  }
+}
+
+}  // namespace staf
