@@ -221,6 +221,54 @@ __device__ inline T wave_sum_to_last(T v) {
     return s;
   }
 }
+// Sums over the 64 lanes of twelve values: halves of the lanes trade values until a row of sixteen lanes holds one value of
+// four, then three prefix sums in the rows (63 instructions for doubles where twelve of wave_scan are 216).  The sum of
+// v[4 q + place] is v[q] of the last lane of row 0, 2, 1, 3 for place 0, 1, 2, 3.
+__device__ inline void lanes_trade32(double& a, double& b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  a = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+  b = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+__device__ inline void lanes_trade16(double& a, double& b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  a = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+  b = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+__device__ inline void lanes_trade32(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+}
+__device__ inline void lanes_trade16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+}
+template <typename T>
+__device__ inline void wave_sums12(T (&v)[12]) {
+#pragma unroll
+  for (int p = 0; p < 6; p++) { lanes_trade32(v[2 * p], v[2 * p + 1]); v[p] = v[2 * p] + v[2 * p + 1]; }
+#pragma unroll
+  for (int q = 0; q < 3; q++) { lanes_trade16(v[2 * q], v[2 * q + 1]); v[q] = v[2 * q] + v[2 * q + 1]; }
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    if constexpr (sizeof(T) == 8) {
+      v[q] += dpp_row<0x111>(v[q]);
+      v[q] += dpp_row<0x112>(v[q]);
+      v[q] += dpp_row<0x114>(v[q]);
+      v[q] += dpp_row<0x118>(v[q]);
+    } else {
+      T s = v[q] + dpp_get<0x111, 0xf>(v[q]);
+      s += dpp_get<0x112, 0xf>(v[q]);
+      s += dpp_get<0x113, 0xf>(v[q]);
+      s += dpp_get<0x114, 0xf>(s);
+      s += dpp_get<0x118, 0xf>(s);
+      v[q] = s;
+    }
+  }
+}
 // Wave-uniform value loaded through a vector path (e.g. from LDS) moved to a scalar register, so that loop
 // bounds and addresses derived from it stay scalar.
 __device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }

@@ -31,7 +31,10 @@
 // are all that has to be summed, and (u_s . V_s) u_s comes off once.  The lanes of the triplets leave A, R_j and R_k in LDS, where
 // the exponential table was, in storage order, and lane s takes them for every p (dealt to the waves): reads of consecutive
 // words for p < s.  Seven operations per (slot, partner) in place of four prefix sums per pass and a loop over the rows of a pass:
-// 236 -> 215 M vector instructions for 24576 atoms (m = 37), 23 -> 15 % of the LDS cycles; launch 535 -> 486 us.
+// 236 -> 215 M vector instructions for 24576 atoms (m = 37), 183 -> 155 M LDS cycles; launch 490 -> 455 us.  The slots lie in LDS as
+// pairs of 16 bytes (two reads for what four separate rows took four reads and addresses for), and the first wave, which holds
+// all slots, forms the centre's own force and virial by itself, twelve sums at once (wave_sums12): 215 -> 200 M, 455 -> 430 us;
+// launches of 4 x 768, 768 and 96 centres 73.5 -> 69.6, 28.0 -> 26.8 and 17.4 -> 16.3 us.
 // The slot forces go to scratch or to the caller's arrays (gslot, and the centre's own force to self); the atoms
 // that receive them collect them in gather_kernel (per op) or force_total_kernel (all species at once) through the
 // neighbour map.
@@ -91,11 +94,12 @@ struct Force3Cfg {
     const int nsig = 2 * nt - 1;
     return (size_t)nsig * rowp(Aa) * 4 /*prm*/ + (size_t)nsig * pitch(Aa) * 2 /*prE*/ +
            table_reals(nr, nt, pull) /*E, then the triplets*/ +
-           (pull ? 0 : (size_t)NW * 4 * nr) /*slot sums per wave*/ + nr /*D*/ + 3 * nr /*grad fc*/ +
-           (size_t)NW * 4 /*the waves' shares of the centre's own force*/ + (fused ? 4 * nr : 0) /*unit vectors, 1/r*/ +
+           (pull ? 0 : (size_t)NW * 4 * nr) /*slot sums per wave*/ + (pull ? 4 * WAVE : nr) /*D, pull: the slots*/ +
+           3 * nr /*grad fc*/ + (size_t)NW * 4 /*the waves' shares of the centre's own force*/ +
+           (pull ? nr : fused ? 4 * nr : 0) /*unit vectors, 1/r, pull: 1/r*/ +
            (Ar2 > 0 ? (size_t)NW * nr + nr + (size_t)2 * nt * Ar2 : 0) /*2-body: the waves' shares of the pair
            weights, D, parameter rows*/ +
-           (fused && Ar2 > 0 ? NW * 9 : 0) /*the waves' shares of the centre's virial*/;
+           (fused && Ar2 > 0 && !pull ? NW * 9 : 0) /*the waves' shares of the centre's virial*/;
   }
   __host__ __device__ static size_t bytes(int nr, int Aa, int nt, bool fused = false, int Ar2 = 0, bool pull = false) {
     return n_reals(nr, Aa, nt, fused, Ar2, pull) * sizeof(real) + (size_t)(16 + (Ar2 > 0 ? NT_MAX : 0) + nr) * sizeof(int);
@@ -166,14 +170,16 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
   real* triA = E;                                          // PULL: [3][TRI] of the sweep's triplets, where the table was
   real* acc = E + L::table_reals(nr, nt, PULL);            // [NW][4 nr]: per wave, slot sums (as j and as k), see accW
   real* sD = acc + (PULL ? (size_t)0 : (size_t)NW * 4 * nr);   // [nr]
-  real* sg = sD + nr;                                      // [3*nr] grad fc (der3bsupp)
+  real2* slots = (real2*)sD;                               // PULL: [2][WAVE] (u_x, u_y) and (u_z, D) of the slots
+  real* sg = sD + (PULL ? 4 * WAVE : nr);                  // [3*nr] grad fc (der3bsupp)
   real* xch = sg + 3 * nr;                                 // [NW][4] the waves' shares of the centre's own force
   real* sU = xch + NW * 4;                                 // FUSED: [4][nr] unit vector, 1/r
-  real* w2p = sU + (FUSED ? 4 * nr : 0);                   // W2B: [NW][nr] the waves' shares of the 2-body pair weights
+  real* rinv = sU + (PULL ? 0 : 3 * nr);                   // FUSED: [nr] 1/r
+  real* w2p = sU + (PULL ? nr : FUSED ? 4 * nr : 0);       // W2B: [NW][nr] the waves' shares of the 2-body pair weights
   real* sD2 = w2p + (W2B ? NW * nr : 0);                   // W2B: [nr] raddescr of the slots
   real* p2 = sD2 + (W2B ? nr : 0);                         // W2B: alpha2b [nt*Ar], dE/dAF2 emb2b [nt*Ar] of the channels of weight != 0
   real* xv = p2 + (W2B ? 2 * nt * B2.Ar : 0);              // VIR: [NW][9] the waves' shares of the centre's virial
-  int* nact = (int*)(xv + (VIR ? NW * 9 : 0));   // [16] active channels per sigma (0 beyond nsig)
+  int* nact = (int*)(xv + (VIR && !PULL ? NW * 9 : 0));   // [16] active channels per sigma (0 beyond nsig)
   int* nact2 = nact + 16;                                  // W2B: [nt] such channels per neighbour species
   int* stp = nact2 + (W2B ? NT_MAX : 0);                   // [nr] species of every slot
 
@@ -319,10 +325,18 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
     }
   }
   if (tid < nr) {
-    sD[tid] = d_s;
+    if constexpr (PULL) {
+      real2 v, w;
+      v.x = u_s[0]; v.y = u_s[1]; w.x = u_s[2]; w.y = d_s;
+      slots[tid] = v;
+      slots[WAVE + tid] = w;
+      rinv[tid] = u_s[3];
+    } else {
+      sD[tid] = d_s;
+    }
 #pragma unroll
     for (int c = 0; c < 3; c++) sg[c * nr + tid] = g_s[c];
-    if constexpr (FUSED) {
+    if constexpr (FUSED && !PULL) {
 #pragma unroll
       for (int c = 0; c < 4; c++) sU[c * nr + tid] = u_s[c];
     }
@@ -389,7 +403,11 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
       if (nn < ntri) {
         int j, k;
         tri_decode(nn, m, j, k);
-        if constexpr (FUSED) {
+        if constexpr (PULL) {
+          const real2 a = slots[j], a2 = slots[WAVE + j], b_ = slots[k], b2 = slots[WAVE + k];
+          const real cs = a.x * b_.x + a.y * b_.y + a2.x * b2.x;
+          T[p] = (real(0.5) * (cs + real(1))) * (a2.y * b2.y);
+        } else if constexpr (FUSED) {
           const real cs = sU[j] * sU[k] + sU[nr + j] * sU[nr + k] + sU[2 * nr + j] * sU[2 * nr + k];
           T[p] = (real(0.5) * (cs + real(1))) * (sD[j] * sD[k]);
         } else {
@@ -421,7 +439,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
           int s_ = r, tb = 0;
           while (s_ >= m) { s_ -= m; tb++; }
           const real2 o = *(const real2*)(prE + (mul24(stp[s_] + tb, Ap) + c0 + ia) * 2);
-          const real d = sD[s_];
+          const real d = PULL ? slots[WAVE + s_].y : sD[s_];
           real2 v;
           v.x = HE::eval(o.x * d);
           v.y = HE::eval(o.y * d);
@@ -512,8 +530,9 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
         if (p >= npass) break;
         const int q = (p * NW + wave) * WAVE + lane;
         const int j = jk[p] & 0xff, k = jk[p] >> 8;
-        const real cs = sU[j] * sU[k] + sU[nr + j] * sU[nr + k] + sU[2 * nr + j] * sU[2 * nr + k];
-        const real fj = sD[j], fk = sD[k], hT = real(0.5) * T[p];
+        const real2 a = slots[j], a2 = slots[WAVE + j], b_ = slots[k], b2 = slots[WAVE + k];
+        const real cs = a.x * b_.x + a.y * b_.y + a2.x * b2.x;
+        const real fj = a2.y, fk = b2.y, hT = real(0.5) * T[p];
         const real sh = Sd[p] * (real(0.5) * (cs + real(1)));
         if (w0 + q < ntri) {
           triA[q] = Sd[p] * (fj * fk);
@@ -532,8 +551,10 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
           int q = low ? mine + p : theirs + lane;
           q = (unsigned)q < (unsigned)n && lane != p ? q : L::SWEEP;
           const real a = triA[q], rad = triA[(low ? L::TRI : 2 * L::TRI) + q];
-#pragma unroll
-          for (int c = 0; c < 3; c++) pull[c] = r_fma(a, sU[c * nr + p], pull[c]);
+          const real2 u01 = slots[p];
+          pull[0] = r_fma(a, u01.x, pull[0]);
+          pull[1] = r_fma(a, u01.y, pull[1]);
+          pull[2] = r_fma(a, slots[WAVE + p].x, pull[2]);
           pull[3] += rad;
         }
       }
@@ -666,6 +687,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
 #pragma unroll
     for (int c = 0; c < 4; c++) triA[(wave * 4 + c) * WAVE + lane] = pull[c];
     __syncthreads();
+    if (wave > 0) return;   // all slots are the first wave's
   }
 
   // ---- slot forces (waves added in a fixed order; one slot per thread: m <= nr < THREADS), centre's own force.
@@ -680,7 +702,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
 #pragma unroll
           for (int c = 0; c < 4; c++) t4[c] += triA[(w * 4 + c) * WAVE + lane];
         // sum of A (u_p - (u_s . u_p) u_s)
-        const real u[3] = {sU[tid], sU[nr + tid], sU[2 * nr + tid]};
+        const real u[3] = {slots[lane].x, slots[lane].y, slots[WAVE + lane].x};
         const real along = u[0] * t4[0] + u[1] * t4[1] + u[2] * t4[2];
 #pragma unroll
         for (int c = 0; c < 3; c++) t4[c] = r_fma(-along, u[c], t4[c]);
@@ -693,7 +715,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
       }
 #pragma unroll
       for (int c = 0; c < 3; c++) {
-        const real t = FUSED ? t4[c] * (real(0.5) * sU[3 * nr + tid]) : t4[c];
+        const real t = FUSED ? t4[c] * (real(0.5) * rinv[tid]) : t4[c];
         f3[c] = t + t4[3] * sg[c * nr + tid];
       }
     }
@@ -709,6 +731,33 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
         for (int c = 0; c < 3; c++) f3[c] += w * B2.dD[rowAtom * 3 * nr + c * nr + tid];
       }
     }
+    if constexpr (PULL) {
+      // the centre's own force and its virial, - sum_s f_s (x) (r_centre - r_s): the separations are the unit vectors times r
+      const real2 u01 = slots[lane];
+      const real2 u23 = slots[WAVE + lane];
+      const real r = tid < cnt2 ? -(real(1) / rinv[tid]) : real(0);
+      const real re[3] = {tid < cnt2 ? r * u01.x : real(0), tid < cnt2 ? r * u01.y : real(0), tid < cnt2 ? r * u23.x : real(0)};
+      real v[12] = {-f3[0], -f3[1], -f3[2]};
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int e = 0; e < 3; e++) v[3 + c * 3 + e] = f3[c] * re[e];
+      wave_sums12(v);
+      if (tid < nr) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) gslot[(rowOut * nr + tid) * 3 + c] = f3[c];
+      }
+      if ((lane & 15) == 15) {
+        const int row = lane >> 4, place = ((row & 1) << 1) | (row >> 1);
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+          const int at = 4 * q + place;
+          if (at < 3) self[rowOut * 3 + at] = v[q];
+          else if (A.vpart) A.vpart[rowOut * 9 + at - 3] = v[q];
+        }
+      }
+      return;
+    }
     real tot[3] = {f3[0], f3[1], f3[2]};
     wave_scan(tot);
 #pragma unroll
@@ -719,7 +768,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
       // (nine sums in a wave that has its operands, 2-3 us of launches per 6144 atoms less than a pass over the
       // slot forces)
       if (A.vpart) {
-        const real r = tid < cnt2 ? real(1) / sU[3 * nr + tid] : real(0);
+        const real r = tid < cnt2 ? real(1) / rinv[tid] : real(0);
 #pragma unroll
         for (int e = 0; e < 3; e++) {
           const real re = tid < cnt2 ? -(r * sU[e * nr + tid]) : real(0);
