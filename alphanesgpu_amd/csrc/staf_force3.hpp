@@ -806,10 +806,10 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
   }
 }
 
-template <typename real, bool FUSED = false, int NWAVES = 4, bool W2B = false, bool PULL = false>
+template <typename real, bool FUSED = false, int NWAVES = 4, bool W2B = false>
 __global__ __launch_bounds__((Force3Cfg<real, NWAVES>::THREADS), (Force3Cfg<real, NWAVES>::MIN_WAVES)) void force3_kernel(
     const Force3Args<real> A) {
-  force3_body<real, FUSED, NWAVES, W2B, PULL>(A, (int)blockIdx.x);
+  force3_body<real, FUSED, NWAVES, W2B, false>(A, (int)blockIdx.x);
 }
 
 // The centres of several species in one launch: entry e takes workgroups first[e] .. first[e + 1].

@@ -56,8 +56,8 @@ PROFILED_NAME = {
     ("desc_fp_kernel", "f64"): "staf::desc_fingerprints_kernel<double>",
     ("desc_kernel", "f32"): "staf::desc_kernel<float>",
     ("desc_kernel", "f64"): "staf::desc_kernel<double>",
-    ("af3_fused", "f64"): "staf::step_fingerprints_kernel<double, 256>",
-    ("force3_fused", "f64"): "staf::force3_species_kernel<double, true, 4, true>",
+    ("af3_fused", "f64"): "staf::step_fingerprints_kernel<double, 256, true>",
+    ("force3_fused", "f64"): "staf::force3_species_kernel<double, true, 4, true, true>",
 }
 
 
