@@ -442,17 +442,15 @@ template <typename real>
 int step_fingerprints(const StepSpecies<real>* sp, int n, const StepRows<real>& R, const int* type_map, int nt,
                       hipStream_t stream) {
   int total = 0;
-  size_t lds = 0, rows_lds = 0;
-  bool rows = step_slots(R.nr, R.na, nt);
+  size_t lds = 0;
+  bool rows = true;
   for (int c = 0; c < n; c++) {
     total += R.nf * sp[c].Nl;
-    rows = rows && (sp[c].table || sp[c].Nl == 0);
-    rows_lds = std::max(rows_lds, RowsCfg<real, 8>::bytes(R.nr, sp[c].Aa, nt) +
-                                      (size_t)2 * nt * sp[c].Ar * sizeof(real) + (size_t)8 * R.nr * (sizeof(real) + sizeof(int)));
+    rows = rows && (sp[c].Nl <= 0 || (sp[c].table && rows_fits<real>(R.nr, R.na, nt, sp[c].Ar, sp[c].Aa)));
     lds = std::max(lds, TriLds<real, 0, true, 512>::bytes(R.nr, sp[c].Aa, nt, true) +
                             (size_t)2 * nt * sp[c].Ar * sizeof(real) + (size_t)8 * R.nr * (sizeof(real) + sizeof(int)));
   }
-  if (rows && rows_lds <= 64 * 1024)
+  if (rows)
     return total <= WIDE_ROWS_CENTRES ? step_fingerprints_launch<real, 512, true>(sp, n, R, type_map, nt, stream)
                                       : step_fingerprints_launch<real, TRI_BLOCK, true>(sp, n, R, type_map, nt, stream);
   if (total <= WIDE_FINGERPRINT_CENTRES && lds <= 64 * 1024) return step_fingerprints_launch<real, 512, false>(sp, n, R, type_map, nt, stream);

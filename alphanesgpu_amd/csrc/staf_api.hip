@@ -250,7 +250,8 @@ static bool load_species_params(StafModel* m) {
       if (!u.d->reserve(u.h->size())) return false;
       if (!upload_sync(u.d->p, u.h->data(), u.h->size() * sizeof(double), m->stream)) return false;
     }
-    if (const size_t n = staf::step_table_reals<double>(nt, m->Aa[k])) {
+    if (staf::rows_fits<double>(m->nr, m->na, nt, m->Ar[k], m->Aa[k])) {
+      const size_t n = staf::step_table_reals<double>(nt, m->Aa[k]);
       if (!m->table[k].reserve(n)) return false;
       std::vector<double> t(n, 0.0);
       staf::step_table_host(t.data(), a3.data(), e3.data(), nt, m->Aa[k]);

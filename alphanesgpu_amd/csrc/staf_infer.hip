@@ -83,7 +83,8 @@ static int frames_plan(const DescConfig<real>& c, int nf, int N, int nt, const S
     P->emb2b[k] = place((size_t)nt * s.nalpha_r * sizeof(real));
     P->emb3b[k] = place((size_t)nt * (nt + 1) / 2 * s.nsmooth_a * sizeof(real));
     P->net[k] = place(block * sizeof(real));
-    P->table[k] = place(step_table_reals<real>(nt, s.nsmooth_a) * sizeof(real));
+    P->table[k] = place(rows_fits<real>(c.nr, c.na, nt, s.nalpha_r, s.nsmooth_a)
+                            ? step_table_reals<real>(nt, s.nsmooth_a) * sizeof(real) : 0);
   }
   return sum == N ? STAF_OK : STAF_E_BAD_ARG;
 }
@@ -129,7 +130,7 @@ static int frames(const real* pos, const real* box, int nf, int N, int nt, const
     parts.insert(parts.end(), mine, mine + 2 + m);
     S[n] = {first, s.n_local, s.nalpha_r, s.nsmooth_a, (const real*)s.alpha2b, (const real*)s.alpha3b, at(P.emb2b[k]),
             at(P.emb3b[k]), at(P.af2[k]), at(P.af3[k]), at(P.g2[k]), at(P.g3[k]), nullptr};
-    if (step_table_reals<real>(nt, s.nsmooth_a)) {
+    if (rows_fits<real>(c.nr, c.na, nt, s.nalpha_r, s.nsmooth_a)) {
       S[n].table = at(P.table[k]);
       tables[n_tables++] = {S[n].alpha3b, (const real*)s.type_emb3b, at(P.table[k]), s.nsmooth_a, 1};
     }

@@ -43,8 +43,7 @@ __host__ __device__ inline size_t step_pair_at(int nsig, int Aa) {
   return step_exp_at<real>(nsig, Aa) + (size_t)nsig * (EXP_ROWS + 1) * step_pitch(Aa);
 }
 template <typename real>
-inline size_t step_table_reals(int nt, int Aa) {   // 0: more channels than a table is made for
-  if (Aa > STEP_CHANNELS || nt > NT_MAX) return 0;
+inline size_t step_table_reals(int nt, int Aa) {
   const int nsig = 2 * nt - 1;
   return sizeof(real) == 8 ? step_pair_at<real>(nsig, Aa) + (size_t)nsig * (EXP_ROWS + 1) * step_pitch(Aa) * 2
                            : step_exp_at<real>(nsig, Aa);
@@ -171,15 +170,15 @@ __host__ __device__ inline bool step_slots(int nr, int na, int nt) {
 }
 
 // Slots grouped by species, by one full wave: lane s holds slot s (its species t_s, anything for lanes that take no part: on
-// false).  off [nt + 1]; returns the place of the lane's slot.
-__device__ inline int group_lane(int nt, int t_s, bool on, int* off) {
+// false).  Behind every group lie `pad` places that hold no slot.  off [nt + 1]; returns the place of the lane's slot.
+__device__ inline int group_lane(int nt, int t_s, bool on, int pad, int* off) {
   const int lane = lane_id();
   int pos = 0, base = 0;
   for (int t = 0; t < nt; t++) {
     const unsigned long long mask = __ballot(on && t_s == t);
     if (lane == 0) off[t] = base;
     if (on && t_s == t) pos = base + __popcll(mask & ((1ull << lane) - 1ull));
-    base += __popcll(mask);
+    base += __popcll(mask) + pad;
   }
   if (lane == 0) off[nt] = base;
   return pos;
@@ -293,14 +292,23 @@ __device__ inline void step_table_body(const StepTablePart<real>& P, int nt, int
 template <typename real, int WAVES>
 struct RowsCfg {
   static constexpr int THREADS = WAVES * WAVE;
-  static constexpr int PAD = 3;            // rows a step of four may read beyond the last one
+  static constexpr int PAD = 3;            // rows of zeros behind every species', which a step of four may read
   static constexpr int MIN_WAVES = sizeof(real) == 8 ? 4 : 8;
+  __host__ __device__ static int rows(int nr, int nt) { return nr + nt * PAD; }
   __host__ __device__ static size_t bytes(int nr, int Aa, int nt) {
-    size_t b = ((size_t)nt * (nr + PAD) * TRI_CAP * 2 + (size_t)5 * nr + (size_t)WAVES * Aa) * sizeof(real);
-    b += (size_t)(nr + NT_MAX + 1) * sizeof(int);
+    const size_t r = rows(nr, nt);
+    size_t b = (nt * r * TRI_CAP * 2 + 5 * r + (size_t)WAVES * Aa) * sizeof(real);
+    b += (r + NT_MAX + 1) * sizeof(int);
     return (b + 15) & ~(size_t)15;
   }
 };
+// True: rows_body takes a species of these sizes (the launch computes the 2-body fingerprints too).
+template <typename real>
+inline bool rows_fits(int nr, int na, int nt, int Ar, int Aa) {
+  const size_t lds = RowsCfg<real, 8>::bytes(nr, Aa, nt) +
+                     (size_t)2 * nt * Ar * sizeof(real) + (size_t)8 * nr * (sizeof(real) + sizeof(int));
+  return step_slots(nr, na, nt) && Aa <= STEP_CHANNELS && lds <= 64 * 1024;
+}
 
 template <typename real, int WAVES>
 __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __restrict__ table, const int first_centre,
@@ -313,13 +321,13 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
   constexpr int THREADS = L::THREADS;
   extern __shared__ __align__(16) unsigned char smem[];
   const int nr = A.nr, Aa = A.Aa, nt = A.nt, nsig = 2 * nt - 1, pitch = step_pitch(Aa);
-  const int EP = nr + L::PAD;                      // rows of a partner species' block of the table
+  const int EP = L::rows(nr, nt);                  // rows of a partner species' block of the table
   real2* E = (real2*)smem;                         // [partner species][grouped slot][channel]
   real2* slots = E + (size_t)nt * EP * TRI_CAP;    // [grouped slot] unit vector, cutoff value
-  real* rst = (real*)(slots + 2 * nr);             // [grouped slot] distance from its row of the pair tables
-  real* outw = rst + nr;
-  int* stp = (int*)(outw + (size_t)WAVES * Aa);    // [grouped slot] species | row of the pair tables << 8
-  int* off = stp + nr;                             // [nt + 1] first grouped slot of a species
+  real* rst = (real*)(slots + 2 * EP);             // [grouped slot] distance from its row of the pair tables
+  real* outw = rst + EP;
+  int* stp = (int*)(outw + (size_t)WAVES * Aa);    // [grouped slot] species | row of the pair tables << 8, -1: none
+  int* off = stp + EP;                             // [nt + 1] first grouped slot of a species
   const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = uniform(tid / WAVE);
   const int ia = lane & (TRI_CAP - 1), r = lane / TRI_CAP;
   real* const my_out = outw + wave * Aa;
@@ -355,7 +363,7 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
       const int m = m_n > nr ? nr : m_n;
       int t_s = 0;
       if (lane < m) t_s = A.type_map[nj_n];
-      const int pos = group_lane(nt, t_s, lane < m, off);
+      const int pos = group_lane(nt, t_s, lane < m, L::PAD, off);
       if (lane < m) {
         real2 v, w;
         v.x = u_n[0]; v.y = u_n[1]; w.x = u_n[2]; w.y = d_n;
@@ -363,9 +371,12 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
         slots[2 * pos + 1] = w;
         stp[pos] = t_s | (pairs.place(d_n, rst[pos]) << 8);
       }
+      __builtin_amdgcn_wave_barrier();
+      __threadfence_block();
+      if (lane < nt * L::PAD) stp[off[lane / L::PAD + 1] - 1 - lane % L::PAD] = -1;
     }
     __syncthreads();
-    const int m = uniform(off[nt]);
+    const int rows = uniform(off[nt]);
     const int next = stride > total - 1 - atom ? -1 : atom + stride;
 
     for (int c0 = 0; c0 < maxact; c0 += TRI_CAP) {
@@ -373,14 +384,13 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
       // ---- table: E[tb][g][ia] = (exp(a1 D), exp(a2 D)) with the parameters of sigma = species + tb
       {
         int g = wave * 4 + r, tb = 0;
-        const int rows = m + L::PAD;
         for (;; g += 4 * WAVES) {
           while (g >= rows && tb < nt) { g -= rows; tb++; }
           if (tb >= nt) break;
           real2 v;
           v.x = v.y = 0;
-          if (g < m) {
-            const int at = stp[g], sg = (at & 255) + tb;
+          if (const int at = stp[g]; at >= 0) {
+            const int sg = (at & 255) + tb;
             const real2 par = *(const real2*)(parA + sg * pitch + c0 + ia);
             v = pairs(par.x, par.y, sg, c0 + ia, slots[2 * g + 1].y, at >> 8, rst[g]);
           }
@@ -394,9 +404,9 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
       // ---- rows, four at a time, of every class, dealt to the waves
       int turn = 0;
       for (int ta = 0; ta < nt; ta++) {
-        const int oa = uniform(off[ta]), na_ = uniform(off[ta + 1]) - oa;
+        const int oa = uniform(off[ta]), na_ = uniform(off[ta + 1]) - oa - L::PAD;
         for (int tb = ta; tb < nt; tb++) {
-          const int ob = uniform(off[tb]), nb_ = uniform(off[tb + 1]) - ob;
+          const int ob = uniform(off[tb]), nb_ = uniform(off[tb + 1]) - ob - L::PAD;
           const bool same = ta == tb;
           if (same ? na_ < 2 : na_ * nb_ == 0) continue;
           const int sg = ta + tb;
