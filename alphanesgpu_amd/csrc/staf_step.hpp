@@ -13,10 +13,10 @@
 //     is summed (two multiply-adds per item instead of four operations), and the row's factors are applied once per row;
 //   * one table entry per item is read from LDS, the same address for the four rows;
 //   * all classes' tables are built at once, the rows of all classes are dealt to the waves: three barriers per centre.
-// Launches of 24576, 4 x 768 (inference), 768 and 96 centres: 366 -> 329, 56.6 -> 51.6, 24.9 -> 18.5 and 12.5 -> 10.7 us in double
-// precision (157 -> 135 M vector instructions, 28 -> 12 M LDS instructions for 24576), 4 x 768 in single 31.8 -> 25.3; a vector
-// instruction in 0.71 of the issue slots, the rest is latency at four waves per SIMD (125 registers; five would need 96, and
-// less than the 36 KB of LDS that 60 slots take).
+// Launches of 24576, 4 x 768 (inference), 768 and 96 centres: 366 -> 335, 56.6 -> 52, 24.9 -> 19 and 12.5 -> 11.0 us in double
+// precision (157 -> 137 M vector instructions, 28 -> 13 M LDS instructions for 24576), 4 x 768 in single 31.8 -> 25.3; a vector
+// instruction in 0.71 of the busy cycles, the rest is latency at four waves per SIMD (127 registers; five would need 96, and
+// less than the 38 KB of LDS that 60 slots take).
 #pragma once
 #include "staf_tri.hpp"
 
