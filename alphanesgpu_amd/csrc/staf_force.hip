@@ -850,10 +850,11 @@ int step_forces(const StepSpecies<real>* sp, int n, const StepRows<real>& R, con
   if (wg == 0) return STAF_OK;
   M.first[M.entries] = wg;
   // A launch of few centres lasts as long as one centre takes, and with eight waves a centre's passes are shared by twice
-  // as many: MD call of 225 atoms 84.8 -> 79.3 us, 432 89.7 -> 86.0, 504 91.6 -> 88.7, 588 101.2 -> 98.5, 768 103.5 -> 99.7.  A
-  // little beyond it they still are no slower (864: 105.1 and 104.1, 960: 112.1 and 109.6, 1152: 126.1 and 123.1, 1215: 125.2 and
-  // 123.8); in longer launches the registers and LDS of the wide ones cost residency.
-  constexpr int FORCE3_WIDE_CENTRES = 768;   // three per CU
+  // as many: MD call of 225 atoms 84.8 -> 79.3 us, 432 89.7 -> 86.0, 504 91.6 -> 88.7, 588 101.2 -> 98.5, 768 103.5 -> 99.7 (before the
+  // slots' lanes summed their triplets).  A CU holds three such workgroups, and launches of a second round of them still gain:
+  // launches of 864, 972, 1200, 1500 and 2160 centres by four and by eight waves 32.5 / 31.6, 32.0 / 30.9, 37.5 / 35.6, 41.3 / 41.3 and
+  // 55.6 / 56.3 us, in single precision 864 and 1152 20.0 / 18.4 and 21.0 / 19.9.
+  constexpr int FORCE3_WIDE_CENTRES = 1280;   // five per CU
   KernelTimer kt_("force3_kernel", stream);
   auto launch = [&](auto pull_c) -> int {
     constexpr bool PULL = decltype(pull_c)::value;
