@@ -405,9 +405,9 @@ static int step_fingerprints_launch(const StepSpecies<real>* sp, int n, const St
     auto& Q = M.rad[M.entries];
     Q.D = R.raddescr + o * R.nr; Q.alpha2b = S.alpha2b; Q.emb2b = S.emb2b; Q.out = S.af2; Q.Ar = S.Ar;
     M.table[M.entries] = S.table;
-    const size_t need3 = ROWS ? RowsCfg<real, WAVES>::bytes(R.nr, S.Aa, nt) : TriLds<real, 0, true, BLOCK>::bytes(R.nr, S.Aa, nt, true);
     const size_t need2 = (size_t)2 * nt * S.Ar * sizeof(real) + (size_t)WAVES * R.nr * (sizeof(real) + sizeof(int));
-    lds = std::max(lds, std::max(need2, need3));
+    lds = std::max(lds, ROWS ? rows_lds<real, WAVES>(R.nr, nt, S.Ar, S.Aa)
+                             : std::max(need2, TriLds<real, 0, true, BLOCK>::bytes(R.nr, S.Aa, nt, true)));
     M.first2[M.entries++] = wg;
     wg += (R.nf * S.Nl + WAVES - 1) / WAVES;
     total += R.nf * S.Nl;
@@ -435,24 +435,24 @@ static int step_fingerprints_launch(const StepSpecies<real>* sp, int n, const St
 // 94.0 -> 88.7.  A CU holds two such workgroups; beyond that 256 threads are as fast (588 atoms: 98.5 and 98.6 us) or faster
 // (768: 99.7 and 101.0, 1080: 119.3 and 123.1, 1215: 125.2 and 130.5).
 constexpr int WIDE_FINGERPRINT_CENTRES = 512;   // two per CU
-// The same of rows_body, whose launches of 4 and of 8 waves per centre take 13.5 and 10.7 us for 96 centres, 13.9 and 10.8 for
-// 225, 15.6 and 13.4 for 378, 16.1 and 16.8 for 504, 17.1 and 19.0 for 576, 18.5 and 21.6 for 768.
-constexpr int WIDE_ROWS_CENTRES = 448;
 template <typename real>
 int step_fingerprints(const StepSpecies<real>* sp, int n, const StepRows<real>& R, const int* type_map, int nt,
                       hipStream_t stream) {
   int total = 0;
   size_t lds = 0;
-  bool rows = true;
+  RowsLaunch<real> rows;
   for (int c = 0; c < n; c++) {
     total += R.nf * sp[c].Nl;
-    rows = rows && (sp[c].Nl <= 0 || (sp[c].table && rows_fits<real>(R.nr, R.na, nt, sp[c].Ar, sp[c].Aa)));
+    rows.add(R.nr, R.na, nt, sp[c].Ar, sp[c].Aa, (long long)R.nf * sp[c].Nl);
+    rows.fits = rows.fits && (sp[c].Nl <= 0 || sp[c].table);
     lds = std::max(lds, TriLds<real, 0, true, 512>::bytes(R.nr, sp[c].Aa, nt, true) +
                             (size_t)2 * nt * sp[c].Ar * sizeof(real) + (size_t)8 * R.nr * (sizeof(real) + sizeof(int)));
   }
-  if (rows)
-    return total <= WIDE_ROWS_CENTRES ? step_fingerprints_launch<real, 512, true>(sp, n, R, type_map, nt, stream)
-                                      : step_fingerprints_launch<real, TRI_BLOCK, true>(sp, n, R, type_map, nt, stream);
+  switch (rows.waves()) {
+    case 8: return step_fingerprints_launch<real, 512, true>(sp, n, R, type_map, nt, stream);
+    case 4: return step_fingerprints_launch<real, TRI_BLOCK, true>(sp, n, R, type_map, nt, stream);
+    default: break;
+  }
   if (total <= WIDE_FINGERPRINT_CENTRES && lds <= 64 * 1024) return step_fingerprints_launch<real, 512, false>(sp, n, R, type_map, nt, stream);
   return step_fingerprints_launch<real, TRI_BLOCK, false>(sp, n, R, type_map, nt, stream);
 }

@@ -20,6 +20,7 @@ struct FramesPlan {
   size_t bytes = 0;
   size_t raddescr, des3bsupp, der2b, der3bsupp, unit, slots, self, vpart, e_atom, intmap2b, numtriplet;
   size_t af2[NT_MAX], af3[NT_MAX], g2[NT_MAX], g3[NT_MAX], net[NT_MAX], emb2b[NT_MAX], emb3b[NT_MAX], table[NT_MAX];
+  bool rows = false;   // the fingerprints' launch reads the species' tables
 };
 
 static DevMlpSource net_source(const StafFramesSpecies& s) {
@@ -68,6 +69,9 @@ static int frames_plan(const DescConfig<real>& c, int nf, int N, int nt, const S
   P->e_atom = place(rows * sizeof(real));
   P->intmap2b = place(rows * (nr + 1) * sizeof(int));
   P->numtriplet = place(rows * sizeof(int));
+  RowsLaunch<real> form;
+  for (int k = 0; k < nt; k++) form.add(c.nr, c.na, nt, sp[k].nalpha_r, sp[k].nsmooth_a, (long long)nf * sp[k].n_local);
+  P->rows = form.waves() > 0;
   long long sum = 0;
   for (int k = 0; k < nt; k++) {
     const StafFramesSpecies& s = sp[k];
@@ -83,8 +87,7 @@ static int frames_plan(const DescConfig<real>& c, int nf, int N, int nt, const S
     P->emb2b[k] = place((size_t)nt * s.nalpha_r * sizeof(real));
     P->emb3b[k] = place((size_t)nt * (nt + 1) / 2 * s.nsmooth_a * sizeof(real));
     P->net[k] = place(block * sizeof(real));
-    P->table[k] = place(rows_fits<real>(c.nr, c.na, nt, s.nalpha_r, s.nsmooth_a)
-                            ? step_table_reals<real>(nt, s.nsmooth_a) * sizeof(real) : 0);
+    P->table[k] = place(P->rows && s.n_local > 0 ? step_table_reals<real>(nt, s.nsmooth_a) * sizeof(real) : 0);
   }
   return sum == N ? STAF_OK : STAF_E_BAD_ARG;
 }
@@ -130,7 +133,7 @@ static int frames(const real* pos, const real* box, int nf, int N, int nt, const
     parts.insert(parts.end(), mine, mine + 2 + m);
     S[n] = {first, s.n_local, s.nalpha_r, s.nsmooth_a, (const real*)s.alpha2b, (const real*)s.alpha3b, at(P.emb2b[k]),
             at(P.emb3b[k]), at(P.af2[k]), at(P.af3[k]), at(P.g2[k]), at(P.g3[k]), nullptr};
-    if (rows_fits<real>(c.nr, c.na, nt, s.nalpha_r, s.nsmooth_a)) {
+    if (P.rows) {
       S[n].table = at(P.table[k]);
       tables[n_tables++] = {S[n].alpha3b, (const real*)s.type_emb3b, at(P.table[k]), s.nsmooth_a, 1};
     }

@@ -166,7 +166,7 @@ __device__ inline const __attribute__((address_space(4))) T* scalar_ptr(const T*
 }
 
 __host__ __device__ inline bool step_slots(int nr, int na, int nt) {
-  return nr <= WAVE && na >= nr * (nr - 1) / 2 && nt <= NT_MAX;
+  return nr > 0 && nr <= WAVE && na >= nr * (nr - 1) / 2 && nt <= NT_MAX;
 }
 
 // Slots grouped by species, by one full wave: lane s holds slot s (its species t_s, anything for lanes that take no part: on
@@ -302,13 +302,67 @@ struct RowsCfg {
     return (b + 15) & ~(size_t)15;
   }
 };
-// True: rows_body takes a species of these sizes (the launch computes the 2-body fingerprints too).
+// LDS of a workgroup of a launch that takes rows_body with WAVES waves per centre for a species of these sizes: that of rows_body, or
+// that of the workgroups of the 2-body fingerprints.
+template <typename real, int WAVES>
+inline size_t rows_lds(int nr, int nt, int Ar, int Aa) {
+  const size_t two_body = (size_t)2 * nt * Ar * sizeof(real) + (size_t)WAVES * nr * (sizeof(real) + sizeof(int));
+  const size_t b = RowsCfg<real, WAVES>::bytes(nr, Aa, nt);
+  return b > two_body ? b : two_body;
+}
+// workgroups whose LDS a CU's 160 KB hold at once: they are handed out in pieces of 1280 bytes
+inline int lds_workgroups(size_t lds) { return (int)(128 / ((lds + 1279) / 1280)); }
+// True: there are launches in which rows_body takes a species of these sizes.  Its table is held to 32 MB.
 template <typename real>
 inline bool rows_fits(int nr, int na, int nt, int Ar, int Aa) {
-  const size_t lds = RowsCfg<real, 8>::bytes(nr, Aa, nt) +
-                     (size_t)2 * nt * Ar * sizeof(real) + (size_t)8 * nr * (sizeof(real) + sizeof(int));
-  return step_slots(nr, na, nt) && Aa <= STEP_CHANNELS && lds <= 64 * 1024;
+  return step_slots(nr, na, nt) && Ar > 0 && Aa > 0 && Aa <= STEP_CHANNELS && lds_workgroups(rows_lds<real, 8>(nr, nt, Ar, Aa)) > 0 &&
+         step_table_reals<real>(nt, Aa) * sizeof(real) <= (size_t)32 << 20;
 }
+// Which form a launch takes.  The tables of rows_body hold nt rows per slot where tri_reduce_body has one: with three species, 60 slots
+// and 40 channels a CU holds two workgroups of four waves in double precision, not four.  Where waves are few the launch is slower than the
+// staged form, unless all its centres are there at once: then it lasts as long as a centre takes.  Launches of the staged form, of
+// rows_body with four and (up to 729) with eight waves per centre, us; the channels dealt to the classes in blocks:
+//                                      centres  512                 729                 2197         5832
+//   double, two species, 60 slots, 4 per CU:    18.3 / 15.3         20.4 / 16.5         38.8 / 36.6  82.7 / 77.3
+//   double, three, 32 slots, 4 per CU:                              20.2 / 16.3         39.7 / 39.2  80.5 / 77.2
+//   double, three, 48 slots, 3 per CU:          21.7 / 16.5 / 17.7  22.1 / 20.4 / 21.7  43.3 / 44.0  90.7 / 100.9
+//   double, three, 60 slots, 2 per CU:          22.6 / 20.2 / 19.0  24.9 / 28.3 / 23.7  51.1 / 85.0  112.7 / 147.7
+//   double, four, 40 slots, 2 per CU:                               26.7 / 30.2         57.8 / 70.5  123.4 / 156.5
+//                                      centres  729                 1458                2916         11664
+//   single, three, 40 slots, 7 per CU:          17.7 / 14.0                             36.4 / 29.7  104.0 / 88.5
+//   single, three, 60 slots, 5 per CU:          18.7 / 15.2         22.6 / 23.3         39.9 / 37.9  114.8 / 110.9
+//   single, four, 60 slots, 4 per CU:           24.1 / 18.2         28.8 / 29.1         52.9 / 46.5  156.4 / 152.9
+//   single, five, 60 slots, 3 per CU:           31.2 / 23.9                                          274.5 / 235.3
+// So rows_body takes launches whose centres are all resident, and others where a CU holds FULL workgroups: four in double precision, what
+// its registers admit, three in single.  (With a weight of every channel in every class, which training does not make of blocks -- a
+// weight of 0 has no gradient --, the last three rows are 36.5 / 31.4 and 49.3 / 39.5 for 729, but 83.3 / 89.7, 111.6 / 112.4 and 146.0 / 168.7
+// for 2916 and 257.9 / 278.2, 349.1 / 390.9 and 648.9 / 626.5 for 11664.)
+// Eight waves per centre up to 448 centres: two species, 60 slots, four and eight waves 13.5 and 10.7 us for 96 centres, 13.9 and 10.8
+// for 225, 15.6 and 13.4 for 378, 16.1 and 16.8 for 504, 17.1 and 19.0 for 576, 18.5 and 21.6 for 768.
+constexpr int ROWS_CUS = 256, WIDE_ROWS_CENTRES = 448;
+template <typename real>
+struct RowsLaunch {
+  bool fits = true;
+  size_t lds4 = 0, lds8 = 0;
+  long long centres = 0;
+  void add(int nr, int na, int nt, int Ar, int Aa, long long n) {   // a species with n centres
+    if (n <= 0) return;
+    fits = fits && rows_fits<real>(nr, na, nt, Ar, Aa);
+    if (!fits) return;
+    const size_t four = rows_lds<real, 4>(nr, nt, Ar, Aa), eight = rows_lds<real, 8>(nr, nt, Ar, Aa);
+    lds4 = four > lds4 ? four : lds4;
+    lds8 = eight > lds8 ? eight : lds8;
+    centres += n;
+  }
+  // waves per centre of rows_body; 0: tri_reduce_body
+  int waves() const {
+    constexpr int FULL = sizeof(real) == 8 ? 4 : 3;
+    if (!fits || centres == 0) return 0;
+    if (centres <= WIDE_ROWS_CENTRES && centres <= ROWS_CUS * lds_workgroups(lds8)) return 8;
+    const int held = lds_workgroups(lds4);
+    return held >= FULL || centres <= ROWS_CUS * held ? 4 : 0;
+  }
+};
 
 template <typename real, int WAVES>
 __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __restrict__ table, const int first_centre,

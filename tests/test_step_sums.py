@@ -17,17 +17,18 @@ def _crowd(edge, spacing, species, seed):
 
 # Neighbours inside the angular cutoff: about 6, 18, 32 and 56 of at most `nr`.  A sweep of the force kernel takes 1024
 # triplets (46 neighbours have 1035), the fingerprints' rows go four by four and their columns sixteen by sixteen.  125 to 1331
-# centres: eight waves each up to 448 for the fingerprints and 1280 for the forces.
+# centres: eight waves each up to 448 for the fingerprints and 1280 for the forces.  Four species with 40 channels: 40 to 84
+# KB of LDS with eight waves, at 64 slots one workgroup per CU, which is enough for 216 centres and not for 343.
 @pytest.mark.gpu
 @pytest.mark.parametrize("edge,spacing,nr", [(5, 3.6, 24), (6, 2.6, 60), (6, 2.1, 64), (9, 2.1, 65), (7, 1.9, 64), (10, 1.9, 64),
                                              (11, 2.6, 60)])
 @pytest.mark.parametrize("species,channels,beta", [(1, (15,), 1.0), (2, (3, 17, 40), 1.0), (2, (14, 13, 13), -12.0),
-                                                   (3, (4, 3, 5, 3, 4, 3), 30.0)])
+                                                   (3, (4, 3, 5, 3, 4, 3), 30.0), (4, (4,) * 10, 1.0)])
 def test_sums_of_a_step(tmp_path, edge, spacing, nr, species, channels, beta):
     """float64, sums in another order: 1e-11.  beta: the largest exponent of the angular descriptor, one channel's."""
     from alphanesgpu_amd import libstaf, model_dir
     from test_oracle_pins import small_model
-    ps = small_model(species, (5, 4, 6)[:species], channels, seed=5, hidden=20, dense=species != 2)
+    ps = small_model(species, (5, 4, 6, 3)[:species], channels, seed=5, hidden=20, dense=species != 2)
     for p in ps:
         p["alpha3b"][0, 2] = beta
     x, box, types = _crowd(edge, spacing, species, seed=edge)
