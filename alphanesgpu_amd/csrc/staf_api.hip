@@ -251,11 +251,8 @@ static bool load_species_params(StafModel* m) {
       if (!upload_sync(u.d->p, u.h->data(), u.h->size() * sizeof(double), m->stream)) return false;
     }
     if (staf::rows_fits<double>(m->nr, m->na, nt, m->Ar[k], m->Aa[k])) {
-      const size_t n = staf::step_table_reals<double>(nt, m->Aa[k]);
-      if (!m->table[k].reserve(n)) return false;
-      std::vector<double> t(n, 0.0);
-      staf::step_table_host(t.data(), a3.data(), e3.data(), nt, m->Aa[k]);
-      if (!upload_sync(m->table[k].p, t.data(), n * sizeof(double), m->stream)) return false;
+      const std::vector<double> t = staf::step_table_host(a3.data(), e3.data(), nt, m->Aa[k]);
+      if (!m->table[k].reserve(t.size()) || !upload_sync(m->table[k].p, t.data(), t.size() * sizeof(double), m->stream)) return false;
     }
   }
   return true;

@@ -71,7 +71,9 @@ static int frames_plan(const DescConfig<real>& c, int nf, int N, int nt, const S
   P->numtriplet = place(rows * sizeof(int));
   RowsLaunch<real> form;
   for (int k = 0; k < nt; k++) form.add(c.nr, c.na, nt, sp[k].nalpha_r, sp[k].nsmooth_a, (long long)nf * sp[k].n_local);
-  P->rows = form.waves() > 0;
+  // (one species in double precision: its launches of few centres, 125, 343 and 512, take 17.4, 22.4 and 25.0 us in the staged form and 18.0,
+  // 21.8 and 25.1 by rows, whose table costs the parameters' launch 0.6 to 1.2)
+  P->rows = form.waves() > 0 && (sizeof(real) == 4 || nt > 1 || form.centres > 512);
   long long sum = 0;
   for (int k = 0; k < nt; k++) {
     const StafFramesSpecies& s = sp[k];

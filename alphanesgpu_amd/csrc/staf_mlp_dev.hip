@@ -582,7 +582,7 @@ constexpr int PACK_BLOCK = 256;
 static_assert(PACK_BLOCK == STEP_TABLE_BLOCK, "one launch");
 template <typename T>
 struct PackArgs {
-  int n, first[PACK_PARTS + 1];   // workgroups of a part; behind the last one's those of the tables
+  int n, first[PACK_PARTS + 1];   // workgroups of a part; before the first one's those of the tables, which take longest
   PackPart part[PACK_PARTS];
   int nt;
   StepTablePart<T> table[NT_MAX];
@@ -591,13 +591,15 @@ template <typename T>
 __host__ __device__ inline size_t pack_elements(const PackPart& p) {
   return p.kind == PACK_TILES ? mlp_tiled<T>(p.K, p.J) : p.kind == PACK_TILES_T ? mlp_tiled<T>(p.J, p.K) : (size_t)p.J;
 }
-// A thread per element of the destination: the order of upload_net's tiles.  Bound by its launch: the two networks of a
-// 60-140-140-1 stack in double precision are 0.9 MB.
+// A thread per element of the destination: the order of upload_net's tiles.  Bound by its launch and the first read of the parameters: the
+// two networks of a 60-140-140-1 stack in double precision are 0.9 MB, and the two tables of exponentials beside them 0.3 MB for
+// exponents up to 2 and 14 channels in use of 40: 5.1 us behind a step of 4 x 768 atoms, 5.6 behind one of 96 (of a step's length each; with tables
+// as wide as all 40 channels, maxima in double precision and divisions per entry 10.1 and 6.8; the networks alone 6.5 and 4.8).
 template <typename T>
 __global__ __launch_bounds__(PACK_BLOCK) void mlp_pack_kernel(const PackArgs<T> A) {
-  if ((int)blockIdx.x >= A.first[A.n]) {
-    const int w = (int)blockIdx.x - A.first[A.n], q = w / STEP_TABLE_PARTS, nsig = 2 * A.nt - 1;
-    step_table_body<T>(A.table[q / nsig], A.nt, q % nsig, w % STEP_TABLE_PARTS, STEP_TABLE_PARTS);
+  if ((int)blockIdx.x < A.first[0]) {
+    const int q = (int)blockIdx.x / STEP_TABLE_PARTS<T>, nsig = 2 * A.nt - 1;
+    step_table_body<T>(A.table[q / nsig], A.nt, q % nsig, (int)blockIdx.x % STEP_TABLE_PARTS<T>, STEP_TABLE_PARTS<T>);
     return;
   }
   int e = 0;
@@ -626,21 +628,24 @@ template <typename T>
 int dev_mlp_pack(const PackPart* parts, int n, const StepTablePart<T>* tables, int n_tables, int nt, hipStream_t stream) {
   for (int at = 0; at < n; at += PACK_PARTS) {
     PackArgs<T> A = {};
-    size_t blocks = 0;
+    size_t blocks = 0, lds = 0;
+    A.nt = nt;
+    if (at == 0) {
+      for (int k = 0; k < n_tables; k++) {
+        A.table[k] = tables[k];
+        lds = std::max(lds, step_table_lds<T>(tables[k].Aa));
+      }
+      blocks = (size_t)n_tables * (2 * nt - 1) * STEP_TABLE_PARTS<T>;
+    }
     for (A.n = 0; A.n < PACK_PARTS && at + A.n < n; A.n++) {
       A.part[A.n] = parts[at + A.n];
       A.first[A.n] = (int)blocks;
       blocks += (pack_elements<T>(A.part[A.n]) + PACK_BLOCK - 1) / PACK_BLOCK;
     }
     A.first[A.n] = (int)blocks;
-    A.nt = nt;
-    if (at == 0) {
-      for (int k = 0; k < n_tables; k++) A.table[k] = tables[k];
-      blocks += (size_t)n_tables * (2 * nt - 1) * STEP_TABLE_PARTS;
-    }
     if (blocks > 0x7fffffff) return STAF_E_LIMIT;
     KernelTimer kt_("mlp_pack_kernel", stream);
-    if (blocks) hipLaunchKernelGGL(mlp_pack_kernel<T>, dim3((unsigned)blocks), dim3(PACK_BLOCK), 0, stream, A);
+    if (blocks) hipLaunchKernelGGL(mlp_pack_kernel<T>, dim3((unsigned)blocks), dim3(PACK_BLOCK), lds, stream, A);
   }
   return hipGetLastError() == hipSuccess ? STAF_OK : STAF_E_HIP;
 }

@@ -18,40 +18,49 @@
 // instruction in 0.71 of the busy cycles, the rest is latency at four waves per SIMD (127 registers; five would need 96, and
 // less than the 38 KB of LDS that 60 slots take).
 #pragma once
+#include <vector>
+
 #include "staf_tri.hpp"
 
 namespace staf {
 
 // What the kernel needs of a species' parameters, laid out once for a loaded model, once a call where the
 // parameters are a caller's tensors: the channels of every sigma whose embedding is not 0, in ascending order, then
-// zeros up to the pitch.
-//   [STEP_HEAD]  N, the largest number of such channels, N', - ; [8 + sigma] the number of such channels
+// zeros up to the pitch, which is the largest number of such channels in whole sixteens.
+//   [STEP_HEAD]  N, the largest number of such channels, N', pitch; [8 + sigma] the number of such channels
 //   [nsig][pitch][4]  alpha1, alpha2, embedding, channel
 //   [nsig][pitch]     beta
-//   double: [nsig][N + 1][pitch]  e^(beta i/N), and [nsig][N' + 1][pitch] of (e^(alpha1 i/N'), e^(alpha2 i/N')), N' in [2]
+//   double: [nsig][N + 1][pitch]  e^(beta i/N), and [nsig][N' + 1][pitch] of (e^(alpha1 i/N'), e^(alpha2 i/N'))
 // The last part: e^(beta T) = g + g p(beta (T - i/N)) with g from the row nearest to T.  What the reduction of HotExp does per
 // triplet and channel -- the integer part, the remainder, the power of two -- is done once per triplet, with exact results: i
 // and T - i/N.  N is the smallest power of two with |beta| / (2 N) <= 2^-7 for every channel (trained values are between -10 and
 // 4; beyond EXP_ROWS / 64 = 16, and where a beta is not a number, N is 0 and HotExp is used); there p, of degree 5 through 0 with
 // slope 1 and the values of e^x at four Chebyshev points, is off by at most 4e-17.
 constexpr int EXP_ROWS = 1024, STEP_HEAD = 32;
-__host__ __device__ inline int step_pitch(int Aa) { return (Aa + 15) & ~15; }
-template <typename real>
-__host__ __device__ inline size_t step_exp_at(int nsig, int Aa) { return STEP_HEAD + (size_t)nsig * step_pitch(Aa) * 5; }
-template <typename real>
-__host__ __device__ inline size_t step_pair_at(int nsig, int Aa) {
-  return step_exp_at<real>(nsig, Aa) + (size_t)nsig * (EXP_ROWS + 1) * step_pitch(Aa);
-}
+__host__ __device__ inline int step_pitch(int channels) { return channels > 16 ? (channels + 15) & ~15 : 16; }
+// where the parts lie, in reals
+struct StepTable {
+  int N, Np, pitch;   // as in the head
+  size_t par, beta, rows, pairs, end;
+  __host__ __device__ StepTable(int nsig, int pitch_, int N_, int Np_) : N(N_), Np(Np_), pitch(pitch_) {
+    const size_t lines = (size_t)nsig * pitch;
+    par = STEP_HEAD;
+    beta = par + 4 * lines;
+    rows = beta + lines;
+    pairs = rows + (N ? lines * (N + 1) : 0);
+    end = pairs + (Np ? lines * (Np + 1) * 2 : 0);
+  }
+};
+// the largest a table of these sizes can be, whatever its parameters
 template <typename real>
 inline size_t step_table_reals(int nt, int Aa) {
-  const int nsig = 2 * nt - 1;
-  return sizeof(real) == 8 ? step_pair_at<real>(nsig, Aa) + (size_t)nsig * (EXP_ROWS + 1) * step_pitch(Aa) * 2
-                           : step_exp_at<real>(nsig, Aa);
+  const int most = sizeof(real) == 8 ? EXP_ROWS : 0;
+  return StepTable(2 * nt - 1, step_pitch(Aa), most, most).end;
 }
-// rows of a table for exponents up to `largest`
-__host__ __device__ inline int exp_rows(double largest) {
+// rows of a table for exponents up to `largest` (which is rounded: 2^-24 of it do not count)
+__host__ __device__ inline int exp_rows(float largest) {
   int N = largest <= EXP_ROWS / 64 ? 1 : 0;
-  while (N && N < 64 * largest) N *= 2;
+  while (N && (float)N < 64 * largest) N *= 2;
   return N;
 }
 // e^(a t): the product's rounding is made good
@@ -59,38 +68,44 @@ __host__ __device__ inline double exp_of(double a, double t) {
   const double hi = a * t, e = exp(hi);
   return fma(e, fma(a, t, -hi), e);
 }
-// The table of a loaded model, on the host: t zeroed, emb3b squared.  step_table_body is the same on the device.
-inline void step_table_host(double* t, const double* alpha3b, const double* emb3b, int nt, int Aa) {
-  const int nsig = 2 * nt - 1, pitch = step_pitch(Aa);
-  double* const par = t + STEP_HEAD;
-  double* const beta = par + (size_t)nsig * pitch * 4;
-  double most[2] = {0, 0};   // of beta, of the alphas
-  int n[2 * NT_MAX] = {0};
+// the larger of `a` and |v|; 1e30 where a v is beyond that or not a number
+__host__ __device__ inline float exp_larger(float a, float v) {
+  return !(fabsf(v) <= 1e30f) ? 1e30f : fmaxf(a, fabsf(v));
+}
+// The table of a loaded model, on the host; emb3b squared.  step_table_body is the same on the device.
+inline std::vector<double> step_table_host(const double* alpha3b, const double* emb3b, int nt, int Aa) {
+  const int nsig = 2 * nt - 1;
+  float most = 0, most_a = 0;
+  std::vector<int> ch[2 * NT_MAX];
+  size_t active = 0;
   for (int s = 0; s < nsig; s++) {
     for (int a = 0; a < Aa; a++) {
       if (emb3b[s * Aa + a] == 0) continue;
       const double* al = alpha3b + 3 * ((size_t)s * Aa + a);
-      for (int c = 0; c < 3; c++) most[c < 2] = !(fabs(al[c]) <= 1e30) ? 1e30 : fmax(most[c < 2], fabs(al[c]));
-      const size_t at = (size_t)s * pitch + n[s]++;
-      par[4 * at] = al[0]; par[4 * at + 1] = al[1]; par[4 * at + 2] = emb3b[s * Aa + a]; par[4 * at + 3] = a;
-      beta[at] = al[2];
+      most_a = exp_larger(exp_larger(most_a, (float)al[0]), (float)al[1]);
+      most = exp_larger(most, (float)al[2]);
+      ch[s].push_back(a);
     }
-    t[8 + s] = n[s];
-    t[1] = fmax(t[1], t[8 + s]);
+    active = ch[s].size() > active ? ch[s].size() : active;
   }
-  const int N = exp_rows(most[0]), Np = exp_rows(most[1]);
-  t[0] = N;
-  t[2] = Np;
-  double* const rows = t + step_exp_at<double>(nsig, Aa);
-  double* const pairs = t + step_pair_at<double>(nsig, Aa);
-  for (int s = 0; s < nsig; s++)
-    for (int c = 0; c < n[s]; c++) {
-      const size_t at = (size_t)s * pitch + c;
-      for (int i = 0; N && i <= N; i++) rows[((size_t)s * (N + 1) + i) * pitch + c] = exp_of(beta[at], (double)i / N);
-      for (int i = 0; Np && i <= Np; i++)
+  const StepTable L(nsig, step_pitch((int)active), exp_rows(most), exp_rows(most_a));
+  std::vector<double> t(L.end, 0.0);
+  t[0] = L.N; t[1] = (double)active; t[2] = L.Np; t[3] = L.pitch;
+  for (int s = 0; s < nsig; s++) {
+    t[8 + s] = (double)ch[s].size();
+    for (size_t c = 0; c < ch[s].size(); c++) {
+      const double* al = alpha3b + 3 * ((size_t)s * Aa + ch[s][c]);
+      const size_t at = (size_t)s * L.pitch + c;
+      double* const par = &t[L.par + 4 * at];
+      par[0] = al[0]; par[1] = al[1]; par[2] = emb3b[s * Aa + ch[s][c]]; par[3] = ch[s][c];
+      t[L.beta + at] = al[2];
+      for (int i = 0; L.N && i <= L.N; i++) t[L.rows + ((size_t)s * (L.N + 1) + i) * L.pitch + c] = exp_of(al[2], (double)i / L.N);
+      for (int i = 0; L.Np && i <= L.Np; i++)
         for (int k = 0; k < 2; k++)
-          pairs[(((size_t)s * (Np + 1) + i) * pitch + c) * 2 + k] = exp_of(par[4 * at + k], (double)i / Np);
+          t[L.pairs + (((size_t)s * (L.Np + 1) + i) * L.pitch + c) * 2 + k] = exp_of(al[k], (double)i / L.Np);
     }
+  }
+  return t;
 }
 // where T lies: its row, and its distance from it
 __device__ inline int exp_place(double T, double n, double inv_n, int N, double& rest) {
@@ -114,8 +129,7 @@ template <typename real>
 struct PairTable {
   const real* rows;
   int n, pitch;
-  __device__ PairTable(const real* table, int n_, int nsig, int Aa)
-      : rows(table + step_pair_at<real>(nsig, Aa)), n(n_), pitch(step_pitch(Aa)) {}
+  __device__ PairTable(const real* table, const StepTable& L) : rows(table + L.pairs), n(L.Np), pitch(L.pitch) {}
   // what a slot's entries have in common: its row and its distance from it
   __device__ int place(real D, real& rest) const {
     if constexpr (sizeof(real) == 8) {
@@ -185,104 +199,101 @@ __device__ inline int group_lane(int nt, int t_s, bool on, int pad, int* off) {
 }
 
 // ---------------------------------------------------------------------------
-// The table, by workgroup `part` of `parts` of sigma sg.  Every workgroup finds the largest exponents of all active channels and
-// the active channels of its sigma for itself; the first one of a sigma writes the parameters, all of them the rows.
+// The table, by workgroup `part` of `parts` of sigma sg.  Every workgroup finds the largest exponents and the numbers of active channels of
+// all sigmas for itself -- their parameters are read at once, whether their channels are active or not: a read that waits for
+// another one is what the launch would last for --, the first one of a sigma writes the parameters, all of them the rows.
 // ---------------------------------------------------------------------------
-constexpr int STEP_TABLE_BLOCK = 256, STEP_TABLE_PARTS = 32;
+constexpr int STEP_TABLE_BLOCK = 256;
+template <typename real>
+inline size_t step_table_lds(int Aa) { return (size_t)Aa * 5 * sizeof(real); }
+template <typename real>
+constexpr int STEP_TABLE_PARTS = sizeof(real) == 8 ? 32 : 1;   // (single precision has no rows)
 template <typename real>
 __device__ inline void step_table_body(const StepTablePart<real>& P, int nt, int sg, int part, int parts) {
-  using real2 = typename Vec2<real>::type;
   using real4 = typename Vec4<real>::type;
   constexpr bool DBL = sizeof(real) == 8;
   constexpr int WAVES = STEP_TABLE_BLOCK / WAVE;
-  __shared__ unsigned short ch[STEP_CHANNELS];
-  __shared__ real top[WAVES][2];
+  extern __shared__ __align__(16) unsigned char smem[];
+  real4* const own = (real4*)smem;                 // [Aa] alpha1, alpha2, embedding, channel of the active channels of sigma sg
+  real* const own_beta = (real*)(own + P.Aa);      // [Aa]
+  __shared__ float top[WAVES][2];
   __shared__ int act[WAVES], active;
-  const int nsig = 2 * nt - 1, Aa = P.Aa, pitch = step_pitch(Aa);
+  const int nsig = 2 * nt - 1, Aa = P.Aa;
   const int tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
-  real4* const par = (real4*)(P.table + STEP_HEAD) + (size_t)sg * pitch;
-  real* const beta = P.table + STEP_HEAD + (size_t)nsig * pitch * 4 + (size_t)sg * pitch;
-  const real* const alpha = P.alpha3b + (size_t)sg * Aa * 3;
-  auto weight = [&](int s, int a) {
-    const real c = a < Aa ? P.emb3b[s * Aa + a] : real(0);
-    return P.raw_emb ? c * c : c;
-  };
-  auto larger = [](real a, real v) { return !(fabs(v) <= real(1e30)) ? real(1e30) : fmax(a, fabs(v)); };
-  real most = 0, most_a = 0;
+  float most = 0, most_a = 0;
   int channels = 0;
   for (int s = wave; s < nsig; s += WAVES) {
     int base = 0;
     for (int a0 = 0; a0 < Aa; a0 += WAVE) {
       const int a = a0 + lane;
-      const bool on = weight(s, a) != real(0);
-      base += __popcll(__ballot(on));
-      if (on) {
+      real4 x;
+      x.x = x.y = x.z = x.w = 0;
+      real be = 0;
+      if (a < Aa) {
         const real* al = P.alpha3b + 3 * ((size_t)s * Aa + a);
-        most_a = larger(larger(most_a, al[0]), al[1]);
-        most = larger(most, al[2]);
+        x.z = P.emb3b[s * Aa + a];
+        x.x = al[0]; x.y = al[1]; be = al[2];
+        x.w = real(a);
+        if (P.raw_emb) x.z *= x.z;
       }
-    }
-    channels = base > channels ? base : channels;
-  }
-#pragma unroll
-  for (int d = WAVE / 2; d > 0; d >>= 1) {
-    most = fmax(most, __shfl_xor(most, d, WAVE));
-    most_a = fmax(most_a, __shfl_xor(most_a, d, WAVE));
-  }
-  if (lane == 0) { top[wave][0] = most; top[wave][1] = most_a; act[wave] = channels; }
-  if (wave == 0) {
-    int base = 0;
-    for (int a0 = 0; a0 < Aa; a0 += WAVE) {
-      const int a = a0 + lane;
-      const real c = weight(sg, a);
-      const bool on = c != real(0);
+      const bool on = x.z != real(0);
       const unsigned long long mask = __ballot(on);
       if (on) {
-        const int at = base + __popcll(mask & ((1ull << lane) - 1ull));
-        ch[at] = (unsigned short)a;
-        if (part == 0) {
-          real4 x;
-          x.x = alpha[3 * a]; x.y = alpha[3 * a + 1]; x.z = c; x.w = real(a);
-          par[at] = x;
-          beta[at] = alpha[3 * a + 2];
+        most_a = exp_larger(exp_larger(most_a, (float)x.x), (float)x.y);
+        most = exp_larger(most, (float)be);
+        if (s == sg) {
+          const int at = base + __popcll(mask & ((1ull << lane) - 1ull));
+          own[at] = x;
+          own_beta[at] = be;
         }
       }
       base += __popcll(mask);
     }
-    if (part == 0) {
-      real4 z;
-      z.x = z.y = z.z = z.w = 0;
-      for (int a = base + lane; a < pitch; a += WAVE) { par[a] = z; beta[a] = 0; }
-      if (lane == 0) P.table[8 + sg] = real(base);
-    }
-    if (lane == 0) active = base;
+    channels = base > channels ? base : channels;
+    if (s == sg && lane == 0) active = base;
   }
+#pragma unroll
+  for (int d = WAVE / 2; d > 0; d >>= 1) {
+    most = fmaxf(most, __shfl_xor(most, d, WAVE));
+    most_a = fmaxf(most_a, __shfl_xor(most_a, d, WAVE));
+  }
+  if (lane == 0) { top[wave][0] = most; top[wave][1] = most_a; act[wave] = channels; }
   __syncthreads();
   for (int w = 0; w < WAVES; w++) {
-    most = fmax(most, top[w][0]);
-    most_a = fmax(most_a, top[w][1]);
+    most = fmaxf(most, top[w][0]);
+    most_a = fmaxf(most_a, top[w][1]);
     channels = act[w] > channels ? act[w] : channels;
   }
-  const int N = DBL ? exp_rows(most) : 0, Np = DBL ? exp_rows(most_a) : 0;
-  if (part == 0 && sg == 0 && tid == 0) {
-    P.table[0] = real(N);
-    P.table[1] = real(channels);
-    P.table[2] = real(Np);
+  const StepTable L(nsig, step_pitch(channels), DBL ? exp_rows(most) : 0, DBL ? exp_rows(most_a) : 0);
+  if (part == 0) {
+    if (tid == 0) {
+      P.table[8 + sg] = real(active);
+      if (sg == 0) { P.table[0] = real(L.N); P.table[1] = real(channels); P.table[2] = real(L.Np); P.table[3] = real(L.pitch); }
+    }
+    real4* const par = (real4*)(P.table + L.par) + (size_t)sg * L.pitch;
+    real* const beta = P.table + L.beta + (size_t)sg * L.pitch;
+    for (int c = tid; c < L.pitch; c += STEP_TABLE_BLOCK) {
+      real4 x;
+      x.x = x.y = x.z = x.w = 0;
+      real be = 0;
+      if (c < active) { x = own[c]; be = own_beta[c]; }
+      par[c] = x;
+      beta[c] = be;
+    }
   }
   if constexpr (DBL) {
-    real* const rows = P.table + step_exp_at<real>(nsig, Aa) + (size_t)sg * (N + 1) * pitch;
-    for (int q = part * STEP_TABLE_BLOCK + tid; N && q < (N + 1) * pitch; q += parts * STEP_TABLE_BLOCK) {
-      const int i = q / pitch, c = q - i * pitch;
-      rows[q] = c < active ? exp_of(alpha[3 * ch[c] + 2], real(i) / N) : real(0);
-    }
-    real2* const pairs = (real2*)(P.table + step_pair_at<real>(nsig, Aa)) + (size_t)sg * (Np + 1) * pitch;
-    for (int q = part * STEP_TABLE_BLOCK + tid; Np && q < (Np + 1) * pitch; q += parts * STEP_TABLE_BLOCK) {
-      const int i = q / pitch, c = q - i * pitch;
-      real2 v;
-      v.x = c < active ? exp_of(alpha[3 * ch[c]], real(i) / Np) : real(0);
-      v.y = c < active ? exp_of(alpha[3 * ch[c] + 1], real(i) / Np) : real(0);
-      pairs[q] = v;
-    }
+    // sixteen values at a time: rows 0 .. N of beta, then those of alpha1 and alpha2 in turn (1/N and 1/N' are exact)
+    const int n = L.N ? L.N + 1 : 0, np = L.Np ? L.Np + 1 : 0;
+    const real inv = real(1) / L.N, inv_p = real(1) / L.Np;
+    real* const rows = P.table + L.rows + (size_t)sg * n * L.pitch;
+    real* const pairs = P.table + L.pairs + (size_t)sg * np * L.pitch * 2;
+    for (int q = part * (STEP_TABLE_BLOCK / 16) + tid / 16; q < n + 2 * np; q += parts * (STEP_TABLE_BLOCK / 16))
+      for (int c = tid & 15; c < L.pitch; c += 16) {
+        const int k = (q - n) & 1, i = q < n ? q : (q - n) >> 1;
+        real v = 0;
+        if (c < active) v = exp_of(q < n ? own_beta[c] : k ? own[c].y : own[c].x, real(i) * (q < n ? inv : inv_p));
+        (q < n ? rows + (size_t)i * L.pitch + c : pairs + ((size_t)i * L.pitch + c) * 2 + k)[0] = v;
+      }
   }
 }
 
@@ -374,7 +385,7 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
   constexpr bool DBL = sizeof(real) == 8;
   constexpr int THREADS = L::THREADS;
   extern __shared__ __align__(16) unsigned char smem[];
-  const int nr = A.nr, Aa = A.Aa, nt = A.nt, nsig = 2 * nt - 1, pitch = step_pitch(Aa);
+  const int nr = A.nr, Aa = A.Aa, nt = A.nt;
   const int EP = L::rows(nr, nt);                  // rows of a partner species' block of the table
   real2* E = (real2*)smem;                         // [partner species][grouped slot][channel]
   real2* slots = E + (size_t)nt * EP * TRI_CAP;    // [grouped slot] unit vector, cutoff value
@@ -386,10 +397,13 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
   const int ia = lane & (TRI_CAP - 1), r = lane / TRI_CAP;
   real* const my_out = outw + wave * Aa;
   const auto head = scalar_ptr(table);
-  const int exp_n = DBL ? (int)head[0] : 0, maxact = (int)head[1];
-  const real4* const parA = (const real4*)(table + STEP_HEAD);
-  const real* const beta = (const real*)(parA + (size_t)nsig * pitch);
-  const PairTable<real> pairs(table, (int)head[2], nsig, Aa);
+  auto size = [&](int i) { return uniform((int)head[i]); };   // (converted by a vector instruction)
+  const int maxact = size(1);
+  const StepTable TL(2 * nt - 1, size(3), DBL ? size(0) : 0, DBL ? size(2) : 0);
+  const int exp_n = TL.N, pitch = TL.pitch;
+  const real4* const parA = (const real4*)(table + TL.par);
+  const real* const beta = table + TL.beta;
+  const PairTable<real> pairs(table, TL);
   const real exp_nr = real(exp_n), exp_inv = real(1) / exp_nr;
   const int exp_row = pitch * (int)sizeof(real);
 
@@ -478,7 +492,7 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
           const real be = beta[at], bes = HE::scale(be);
           const real4 par = parA[at];
           const unsigned char* const exp_base =
-              (const unsigned char*)(table + step_exp_at<real>(nsig, Aa) + c0) + (size_t)sg * (exp_n + 1) * exp_row;
+              (const unsigned char*)(table + TL.rows + c0) + (size_t)sg * (exp_n + 1) * exp_row;
           const unsigned exp_lane = (unsigned)ia * sizeof(real);
           real acc = 0;
           for (; blk < blocks; blk += WAVES) {
