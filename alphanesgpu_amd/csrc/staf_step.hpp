@@ -34,7 +34,7 @@ namespace staf {
 // The last part: e^(beta T) = g + g p(beta (T - i/N)) with g from the row nearest to T.  What the reduction of HotExp does per
 // triplet and channel -- the integer part, the remainder, the power of two -- is done once per triplet, with exact results: i
 // and T - i/N.  N is the smallest power of two with |beta| / (2 N) <= 2^-7 for every channel (trained values are between -10 and
-// 4; beyond EXP_ROWS / 64 = 16, and where a beta is not a number, N is 0 and HotExp is used); there p, of degree 5 through 0 with
+// 4; beyond EXP_ROWS / 64 = 16, and where a beta is not a number, N is 0 and HotExp::product is used); there p, of degree 5 through 0 with
 // slope 1 and the values of e^x at four Chebyshev points, is off by at most 4e-17.
 constexpr int EXP_ROWS = 1024, STEP_HEAD = 32;
 __host__ __device__ inline int step_pitch(int channels) { return channels > 16 ? (channels + 15) & ~15 : 16; }
@@ -123,7 +123,7 @@ __device__ inline double exp_near(double x, double g) {
   return fma(g, q * x, g);
 }
 
-// A slot's entry of the pair tables, (e^(alpha1 D), e^(alpha2 D)) of one channel, by the table's rows (n > 0) or HotExp.  D is a
+// A slot's entry of the pair tables, (e^(alpha1 D), e^(alpha2 D)) of one channel, by the table's rows (n > 0) or HotExp::product.  D is a
 // cutoff function's value, between 0 and 1.
 template <typename real>
 struct PairTable {
@@ -147,15 +147,11 @@ struct PairTable {
         const auto g = ((const typename Vec2<real>::type*)rows)[(unsigned)(sg * (n + 1) + row) * (unsigned)pitch + channel];
         v.x = exp_near(a1 * rest, g.x);
         v.y = exp_near(a2 * rest, g.y);
-      } else {
-        auto eval = [&](real a) { const real x = a * D, e = HE::eval(x); return r_fma(e, r_fma(a, D, -x), e); };
-        v.x = eval(a1);
-        v.y = eval(a2);
+        return v;
       }
-    } else {
-      v.x = HE::eval(HE::scale(a1) * D);
-      v.y = HE::eval(HE::scale(a2) * D);
     }
+    v.x = HE::product(a1, D);
+    v.y = HE::product(a2, D);
     return v;
   }
 };
@@ -489,7 +485,7 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
           turn = (turn + blocks) & (WAVES - 1);
           if (blk >= blocks) continue;
           const int at = sg * pitch + c0 + ia;
-          const real be = beta[at], bes = HE::scale(be);
+          const real be = beta[at];
           const real4 par = parA[at];
           const unsigned char* const exp_base =
               (const unsigned char*)(table + TL.rows + c0) + (size_t)sg * (exp_n + 1) * exp_row;
@@ -538,7 +534,7 @@ __device__ __forceinline__ void rows_body(const TriArgs<real>& A, const real* __
                 for (int u = 0; u < 4; u++) {
                   real e;
                   if constexpr (NEAR) e = exp_near(be * rb[u], g[u]);
-                  else e = HE::eval(bes * Tb[u]);
+                  else e = HE::product(be, Tb[u]);
                   const real w = Tb[u] * e;
                   F2 = r_fma(w, e2[u].y, F2);
                   F1 = r_fma(w, e2[u].x, F1);

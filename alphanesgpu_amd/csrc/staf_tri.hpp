@@ -145,6 +145,7 @@ template <> struct HotExp<float> {
   __device__ static Factor factor(float a) { return {scale(a)}; }
   template <bool ONCE>
   __device__ static float eval(Factor f, float y, const float*) { return __builtin_amdgcn_exp2f(f.a * y); }
+  __device__ static float product(float a, float y) { return eval(scale(a) * y); }
 };
 // 2^(i/128), i = 0..127, correctly rounded
 static __device__ const double exp2_frac_128[128] = {
@@ -250,6 +251,12 @@ template <> struct HotExp<double> {
     q = fma(q, r, c(1.466226238763974e-05));
     q = fma(q, r, c(0.0054152123481238145));
     return ldexp(fma(g, q * r, g), i >> 7);
+  }
+  // e^(a y) without a table, for exponents beyond the rows of the fingerprints' tables: the rounding of the product is made good
+  // (an overflow stays inf)
+  __device__ static double product(double a, double y) {
+    const double x = a * y, e = eval(x);
+    return e <= 1.7976931348623157e308 ? fma(e, fma(a, y, -x), e) : e;
   }
   __device__ static double unscale() { return 1.0; }
   __device__ static void fill(double* tab, int tid, int nthreads) {
