@@ -252,6 +252,7 @@ static bool load_species_params(StafModel* m) {
     }
     if (staf::rows_fits<double>(m->nr, m->na, nt, m->Ar[k], m->Aa[k])) {
       const std::vector<double> t = staf::step_table_host(a3.data(), e3.data(), nt, m->Aa[k]);
+      if (t[0] == 0) continue;   // (exponents beyond its rows: the staged form is faster)
       if (!m->table[k].reserve(t.size()) || !upload_sync(m->table[k].p, t.data(), t.size() * sizeof(double), m->stream)) return false;
     }
   }

@@ -586,6 +586,7 @@ template <typename real>
 struct StepTablePart {
   const real *alpha3b, *emb3b;
   real* table;
+  size_t reals;      // what it may take up
   int Aa, raw_emb;   // emb3b is to be squared
 };
 // 2-body and 3-body fingerprints

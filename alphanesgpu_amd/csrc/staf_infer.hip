@@ -137,7 +137,8 @@ static int frames(const real* pos, const real* box, int nf, int N, int nt, const
             at(P.emb3b[k]), at(P.af2[k]), at(P.af3[k]), at(P.g2[k]), at(P.g3[k]), nullptr};
     if (P.rows) {
       S[n].table = at(P.table[k]);
-      tables[n_tables++] = {S[n].alpha3b, (const real*)s.type_emb3b, at(P.table[k]), s.nsmooth_a, 1};
+      tables[n_tables++] = {S[n].alpha3b, (const real*)s.type_emb3b, at(P.table[k]),
+                            step_table_reals<real>(nt, s.nsmooth_a), s.nsmooth_a, 1};
     }
     calls[n] = {&nets[n], S[n].af2, S[n].af3, at(P.e_atom) + (size_t)nf * first, S[n].g2, S[n].g3, S[n].Ar, S[n].Aa,
                 nf * s.n_local};

@@ -34,9 +34,12 @@ namespace staf {
 // The last part: e^(beta T) = g + g p(beta (T - i/N)) with g from the row nearest to T.  What the reduction of HotExp does per
 // triplet and channel -- the integer part, the remainder, the power of two -- is done once per triplet, with exact results: i
 // and T - i/N.  N is the smallest power of two with |beta| / (2 N) <= 2^-7 for every channel (trained values are between -10 and
-// 4; beyond EXP_ROWS / 64 = 16, and where a beta is not a number, N is 0 and HotExp::product is used); there p, of degree 5 through 0 with
-// slope 1 and the values of e^x at four Chebyshev points, is off by at most 4e-17.
-constexpr int EXP_ROWS = 1024, STEP_HEAD = 32;
+// 4; beyond EXP_ROWS / 64 = 64, and where a beta is not a number, N is 0 and HotExp::product is used); there p, of degree 5 through 0 with
+// slope 1 and the values of e^x at four Chebyshev points, is off by at most 4e-17.  N' likewise, up to PAIR_ROWS / 64 = 16: a slot's
+// entries are few beside the triplets.  Launch of 5832 centres of two species with a beta of -20 and -60: 82.7 us in the staged form, 90.1
+// without rows, 78.0 and 78.4 with them.  A loaded model whose N is 0 takes the staged form; the batch inference, whose host does not
+// know, does not: 46.5 -> 59.4 us for 4 x 729 centres.
+constexpr int EXP_ROWS = 4096, PAIR_ROWS = 1024, STEP_HEAD = 32;
 __host__ __device__ inline int step_pitch(int channels) { return channels > 16 ? (channels + 15) & ~15 : 16; }
 // where the parts lie, in reals
 struct StepTable {
@@ -51,15 +54,16 @@ struct StepTable {
     end = pairs + (Np ? lines * (Np + 1) * 2 : 0);
   }
 };
-// the largest a table of these sizes can be, whatever its parameters
+// What is kept for a table whose parameters are a caller's tensors, which the host does not read: the most rows of beta and 128 of the
+// alphas with every channel in use, or what takes no more.  A table that does not fit is laid out without the rows of the alphas.
 template <typename real>
 inline size_t step_table_reals(int nt, int Aa) {
-  const int most = sizeof(real) == 8 ? EXP_ROWS : 0;
-  return StepTable(2 * nt - 1, step_pitch(Aa), most, most).end;
+  constexpr bool rows = sizeof(real) == 8;
+  return StepTable(2 * nt - 1, step_pitch(Aa), rows ? EXP_ROWS : 0, rows ? 128 : 0).end;
 }
-// rows of a table for exponents up to `largest` (which is rounded: 2^-24 of it do not count)
-__host__ __device__ inline int exp_rows(float largest) {
-  int N = largest <= EXP_ROWS / 64 ? 1 : 0;
+// rows of a table for exponents up to `largest` (which is rounded: 2^-24 of it do not count), 0 where they would be more than `rows`
+__host__ __device__ inline int exp_rows(float largest, int rows) {
+  int N = largest <= (float)(rows / 64) ? 1 : 0;
   while (N && (float)N < 64 * largest) N *= 2;
   return N;
 }
@@ -88,7 +92,7 @@ inline std::vector<double> step_table_host(const double* alpha3b, const double* 
     }
     active = ch[s].size() > active ? ch[s].size() : active;
   }
-  const StepTable L(nsig, step_pitch((int)active), exp_rows(most), exp_rows(most_a));
+  const StepTable L(nsig, step_pitch((int)active), exp_rows(most, EXP_ROWS), exp_rows(most_a, PAIR_ROWS));
   std::vector<double> t(L.end, 0.0);
   t[0] = L.N; t[1] = (double)active; t[2] = L.Np; t[3] = L.pitch;
   for (int s = 0; s < nsig; s++) {
@@ -260,7 +264,9 @@ __device__ inline void step_table_body(const StepTablePart<real>& P, int nt, int
     most_a = fmaxf(most_a, top[w][1]);
     channels = act[w] > channels ? act[w] : channels;
   }
-  const StepTable L(nsig, step_pitch(channels), DBL ? exp_rows(most) : 0, DBL ? exp_rows(most_a) : 0);
+  const int N = DBL ? exp_rows(most, EXP_ROWS) : 0, Np = DBL ? exp_rows(most_a, PAIR_ROWS) : 0;
+  StepTable L(nsig, step_pitch(channels), N, Np);
+  if (L.end > P.reals) L = StepTable(nsig, L.pitch, N, 0);
   if (part == 0) {
     if (tid == 0) {
       P.table[8 + sg] = real(active);

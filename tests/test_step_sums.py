@@ -51,8 +51,8 @@ def test_sums_of_a_step(tmp_path, edge, spacing, nr, species, channels, beta):
 @pytest.mark.parametrize("edge,spacing,nr,frames", [(5, 3.6, 24, 1), (6, 2.6, 60, 2), (7, 2.1, 65, 1), (9, 1.9, 64, 1), (7, 1.9, 64, 4),
                                                     (11, 2.6, 60, 2)])
 @pytest.mark.parametrize("species,channels,exponents", [(1, (15,), (1.0, 0.5, 1.0)), (2, (3, 17, 40), (12.0, -12.0, -7.0)),
-                                                        (2, (14, 13, 13), (-20.0, 4.0, 16.0)), (3, (4, 3, 5, 3, 4, 3), (16.0, 20.0, 30.0)),
-                                                        (4, (4,) * 10, (2.0, -5.0, -10.0))])
+                                                        (2, (14, 13, 13), (-20.0, 4.0, 64.0)), (2, (20, 19, 1), (4.0, 1.0, -70.0)), (3, (4, 3, 5, 3, 4, 3), (16.0, 20.0, 30.0)),
+                                                        (4, (4,) * 10, (2.0, -5.0, -40.0))])
 def test_sums_of_a_batch(tmp_path, edge, spacing, nr, frames, species, channels, exponents):
     """float64 against the layers' ops and against the MD entry, whose table is the host's: other summation orders, 1e-11.  float32
     against the float64 layers: an exponential of exponent a D carries a times the rounding of D (the sum of the three here, 6e-8
