@@ -71,9 +71,14 @@ static int frames_plan(const DescConfig<real>& c, int nf, int N, int nt, const S
   P->numtriplet = place(rows * sizeof(int));
   RowsLaunch<real> form;
   for (int k = 0; k < nt; k++) form.add(c.nr, c.na, nt, sp[k].nalpha_r, sp[k].nsmooth_a, (long long)nf * sp[k].n_local);
-  // (one species in double precision: its launches of few centres, 125, 343 and 512, take 17.4, 22.4 and 25.0 us in the staged form and 18.0,
-  // 21.8 and 25.1 by rows, whose table costs the parameters' launch 0.6 to 1.2)
-  P->rows = form.waves() > 0 && (sizeof(real) == 4 || nt > 1 || form.centres > 512);
+  // Up to 512 centres of one or two species in double precision the tables cost the parameters' launch what the fingerprints gain by
+  // them, or more: both launches, in the staged form and by rows, exponents up to 2 and trained ones (up to 10), us:
+  //                            centres  125                  343                  512
+  //   one species                       24.3 / 26.4          29.2 / 28.6          32.4 / 33.4
+  //   two, channels in blocks           19.8 / 20.0, 21.8    22.2 / 21.4, 23.0    25.3 / 23.9
+  //   two, all channels in all classes  31.0 / 31.6, 36.7    36.3 / 35.3, 39.3    39.6 / 42.0
+  //   three, in blocks                  25.2 / 23.7, 25.6    28.1 / 25.0, 27.4
+  P->rows = form.waves() > 0 && (sizeof(real) == 4 || nt > 2 || form.centres > 512);
   long long sum = 0;
   for (int k = 0; k < nt; k++) {
     const StafFramesSpecies& s = sp[k];
