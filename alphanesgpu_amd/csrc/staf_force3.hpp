@@ -72,7 +72,7 @@ struct Force3Cfg {
   static constexpr bool PREFETCH = false;
   // waves per SIMD the register allocation is held to: with four waves per workgroup what the LDS footprint of the
   // reference's sizes admits (six workgroups per CU in single precision, four in double); with eight waves three
-  // workgroups per CU, so that launches of up to 768 of the centres that take them (FORCE3_WIDE_CENTRES) have all of them resident: 768 atoms
+  // workgroups per CU, so that launches of up to 768 of the centres that take them (step_forces) have all of them resident: 768 atoms
   // in double precision 33.8 us at 87 registers and two workgroups, 28.0 at 80
   static constexpr int MIN_WAVES = NW == 8 ? 6 : (sizeof(real) == 8 ? 4 : 6);
   __host__ __device__ static bool fits(int nr, int nt) { return nr <= 255 && nt <= NT_MAX; }   // slots packed in 8 bits

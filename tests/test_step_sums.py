@@ -17,10 +17,10 @@ def _crowd(edge, spacing, species, seed):
 
 # Neighbours inside the angular cutoff: about 6, 18, 32 and 56 of at most `nr`.  A sweep of the force kernel takes 1024
 # triplets (46 neighbours have 1035), the fingerprints' rows go four by four and their columns sixteen by sixteen.  125 to 1331
-# centres: eight waves each up to 448 for the fingerprints and 1280 for the forces.  Four species with 40 channels: 40 to 84
+# centres: eight waves each up to 448 for the fingerprints and 1280 (65 slots: 768) for the forces.  Four species with 40 channels: 40 to 84
 # KB of LDS with eight waves, at 64 slots one workgroup per CU, which is enough for 216 centres and not for 343.
 @pytest.mark.gpu
-@pytest.mark.parametrize("edge,spacing,nr", [(5, 3.6, 24), (6, 2.6, 60), (6, 2.1, 64), (9, 2.1, 65), (7, 1.9, 64), (10, 1.9, 64),
+@pytest.mark.parametrize("edge,spacing,nr", [(5, 3.6, 24), (6, 2.6, 60), (6, 2.1, 64), (9, 2.1, 65), (10, 2.1, 65), (7, 1.9, 64), (10, 1.9, 64),
                                              (11, 2.6, 60)])
 @pytest.mark.parametrize("species,channels,beta", [(1, (15,), 1.0), (2, (3, 17, 40), 1.0), (2, (14, 13, 13), -12.0),
                                                    (3, (4, 3, 5, 3, 4, 3), 30.0), (4, (4,) * 10, 1.0)])
