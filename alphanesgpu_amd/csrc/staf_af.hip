@@ -353,7 +353,9 @@ struct StepFingerprintArgs {
 };
 
 template <typename real, int BLOCK, bool ROWS>
-__global__ __launch_bounds__(BLOCK, (ROWS ? RowsCfg<real, BLOCK / WAVE>::MIN_WAVES : TriCfg<real, 0, true, BLOCK>::MIN_WAVES)) void step_fingerprints_kernel(
+constexpr int STEP_MIN_WAVES = ROWS ? RowsCfg<real, BLOCK / WAVE>::MIN_WAVES : TriCfg<real, 0, true, BLOCK>::MIN_WAVES;
+template <typename real, int BLOCK, bool ROWS>
+__global__ __launch_bounds__(BLOCK, (STEP_MIN_WAVES<real, BLOCK, ROWS>)) void step_fingerprints_kernel(
     const StepFingerprintArgs<real> M) {
   constexpr int WAVES = BLOCK / WAVE;
   const int wg = (int)blockIdx.x;
@@ -453,7 +455,8 @@ int step_fingerprints(const StepSpecies<real>* sp, int n, const StepRows<real>& 
     case 4: return step_fingerprints_launch<real, TRI_BLOCK, true>(sp, n, R, type_map, nt, stream);
     default: break;
   }
-  if (total <= WIDE_FINGERPRINT_CENTRES && lds <= 64 * 1024) return step_fingerprints_launch<real, 512, false>(sp, n, R, type_map, nt, stream);
+  if (total <= WIDE_FINGERPRINT_CENTRES && lds <= 64 * 1024)
+    return step_fingerprints_launch<real, 512, false>(sp, n, R, type_map, nt, stream);
   return step_fingerprints_launch<real, TRI_BLOCK, false>(sp, n, R, type_map, nt, stream);
 }
 template int step_fingerprints<float>(const StepSpecies<float>*, int, const StepRows<float>&, const int*, int, hipStream_t);

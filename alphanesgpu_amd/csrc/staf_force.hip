@@ -855,7 +855,8 @@ int step_forces(const StepSpecies<real>* sp, int n, const StepRows<real>& R, con
   // launches of 864, 972, 1200, 1500 and 2160 centres by four and by eight waves 32.5 / 31.6, 32.0 / 30.9, 37.5 / 35.6, 41.3 / 41.3 and
   // 55.6 / 56.3 us, in single precision 864 and 1152 20.0 / 18.4 and 21.0 / 19.9.
   // Without the sums in the slots' lanes (more than 64 slots) a second round loses, most in single precision: 1000 and 1280 centres of two
-  // species with 65 slots 18.1 / 21.1 and 19.9 / 23.7 us, of one 25.1 / 27.8 and 27.8 / 31.1; in double precision 28.1 / 29.7 and 37.1 / 34.8.
+  // species with 65 slots 18.1 / 21.1 and 19.9 / 23.7 us, of one 25.1 / 27.8 and 27.8 / 31.1; in double precision, two species,
+  // 28.1 / 29.7 and 37.1 / 34.8.
   const int wide_centres = pull ? 1280 : 768;   // five per CU, three
   KernelTimer kt_("force3_kernel", stream);
   auto launch = [&](auto pull_c) -> int {

@@ -45,8 +45,8 @@
 
 namespace staf {
 
-// NW_: waves per workgroup, 4 or 8 (step_forces takes 8 for few centres; for the others see force_tripl).  A sweep takes 16 passes of 64 triplets
-// either way; with eight waves a wave holds two of them, so that a centre's critical path and a wave's registers
+// NW_: waves per workgroup, 4 or 8 (step_forces takes 8 for few centres; for the others see force_tripl).  A sweep takes 16
+// passes of 64 triplets either way; with eight waves a wave holds two of them, so that a centre's critical path and a wave's registers
 // are about half of what they are with four.
 template <typename real, int NW_ = 4>
 struct Force3Cfg {
@@ -72,8 +72,10 @@ struct Force3Cfg {
   static constexpr bool PREFETCH = false;
   // waves per SIMD the register allocation is held to: with four waves per workgroup what the LDS footprint of the
   // reference's sizes admits (six workgroups per CU in single precision, four in double); with eight waves three
-  // workgroups per CU, so that launches of up to 768 of the centres that take them (step_forces) have all of them resident: 768 atoms
-  // in double precision 33.8 us at 87 registers and two workgroups, 28.0 at 80
+  // workgroups per CU, so that launches of up to 768 of the centres that take them (step_forces) have all of them resident.
+  // PULL in double precision would take 87 registers, and has two workgroups then; of its 80 two lie in scratch (12 bytes per
+  // lane).  Launches of 125, 512, 729, 1000 and 1210 centres of two species by 87 and by 80: 12.9 / 12.8, 17.5 / 17.5, 23.0 / 20.7,
+  // 27.2 / 25.3 and 32.4 / 28.8 us.
   static constexpr int MIN_WAVES = NW == 8 ? 6 : (sizeof(real) == 8 ? 4 : 6);
   __host__ __device__ static bool fits(int nr, int nt) { return nr <= 255 && nt <= NT_MAX; }   // slots packed in 8 bits
   __host__ __device__ static int pitch(int Aa) { return (Aa + 3) & ~3; }   // parameter row pitch (channels)
@@ -95,7 +97,7 @@ struct Force3Cfg {
     return (size_t)nsig * rowp(Aa) * 4 /*prm*/ + (size_t)nsig * pitch(Aa) * 2 /*prE*/ +
            table_reals(nr, nt, pull) /*E, then the triplets*/ +
            (pull ? 0 : (size_t)NW * 4 * nr) /*slot sums per wave*/ + (pull ? 4 * WAVE : nr) /*D, pull: the slots*/ +
-           3 * nr /*grad fc*/ + (size_t)NW * 4 /*the waves' shares of the centre's own force*/ +
+           3 * nr /*grad fc*/ + (pull ? 0 : (size_t)NW * 4) /*the waves' shares of the centre's own force*/ +
            (pull ? nr : fused ? 4 * nr : 0) /*unit vectors, 1/r, pull: 1/r*/ +
            (Ar2 > 0 ? (size_t)NW * nr + nr + (size_t)2 * nt * Ar2 : 0) /*2-body: the waves' shares of the pair
            weights, D, parameter rows*/ +
@@ -173,7 +175,7 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
   real2* slots = (real2*)sD;                               // PULL: [2][WAVE] (u_x, u_y) and (u_z, D) of the slots
   real* sg = sD + (PULL ? 4 * WAVE : nr);                  // [3*nr] grad fc (der3bsupp)
   real* xch = sg + 3 * nr;                                 // [NW][4] the waves' shares of the centre's own force
-  real* sU = xch + NW * 4;                                 // FUSED: [4][nr] unit vector, 1/r
+  real* sU = xch + (PULL ? 0 : NW * 4);                    // FUSED: [4][nr] unit vector, 1/r
   real* rinv = sU + (PULL ? 0 : 3 * nr);                   // FUSED: [nr] 1/r
   real* w2p = sU + (PULL ? nr : FUSED ? 4 * nr : 0);       // W2B: [NW][nr] the waves' shares of the 2-body pair weights
   real* sD2 = w2p + (W2B ? NW * nr : 0);                   // W2B: [nr] raddescr of the slots
@@ -708,10 +710,10 @@ __device__ __forceinline__ void force3_body(const Force3Args<real>& A, const int
         for (int c = 0; c < 3; c++) t4[c] = r_fma(-along, u[c], t4[c]);
       } else {
 #pragma unroll
-      for (int w = 0; w < NW; w++) {
-        const real4 a = acc_get(acc + (size_t)w * 4 * nr, tid);
-        t4[0] += a.x; t4[1] += a.y; t4[2] += a.z; t4[3] += a.w;
-      }
+        for (int w = 0; w < NW; w++) {
+          const real4 a = acc_get(acc + (size_t)w * 4 * nr, tid);
+          t4[0] += a.x; t4[1] += a.y; t4[2] += a.z; t4[3] += a.w;
+        }
       }
 #pragma unroll
       for (int c = 0; c < 3; c++) {

@@ -348,8 +348,8 @@ inline bool rows_fits(int nr, int na, int nt, int Ar, int Aa) {
 //   single, five, 60 slots, 3 per CU:           31.2 / 23.9                                          274.5 / 235.3
 // So rows_body takes launches whose centres are all resident, and others where a CU holds FULL workgroups: four in double precision, what
 // its registers admit, three in single.  (With a weight of every channel in every class, which training does not make of blocks -- a
-// weight of 0 has no gradient --, the last three rows are 36.5 / 31.4 and 49.3 / 39.5 for 729, but 83.3 / 89.7, 111.6 / 112.4 and 146.0 / 168.7
-// for 2916 and 257.9 / 278.2, 349.1 / 390.9 and 648.9 / 626.5 for 11664.)
+// weight of 0 has no gradient --, the last three rows are 36.5 / 31.4 and 49.3 / 39.5 for 729, but 83.3 / 89.7, 111.6 / 112.4 and
+// 146.0 / 168.7 for 2916 and 257.9 / 278.2, 349.1 / 390.9 and 648.9 / 626.5 for 11664.)
 // Eight waves per centre up to 448 centres: two species, 60 slots, four and eight waves 13.5 and 10.7 us for 96 centres, 13.9 and 10.8
 // for 225, 15.6 and 13.4 for 378, 16.1 and 16.8 for 504, 17.1 and 19.0 for 576, 18.5 and 21.6 for 768.
 constexpr int ROWS_CUS = 256, WIDE_ROWS_CENTRES = 448;

@@ -76,8 +76,8 @@ def test_a_launch_whose_tables_leave_few_waves_takes_the_staged_form(rule, f64, 
     assert rule(f64, nr, nt, 20, 40, centres)[0] == waves
 
 
-@pytest.mark.parametrize("active,largest,rows", [((14, 13, 13), 2.0, (128, 64)), ((3, 17, 0), 16.0, (1024, 1024)), ((1, 0, 5), 16.5, (2048, 0)),
-                                                 ((20, 1, 5), 64.0, (4096, 0)), ((1, 0, 5), 64.5, (0, 0)),
+@pytest.mark.parametrize("active,largest,rows", [((14, 13, 13), 2.0, (128, 64)), ((3, 17, 0), 16.0, (1024, 1024)),
+                                                 ((1, 0, 5), 16.5, (2048, 0)), ((20, 1, 5), 64.0, (4096, 0)), ((1, 0, 5), 64.5, (0, 0)),
                                                  ((40, 40, 40), 0.01, (1, 1)), ((0, 0, 0), 2.0, (1, 1))])
 def test_a_table_is_as_wide_as_the_channels_in_use(rule, active, largest, rows):
     """Two species, forty channels of which a class has `active`: the pitch is the largest number in whole sixteens, the rows those

@@ -20,8 +20,8 @@ def _crowd(edge, spacing, species, seed):
 # centres: eight waves each up to 448 for the fingerprints and 1280 (65 slots: 768) for the forces.  Four species with 40 channels: 40 to 84
 # KB of LDS with eight waves, at 64 slots one workgroup per CU, which is enough for 216 centres and not for 343.
 @pytest.mark.gpu
-@pytest.mark.parametrize("edge,spacing,nr", [(5, 3.6, 24), (6, 2.6, 60), (6, 2.1, 64), (9, 2.1, 65), (10, 2.1, 65), (7, 1.9, 64), (10, 1.9, 64),
-                                             (11, 2.6, 60)])
+@pytest.mark.parametrize("edge,spacing,nr", [(5, 3.6, 24), (6, 2.6, 60), (6, 2.1, 64), (9, 2.1, 65), (10, 2.1, 65), (7, 1.9, 64),
+                                             (10, 1.9, 64), (11, 2.6, 60)])
 @pytest.mark.parametrize("species,channels,beta", [(1, (15,), 1.0), (2, (3, 17, 40), 1.0), (2, (14, 13, 13), -12.0),
                                                    (3, (4, 3, 5, 3, 4, 3), 30.0), (4, (4,) * 10, 1.0)])
 def test_sums_of_a_step(tmp_path, edge, spacing, nr, species, channels, beta):
@@ -51,7 +51,8 @@ def test_sums_of_a_step(tmp_path, edge, spacing, nr, species, channels, beta):
 @pytest.mark.parametrize("edge,spacing,nr,frames", [(5, 3.6, 24, 1), (6, 2.6, 60, 2), (7, 2.1, 65, 1), (9, 1.9, 64, 1), (7, 1.9, 64, 4),
                                                     (11, 2.6, 60, 2)])
 @pytest.mark.parametrize("species,channels,exponents", [(1, (15,), (1.0, 0.5, 1.0)), (2, (3, 17, 40), (12.0, -12.0, -7.0)),
-                                                        (2, (14, 13, 13), (-20.0, 4.0, 64.0)), (2, (20, 19, 1), (4.0, 1.0, -70.0)), (3, (4, 3, 5, 3, 4, 3), (16.0, 20.0, 30.0)),
+                                                        (2, (14, 13, 13), (-20.0, 4.0, 64.0)), (2, (20, 19, 1), (4.0, 1.0, -70.0)),
+                                                        (3, (4, 3, 5, 3, 4, 3), (16.0, 20.0, 30.0)),
                                                         (4, (4,) * 10, (2.0, -5.0, -40.0))])
 def test_sums_of_a_batch(tmp_path, edge, spacing, nr, frames, species, channels, exponents):
     """float64 against the layers' ops and against the MD entry, whose table is the host's: other summation orders, 1e-11.  float32
