@@ -593,9 +593,9 @@ __host__ __device__ inline size_t pack_elements(const PackPart& p) {
 }
 // A thread per element of the destination: the order of upload_net's tiles.  Bound by its launch and the first read of the
 // parameters: the two networks of a 60-140-140-1 stack in double precision are 0.9 MB, and the two tables of exponentials beside
-// them 0.3 MB for exponents up to 2 and 14 channels in use of 40.  Trace of an inference of 4 x 768 atoms 5.1 us, of one of 96 5.6
-// (with tables as wide as all 40 channels, maxima in double precision and divisions per entry 10.1 and 6.8; the networks alone 6.6
-// and 4.8).  Trained exponents, up to 10: 1025 and 513 rows, 1.2 MB, 8.5 us between events (11.7; the networks alone 6.8).
+// them 0.3 MB for exponents up to 2 and 14 channels in use of 40, 1.2 MB for trained ones (up to 10: 1025 and 513 rows).  Between
+// events, four frames of 729 atoms: the networks alone 6.9 us, with the tables 7.6 and 8.5 (as wide as all 40 channels, with maxima in
+// double precision and divisions per entry, 8.8 and 11.7).
 template <typename T>
 __global__ __launch_bounds__(PACK_BLOCK) void mlp_pack_kernel(const PackArgs<T> A) {
   if ((int)blockIdx.x < A.first[0]) {
