@@ -1,6 +1,6 @@
 // 3-body fingerprints of the paths that hold no tensor of the angular buffer's width (the MD entry, the batch inference), from
 // the nr-wide rows of the radial-only descriptor launch, for up to 64 neighbours and angular buffers that hold all their
-// pairs (step_slots); other buffers go through tri_reduce_body.
+// pairs (step_slots), in launches that it leaves enough waves (RowsLaunch); the others go through tri_reduce_body.
 //
 // tri_reduce_body, which also rebuilds T where no angular tensor exists, stages the triplets of a class in LDS and reads a
 // record and two table rows per (triplet, channel): its inner loop is as long as its LDS reads take, whatever it computes (the
@@ -14,9 +14,9 @@
 //   * one table entry per item is read from LDS, the same address for the four rows;
 //   * all classes' tables are built at once, the rows of all classes are dealt to the waves: three barriers per centre.
 // Launches of 24576, 4 x 768 (inference), 768 and 96 centres: 366 -> 335, 56.6 -> 52, 24.9 -> 19 and 12.5 -> 11.0 us in double
-// precision (157 -> 137 M vector instructions, 28 -> 13 M LDS instructions for 24576), 4 x 768 in single 31.8 -> 25.3; a vector
-// instruction in 0.71 of the busy cycles, the rest is latency at four waves per SIMD (127 registers; five would need 96, and
-// less than the 38 KB of LDS that 60 slots take).
+// precision (157 -> 137 M vector instructions, 28 -> 13 M LDS instructions for 24576), 4 x 768 in single 31.8 -> 25.3; the vector
+// instructions of 24576 centres fill 0.66 of the issue slots, the rest is latency at four waves per SIMD (127 registers; five would
+// need 96, and less than the 38 KB of LDS that 60 slots of two species take).
 #pragma once
 #include <vector>
 
